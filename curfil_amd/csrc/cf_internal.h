@@ -136,6 +136,26 @@ struct FeatGenJob {
     int pad;
 };
 
+// A feature generation job's place in its candidates and its stream of sample-index draws (absolute draw
+// numbers; draw i lies in slot i mod the ring's size).
+struct WalkState {
+    int head, tail;             // next draw of the walk, draws produced
+    int recorded, steps;        // draws produced before the last production, and the steps of that
+    int k, generated;           // next candidate, features generated
+    int t, tries;               // thresholds found and tries left of a candidate that ran past its band
+    int drawsDone, candsDone;   // draws used by the candidates that have ended
+    int openDraws;              // draws used so far by the candidate that ran past its band
+    int err, done;
+    float guess;                // expected draws of a candidate before any has ended
+};
+
+// the sample behind a draw: depthReciprocal of its depth, x | y << 16, its image (-1: no valid depth)
+struct DrawRec {
+    double rinv;
+    int xy;
+    int image;
+};
+
 // Per-(tree, level) feature tables on the device, slot = tree * F + f.
 struct FeatTables {
     DevBuf<FeatRec> feat;      // sorted features [trees*F]
@@ -150,6 +170,9 @@ struct FeatTables {
     DevBuf<float> unsortedThr;
     DevBuf<int> unsortedKey;
     DevBuf<int> err;
+    // the walk over the draws (k_features.hip)
+    DevBuf<uint8_t> walkSpace;
+    float meanDraws = 0;       // draws per candidate in the last generation (0: none yet)
     int trees = 0, F = 0, T = 0;
 };
 

@@ -8,20 +8,31 @@
 // RandomSource(seed) hands seed to the sample-index sampler and seeds
 // seed+1+4k .. seed+4+4k to candidate k's four samplers (type, offset,
 // region, channel).  Candidates are therefore independent and are drawn in
-// parallel (k_fg_candidates).  Thresholds consume one shared draw stream in
-// order, and how many draws a candidate consumes depends on which responses
-// are NaN; k_fg_walk keeps that order exactly: one workgroup per (tree, level)
-// owns the sample-index generator (MT19937 state twisted in parallel in LDS),
-// evaluates the next 16 candidates, each in a band of 128 of the next 512
-// queued draws, in parallel, and lets one wave walk them with the reference's
-// retry rules.
+// parallel (k_fg_candidates), and so is the stream of sample-index draws
+// (k_fg_draws, k_fg_records).  Thresholds consume that one stream in order, and
+// how many draws a candidate consumes depends on which responses are NaN, so a
+// candidate's first draw is known only after its predecessor's last.  That
+// chain is taken in rounds of two launches:
+//   k_fg_round    a workgroup per candidate evaluates it on a band of draws
+//                 around its expected first draw and, from the finite bits,
+//                 tabulates for every start in the band where the candidate
+//                 would end and whether it would be accepted;
+//   k_fg_advance  a workgroup per tree follows the chain through the tables
+//                 (one LDS read per candidate) and writes the accepted
+//                 candidates' thresholds.
+// The bands only decide how far a round gets, never which draws a candidate
+// uses.  Per level of 5 trees with F = 4000, T = 32 on 50 frames of 640x480 the
+// walk takes 1.7 ms (about 40 rounds of 112 candidates: 15 us + 18 us each);
+// one workgroup per tree that evaluated 16 candidates a round on its own CU
+// took 15.2 ms, bound by that CU's gathers.
+#include <algorithm>
+
 #include "cf_internal.h"
 #include "cf_rng.h"
 
 namespace cf {
 
 constexpr int kPrefixDraws = 24;   // engine outputs available to one feature sampler
-constexpr int kDrawQueue = 2048;   // ring of pending sample-index draws
 
 // g++ on x86-64 evaluates the two getNext() calls of `Offset(rgen.getNext(),
 // rgen.getNext())` right to left, so the second coordinate is drawn first
@@ -100,345 +111,465 @@ __device__ __forceinline__ int featureSortKey(const FeatRec& f) {
     return k;
 }
 
-constexpr int kWalkCand = 16;   // candidates evaluated per round
-constexpr int kWalkDraws = 512; // queued draws a round can reach
-constexpr int kWalkBand = 128;  // draws evaluated per candidate per round
-constexpr int kWalkWords = kWalkDraws / 64;
-static_assert(kDrawQueue >= kWalkDraws + 624, "the draw ring holds a round's window and one refill");
+// A candidate uses at least this many draws: T thresholds, or the 10 NaN responses that reject it.
+__host__ __device__ __forceinline__ int minDraws(int T) { return T < 10 ? T : 10; }
 
-// What the walk did with candidate j of a round: window positions
-// [begin, end) were consumed with st = 0 (still open at its band's end),
-// 1 (accepted into output slot `slot`) or 2 (rejected, or not reached); t0
-// thresholds had been found before the round.
+// The next words of each job's index generator: as many as the features still missing are expected to
+// take, tempered, and per wave the mask of those that uniform_int accepts.  MT19937 as the recurrence
+// x[n + 624] = mix(x[n], x[n + 1], x[n + 397]), 227 words a step (no word of a step depends on another) in
+// an LDS ring with one barrier a step.  One workgroup per job: bound by the latency of a step.  uniform_int
+// accepts a word w iff w / bucket <= range, that is iff w < bucket (range + 1).
+constexpr int kMtStep = 227;
+constexpr int kMtRing = 2048;
+__global__ void __launch_bounds__(256) k_fg_draws(const FeatGenJob* __restrict__ jobs, int F, int T, int ring,
+        int fresh, float guess, WalkState* __restrict__ states, uint32_t* __restrict__ mtState, uint32_t* __restrict__ raw,
+        unsigned long long* __restrict__ masks, int maxSteps) {
+    __shared__ uint32_t x[kMtRing];
+    __shared__ int counts[4];
+    const FeatGenJob job = jobs[blockIdx.x];
+    WalkState st = states[blockIdx.x];
+    if (fresh) {
+        st = WalkState{};
+        st.tries = 10;
+        st.guess = guess;
+    }
+    if (st.done) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const UniformIntParams up = uniformIntParams(0, job.n - 1);
+    uint32_t* saved = mtState + static_cast<size_t>(blockIdx.x) * 624;
+    if (!fresh) {
+        for (int i = tid; i < 624; i += 256) x[i] = saved[i];
+    } else if (tid == 0) {
+        uint32_t v = static_cast<uint32_t>(job.seed);
+        x[0] = v;
+        for (uint32_t i = 1; i < 624; i++) {
+            v = mtInitStep(v, i);
+            x[i] = v;
+        }
+    }
+    __syncthreads();
+    // draws per feature so far, with the rejected candidates' share
+    const double perFeature = st.generated > 0 ? static_cast<double>(st.drawsDone) / st.generated : st.guess;
+    const double want = (F - st.generated) * perFeature * 1.06 + 2048.0;
+    const int target = st.head + static_cast<int>(fmin(want, static_cast<double>(ring - 512)));
+    const int missing = max(0, target - st.tail);
+    int steps = 0, made = missing;   // a range of one value takes no words
+    if (up.range != 0) {
+        const unsigned long long limit = static_cast<unsigned long long>(up.bucket) * (up.range + 1ull);
+        const double share = limit >= (1ull << 32) ? 1.0 : static_cast<double>(limit) / 4294967296.0;
+        // at least half of the words are accepted, so the ring (at most ring - 512 ahead of the walk before
+        // this, and no more than `missing` words over that) never overruns
+        steps = min(maxSteps, min(static_cast<int>(missing / share), ring - 512 - (st.tail - st.head)) / kMtStep + (missing > 0 ? 1 : 0));
+        uint32_t* out = raw + static_cast<size_t>(blockIdx.x) * maxSteps * 256;
+        unsigned long long* mk = masks + static_cast<size_t>(blockIdx.x) * maxSteps * 4;
+        int base = 0;
+        made = 0;
+        for (int s = 0; s < steps; s++) {
+            bool acc = false;
+            if (tid < kMtStep) {
+                const int i = base + tid;
+                const uint32_t w = mtMix(x[i & (kMtRing - 1)], x[(i + 1) & (kMtRing - 1)], x[(i + 397) & (kMtRing - 1)]);
+                x[(i + 624) & (kMtRing - 1)] = w;
+                const uint32_t v = mtTemper(w);
+                acc = v < limit;
+                out[s * 256 + tid] = v;
+            }
+            const unsigned long long mask = __ballot(acc);
+            if (lane == 0) mk[s * 4 + wave] = mask;
+            made += __popcll(mask);
+            base += kMtStep;
+            __syncthreads();
+        }
+        if (lane == 0) counts[wave] = made;
+        __syncthreads();
+        made = counts[0] + counts[1] + counts[2] + counts[3];
+        for (int i = tid; i < 624; i += 256) saved[i] = x[(base + i) & (kMtRing - 1)];
+    }
+    if (tid == 0) {
+        st.recorded = st.tail;
+        st.tail += made;
+        st.steps = steps;
+        states[blockIdx.x] = st;
+    }
+}
+
+// The sample records behind the draws produced last, in draw order in the job's ring, so that every
+// candidate whose band holds a draw reads its sample coalesced.  A workgroup takes a step's words; their
+// place among the accepted ones is the count of the mask bits before them.
+__global__ void __launch_bounds__(256) k_fg_records(const FeatGenJob* __restrict__ jobs,
+        const WalkState* __restrict__ states, int ring, const uint32_t* __restrict__ raw,
+        const unsigned long long* __restrict__ masks, int maxSteps, DrawRec* __restrict__ recs) {
+    __shared__ int part[4];
+    const WalkState st = states[blockIdx.y];
+    if (st.done) return;
+    const FeatGenJob job = jobs[blockIdx.y];
+    const UniformIntParams up = uniformIntParams(0, job.n - 1);
+    DrawRec* out = recs + static_cast<size_t>(blockIdx.y) * ring;
+    auto record = [&](int index, int at) {
+        const cf_sample s = job.samples[index];
+        DrawRec r;
+        const bool valid = s.depth_mm > 0;
+        r.rinv = valid ? depthReciprocal(depthToFloat(s.depth_mm)) : 0.0;
+        r.xy = s.x | (s.y << 16);
+        r.image = valid ? static_cast<int>(s.image) : -1;
+        out[at & (ring - 1)] = r;
+    };
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (up.range == 0) {
+        for (int i = st.recorded + blockIdx.x * 256 + tid; i < st.tail; i += gridDim.x * 256) record(up.lo, i);
+        return;
+    }
+    const uint32_t* words = raw + static_cast<size_t>(blockIdx.y) * maxSteps * 256;
+    const unsigned long long* mk = masks + static_cast<size_t>(blockIdx.y) * maxSteps * 4;
+    for (int s = blockIdx.x; s < st.steps; s += gridDim.x) {
+        int before = 0;
+        for (int i = tid; i < 4 * s; i += 256) before += __popcll(mk[i]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+        if (lane == 0) part[wave] = before;
+        __syncthreads();
+        int at = st.recorded + part[0] + part[1] + part[2] + part[3];
+        __syncthreads();
+        unsigned long long own = 0;
+        for (int w = 0; w <= wave; w++) {
+            own = mk[4 * s + w];
+            if (w < wave) at += __popcll(own);
+        }
+        if ((own >> lane) & 1ull) {
+            record(static_cast<int>(static_cast<uint32_t>(up.lo) + words[s * 256 + tid] / up.bucket),
+                    at + __popcll(own & ((1ull << lane) - 1ull)));
+        }
+    }
+}
+
+// position of the n-th set bit of w (n from 1, at most popcount(w))
+__device__ __forceinline__ int nthBit(unsigned long long w, int n) {
+    int pos = 0;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) {
+        const int c = __popcll(w & ((1ull << s) - 1ull));
+        if (n > c) {
+            n -= c;
+            w >>= s;
+            pos += s;
+        }
+    }
+    return pos;
+}
+
+constexpr int kBandMax = 2048;            // draws of the widest band
+constexpr int kRoundTable = 28672;        // table entries of a round (two bytes each, in the walker's LDS)
+constexpr int kRoundCandMax = 224;        // candidates of a round (kRoundTable / the narrowest band)
+constexpr int kAdvanceLanes = 1024;
+constexpr int kGroup = 8;                 // consecutive candidates that k_fg_advance composes
+constexpr uint16_t kOpen = 0x8000;        // the candidate does not end inside its band
+constexpr uint16_t kAccept = 0x4000;      // it ends with its T-th threshold (else rejected)
+
+// Band of a round for T thresholds: a power of two of at least 8 T draws.  A candidate uses about 1.25 T
+// draws with a spread of T / 8, so the start of the round's j-th candidate is known to about sqrt(j) T / 8;
+// with 28672 / band candidates a round that is covered to its end (measured on 640x480 frames: T = 32,
+// 112 candidates, starts within 80 draws of the mean in nine rounds of ten).
+static int bandDraws(int T) {
+    int b = 128;
+    while (b < 8 * T && b < kBandMax) b *= 2;
+    return b;
+}
+
+// One candidate of a round on its band (see the head of this file).  Bound by the latency of the corner
+// gathers, which the round's candidates x trees workgroups overlap on all CUs.
+__global__ void __launch_bounds__(256) k_fg_round(const WalkState* __restrict__ states, ImageSet imgs,
+        const FeatRec* __restrict__ cand, int numCand, int T, int ring, int band, const DrawRec* __restrict__ recs,
+        float* __restrict__ resp, uint16_t* __restrict__ next, int4* __restrict__ bands) {
+    constexpr int kWords = kBandMax / 64;
+    __shared__ unsigned long long finite[kWords], rejects[kWords];   // not NaN; tenth NaN of a run
+    const WalkState st = states[blockIdx.y];
+    const int j = blockIdx.x;
+    if (st.done || st.k + j >= numCand) return;
+    const size_t row = static_cast<size_t>(blockIdx.y) * gridDim.x + j;
+    // the band: around j times the draws that a candidate has used so far, wider the later the candidate
+    const float avg = (st.drawsDone + 16.0f * st.guess) / (st.candsDone + 16.0f);
+    const float dev = 8.0f + 0.19f * avg * sqrtf(static_cast<float>(j));
+    const int lo = j == 0 ? 0 : max(j * minDraws(T), static_cast<int>(j * avg - dev));
+    int width = j == 0 ? band : min(band, static_cast<int>(2.0f * dev + 1.25f * avg) + 8);
+    width = max(0, min(width, st.tail - st.head - lo));
+    const Feat f = loadFeat(cand + static_cast<size_t>(blockIdx.y) * numCand + st.k + j);
+    const DrawRec* rec = recs + static_cast<size_t>(blockIdx.y) * ring;
+    const size_t plane = static_cast<size_t>(imgs.W) * imgs.H;
+    for (int i = threadIdx.x; i < band; i += blockDim.x) {
+        float v = __builtin_nanf("");
+        if (i < width) {
+            const DrawRec r = rec[(st.head + lo + i) & (ring - 1)];
+            int idx[8];
+            if (r.image >= 0 && responseCorners(f, r.xy & 0xffff, static_cast<int>(static_cast<uint32_t>(r.xy) >> 16),
+                    imgs.W, imgs.H, r.rinv, false, idx)) {
+                if (f.type == T_DEPTH) {
+                    const int2* dep = imgs.dep + static_cast<size_t>(r.image) * plane;
+                    int2 cv[8];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) cv[e] = planeAt(dep, idx[e]);
+                    v = static_cast<float>(depthResponseFromCorners(cv));
+                } else {
+                    const float* col = imgs.col + static_cast<size_t>(r.image) * 3 * plane;
+                    const float* colA = col + static_cast<size_t>(f.c1) * plane;
+                    const float* colB = col + static_cast<size_t>(f.c2) * plane;
+                    float c8[8];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) c8[e] = planeAt(colA, idx[e]);
+#pragma unroll
+                    for (int e = 4; e < 8; e++) c8[e] = planeAt(colB, idx[e]);
+                    v = static_cast<float>(colorResponseFromCorners(c8));
+                }
+            }
+            resp[row * band + i] = v;
+        }
+        const unsigned long long fm = __ballot(i < width && !__builtin_isnan(v));
+        if ((i & 63) == 0) finite[i >> 6] = fm;
+    }
+    __syncthreads();
+    const int words = band / 64;
+    // NaN draws of word w inside the band
+    auto nanWord = [&](int w) -> unsigned long long {
+        if (w < 0 || width <= w * 64) return 0ull;
+        const int n = width - w * 64;
+        return ~finite[w] & (n >= 64 ? ~0ull : ((1ull << n) - 1ull));
+    };
+    if (static_cast<int>(threadIdx.x) < words) {
+        // runs of 10 on the pair (previous word, word): ends of runs of 2, 4, 8, then 8 + 2
+        unsigned long long hi = nanWord(threadIdx.x), lw = nanWord(static_cast<int>(threadIdx.x) - 1);
+        auto andShifted = [&](int s, unsigned long long h2, unsigned long long l2) {
+            hi &= (h2 << s) | (l2 >> (64 - s));
+            lw &= l2 << s;
+        };
+        andShifted(1, hi, lw);
+        const unsigned long long h2 = hi, l2 = lw;
+        andShifted(2, hi, lw);
+        andShifted(4, hi, lw);
+        andShifted(8, h2, l2);
+        rejects[threadIdx.x] = hi;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < width; i += blockDim.x) {
+        // the first of: the T-th finite draw from i on, the tenth NaN of a run that starts at i or later
+        int need = T, end = 0;
+        uint16_t how = kOpen;
+        if (j == 0 && i == 0) {
+            // thresholds found and tries left when the candidate ran past the last round's band
+            need = T - st.t;
+            const unsigned long long n0 = nanWord(0);
+            const int lead = ~n0 ? __builtin_ctzll(~n0) : 64;
+            if (lead >= st.tries) {
+                end = st.tries;
+                how = 0;
+            }
+        }
+        for (int w = i >> 6; how == kOpen && w < words; w++) {
+            unsigned long long fw = finite[w], rw = rejects[w];
+            const int from = i - w * 64, rejFrom = from + 9;
+            if (from > 0) fw &= ~0ull << from;
+            if (rejFrom >= 64) rw = 0ull;
+            else if (rejFrom > 0) rw &= ~0ull << rejFrom;
+            const int c = __popcll(fw);
+            const int a = c >= need ? nthBit(fw, need) : 64;
+            const int r = rw ? __builtin_ctzll(rw) : 64;
+            if (a < 64 || r < 64) {
+                how = a < r ? kAccept : 0;
+                end = w * 64 + min(a, r) + 1;
+            }
+            need -= c;
+        }
+        next[row * band + i] = static_cast<uint16_t>(how | end);
+    }
+    if (threadIdx.x == 0) {
+        // the band's finite draws and the NaN draws after the last of them, for a candidate that runs past it
+        int found = 0, last = -1;
+        if (j == 0) {
+            for (int w = 0; w < words; w++) {
+                found += __popcll(finite[w]);
+                if (finite[w]) last = w * 64 + 63 - __clzll(finite[w]);
+            }
+        }
+        bands[row] = make_int4(lo, width, found, width - 1 - last);
+    }
+}
+
+// What the walk did with candidate j of a round: it used the band's draws [begin, end) and ended with
+// st = 1 (accepted into output slot `slot`), 0 (still open at its band's end), or 2 (rejected, or not
+// reached).
 struct WalkStep {
     int st, begin, end, t0, slot;
 };
 
-struct WalkShared {
-    uint32_t mt[624];
-    int dq[kDrawQueue];
-    float resp[kWalkCand][kWalkDraws];
-    unsigned long long finite[kWalkCand][kWalkWords];   // bit: response is not NaN (set inside the band only)
-    FeatRec cand[kWalkCand];
-    WalkStep step[kWalkCand];
-    int waveCounts[4];
-    // walk state after a round: next draw, next candidate, features generated,
-    // thresholds found and tries left for a candidate that ran past the round;
-    // band spacing of the next round and the draws / candidates finished so far
-    int head, k, generated, t, tries, err;
-    int spacing, drawsDone, candsDone;
-};
-
-// One MT19937 twist of the LDS state, in three dependency-free phases.
-__device__ void mtTwistShared(uint32_t* mt) {
-    const int tid = threadIdx.x;
-    uint32_t v = 0;
-    if (tid < 227) v = mtMix(mt[tid], mt[tid + 1], mt[tid + 397]);
-    __syncthreads();
-    if (tid < 227) mt[tid] = v;
-    __syncthreads();
-    if (tid < 227) v = mtMix(mt[227 + tid], mt[228 + tid], mt[tid]);
-    __syncthreads();
-    if (tid < 227) mt[227 + tid] = v;
-    __syncthreads();
-    if (tid < 169) v = mtMix(mt[454 + tid], mt[455 + tid], mt[227 + tid]);
-    __syncthreads();
-    if (tid < 169) mt[454 + tid] = v;
-    __syncthreads();
-    if (tid == 0) mt[623] = mtMix(mt[623], mt[0], mt[396]);
-    __syncthreads();
-}
-
-// Appends the accepted uniform_int draws of one engine block to the queue.
-__device__ int refillDraws(WalkShared& sh, int tail, const UniformIntParams& up) {
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    if (up.range == 0) {
-        for (int i = tid; i < 624; i += 256) sh.dq[(tail + i) % kDrawQueue] = up.lo;
-        __syncthreads();
-        return tail + 624;
+// Follows the candidates of a round through their tables, from the state's next draw and candidate on.  The
+// round ends at the first candidate that starts outside its band or does not end inside it; the round's first
+// candidate, which starts at its band's first draw, then carries its thresholds and tries into the next.
+// Bound by the chain of dependent LDS reads, about 0.2 us each.  The chain is shortened by composing the
+// tables of kGroup consecutive candidates for every start of the first's band, all in parallel: the walk then
+// takes a read per group, and the groups it passed are expanded in parallel (F = 4000, T = 32: 18 us a launch,
+// 32 us with a read per candidate).
+__global__ void __launch_bounds__(kAdvanceLanes) k_fg_advance(const FeatGenJob* __restrict__ jobs,
+        WalkState* __restrict__ states, const FeatRec* __restrict__ cand, int numCand, int F, int T, int band, int m,
+        const float* __restrict__ resp, const uint16_t* __restrict__ next, const int4* __restrict__ bands,
+        FeatRec* __restrict__ outFeat, float* __restrict__ outThr, int* __restrict__ outKey) {
+    // uint16 [m][band], then per group of kGroup candidates uint32 [band]: the end of the group's last
+    // candidate (20 bits), its accepted candidates << 20, or kGroupStop if the walk ends inside the group
+    extern __shared__ uint4 tableWords[];
+    __shared__ int4 bd[kRoundCandMax];
+    __shared__ WalkStep steps[kRoundCandMax];
+    __shared__ int groupStart[kRoundCandMax / kGroup], groupGen[kRoundCandMax / kGroup];   // start -1: not passed whole
+    constexpr uint32_t kGroupStop = 0xffffffffu;
+    const WalkState st = states[blockIdx.x];
+    if (st.done) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const size_t row0 = static_cast<size_t>(blockIdx.x) * m;
+    const uint4* src = reinterpret_cast<const uint4*>(next + row0 * band);
+    const int words = m * band / 8, groups = m / kGroup;
+    for (int i = tid; i < words; i += kAdvanceLanes) tableWords[i] = src[i];
+    for (int i = tid; i < m; i += kAdvanceLanes) {
+        // rows of candidates past the last are never written: empty bands
+        bd[i] = st.k + i < numCand ? bands[row0 + i] : make_int4(0, 0, 0, 0);
+        steps[i].st = 2;
     }
-    mtTwistShared(sh.mt);
-    for (int r = 0; r < 3; r++) {
-        const int i = r * 256 + tid;
-        bool acc = false;
-        uint32_t v = 0;
-        if (i < 624) {
-            v = mtTemper(sh.mt[i]) / up.bucket;
-            acc = v <= up.range;
-        }
-        const unsigned long long mask = __ballot(acc);
-        const int lanePrefix = __popcll(mask & ((1ull << lane) - 1ull));
-        if (lane == 0) sh.waveCounts[wave] = __popcll(mask);
-        __syncthreads();
-        int wavePrefix = 0, total = 0;
-        for (int w = 0; w < 4; w++) {
-            if (w < wave) wavePrefix += sh.waveCounts[w];
-            total += sh.waveCounts[w];
-        }
-        if (acc) sh.dq[(tail + wavePrefix + lanePrefix) % kDrawQueue] = static_cast<int>(static_cast<uint32_t>(up.lo) + v);
-        tail += total;
-        __syncthreads();
-    }
-    return tail;
-}
-
-// Per round: candidate j of the next kWalkCand is evaluated at the draws
-// [j S, j S + kWalkBand) of the next kWalkDraws queued draws (S: about 7/8 of
-// the draws a finished candidate has used, at least min(T, 10), the fewest a
-// candidate can use), 2 candidates x 2 draws per lane and wave; then wave 0
-// walks the candidates in order with the reference's rules
-// (random_tree_image.cpp:648-700: a NaN response costs one of 10 tries, a
-// finite one is a threshold and resets the tries; T thresholds accept the
-// candidate, 10 NaN in a row reject it).  A candidate's first draw is the one
-// after its predecessor's last.  The round ends at the first candidate whose
-// first draw lies outside its band or which runs to its band's end; that
-// candidate carries its state into the next round, which starts with it.
-// The bands only decide how far a round gets, never which draws a candidate
-// uses.
-__global__ void __launch_bounds__(256) k_fg_walk(const FeatGenJob* __restrict__ jobs, ImageSet imgs,
-        const FeatRec* __restrict__ cand, int numCand, int F, int T, FeatRec* __restrict__ outFeat,
-        float* __restrict__ outThr, int* __restrict__ outKey, int* __restrict__ err) {
-    __shared__ WalkShared sh;
-    const FeatGenJob job = jobs[blockIdx.x];
-    const FeatRec* myCand = cand + static_cast<size_t>(blockIdx.x) * numCand;
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const UniformIntParams up = uniformIntParams(0, job.n - 1);
-    const int minUse = min(T, 10);
-    if (tid == 0) {
-        uint32_t v = static_cast<uint32_t>(job.seed);
-        sh.mt[0] = v;
-        for (uint32_t i = 1; i < 624; i++) {
-            v = mtInitStep(v, i);
-            sh.mt[i] = v;
-        }
-        sh.head = 0;
-        sh.k = 0;
-        sh.generated = 0;
-        sh.t = 0;
-        sh.tries = 10;
-        sh.err = 0;
-        sh.spacing = minUse;
-        sh.drawsDone = 0;
-        sh.candsDone = 0;
-    }
+    for (int i = tid; i < groups; i += kAdvanceLanes) groupStart[i] = -1;
     __syncthreads();
-    constexpr int kPerWave = kWalkCand / 4;          // candidates per wave: wave, wave + 4, ...
-    constexpr int kReps = kWalkBand / 64;            // draws per lane and candidate
-    constexpr int kSlots = kPerWave * kReps;
-    int tail = 0;
-    for (;;) {
-        const int head = sh.head, k0 = sh.k, S = sh.spacing;
-        const bool done = sh.generated >= F || sh.err != 0;
-        __syncthreads();
-        if (done) break;
-        while (tail - head < kWalkDraws) tail = refillDraws(sh, tail, up);
-        for (int i = tid; i < kWalkCand * kWalkWords; i += 256) (&sh.finite[0][0])[i] = 0ull;
-        if (tid < kWalkCand && k0 + tid < numCand) sh.cand[tid] = myCand[k0 + tid];
-        __syncthreads();
-        {
-            // two rounds of loads for all slots together: first every slot's sample record, then every
-            // slot's corner gathers (planes addressed from the image index, no descriptor load); a
-            // response is formed only after all of them are in flight
-            bool ok[kSlots], isDepth[kSlots], active[kSlots];
-            int2 cv[kSlots][8];   // depth corners, or colour corners' bits in .x
-            cf_sample smp[kSlots];
-#pragma unroll
-            for (int q = 0; q < kPerWave; q++) {
-                const int c = wave + 4 * q;
-                const bool candOk = k0 + c < numCand;
-#pragma unroll
-                for (int r = 0; r < kReps; r++) {
-                    const int i = q * kReps + r;
-                    const int dpos = c * S + 64 * r + lane;
-                    active[i] = candOk && dpos < kWalkDraws;
-                    // inactive slots read the level's first sample (in range) and issue no gathers
-                    const int d = active[i] ? sh.dq[(head + dpos) % kDrawQueue] : 0;
-                    smp[i] = job.samples[d];
-                }
+    const uint16_t* table = reinterpret_cast<const uint16_t*>(tableWords);
+    uint32_t* composed = reinterpret_cast<uint32_t*>(tableWords + words);
+    for (int i = tid; i < groups * band; i += kAdvanceLanes) {
+        const int g = i / band, j0 = g * kGroup;
+        uint32_t accepted = 0;
+        int p = bd[j0].x + (i - g * band);
+        bool whole = true;
+        for (int q = 0; whole && q < kGroup; q++) {
+            const int lo = bd[j0 + q].x, at = p - lo;
+            whole = at >= 0 && at < bd[j0 + q].y;
+            if (whole) {
+                const int e = table[(j0 + q) * band + at];
+                whole = (e & kOpen) == 0;
+                accepted += (e & kAccept) ? 1u : 0u;
+                p = lo + (e & (kAccept - 1));
             }
-            const size_t plane = static_cast<size_t>(imgs.W) * imgs.H;
-#pragma unroll
-            for (int q = 0; q < kPerWave; q++) {
-                const int c = wave + 4 * q;
-                const bool candOk = k0 + c < numCand;
-                Feat ff{};
-                if (candOk) ff = loadFeat(&sh.cand[c]);
-#pragma unroll
-                for (int r = 0; r < kReps; r++) {
-                    const int i = q * kReps + r;
-                    isDepth[i] = ff.type == T_DEPTH;
-                    const bool valid = smp[i].depth_mm > 0;
-                    const double rinv = valid ? depthReciprocal(depthToFloat(smp[i].depth_mm)) : 0.0;
-                    int idx[8];
-                    ok[i] = active[i] && valid && responseCorners(ff, smp[i].x, smp[i].y, imgs.W, imgs.H, rinv, false,
-                            idx);
-                    if (ok[i]) {
-                        if (isDepth[i]) {
-                            const int2* dep = imgs.dep + static_cast<size_t>(smp[i].image) * plane;
-#pragma unroll
-                            for (int e = 0; e < 8; e++) cv[i][e] = planeAt(dep, idx[e]);
-                        } else {
-                            const float* col = imgs.col + static_cast<size_t>(smp[i].image) * 3 * plane;
-                            const float* colA = col + static_cast<size_t>(ff.c1) * plane;
-                            const float* colB = col + static_cast<size_t>(ff.c2) * plane;
-#pragma unroll
-                            for (int e = 0; e < 4; e++) cv[i][e].x = __float_as_int(planeAt(colA, idx[e]));
-#pragma unroll
-                            for (int e = 4; e < 8; e++) cv[i][e].x = __float_as_int(planeAt(colB, idx[e]));
+        }
+        composed[i] = whole && p < (1 << 20) ? static_cast<uint32_t>(p) | (accepted << 20) : kGroupStop;
+    }
+    __syncthreads();
+    const int outOffset = jobs[blockIdx.x].outOffset;
+    if (tid < 64) {
+        // wave 0, all lanes in step: the walk's state is uniform
+        int p = 0, j = 0, gen = st.generated, err = 0;
+        bool open = false, stop = false;
+        while (j < m && !stop) {
+            // a whole group, unless the features or candidates may run out in it
+            const int g = j / kGroup;
+            if (j % kGroup == 0 && gen + kGroup < F && st.k + j + kGroup < 3 * F && g < groups) {
+                const int lo = __builtin_amdgcn_readfirstlane(bd[j].x), at = p - lo;
+                if (at >= 0 && at < __builtin_amdgcn_readfirstlane(bd[j].y)) {
+                    const uint32_t c = __builtin_amdgcn_readfirstlane(composed[g * band + at]);
+                    if (c != kGroupStop) {
+                        if (lane == 0) {
+                            groupStart[g] = p;
+                            groupGen[g] = gen;
                         }
+                        p = static_cast<int>(c & ((1u << 20) - 1u));
+                        gen += static_cast<int>(c >> 20);
+                        j += kGroup;
+                        continue;
                     }
                 }
             }
-#pragma unroll
-            for (int q = 0; q < kPerWave; q++) {
-                const int c = wave + 4 * q;
-#pragma unroll
-                for (int r = 0; r < kReps; r++) {
-                    const int i = q * kReps + r;
-                    const int start = c * S + 64 * r;   // draw of lane 0
-                    const int dpos = start + lane;
-                    float v = __builtin_nanf("");
-                    if (ok[i]) {
-                        if (isDepth[i]) {
-                            v = static_cast<float>(depthResponseFromCorners(cv[i]));
-                        } else {
-                            float c8[8];
-#pragma unroll
-                            for (int e = 0; e < 8; e++) c8[e] = __int_as_float(cv[i][e].x);
-                            v = static_cast<float>(colorResponseFromCorners(c8));
-                        }
-                    }
-                    if (active[i]) sh.resp[c][dpos] = v;
-                    // the wave's 64 draws start at `start`, which need not be word aligned
-                    const unsigned long long fm = __ballot(active[i] && !__builtin_isnan(v));
-                    if (lane == 0 && fm != 0ull) {
-                        const int w = start >> 6, off = start & 63;
-                        atomicOr(&sh.finite[c][w], fm << off);
-                        if (off != 0 && w + 1 < kWalkWords) atomicOr(&sh.finite[c][w + 1], fm >> (64 - off));
-                    }
+            // `--maxLoops <= 0` with maxLoops = 3F, checked right after sampling candidate k
+            if (gen >= F || st.k + j + 1 >= 3 * F) {
+                err = gen < F;
+                break;
+            }
+            const int lo = __builtin_amdgcn_readfirstlane(bd[j].x), width = __builtin_amdgcn_readfirstlane(bd[j].y);
+            const int at = p - lo;
+            if (at < 0 || at >= width) break;   // its first draw was not evaluated: the next round starts here
+            const int e = __builtin_amdgcn_readfirstlane(table[j * band + at]);
+            if (e & kOpen) {
+                open = j == 0;
+                if (open) {
+                    if (lane == 0) steps[0] = WalkStep{0, p, width, st.t, outOffset + gen};
+                    p = width;
                 }
+                break;
+            }
+            const int end = lo + (e & (kAccept - 1));
+            if (e & kAccept) {
+                if (lane == 0) steps[j] = WalkStep{1, p, end, j == 0 ? st.t : 0, outOffset + gen};
+                gen++;
+            }
+            p = end;
+            j++;
+        }
+        if (lane == 0) {
+            WalkState ns = st;
+            ns.head = st.head + p;
+            ns.k = st.k + j;
+            ns.generated = gen;
+            ns.err = err;
+            ns.done = gen >= F || err != 0;
+            if (open) {   // its draws count once it has ended
+                ns.openDraws = st.openDraws + p;
+                ns.t = st.t + bd[0].z;
+                ns.tries = bd[0].z > 0 ? 10 - bd[0].w : st.tries - bd[0].w;
+            } else if (j > 0) {
+                ns.drawsDone = st.drawsDone + st.openDraws + p;
+                ns.candsDone = st.candsDone + j;
+                ns.openDraws = 0;
+                ns.t = 0;
+                ns.tries = 10;
+            }
+            states[blockIdx.x] = ns;
+        }
+    }
+    __syncthreads();
+    if (tid < groups && groupStart[tid] >= 0) {
+        int p = groupStart[tid], slot = outOffset + groupGen[tid];
+        for (int j = tid * kGroup; j < tid * kGroup + kGroup; j++) {
+            const int lo = bd[j].x;
+            const int e = table[j * band + (p - lo)];
+            const int end = lo + (e & (kAccept - 1));
+            if (e & kAccept) steps[j] = WalkStep{1, p, end, j == 0 ? st.t : 0, slot++};
+            p = end;
+        }
+    }
+    __syncthreads();
+    for (int j = tid; j < m; j += kAdvanceLanes) {
+        if (steps[j].st != 1) continue;
+        const FeatRec fr = cand[static_cast<size_t>(blockIdx.x) * numCand + st.k + j];
+        outFeat[steps[j].slot] = fr;
+        outKey[steps[j].slot] = featureSortKey(fr);
+    }
+    // thresholds of the accepted and the still open candidates: their finite draws in order, a wave per
+    // candidate, the first 64 draws of kAhead candidates loaded together
+    constexpr int kWaves = kAdvanceLanes / 64, kAhead = 7;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    for (int ja = tid >> 6; ja < m; ja += kWaves * kAhead) {
+        float v[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            const int j = ja + u * kWaves;
+            v[u] = __builtin_nanf("");
+            if (j < m && steps[j].st != 2) {
+                const int i = steps[j].begin + lane;
+                if (i < steps[j].end) v[u] = resp[(row0 + j) * band + (i - bd[j].x)];
             }
         }
-        __syncthreads();
-        if (tid < 64) {
-            // wave 0 walks the finite-response bits a 64-draw word at a time: lane q
-            // stands for draw q of the word and tests whether the walk stops there
-            // (the T-th threshold, or the NaN that uses up the tries: a NaN run
-            // costs one try per draw, a finite response is the next threshold and
-            // resets the tries to 10); the first such lane ends the candidate
-            const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));   // bits [0, lane)
-            int p = 0;
-            int k = k0;
-            int gen = __builtin_amdgcn_readfirstlane(sh.generated);
-            int t = __builtin_amdgcn_readfirstlane(sh.t);
-            int tries = __builtin_amdgcn_readfirstlane(sh.tries);
-            if (tid < kWalkCand) sh.step[tid].st = 2;   // not walked: nothing to copy
-            while (k < k0 + kWalkCand && gen < F) {
-                const int j = k - k0;
-                const int lo = j * S, hi = min(lo + kWalkBand, kWalkDraws);
-                if (p < lo || p >= hi) break;   // its first draw was not evaluated: the next round starts here
-                // `--maxLoops <= 0` with maxLoops = 3F, checked right after sampling candidate k
-                if (k + 1 >= 3 * F) {
-                    if (tid == 0) {
-                        sh.err = 1;
-                        atomicExch(err, 1);
-                    }
-                    break;
-                }
-                const int begin = p, t0 = t, slot = job.outOffset + gen;
-                int st = 0;
-                while (st == 0 && p < hi) {
-                    const int w = p >> 6, o = p & 63;
-                    const int e = min(64, hi - (w << 6));   // lanes [o, e) lie in the band
-                    const unsigned long long word = sh.finite[j][w];
-                    const uint32_t lo32 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word));
-                    const uint32_t hi32 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word >> 32));
-                    const unsigned long long inBand = (~0ull << o) & (e == 64 ? ~0ull : ((1ull << e) - 1ull));
-                    const unsigned long long m = ((static_cast<unsigned long long>(hi32) << 32) | lo32) & inBand;
-                    // finite draws in [p, q) and the NaN run that ends at q: it starts after the last of
-                    // them and is held to 10 tries, or, with none, starts at p with the tries carried in
-                    const unsigned long long prevF = m & below;
-                    const bool fin = (m >> lane) & 1ull;
-                    const int run = prevF ? lane - (63 - __clzll(prevF)) : lane - o + 1;
-                    const bool accept = fin && t + __popcll(prevF) + 1 == T;
-                    const bool reject = lane >= o && lane < e && !fin && run == (prevF ? 10 : tries);
-                    const unsigned long long stop = __ballot(accept || reject);
-                    if (stop) {
-                        const int q = __builtin_ctzll(stop);
-                        st = ((m >> q) & 1ull) ? 1 : 2;
-                        p = (w << 6) + q + 1;
-                    } else {
-                        // no stop before e: its thresholds count, and the NaN draws after the last
-                        // finite one (fewer than the tries left) carry on
-                        t += __popcll(m);
-                        tries = m ? 10 - (e - 1 - (63 - __clzll(m))) : tries - (e - o);
-                        p = (w << 6) + e;
-                    }
-                }
-                if (tid == 0) {
-                    WalkStep ws;
-                    ws.st = st;
-                    ws.begin = begin;
-                    ws.end = p;
-                    ws.t0 = t0;
-                    ws.slot = slot;
-                    sh.step[j] = ws;
-                    if (st == 1) {
-                        const FeatRec fr = sh.cand[j];
-                        outFeat[slot] = fr;
-                        outKey[slot] = featureSortKey(fr);
-                    }
-                }
-                if (st == 0) break;   // the band ran out inside candidate k
-                if (st == 1) gen++;
-                k++;
-                t = 0;
-                tries = 10;
-            }
-            if (tid == 0) {
-                sh.head = head + p;
-                sh.k = k;
-                sh.generated = gen;
-                sh.t = t;
-                sh.tries = tries;
-                // draws and candidates finished this round (an open candidate's draws count with it later)
-                int used = p;
-                if (k < k0 + kWalkCand) {
-                    const WalkStep& open = sh.step[k - k0];
-                    if (open.st == 0) used = open.begin;
-                }
-                const int drawsDone = sh.drawsDone + used, candsDone = sh.candsDone + (k - k0);
-                sh.drawsDone = drawsDone;
-                sh.candsDone = candsDone;
-                sh.spacing = candsDone > 0 ? max(minUse, (7 * drawsDone) / (8 * candsDone)) : minUse;
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            const int j = ja + u * kWaves;
+            if (j >= m || steps[j].st == 2) continue;
+            const WalkStep ws = steps[j];
+            float* to = outThr + static_cast<size_t>(ws.slot) * T + ws.t0;
+            float cur = v[u];
+            for (int i0 = ws.begin;;) {
+                const unsigned long long fm = __ballot(!__builtin_isnan(cur));
+                if (!__builtin_isnan(cur)) to[__popcll(fm & below)] = cur;
+                to += __popcll(fm);
+                i0 += 64;
+                if (i0 >= ws.end) break;
+                cur = i0 + lane < ws.end ? resp[(row0 + j) * band + (i0 + lane - bd[j].x)] : __builtin_nanf("");
             }
         }
-        __syncthreads();
-        // thresholds of the accepted and still open candidates: the finite
-        // draws of [begin, end) in order, after the t0 found earlier
-#pragma unroll
-        for (int q = 0; q < kPerWave; q++) {
-            const int c = wave + 4 * q;
-            const WalkStep ws = sh.step[c];
-            if (ws.st == 2) continue;
-#pragma unroll
-            for (int r = 0; r < kReps; r++) {
-                const int dpos = c * S + 64 * r + lane;
-                if (dpos < ws.begin || dpos >= ws.end) continue;
-                if (!((sh.finite[c][dpos >> 6] >> (dpos & 63)) & 1ull)) continue;
-                int before = 0;   // finite draws in [begin, dpos)
-                for (int w = ws.begin >> 6; w <= (dpos >> 6); w++) {
-                    unsigned long long m = sh.finite[c][w];
-                    if (w == (ws.begin >> 6)) m &= ~0ull << (ws.begin & 63);
-                    if (w == (dpos >> 6)) m &= (1ull << (dpos & 63)) - 1ull;
-                    before += __popcll(m);
-                }
-                outThr[static_cast<size_t>(ws.slot) * T + ws.t0 + before] = sh.resp[c][dpos];
-            }
-        }
-        __syncthreads();
     }
 }
 
@@ -539,21 +670,86 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     tabs.order.resize(static_cast<size_t>(numJobs) * F * T);
     tabs.err.resize(1);
     CF_HIP(hipMemsetAsync(tabs.err.get(), 0, sizeof(int), s));
-    DevBuf<int> seeds(numJobs);
-    CF_HIP(hipMemcpyAsync(seeds.get(), seedsHost, numJobs * sizeof(int), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_fg_candidates, dim3((numCand + 255) / 256, numJobs), dim3(256), 0, s, seeds.get(), numCand,
+    const int band = bandDraws(T);
+    const int m = std::min(kRoundTable / band, kRoundCandMax);   // candidates of a round
+    int ring = 1 << 14;
+    while (ring < (1 << 19) && ring < 2.0 * F * T) ring *= 2;
+    const int maxSteps = ring / kMtStep + 1;
+    // the walk's buffers in one allocation (hipMalloc and hipFree cost a small training more than the walk)
+    const size_t n = static_cast<size_t>(numJobs), perRound = n * m * band;
+    size_t bytes = 0;
+    auto part = [&](size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 255) & ~static_cast<size_t>(255);
+        return at;
+    };
+    const size_t oSeeds = part(n * sizeof(int)), oWalk = part(n * sizeof(WalkState)), oMt = part(n * 624 * sizeof(uint32_t)),
+            oRaw = part(n * maxSteps * 256 * sizeof(uint32_t)), oMasks = part(n * maxSteps * 4 * sizeof(uint64_t)),
+            oRecs = part(n * ring * sizeof(DrawRec)), oResp = part(perRound * sizeof(float)),
+            oNext = part(perRound * sizeof(uint16_t)), oBands = part(n * m * sizeof(int4));
+    tabs.walkSpace.resize(bytes);
+    uint8_t* space = tabs.walkSpace.get();
+    int* dSeeds = reinterpret_cast<int*>(space + oSeeds);
+    WalkState* dWalk = reinterpret_cast<WalkState*>(space + oWalk);
+    uint32_t* dMt = reinterpret_cast<uint32_t*>(space + oMt);
+    uint32_t* dRaw = reinterpret_cast<uint32_t*>(space + oRaw);
+    unsigned long long* dMasks = reinterpret_cast<unsigned long long*>(space + oMasks);
+    DrawRec* dRecs = reinterpret_cast<DrawRec*>(space + oRecs);
+    float* dResp = reinterpret_cast<float*>(space + oResp);
+    uint16_t* dNext = reinterpret_cast<uint16_t*>(space + oNext);
+    int4* dBands = reinterpret_cast<int4*>(space + oBands);
+    CF_HIP(hipMemcpyAsync(dSeeds, seedsHost, numJobs * sizeof(int), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_fg_candidates, dim3((numCand + 255) / 256, numJobs), dim3(256), 0, s, dSeeds, numCand,
             boxRadius, regionSize, useDepth, tabs.cand.get(), tabs.err.get());
-    hipLaunchKernelGGL(k_fg_walk, dim3(numJobs), dim3(256), 0, s, jobsDev, imgs, tabs.cand.get(), numCand, F, T,
-            tabs.unsortedFeat.get(), tabs.unsortedThr.get(), tabs.unsortedKey.get(), tabs.err.get());
-    hipLaunchKernelGGL(k_fg_sort, dim3((F + 255) / 256, numJobs), dim3(256), F * sizeof(int), s, tabs.unsortedKey.get(),
-            tabs.unsortedFeat.get(), tabs.unsortedThr.get(), F, T, tabs.feat.get(), tabs.thrFT.get(),
-            tabs.thrTF.get(), tabs.soa.get());
     const int total = numJobs * F;
-    hipLaunchKernelGGL(k_threshold_ranks, dim3((total + 255) / 256), dim3(256), 0, s, tabs.thrFT.get(), total, T,
-            tabs.rank.get(), tabs.order.get());
+    std::vector<WalkState> states(numJobs);
     int errHost = 0;
-    CF_HIP(hipMemcpyAsync(&errHost, tabs.err.get(), sizeof(int), hipMemcpyDeviceToHost, s));
-    CF_HIP(hipStreamSynchronize(s));
+    // draws of a candidate: the mean of these tables' last generation (the level before), or 5/4 T
+    const float guess = tabs.meanDraws > 0 ? tabs.meanDraws : 1.25f * T;
+    // The rounds the missing features are expected to take are enqueued together with the sort that
+    // follows (rounds after a job's last feature return at once); in the rare case that a job needs
+    // more, they and the sort are enqueued again.
+    for (bool fresh = true, more = true; more; fresh = false) {
+        int missing = 0;
+        for (const WalkState& st : states) missing = std::max(missing, st.done ? 0 : F - st.generated);
+        // (without a table before this one to go by, the first rounds are short: a candidate's mean use is
+        // only guessed)
+        const int rounds = std::min(64, missing / std::max(1, m * 9 / 10) + (fresh && tabs.meanDraws > 0 ? 2 : 4));
+        hipLaunchKernelGGL(k_fg_draws, dim3(numJobs), dim3(256), 0, s, jobsDev, F, T, ring, fresh ? 1 : 0, guess,
+                dWalk, dMt, dRaw, dMasks, maxSteps);
+        const int steps = static_cast<int>(std::min<double>(maxSteps, 1.4 * missing * T / kMtStep + 12));
+        hipLaunchKernelGGL(k_fg_records, dim3(steps, numJobs), dim3(256), 0, s, jobsDev, dWalk, ring, dRaw,
+                dMasks, maxSteps, dRecs);
+        const size_t lds = static_cast<size_t>(m) * band * 2 + static_cast<size_t>(m / kGroup) * band * 4;
+        allowLds(reinterpret_cast<const void*>(&k_fg_advance), lds);
+        for (int r = 0; r < rounds; r++) {
+            hipLaunchKernelGGL(k_fg_round, dim3(m, numJobs), dim3(std::min(band, 256)), 0, s, dWalk, imgs,
+                    tabs.cand.get(), numCand, T, ring, band, dRecs, dResp, dNext, dBands);
+            hipLaunchKernelGGL(k_fg_advance, dim3(numJobs), dim3(kAdvanceLanes), lds, s, jobsDev, dWalk,
+                    tabs.cand.get(), numCand, F, T, band, m, dResp, dNext, dBands, tabs.unsortedFeat.get(),
+                    tabs.unsortedThr.get(), tabs.unsortedKey.get());
+        }
+        hipLaunchKernelGGL(k_fg_sort, dim3((F + 255) / 256, numJobs), dim3(256), F * sizeof(int), s,
+                tabs.unsortedKey.get(), tabs.unsortedFeat.get(), tabs.unsortedThr.get(), F, T, tabs.feat.get(),
+                tabs.thrFT.get(), tabs.thrTF.get(), tabs.soa.get());
+        hipLaunchKernelGGL(k_threshold_ranks, dim3((total + 255) / 256), dim3(256), 0, s, tabs.thrFT.get(), total, T,
+                tabs.rank.get(), tabs.order.get());
+        CF_HIP(hipMemcpyAsync(states.data(), dWalk, numJobs * sizeof(WalkState), hipMemcpyDeviceToHost, s));
+        CF_HIP(hipMemcpyAsync(&errHost, tabs.err.get(), sizeof(int), hipMemcpyDeviceToHost, s));
+        CF_HIP(hipStreamSynchronize(s));
+        more = false;
+        for (const WalkState& st : states) {
+            if (st.err != 0 && errHost == 0) errHost = st.err;
+            more = more || !st.done;
+        }
+        if (errHost != 0) break;
+    }
+    double draws = 0, cands = 0;
+    for (const WalkState& st : states) {
+        draws += st.drawsDone;
+        cands += st.candsDone;
+    }
+    tabs.meanDraws = cands > 0 ? static_cast<float>(draws / cands) : 0.0f;
     if (errHost == 1) throw Error(CF_ERR_RUNTIME, "failed to generate random features. max loops exceeded");
     if (errHost == 2) throw Error(CF_ERR_RUNTIME, "feature sampler needed more engine outputs than provisioned");
 }

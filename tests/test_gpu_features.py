@@ -1,0 +1,46 @@
+"""GPU feature generation against the oracle at the edges of the walk over the sample-index draws."""
+import numpy as np
+import pytest
+
+import curfil_amd as cf
+import oracle as orc
+from helpers import config0_dataset, random_samples
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def frames(ctx):
+    rgb, depth, labels = config0_dataset()
+    im = cf.Images(ctx, 4, 160, 120)
+    for i in range(4):
+        im.set_rgbd_u8(i, rgb[i], depth[i])
+    return depth, labels, im, orc.Dataset.from_u8(rgb, depth, labels)
+
+
+# T around the band widths (128 draws up to T = 16, then 256 ... 2048) and the 10 tries; with boxRadius 127 most
+# responses of 160x120 frames are NaN, so candidates are rejected and (T = 255) run past the widest band;
+# 8192 x 64 thresholds need more draws than the ring holds; one sample makes every draw the same
+@pytest.mark.parametrize("n,F,T,br,rs", [(700, 40, 1, 60, 10), (700, 90, 9, 127, 20), (700, 90, 10, 60, 10),
+                                         (1500, 400, 16, 60, 10), (1500, 400, 17, 127, 10), (900, 1, 33, 60, 10),
+                                         (2000, 113, 32, 60, 10), (2000, 60, 65, 127, 20), (2000, 30, 129, 60, 10),
+                                         (2000, 16, 255, 127, 20), (3000, 8192, 64, 30, 10), (1, 50, 20, 10, 5)])
+@pytest.mark.parametrize("missing", [False, True])
+def test_feature_walk_edges_match_oracle(ctx, frames, n, F, T, br, rs, missing):
+    depth, labels, im, ds = frames
+    rng = np.random.default_rng(1000 * F + T)
+    s = random_samples(rng, 4 * n, 4, 160, 120, depth.astype(np.int32), labels=labels)
+    s = s[s["depth_mm"] > 0][:n]
+    if missing and n > 1:
+        s["depth_mm"][rng.random(n) < 0.3] = -1   # samples without valid depth: NaN for every feature
+    try:
+        want = ds.generate_features(s, F + T, F, T, br, rs)
+    except Exception:
+        want = None   # more than 3 F candidates
+    if want is None:
+        with pytest.raises(cf.CurfilError):
+            cf.generate_features(ctx, im, s, F + T, F, T, br, rs)
+        return
+    feats, thr = cf.generate_features(ctx, im, s, F + T, F, T, br, rs)
+    assert np.array_equal(feats, want[0])
+    assert np.array_equal(thr.view(np.uint32), want[1].view(np.uint32))
