@@ -243,14 +243,13 @@ void launchFillU32(hipStream_t s, uint32_t* p, size_t n, uint32_t v);
 size_t levelSortScanBlocks(int numSegs, int yBits);
 void levelCountingSort(hipStream_t s, const uint32_t* keys, const uint32_t* vals, int n, int numSegs, int yBits,
         uint32_t* count, uint32_t* cursor, uint32_t* blockSum, uint32_t* out, int* starts);
-// Work list of pass 1 for ngb feature groups, built on the device: segment i (its blocks
-// segFirst[i] .. + segCount[i]) belongs to XCD i % 8; XCD x takes its segments in order, all groups
-// of a segment (group major, block minor) before the next, and workgroup w of the launch runs on
-// XCD w % 8, so work[pos * 8 + x] is XCD x's item pos, (-1, 0) past its end.  xcdPrefix[i] counts
-// the blocks of XCD x's segments before segment i; xcdBlocks[x] all of them; maxLen is the longest
-// XCD list in items.
-void launchBuildWork(hipStream_t s, const int* segFirst, const int* segCount, const int* xcdPrefix,
-        const int* xcdBlocks, int numSegs, int ngb, int maxLen, int2* work);
+// Work list of pass 1 for ngb feature groups, built on the device.  The items are ordered by image group
+// (segment i: its blocks segFirst[i] .. + segCount[i], segPrefix[i] blocks before them), feature group and
+// block; XCD x takes the x-th eighth of them, and workgroup w of the launch runs on XCD w % 8, so
+// work[pos * 8 + x] is XCD x's item pos, (-1, 0) past the end.  buildWorkLength: entries of the list.
+int buildWorkLength(int blocks, int ngb);
+void launchBuildWork(hipStream_t s, const int* segFirst, const int* segCount, const int* segPrefix, int numSegs,
+        int blocks, int ngb, int2* work);
 // bins[g][level index] for the work items (block, g) of feature groups g0 + g of the evaluation order;
 // permutation entries with kFlipEntry are evaluated flipped into bins[flipOffset + g * N + index]
 // with launch shape `shape` (evalShape): blocks of shape.lanes * shape.perLane samples

@@ -45,8 +45,8 @@ struct ActiveTree {
 struct BlockSet {
     int level = -1;        // level the blocks were built for
     DevBuf<BinBlock> blocks;
-    DevBuf<int> segInfo;   // per image group: first block, block count, XCD prefix; then the XCD totals
-    int numSegs = 0, maxXcdBlocks = 0;
+    DevBuf<int> segInfo;   // per image group: first block, block count, blocks before it
+    int numSegs = 0, numBlocks = 0;
     DevBuf<int2> work;
     int workGroups = -1;   // feature groups the work list was built for
     int numWork = 0;
@@ -510,10 +510,9 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             // blocks of one pass-1 block size: consecutive runs of <= blockSamples entries within a (image, tree)
             // segment; the segments of one image form a group of consecutive blocks.  Built on the host from the
             // segment starts for each block size the tuner asks for; the work list of a batch of ngb feature
-            // groups is then built on the device: image group i goes to XCD i % 8; each XCD takes its image
-            // groups in order, all feature groups of an image group (feature group major, then tree, then block)
-            // before the next, so the trees' workgroups of one feature group read the same planes of one image
-            // from the XCD's L2; workgroup w runs on XCD w % 8, so the lists are interleaved
+            // groups is then built on the device: each XCD takes an eighth of it in order, all feature groups of an
+            // image group (feature group major, then tree, then block) before the next image group, so the trees'
+            // workgroups of one feature group read the same planes of one image from the XCD's L2; workgroup w runs on XCD w % 8, so the lists are interleaved
             for (auto& kv : blockSets) kv.second.level = -1;
             auto blocksFor = [&](int blockSamples) -> BlockSet& {
                 BlockSet& bs = blockSets[blockSamples];
@@ -545,31 +544,27 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                     CF_HIP(hipMemcpyAsync(bs.blocks.get(), blocks.data(), blocks.size() * sizeof(BinBlock),
                             hipMemcpyHostToDevice, s));
                 }
-                constexpr int kXcds = 8;
                 bs.numSegs = static_cast<int>(segBlocks.size());
-                // first, count, XCD prefix per image group; XCD totals
-                std::vector<int> segInfo(3 * static_cast<size_t>(bs.numSegs) + kXcds, 0);
-                int* xcdBlocks = segInfo.data() + 3 * static_cast<size_t>(bs.numSegs);
-                for (int i = 0; i < bs.numSegs; i++) {
+                bs.numBlocks = static_cast<int>(blocks.size());
+                std::vector<int> segInfo(3 * static_cast<size_t>(bs.numSegs), 0);
+                for (int i = 0, before = 0; i < bs.numSegs; i++) {
                     segInfo[i] = segBlocks[i].first;
                     segInfo[bs.numSegs + i] = segBlocks[i].second;
-                    segInfo[2 * static_cast<size_t>(bs.numSegs) + i] = xcdBlocks[i % kXcds];
-                    xcdBlocks[i % kXcds] += segBlocks[i].second;
+                    segInfo[2 * static_cast<size_t>(bs.numSegs) + i] = before;
+                    before += segBlocks[i].second;
                 }
-                bs.maxXcdBlocks = *std::max_element(xcdBlocks, xcdBlocks + kXcds);
-                bs.segInfo.resize(segInfo.size());
+                bs.segInfo.resize(std::max<size_t>(segInfo.size(), 1));
                 CF_HIP(hipMemcpyAsync(bs.segInfo.get(), segInfo.data(), segInfo.size() * sizeof(int),
                         hipMemcpyHostToDevice, s));
                 return bs;
             };
             // the work list of a batch of ngb feature groups into `work`; returns its length
             auto buildWork = [&](BlockSet& bs, int ngb, DevBuf<int2>& work) {
-                const int maxLen = bs.maxXcdBlocks * ngb;
-                const int numWork = maxLen * kNumXcds;
+                const int numWork = buildWorkLength(bs.numBlocks, ngb);
                 work.resize(std::max<size_t>(static_cast<size_t>(numWork), 1));
                 const int ns = bs.numSegs;
-                launchBuildWork(s, bs.segInfo.get(), bs.segInfo.get() + ns, bs.segInfo.get() + 2 * ns,
-                        bs.segInfo.get() + 3 * ns, ns, ngb, maxLen, work.get());
+                launchBuildWork(s, bs.segInfo.get(), bs.segInfo.get() + ns, bs.segInfo.get() + 2 * ns, ns, bs.numBlocks, ngb,
+                        work.get());
                 return numWork;
             };
             auto workFor = [&](BlockSet& bs, int ngb) {
