@@ -162,6 +162,7 @@ struct FeatTables {
     DevBuf<float> thrFT;       // thresholds feature-major [trees*F][T]
     DevBuf<float> thrTF;       // thresholds threshold-major [trees][T][F] (reference layout)
     DevBuf<uint16_t> rank;     // rank[tf*T + t] = #{k : thr[k] < thr[t]} within the feature
+    DevBuf<float> thrPad;      // thresholds padded with +inf to binThresholdWidth(T), for pass 1 [trees*F][width]
     DevBuf<uint16_t> order;    // thresholds of each feature in non-decreasing rank order
     DevBuf<int8_t> soa;        // [trees][11][F] (reference SoA layout)
     // candidate / unsorted staging
@@ -177,7 +178,8 @@ struct FeatTables {
 };
 
 void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJob* jobsDev, int numJobs,
-        int F, int T, int boxRadius, int regionSize, int useDepth, const int* seedsHost, FeatTables& tabs);
+        int F, int T, int boxRadius, int regionSize, int useDepth, const int* seedsHost, FeatTables& tabs,
+        bool referenceLayouts = false);
 // thresholds given in reference layout [trees][T][F] + features SoA [trees][11][F] -> tables
 void launchPrepareTables(hipStream_t s, int trees, int F, int T, FeatTables& tabs);
 
@@ -224,7 +226,6 @@ struct BinBlock {
     int count;
     int image;   // the image of every sample in the block
 };
-void launchFeatureEvalOrder(hipStream_t s, const FeatTables& tabs, int trees, uint16_t* evalOrder);
 // keys ((image * keyMul + keyBase) << yBits | y) and values (level index) of one tree's level segment;
 // with flipN > 0 also the flipped evaluation of every Both sample at flipN + index (value |
 // kFlipEntry), and segment absentKey for the other samples there
@@ -250,11 +251,11 @@ void levelCountingSort(hipStream_t s, const uint32_t* keys, const uint32_t* vals
 int buildWorkLength(int blocks, int ngb);
 void launchBuildWork(hipStream_t s, const int* segFirst, const int* segCount, const int* segPrefix, int numSegs,
         int blocks, int ngb, int2* work);
-// bins[g][level index] for the work items (block, g) of feature groups g0 + g of the evaluation order;
+// bins[g][level index] for the work items (block, g) of feature groups g0 + g;
 // permutation entries with kFlipEntry are evaluated flipped into bins[flipOffset + g * N + index]
 // with launch shape `shape` (evalShape): blocks of shape.lanes * shape.perLane samples
 void launchEvalBins(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const uint32_t* perm,
-        const BinBlock* blocks, const int2* work, int numWork, int g0, const FeatRec* gFeat, const float* gThr,
+        const BinBlock* blocks, const int2* work, int numWork, int g0,
         const FeatTables& tabs, int N, uint4* bins, size_t flipOffset, int shape);
 // A launch shape of pass 1: lanes per workgroup, samples per lane (a workgroup's block holds
 // lanes * perLane samples), features whose corner gathers are issued together, workgroups per CU (held
@@ -272,9 +273,6 @@ int evalTunerChoose(int TM, size_t entries, bool* measure);
 void evalTunerRecord(int TM, size_t entries, int shape, double ms, double responses);
 // padded threshold width of the bin kernel for T thresholds
 int binThresholdWidth(int T);
-// features and +inf-padded thresholds in evaluation order: gFeat[trees * F], gThr[trees * F * binThresholdWidth(T)]
-void launchBinTables(hipStream_t s, const FeatTables& tabs, int trees, const uint16_t* evalOrder, FeatRec* gFeat,
-        float* gThr);
 // G[slot][ng * 16][T + 1][C] from the bin rows of the chunks' samples
 // (samples still set to Both also count their flipped row at flipOffset)
 void launchHistBins(hipStream_t s, const uint4* bins, const uint8_t* labels, const Chunk* chunks, int numChunks,
@@ -283,7 +281,7 @@ void launchHistBins(hipStream_t s, const uint4* bins, const uint8_t* labels, con
 // allScores[T][F] of slot onlySlot alone, or allScores[slot][T][F] of all slots (onlySlot < 0).
 void launchScores(hipStream_t s, const uint32_t* G, const uint32_t* nodeHist, const int* slotTree, int numSlots,
         const FeatTables& tabs, int C, FeatSummary* summ, double* allScores, int onlySlot, int fOffset = 0,
-        int Fb = -1, const uint16_t* evalOrder = nullptr);
+        int Fb = -1);
 void launchScoresFromCounters(hipStream_t s, const uint32_t* counters, const uint32_t* hist, int F, int T, int C,
         double* scores);
 void launchReduce(hipStream_t s, const FeatSummary* summ, int numSlots, int F, NodeBest* best);

@@ -102,58 +102,53 @@ private:
     int seed_;
 };
 
-// Device generator for the first K outputs of MT19937(seed) without the full
-// state: output k (k < 227) is temper(mix(s[k], s[k+1], s[k+397])) over the
-// initial state s, so only s[0..K] and s[397..397+K) are kept.  Samplers of
-// the feature generator draw a handful of values each.
+// The first K outputs of MT19937(seed) without the full state: output k (k < 227) is
+// temper(mix(s[k], s[k+1], s[k+397])) over the initial state s, a chain of which only s[0..K] has to be kept.
+// Samplers of the feature generator draw a handful of values each.
 template<int K>
-struct DevMTPrefix {
+__device__ __forceinline__ void mtPrefix(uint32_t seed, uint32_t* out) {
     uint32_t lo[K + 1];
-    uint32_t hi[K];
-    int pos;
-
-    __device__ void init(uint32_t seed) {
-        uint32_t v = seed;
-        lo[0] = v;
-#pragma unroll 1
-        for (uint32_t i = 1; i < 397u + K; i++) {
-            v = mtInitStep(v, i);
-            if (i <= static_cast<uint32_t>(K)) lo[i] = v;
-            if (i >= 397u) hi[i - 397u] = v;
-        }
-        pos = 0;
+    uint32_t v = seed;
+    lo[0] = v;
+#pragma unroll
+    for (uint32_t i = 1; i <= static_cast<uint32_t>(K); i++) {
+        v = mtInitStep(v, i);
+        lo[i] = v;
     }
-    // false when more than K outputs would be needed
-    __device__ bool next(uint32_t& out) {
-        if (pos >= K) return false;
-        out = mtTemper(mtMix(lo[pos], lo[pos + 1], hi[pos]));
-        pos++;
-        return true;
+#pragma unroll 4
+    for (uint32_t i = K + 1; i < 397u; i++) v = mtInitStep(v, i);
+#pragma unroll
+    for (uint32_t k = 0; k < static_cast<uint32_t>(K); k++) {
+        v = mtInitStep(v, 397u + k);
+        out[k] = mtTemper(mtMix(lo[k], lo[k + 1], v));
     }
-};
+}
 
+// Sampler(lower, upper) over K engine outputs in memory.
 template<int K>
 struct DevPrefixSampler {
-    DevMTPrefix<K> mt;
+    const uint32_t* outputs;
+    int pos;
     UniformIntParams p;
-    __device__ void init(int seed, int lo, int hi) {
-        mt.init(static_cast<uint32_t>(seed));
+    __device__ void init(const uint32_t* engineOutputs, int lo, int hi) {
+        outputs = engineOutputs;
+        pos = 0;
         p = uniformIntParams(lo, hi);
     }
+    // false when more than K outputs would be needed
     __device__ bool next(int& out) {
         if (p.range == 0) {
             out = p.lo;
             return true;
         }
-        for (;;) {
-            uint32_t r;
-            if (!mt.next(r)) return false;
-            const uint32_t v = r / p.bucket;
+        while (pos < K) {
+            const uint32_t v = outputs[pos++] / p.bucket;
             if (v <= p.range) {
                 out = static_cast<int>(static_cast<uint32_t>(p.lo) + v);
                 return true;
             }
         }
+        return false;
     }
 };
 

@@ -119,7 +119,7 @@ template<int TM, int LANES, int SPL, int FPS>
 __global__ void __launch_bounds__(LANES) k_eval_bins(const float* __restrict__ colBase,
         const int2* __restrict__ depBase, int W, int H, const cf_sample* __restrict__ samples,
         const uint32_t* __restrict__ perm, const BinBlock* __restrict__ blocks, const int2* __restrict__ work,
-        int g0, const FeatRec* __restrict__ gFeat, const float* __restrict__ gThr, int F, int T, int N,
+        int g0, const FeatRec* __restrict__ feat, const float* __restrict__ thrPad, int F, int T, int N,
         uint4* __restrict__ bins, size_t flipOffset) {
     static_assert(kBinGroup % FPS == 0, "features per step divide the group");
     // work[blockIdx] = (sample block, feature group within the batch); the
@@ -186,10 +186,10 @@ __global__ void __launch_bounds__(LANES) k_eval_bins(const float* __restrict__ c
             for (int j = 0; j < FPS; j++) {
                 const size_t tp = static_cast<size_t>(bb.tree) * F + pos0 + fi + j;
                 live[j] = pos0 + fi + j < F;   // uniform: the last group of the table may be partial
-                fr[j] = live[j] ? loadFeat(gFeat + tp) : Feat{};
+                fr[j] = live[j] ? loadFeat(feat + tp) : Feat{};
                 if (kThFirst && live[j]) {
 #pragma unroll
-                    for (int t = 0; t < TM; t++) th[kThFirst ? j : 0][t] = gThr[tp * TM + t];
+                    for (int t = 0; t < TM; t++) th[kThFirst ? j : 0][t] = thrPad[tp * TM + t];
                 }
 #pragma unroll
                 for (int k = 0; k < SPL; k++) {
@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(LANES) k_eval_bins(const float* __restrict__ c
                 if (!kThFirst) {
                     const size_t tp = static_cast<size_t>(bb.tree) * F + pos0 + fi + j;
 #pragma unroll
-                    for (int t = 0; t < TM; t++) th[tj][t] = gThr[tp * TM + t];
+                    for (int t = 0; t < TM; t++) th[tj][t] = thrPad[tp * TM + t];
                 }
 #pragma unroll
                 for (int k = 0; k < SPL; k++) {
@@ -224,25 +224,6 @@ __global__ void __launch_bounds__(LANES) k_eval_bins(const float* __restrict__ c
                 __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(o + outIdx[k]));
             }
         }
-    }
-}
-
-// Feature records and thresholds in evaluation order, thresholds padded to
-// TM per feature with +inf: gFeat[tree][pos], gThr[tree][pos][TM].  A NaN
-// threshold becomes +inf and -0 becomes +0; neither changes any comparison
-// th < q (NaN < q and +inf < q are false for every q, and -0 and +0 compare
-// equal).
-__global__ void __launch_bounds__(256) k_bin_tables(const FeatRec* __restrict__ feat, const float* __restrict__ thrFT,
-        const uint16_t* __restrict__ evalOrder, int total, int F, int T, int TM, FeatRec* __restrict__ gFeat,
-        float* __restrict__ gThr) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const int tree = i / F;
-    const size_t tf = static_cast<size_t>(tree) * F + evalOrder[i];
-    gFeat[i] = feat[tf];
-    for (int t = 0; t < TM; t++) {
-        const float v = t < T ? thrFT[tf * T + t] : __builtin_inff();
-        gThr[static_cast<size_t>(i) * TM + t] = (v != v) ? __builtin_inff() : v + 0.0f;
     }
 }
 
@@ -302,48 +283,6 @@ __global__ void __launch_bounds__(256) k_hist_bins(const uint4* __restrict__ bin
     for (int k = threadIdx.x; k < nb; k += 256) {
         const uint32_t v = h[k];
         if (v) atomicAdd(&out[k], v);
-    }
-}
-
-// Per tree: feature evaluation order grouped by the planes a feature reads
-// (depth first, then colour by (channel1, channel2)), stable in feature index.
-// One wave per table: a stable counting sort over the 10 keys, 64 features at a time -- a lane's place
-// among the lanes of its key is the count of its key's ballot bits below it.
-__global__ void __launch_bounds__(64) k_feature_eval_order(const FeatRec* __restrict__ feat, int F,
-        uint16_t* __restrict__ evalOrder) {
-    constexpr int kKeys = 10;
-    const FeatRec* ft = feat + static_cast<size_t>(blockIdx.x) * F;
-    uint16_t* eo = evalOrder + static_cast<size_t>(blockIdx.x) * F;
-    const int lane = threadIdx.x;
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    auto keyOf = [&](int f) {
-        if (f >= F) return -1;
-        const Feat x = loadFeat(ft + f);
-        return x.type == T_DEPTH ? 0 : 1 + x.c1 * 3 + x.c2;
-    };
-    int start[kKeys];
-#pragma unroll
-    for (int k = 0; k < kKeys; k++) start[k] = 0;
-    for (int f0 = 0; f0 < F; f0 += 64) {
-        const int key = keyOf(f0 + lane);
-#pragma unroll
-        for (int k = 0; k < kKeys; k++) start[k] += __popcll(__ballot(key == k));
-    }
-    int acc = 0;
-#pragma unroll
-    for (int k = 0; k < kKeys; k++) {
-        const int c = start[k];
-        start[k] = acc;
-        acc += c;
-    }
-    for (int f0 = 0; f0 < F; f0 += 64) {
-        const int key = keyOf(f0 + lane);
-#pragma unroll
-        for (int k = 0; k < kKeys; k++) {
-            const uint64_t m = __ballot(key == k);
-            if (key == k) eo[start[k] + __popcll(m & below)] = static_cast<uint16_t>(f0 + lane);
-            start[k] += __popcll(m);
-        }
     }
 }
 
@@ -425,18 +364,6 @@ int binThresholdWidth(int T) {
     throw Error(CF_ERR_ARG, "too many thresholds for 8-bit bins");
 }
 
-void launchBinTables(hipStream_t s, const FeatTables& tabs, int trees, const uint16_t* evalOrder, FeatRec* gFeat,
-        float* gThr) {
-    const int total = trees * tabs.F;
-    if (total == 0) return;
-    hipLaunchKernelGGL(k_bin_tables, dim3((total + 255) / 256), dim3(256), 0, s, tabs.feat.get(), tabs.thrFT.get(),
-            evalOrder, total, tabs.F, tabs.T, binThresholdWidth(tabs.T), gFeat, gThr);
-}
-
-void launchFeatureEvalOrder(hipStream_t s, const FeatTables& tabs, int trees, uint16_t* evalOrder) {
-    hipLaunchKernelGGL(k_feature_eval_order, dim3(trees), dim3(64), 0, s, tabs.feat.get(), tabs.F, evalOrder);
-}
-
 void launchLevelKeys(hipStream_t s, const cf_sample* samples, int begin, int n, uint32_t keyBase, uint32_t keyMul,
         uint32_t* keys, uint32_t* vals, int flipN, uint32_t absentKey, int yBits) {
     if (n == 0) return;
@@ -514,13 +441,13 @@ static size_t evalBinsLdsBytes(int w) {
 
 template<int LANES, int SPL, int FPS>
 static void launchEvalBinsShape(hipStream_t s, int TM, size_t lds, const ImageSet& imgs, const cf_sample* samples,
-        const uint32_t* perm, const BinBlock* blocks, const int2* work, int numWork, int g0, const FeatRec* gFeat,
-        const float* gThr, const FeatTables& tabs, int N, uint4* bins, size_t flipOffset) {
+        const uint32_t* perm, const BinBlock* blocks, const int2* work, int numWork, int g0,
+        const FeatTables& tabs, int N, uint4* bins, size_t flipOffset) {
     const dim3 grid(static_cast<unsigned>(numWork)), block(LANES);
 #define CF_EVAL_BINS(TMV)                                                                                        \
     allowLds(reinterpret_cast<const void*>(&k_eval_bins<TMV, LANES, SPL, FPS>), lds);                            \
     hipLaunchKernelGGL((k_eval_bins<TMV, LANES, SPL, FPS>), grid, block, lds, s, imgs.col, imgs.dep, imgs.W,     \
-            imgs.H, samples, perm, blocks, work, g0, gFeat, gThr, tabs.F, tabs.T, N, bins, flipOffset)
+            imgs.H, samples, perm, blocks, work, g0, tabs.feat.get(), tabs.thrPad.get(), tabs.F, tabs.T, N, bins, flipOffset)
     switch (TM) {
         case 8: CF_EVAL_BINS(8); break;
         case 12: CF_EVAL_BINS(12); break;
@@ -535,15 +462,14 @@ static void launchEvalBinsShape(hipStream_t s, int TM, size_t lds, const ImageSe
 }
 
 void launchEvalBins(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const uint32_t* perm,
-        const BinBlock* blocks, const int2* work, int numWork, int g0, const FeatRec* gFeat, const float* gThr,
-        const FeatTables& tabs, int N, uint4* bins, size_t flipOffset, int shape) {
+        const BinBlock* blocks, const int2* work, int numWork, int g0, const FeatTables& tabs, int N, uint4* bins, size_t flipOffset, int shape) {
     if (numWork == 0) return;
     const int TM = binThresholdWidth(tabs.T);
     const EvalShape& sh = evalShape(shape);
     const size_t lds = evalBinsLdsBytes(sh.wgPerCu);
 #define CF_SHAPE(L, S, F)                                                                                         \
     if (sh.lanes == L && sh.perLane == S && sh.featPerStep == F) {                                               \
-        launchEvalBinsShape<L, S, F>(s, TM, lds, imgs, samples, perm, blocks, work, numWork, g0, gFeat, gThr, tabs, \
+        launchEvalBinsShape<L, S, F>(s, TM, lds, imgs, samples, perm, blocks, work, numWork, g0, tabs, \
                 N, bins, flipOffset);                                                                            \
         return;                                                                                                  \
     }

@@ -34,15 +34,30 @@ namespace cf {
 
 constexpr int kPrefixDraws = 24;   // engine outputs available to one feature sampler
 
+// Candidates [first, first + count) of every job.  A lane per (candidate, sampler) runs the chain of 420
+// seeding steps that a sampler's first outputs need (the bound: with the four samplers one after another in
+// one lane, and the outputs indexed in scratch memory, 71 us a launch), then a lane per candidate draws from
+// the outputs in LDS.
+//
 // g++ on x86-64 evaluates the two getNext() calls of `Offset(rgen.getNext(),
 // rgen.getNext())` right to left, so the second coordinate is drawn first
 // (pinned by the reference's golden feature hash).
-__global__ void __launch_bounds__(256) k_fg_candidates(const int* __restrict__ seeds, int numCand, int boxRadius,
-        int regionSize, int useDepth, FeatRec* __restrict__ cand, int* __restrict__ err) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) k_fg_candidates(const int* __restrict__ seeds, int numCand, int first, int count,
+        int boxRadius, int regionSize, int useDepth, FeatRec* __restrict__ cand, int* __restrict__ err) {
+    constexpr int kStride = kPrefixDraws + 1;
+    __shared__ uint32_t outputs[256 * kStride];
     const int job = blockIdx.y;
-    if (k >= numCand) return;
-    const int base = seeds[job] + 1 + 4 * k;
+    {
+        const int k = first + blockIdx.x * 64 + static_cast<int>(threadIdx.x >> 2);
+        uint32_t out[kPrefixDraws];
+        mtPrefix<kPrefixDraws>(static_cast<uint32_t>(seeds[job] + 1 + 4 * k + static_cast<int>(threadIdx.x & 3)), out);
+#pragma unroll
+        for (int i = 0; i < kPrefixDraws; i++) outputs[threadIdx.x * kStride + i] = out[i];
+    }
+    __syncthreads();
+    const int k = first + blockIdx.x * 64 + threadIdx.x;
+    if (threadIdx.x >= 64 || k >= first + count) return;
+    const uint32_t* mine = outputs + threadIdx.x * 4 * kStride;   // samplers: type, offset, region, channel
     FeatRec f;
 #pragma unroll
     for (int i = 0; i < 16; i++) f.p[i] = 0;
@@ -50,7 +65,7 @@ __global__ void __launch_bounds__(256) k_fg_candidates(const int* __restrict__ s
     int a, b;
     {
         DevPrefixSampler<kPrefixDraws> xy;
-        xy.init(base + 1, -boxRadius, boxRadius);
+        xy.init(mine + kStride, -boxRadius, boxRadius);
         int o1x = 0, o1y = 0, o2x = 0, o2y = 0;
         ok &= xy.next(b);
         ok &= xy.next(a);
@@ -69,7 +84,7 @@ __global__ void __launch_bounds__(256) k_fg_candidates(const int* __restrict__ s
     }
     {
         DevPrefixSampler<kPrefixDraws> rg;
-        rg.init(base + 2, 1, regionSize);
+        rg.init(mine + 2 * kStride, 1, regionSize);
         ok &= rg.next(b);
         ok &= rg.next(a);
         f.p[P_R1X] = static_cast<int8_t>(a);
@@ -82,7 +97,7 @@ __global__ void __launch_bounds__(256) k_fg_candidates(const int* __restrict__ s
     int type = T_COLOR;
     if (useDepth) {
         DevPrefixSampler<kPrefixDraws> ft;
-        ft.init(base, 0, 1);
+        ft.init(mine, 0, 1);
         int v = 0;
         ok &= ft.next(v);
         type = (v == 0) ? T_DEPTH : T_COLOR;
@@ -90,7 +105,7 @@ __global__ void __launch_bounds__(256) k_fg_candidates(const int* __restrict__ s
     f.p[P_TYPE] = static_cast<int8_t>(type);
     if (type == T_COLOR) {
         DevPrefixSampler<kPrefixDraws> cc;
-        cc.init(base + 3, 0, 2);
+        cc.init(mine + 3 * kStride, 0, 2);
         ok &= cc.next(b);
         ok &= cc.next(a);
         f.p[P_C1] = static_cast<int8_t>(a);
@@ -278,7 +293,7 @@ static int bandDraws(int T) {
 // One candidate of a round on its band (see the head of this file).  Bound by the latency of the corner
 // gathers, which the round's candidates x trees workgroups overlap on all CUs.
 __global__ void __launch_bounds__(256) k_fg_round(const WalkState* __restrict__ states, ImageSet imgs,
-        const FeatRec* __restrict__ cand, int numCand, int T, int ring, int band, const DrawRec* __restrict__ recs,
+        const FeatRec* __restrict__ cand, int numCand, int drawn, int T, int ring, int band, const DrawRec* __restrict__ recs,
         float* __restrict__ resp, uint16_t* __restrict__ next, int4* __restrict__ bands) {
     constexpr int kWords = kBandMax / 64;
     __shared__ unsigned long long finite[kWords], rejects[kWords];   // not NaN; tenth NaN of a run
@@ -292,6 +307,7 @@ __global__ void __launch_bounds__(256) k_fg_round(const WalkState* __restrict__ 
     const int lo = j == 0 ? 0 : max(j * minDraws(T), static_cast<int>(j * avg - dev));
     int width = j == 0 ? band : min(band, static_cast<int>(2.0f * dev + 1.25f * avg) + 8);
     width = max(0, min(width, st.tail - st.head - lo));
+    if (st.k + j >= drawn) width = 0;   // not drawn yet: the walk stops here
     const Feat f = loadFeat(cand + static_cast<size_t>(blockIdx.y) * numCand + st.k + j);
     const DrawRec* rec = recs + static_cast<size_t>(blockIdx.y) * ring;
     const size_t plane = static_cast<size_t>(imgs.W) * imgs.H;
@@ -573,37 +589,87 @@ __global__ void __launch_bounds__(kAdvanceLanes) k_fg_advance(const FeatGenJob* 
     }
 }
 
-// Stable sort of each job's F features by key (rank = #smaller keys + #equal
-// keys earlier), scattering features and thresholds into both layouts.  The
-// grid is (F / 256 blocks, jobs): every workgroup holds all of its job's keys
-// in LDS and ranks 256 of its features.
+// Place of threshold t among its feature's T: rank = #{k : th[k] < th[t]}, and its position in the order by
+// (value, index), NaN after every number, so that the order is a permutation whatever the table holds (the
+// callers refuse NaN thresholds).  A sample with float key q goes left at threshold t iff q <= th[t] iff
+// #{k : th[k] < q} <= rank[t].
+__device__ __forceinline__ int2 thresholdPlace(const float* __restrict__ th, int T, int t) {
+    const float v = th[t];
+    const bool vNan = v != v;
+    int r = 0, pos = 0;
+#pragma unroll 8
+    for (int k = 0; k < T; k++) {
+        const float u = th[k];
+        const bool uNan = u != u;
+        const bool below = vNan ? !uNan : u < v;
+        const bool same = vNan ? uNan : u == v;
+        r += (u < v) ? 1 : 0;
+        pos += (below || (same && k < t)) ? 1 : 0;
+    }
+    return make_int2(r, pos);
+}
+
+// Stable sort of each job's F features by key (rank = #smaller keys + #equal keys earlier), scattering the
+// features and their threshold tables: values, ranks, order, the rows padded to TM with +inf that pass 1
+// compares against (a NaN threshold becomes +inf and -0 becomes +0; neither changes any comparison
+// th < q), and, where asked for, the reference's layouts.  The keys start with (type, channel1, channel2), so
+// the sorted order also groups the features by the planes they read.
+//
+// A workgroup ranks kSortFeat features: lane l of each wave takes feature l and a quarter of the keys, which
+// lie in LDS (one feature per lane over all keys, and a lane per feature for the threshold tables, took
+// 136 + 218 us for 5 x 4000 features with 32 thresholds).
+constexpr int kSortFeat = 64;
 __global__ void __launch_bounds__(256) k_fg_sort(const int* __restrict__ keys, const FeatRec* __restrict__ inFeat,
-        const float* __restrict__ inThr, int F, int T, FeatRec* __restrict__ feat, float* __restrict__ thrFT,
+        const float* __restrict__ inThr, int F, int T, int TM, FeatRec* __restrict__ feat, float* __restrict__ thrFT,
+        uint16_t* __restrict__ rank, uint16_t* __restrict__ order, float* __restrict__ thrPad,
         float* __restrict__ thrTF, int8_t* __restrict__ soa) {
     extern __shared__ int sk[];
-    const int job = blockIdx.y;
-    const int* jk = keys + static_cast<size_t>(job) * F;
-    for (int i = threadIdx.x; i < F; i += blockDim.x) sk[i] = jk[i];
+    __shared__ int part[4][kSortFeat];
+    const size_t jobF = static_cast<size_t>(blockIdx.y) * F;
+    for (int i = threadIdx.x; i < F; i += 256) sk[i] = keys[jobF + i];
     __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i0 = blockIdx.x * kSortFeat, i = i0 + lane;
     {
-        const int i = blockIdx.x * blockDim.x + threadIdx.x;
-        if (i >= F) return;
-        const int ki = sk[i];
-        int rank = 0;
-        for (int j = 0; j < F; j++) {
-            const int kj = sk[j];
-            rank += (kj < ki || (kj == ki && j < i)) ? 1 : 0;
+        const int ki = i < F ? sk[i] : 0;
+        const int a = static_cast<int>(static_cast<int64_t>(F) * wave / 4), b = static_cast<int>(static_cast<int64_t>(F) * (wave + 1) / 4);
+        const int m1 = min(max(a, i0), b), m2 = min(max(a, i0 + kSortFeat), b);   // [m1, m2): the workgroup's own
+        int r = 0;
+#pragma unroll 8
+        for (int j = a; j < m1; j++) r += sk[j] <= ki ? 1 : 0;
+        for (int j = m1; j < m2; j++) r += (sk[j] < ki || (sk[j] == ki && j < i)) ? 1 : 0;
+#pragma unroll 8
+        for (int j = m2; j < b; j++) r += sk[j] < ki ? 1 : 0;
+        part[wave][lane] = r;
+    }
+    __syncthreads();
+    const int nf = min(kSortFeat, F - i0);
+    if (threadIdx.x < nf) {
+        const int r = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+        part[0][lane] = r;
+        const FeatRec fr = inFeat[jobF + i];
+        feat[jobF + r] = fr;
+        if (soa) {
+            for (int p = 0; p < kFeatParams; p++) soa[(static_cast<size_t>(blockIdx.y) * kFeatParams + p) * F + r] = fr.p[p];
         }
-        const size_t src = static_cast<size_t>(job) * F + i;
-        const size_t dst = static_cast<size_t>(job) * F + rank;
-        const FeatRec fr = inFeat[src];
-        feat[dst] = fr;
-        for (int p = 0; p < kFeatParams; p++) soa[(static_cast<size_t>(job) * kFeatParams + p) * F + rank] = fr.p[p];
-        for (int t = 0; t < T; t++) {
-            const float v = inThr[src * T + t];
-            thrFT[dst * T + t] = v;
-            thrTF[(static_cast<size_t>(job) * T + t) * F + rank] = v;
-        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < nf * T; e += 256) {
+        const int l = e / T, t = e - l * T, dst = part[0][l];
+        const float* th = inThr + (jobF + i0 + l) * T;
+        const float v = th[t];
+        const int2 place = thresholdPlace(th, T, t);
+        const size_t row = (jobF + dst) * T;
+        thrFT[row + t] = v;
+        rank[row + t] = static_cast<uint16_t>(place.x);
+        order[row + place.y] = static_cast<uint16_t>(t);
+        if (TM > 0) thrPad[(jobF + dst) * TM + t] = (v != v) ? __builtin_inff() : v + 0.0f;
+        if (thrTF) thrTF[(static_cast<size_t>(blockIdx.y) * T + t) * F + dst] = v;
+    }
+    const int padT = max(0, TM - T);
+    for (int e = threadIdx.x; e < nf * padT; e += 256) {
+        const int l = e / padT;
+        thrPad[(jobF + part[0][l]) * TM + T + (e - l * padT)] = __builtin_inff();
     }
 }
 
@@ -622,35 +688,20 @@ __global__ void __launch_bounds__(256) k_tables_from_reference(const int8_t* __r
     for (int t = 0; t < T; t++) thrFT[static_cast<size_t>(i) * T + t] = thrTF[(static_cast<size_t>(job) * T + t) * F + f];
 }
 
-// Per feature: rank[t] = #{k : thr[k] < thr[t]} and the thresholds ordered by
-// (value, index).  A sample with float key q goes left at threshold t iff
-// q <= thr[t] iff #{k : thr[k] < q} <= rank[t].
+// rank[t] and the order of every feature's thresholds, one lane per threshold.
 __global__ void __launch_bounds__(256) k_threshold_ranks(const float* __restrict__ thrFT, int total, int T,
         uint16_t* __restrict__ rank, uint16_t* __restrict__ order) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const float* th = thrFT + static_cast<size_t>(i) * T;
-    // order: by (value, index) with NaN after every number, so `order` is a permutation
-    // whatever the table holds (the callers refuse NaN thresholds)
-    for (int t = 0; t < T; t++) {
-        const float v = th[t];
-        const bool vNan = v != v;
-        int r = 0, pos = 0;
-        for (int k = 0; k < T; k++) {
-            const float u = th[k];
-            const bool uNan = u != u;
-            const bool below = vNan ? !uNan : u < v;
-            const bool same = vNan ? uNan : u == v;
-            r += (u < v) ? 1 : 0;
-            pos += (below || (same && k < t)) ? 1 : 0;
-        }
-        rank[static_cast<size_t>(i) * T + t] = static_cast<uint16_t>(r);
-        order[static_cast<size_t>(i) * T + pos] = static_cast<uint16_t>(t);
-    }
+    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= static_cast<size_t>(total) * T) return;
+    const size_t row = i / T * T;
+    const int t = static_cast<int>(i - row);
+    const int2 place = thresholdPlace(thrFT + row, T, t);
+    rank[i] = static_cast<uint16_t>(place.x);
+    order[row + place.y] = static_cast<uint16_t>(t);
 }
 
 void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJob* jobsDev, int numJobs, int F,
-        int T, int boxRadius, int regionSize, int useDepth, const int* seedsHost, FeatTables& tabs) {
+        int T, int boxRadius, int regionSize, int useDepth, const int* seedsHost, FeatTables& tabs, bool referenceLayouts) {
     if (T > kMaxThresholds) throw Error(CF_ERR_ARG, "too many thresholds (max 256)");
     if (F > 8192) throw Error(CF_ERR_ARG, "too many features (max 8192)");
     if (boxRadius > 127 || regionSize > 127) throw Error(CF_ERR_ARG, "boxRadius/regionSize must fit int8");
@@ -664,10 +715,14 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     tabs.unsortedKey.resize(static_cast<size_t>(numJobs) * F);
     tabs.feat.resize(static_cast<size_t>(numJobs) * F);
     tabs.thrFT.resize(static_cast<size_t>(numJobs) * F * T);
-    tabs.thrTF.resize(static_cast<size_t>(numJobs) * F * T);
-    tabs.soa.resize(static_cast<size_t>(numJobs) * F * kFeatParams);
+    if (referenceLayouts) {
+        tabs.thrTF.resize(static_cast<size_t>(numJobs) * F * T);
+        tabs.soa.resize(static_cast<size_t>(numJobs) * F * kFeatParams);
+    }
     tabs.rank.resize(static_cast<size_t>(numJobs) * F * T);
     tabs.order.resize(static_cast<size_t>(numJobs) * F * T);
+    const int TM = T <= kMaxBinThresholds ? binThresholdWidth(T) : 0;
+    tabs.thrPad.resize(static_cast<size_t>(numJobs) * F * TM);
     tabs.err.resize(1);
     CF_HIP(hipMemsetAsync(tabs.err.get(), 0, sizeof(int), s));
     const int band = bandDraws(T);
@@ -699,9 +754,15 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     uint16_t* dNext = reinterpret_cast<uint16_t*>(space + oNext);
     int4* dBands = reinterpret_cast<int4*>(space + oBands);
     CF_HIP(hipMemcpyAsync(dSeeds, seedsHost, numJobs * sizeof(int), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_fg_candidates, dim3((numCand + 255) / 256, numJobs), dim3(256), 0, s, dSeeds, numCand,
-            boxRadius, regionSize, useDepth, tabs.cand.get(), tabs.err.get());
-    const int total = numJobs * F;
+    // a candidate in twenty or fewer is rejected on ordinary frames: the rest are drawn if they are needed
+    auto drawCandidates = [&](int first, int count) {
+        if (count > 0) {
+            hipLaunchKernelGGL(k_fg_candidates, dim3((count + 63) / 64, numJobs), dim3(256), 0, s, dSeeds, numCand, first,
+                    count, boxRadius, regionSize, useDepth, tabs.cand.get(), tabs.err.get());
+        }
+    };
+    int drawn = std::min(numCand, F + F / 8 + 64);
+    drawCandidates(0, drawn);
     std::vector<WalkState> states(numJobs);
     int errHost = 0;
     // draws of a candidate: the mean of these tables' last generation (the level before), or 5/4 T
@@ -724,16 +785,15 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
         allowLds(reinterpret_cast<const void*>(&k_fg_advance), lds);
         for (int r = 0; r < rounds; r++) {
             hipLaunchKernelGGL(k_fg_round, dim3(m, numJobs), dim3(std::min(band, 256)), 0, s, dWalk, imgs,
-                    tabs.cand.get(), numCand, T, ring, band, dRecs, dResp, dNext, dBands);
+                    tabs.cand.get(), numCand, drawn, T, ring, band, dRecs, dResp, dNext, dBands);
             hipLaunchKernelGGL(k_fg_advance, dim3(numJobs), dim3(kAdvanceLanes), lds, s, jobsDev, dWalk,
                     tabs.cand.get(), numCand, F, T, band, m, dResp, dNext, dBands, tabs.unsortedFeat.get(),
                     tabs.unsortedThr.get(), tabs.unsortedKey.get());
         }
-        hipLaunchKernelGGL(k_fg_sort, dim3((F + 255) / 256, numJobs), dim3(256), F * sizeof(int), s,
-                tabs.unsortedKey.get(), tabs.unsortedFeat.get(), tabs.unsortedThr.get(), F, T, tabs.feat.get(),
-                tabs.thrFT.get(), tabs.thrTF.get(), tabs.soa.get());
-        hipLaunchKernelGGL(k_threshold_ranks, dim3((total + 255) / 256), dim3(256), 0, s, tabs.thrFT.get(), total, T,
-                tabs.rank.get(), tabs.order.get());
+        hipLaunchKernelGGL(k_fg_sort, dim3((F + kSortFeat - 1) / kSortFeat, numJobs), dim3(256), F * sizeof(int), s,
+                tabs.unsortedKey.get(), tabs.unsortedFeat.get(), tabs.unsortedThr.get(), F, T, TM, tabs.feat.get(),
+                tabs.thrFT.get(), tabs.rank.get(), tabs.order.get(), tabs.thrPad.get(),
+                referenceLayouts ? tabs.thrTF.get() : nullptr, referenceLayouts ? tabs.soa.get() : nullptr);
         CF_HIP(hipMemcpyAsync(states.data(), dWalk, numJobs * sizeof(WalkState), hipMemcpyDeviceToHost, s));
         CF_HIP(hipMemcpyAsync(&errHost, tabs.err.get(), sizeof(int), hipMemcpyDeviceToHost, s));
         CF_HIP(hipStreamSynchronize(s));
@@ -743,6 +803,10 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
             more = more || !st.done;
         }
         if (errHost != 0) break;
+        if (more && drawn < numCand) {
+            drawCandidates(drawn, numCand - drawn);
+            drawn = numCand;
+        }
     }
     double draws = 0, cands = 0;
     for (const WalkState& st : states) {
@@ -766,8 +830,9 @@ void launchPrepareTables(hipStream_t s, int trees, int F, int T, FeatTables& tab
     const int total = trees * F;
     hipLaunchKernelGGL(k_tables_from_reference, dim3((total + 255) / 256), dim3(256), 0, s, tabs.soa.get(),
             tabs.thrTF.get(), trees, F, T, tabs.feat.get(), tabs.thrFT.get());
-    hipLaunchKernelGGL(k_threshold_ranks, dim3((total + 255) / 256), dim3(256), 0, s, tabs.thrFT.get(), total, T,
-            tabs.rank.get(), tabs.order.get());
+    const size_t thresholds = static_cast<size_t>(total) * T;
+    hipLaunchKernelGGL(k_threshold_ranks, dim3(static_cast<unsigned>((thresholds + 255) / 256)), dim3(256), 0, s,
+            tabs.thrFT.get(), total, T, tabs.rank.get(), tabs.order.get());
 }
 
 }  // namespace cf

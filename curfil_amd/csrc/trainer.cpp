@@ -300,10 +300,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
     DevBuf<int> dRepTree;
     DevBuf<FeatSummary> dRepSumm;
     DevBuf<NodeBest> dRepBest;
-    DevBuf<FeatRec> dGFeat;
-    DevBuf<float> dGThr;
     DevBuf<int> dStarts;
-    DevBuf<uint16_t> dEvalOrder;
     DevBuf<uint4> dBins;
     const size_t binsBudget = binsBudgetBytes();
     // CURFIL_LEVEL_GRAPH=1: levels whose pass-1 shape is settled run as one captured graph.  Off by default:
@@ -572,11 +569,6 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 bs.workGroups = ngb;
                 bs.numWork = buildWork(bs, ngb, bs.work);
             };
-            dEvalOrder.resize(static_cast<size_t>(numActive) * F);
-            launchFeatureEvalOrder(s, tabs, numActive, dEvalOrder.get());
-            dGFeat.resize(static_cast<size_t>(numActive) * F);
-            dGThr.resize(static_cast<size_t>(numActive) * F * binThresholdWidth(T));
-            launchBinTables(s, tabs, numActive, dEvalOrder.get(), dGFeat.get(), dGThr.get());
             // node histograms and trees of the whole level
             std::vector<uint32_t> nh(static_cast<size_t>(numNodes) * C);
             std::vector<int> st(numNodes);
@@ -660,7 +652,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 for (const Batch& b : batches) {
                     timer.begin();
                     launchEvalBins(s, images->set(), level[cur].get(), dPerm.get(), bs.blocks.get(), b.work->get(),
-                            b.numWork, b.g0, dGFeat.get(), dGThr.get(), tabs, N, dBins.get(), flipOffset, levelShape);
+                            b.numWork, b.g0, tabs, N, dBins.get(), flipOffset, levelShape);
                     timer.end(stats.evalKernelMs);
                     stats.evalLaunches += 1;
                     stats.shapeLaunches[levelShape] += 1;
@@ -677,7 +669,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                         timer.begin();
                         launchScores(s, dG.get(), dNodeHist.get() + static_cast<size_t>(s0) * C, dSlotTree.get() + s0,
                                 ns, tabs, C, dSumm.get() + static_cast<size_t>(s0) * F, nullptr, -1, b.g0 * kBinGroup,
-                                b.ngb * kBinGroup, dEvalOrder.get());
+                                b.ngb * kBinGroup);
                         timer.end(stats.scoreMs);
                         k++;
                     }
@@ -698,7 +690,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 if (measure) CF_HIP(hipEventRecord(tuneStart, s));
                 timer.begin();
                 launchEvalBins(s, images->set(), level[cur].get(), dPerm.get(), bs.blocks.get(), bs.work.get(),
-                        bs.numWork, g0, dGFeat.get(), dGThr.get(), tabs, N, dBins.get(), flipOffset, shape);
+                        bs.numWork, g0, tabs, N, dBins.get(), flipOffset, shape);
                 timer.end(stats.evalKernelMs);
                 if (measure) {
                     CF_HIP(hipEventRecord(tuneEnd, s));
@@ -730,7 +722,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                     timer.begin();
                     launchScores(s, dG.get(), dNodeHist.get() + static_cast<size_t>(s0) * C, dSlotTree.get() + s0, ns,
                             tabs, C, dSumm.get() + static_cast<size_t>(s0) * F, nullptr, -1, g0 * kBinGroup,
-                            ngb * kBinGroup, dEvalOrder.get());
+                            ngb * kBinGroup);
                     timer.end(stats.scoreMs);
                     s0 = s1;
                 }
