@@ -31,14 +31,12 @@ typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 
-// element i of a depth integral plane / a colour integral plane (a plane is far below 4 GiB)
-__device__ __forceinline__ int2 depthAt(const int2* plane, int i) {
-    const uint32_t off = static_cast<uint32_t>(i) * 8u;
+// the element at a byte offset of a depth integral plane / a colour integral plane (below 4 GiB)
+__device__ __forceinline__ int2 depthAtOffset(const int2* plane, uint32_t off) {
     const i32x2 v = *(const CF_GLOBAL i32x2*)((const CF_GLOBAL char*)plane + off);
     return make_int2(v.x, v.y);
 }
-__device__ __forceinline__ float colorAt(const float* plane, int i) {
-    const uint32_t off = static_cast<uint32_t>(i) * 4u;
+__device__ __forceinline__ float colorAtOffset(const float* plane, uint32_t off) {
     return *(const CF_GLOBAL float*)((const CF_GLOBAL char*)plane + off);
 }
 // record s of block b of the forest
@@ -73,7 +71,7 @@ __device__ __forceinline__ Feat unpackNode(const uint4& w) {
 // the depth in mm when the pixel's depth is valid.
 __device__ __forceinline__ bool pixelDepthAt(const DevImage& im, int x, int y, int32_t& depth) {
     const int W = im.W;
-    auto at = [&](int xx, int yy) -> int2 { return depthAt(im.dep, yy * W + xx); };
+    auto at = [&](int xx, int yy) -> int2 { return depthAtOffset(im.dep, static_cast<uint32_t>(yy * W + xx) * 8u); };
     const int2 c00 = at(x, y);
     const int2 cl = x > 0 ? at(x - 1, y) : make_int2(0, 0);
     const int2 ca = y > 0 ? at(x, y - 1) : make_int2(0, 0);
@@ -86,6 +84,50 @@ __device__ __forceinline__ bool pixelDepthAt(const DevImage& im, int x, int y, i
                 (static_cast<uint32_t>(cl.x) + static_cast<uint32_t>(ca.x) - static_cast<uint32_t>(cal.x)));
     }
     return depth > 0;
+}
+
+// Byte offsets of the 8 corners (as responseCorners' indices) in planes of 1 << sh byte elements; false if a
+// box leaves the image.  Rows and widths fit 24 bits (a coordinate is at most 127 px scaled by 1000 / mm), so
+// an offset is one 24-bit multiply-add; 32-bit products run at a quarter of the rate.
+__device__ __forceinline__ bool cornerOffsets(const Feat& f, int px, int py, int W, int H, double rinv, int sh,
+        uint32_t* off) {
+    const uint32_t pitch = static_cast<uint32_t>(W) << sh;
+    auto box = [&](int o1, int o2, int r1, int r2, uint32_t* to) {
+        const int w = max(normalizeCoord(r1, rinv), 1), h = max(normalizeCoord(r2, rinv), 1);
+        const int x = px + normalizeCoord(o1, rinv), y = py + normalizeCoord(o2, rinv);
+        const int lx = x - w, hx = x + w, uy = y - h, ly = y + h;
+        const uint32_t r = static_cast<uint32_t>(hx) << sh, l = static_cast<uint32_t>(lx) << sh;
+        to[0] = __umul24(ly, pitch) + r;
+        to[1] = __umul24(ly, pitch) + l;
+        to[2] = __umul24(uy, pitch) + r;
+        to[3] = __umul24(uy, pitch) + l;
+        return (lx | uy) >= 0 && hx < W && ly < H;
+    };
+    const bool a = box(f.o1x, f.o1y, f.r1x, f.r1y, off);
+    const bool b = box(f.o2x, f.o2y, f.r2x, f.r2y, off + 4);
+    return a && b;
+}
+
+// depthResponseFromCorners(d) <= thr.  The kernel keeps the vector units as busy as the vector L1 (170
+// instructions a pixel, tree and level before), and two correctly rounded double divisions are a third of a
+// depth split's (with the 24-bit offsets: 64 frames of 640x480, 10 trees of depth 18, 15.14 -> 14.45 ms).  The means in mm are first formed in float:
+// relative error below 2^-21 each (the sums rounded to float, a reciprocal of 1 ulp, a product), so a
+// difference that clears the threshold by 2^-20 of the operands' sizes decides as the double one does.  Else
+// (and where a count is zero or anything is not finite: the comparison with NaN fails) the exact form.
+__device__ __forceinline__ bool depthGoesLeft(const int2* d, float thr) {
+    auto boxOf = [](const int2* e) {
+        return make_int2(static_cast<int>((static_cast<uint32_t>(e[0].x) - static_cast<uint32_t>(e[2].x)) +
+                                 (static_cast<uint32_t>(e[3].x) - static_cast<uint32_t>(e[1].x))),
+                static_cast<int>((static_cast<uint32_t>(e[0].y) - static_cast<uint32_t>(e[2].y)) +
+                        (static_cast<uint32_t>(e[3].y) - static_cast<uint32_t>(e[1].y))));
+    };
+    const int2 a = boxOf(d), b = boxOf(d + 4);
+    const float ma = static_cast<float>(a.x) * __builtin_amdgcn_rcpf(static_cast<float>(a.y));
+    const float mb = static_cast<float>(b.x) * __builtin_amdgcn_rcpf(static_cast<float>(b.y));
+    const float t = thr * 1000.0f;
+    const float gap = (ma - mb) - t;
+    if (fabsf(gap) > (fabsf(ma) + fabsf(mb) + fabsf(t)) * 0x1p-20f) return gap < 0.0f;
+    return depthResponseFromCorners(d) <= static_cast<double>(thr);
 }
 
 // The leaf index one tree sends the pixel to, from the tree's root reference.  Per split the 8 corner
@@ -106,33 +148,43 @@ __device__ __forceinline__ int walkTree(const DevImage& im, int x, int y, bool d
         // branch that uses them, and every load instruction costs a tag lookup per line its lanes touch
         __asm__ volatile("" : : "v"(rec.x), "v"(rec.y), "v"(rec.z), "v"(rec.w));
         const Feat f = unpackNode(rec);
-        int idx[8];
         const bool isDepth = f.type == T_DEPTH;
-        const bool ok = depthOk && responseCorners(f, x, y, W, H, rinv, false, idx);
-        // one 8-byte load per depth corner and one 4-byte load per colour corner, in separate branches
-        // (a shared corner array makes the compiler split the depth loads in two)
-        double r = cf_nan();
-        if (ok && isDepth) {
-            int2 dv[8];
-#pragma unroll
-            for (int c = 0; c < 8; c++) dv[c] = depthAt(im.dep, idx[c]);
-            // all 8 corners are needed here: the compiler may not split a corner's two halves and sink the
-            // sums behind the count check (that doubles the loads and serialises them)
-#pragma unroll
-            for (int c = 0; c < 8; c++) __asm__ volatile("" : : "v"(dv[c].x), "v"(dv[c].y));
-            r = depthResponseFromCorners(dv);
-        } else if (ok) {
-            const float* colA = im.col + static_cast<size_t>(f.c1) * plane;
-            const float* colB = im.col + static_cast<size_t>(f.c2) * plane;
-            float cv[8];
-#pragma unroll
-            for (int c = 0; c < 4; c++) cv[c] = colorAt(colA, idx[c]);
-#pragma unroll
-            for (int c = 4; c < 8; c++) cv[c] = colorAt(colB, idx[c]);
-            r = colorResponseFromCorners(cv);
-        }
         const float thr = __uint_as_float(rec.x);
-        const int q = 2 * p + ((r <= static_cast<double>(thr)) ? 1 : 2);
+        // NaN goes right: invalid depth, a box outside the image
+        bool left = false;
+        uint32_t off[8];
+        if (depthOk && cornerOffsets(f, x, y, W, H, rinv, isDepth ? 3 : 2, off)) {
+            if (isDepth) {
+                int2 dv[8];
+#pragma unroll
+                for (int c = 0; c < 8; c++) dv[c] = depthAtOffset(im.dep, off[c]);
+                // all 8 corners are needed here: the compiler may not split a corner's two halves and sink the
+                // sums behind the count check (that doubles the loads and serialises them)
+#pragma unroll
+                for (int c = 0; c < 8; c++) __asm__ volatile("" : : "v"(dv[c].x), "v"(dv[c].y));
+                left = depthGoesLeft(dv, thr);
+            } else {
+                float cv[8];
+                if (plane <= (1u << 28)) {   // (uniform) three planes within 32-bit byte offsets
+                    const uint32_t p4 = static_cast<uint32_t>(plane) * 4u;
+                    const uint32_t a0 = f.c1 == 0 ? 0u : (f.c1 == 1 ? p4 : 2u * p4);
+                    const uint32_t b0 = f.c2 == 0 ? 0u : (f.c2 == 1 ? p4 : 2u * p4);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) cv[c] = colorAtOffset(im.col, a0 + off[c]);
+#pragma unroll
+                    for (int c = 4; c < 8; c++) cv[c] = colorAtOffset(im.col, b0 + off[c]);
+                } else {
+                    const float* colA = im.col + static_cast<size_t>(f.c1) * plane;
+                    const float* colB = im.col + static_cast<size_t>(f.c2) * plane;
+#pragma unroll
+                    for (int c = 0; c < 4; c++) cv[c] = colorAtOffset(colA, off[c]);
+#pragma unroll
+                    for (int c = 4; c < 8; c++) cv[c] = colorAtOffset(colB, off[c]);
+                }
+                left = colorResponseFromCorners(cv) <= static_cast<double>(thr);
+            }
+        }
+        const int q = 2 * p + (left ? 1 : 2);
         const uint32_t below = (1u << q) - 1u;
         if ((tail.z >> q) & 1u) return static_cast<int>(tail.y + __popc(tail.z & below));
         if (q < static_cast<int>(tail.w >> 16)) {
