@@ -163,7 +163,6 @@ struct FeatTables {
     DevBuf<float> thrTF;       // thresholds threshold-major [trees][T][F] (reference layout)
     DevBuf<uint16_t> rank;     // rank[tf*T + t] = #{k : thr[k] < thr[t]} within the feature
     DevBuf<float> thrPad;      // thresholds padded with +inf to binThresholdWidth(T), for pass 1 [trees*F][width]
-    DevBuf<uint16_t> order;    // thresholds of each feature in non-decreasing rank order
     DevBuf<int8_t> soa;        // [trees][11][F] (reference SoA layout)
     // candidate / unsorted staging
     DevBuf<FeatRec> cand;

@@ -9,7 +9,7 @@
 //                 (random_tree_image_gpu.cu:1455-1720) and the CPU counter
 //                 loop (random_tree_image.cpp:97-153): the response is never
 //                 stored and never re-read per threshold.
-//   k_scores      one thread per (node, feature): prefix sums over the bins
+//   k_scores      one thread per (node, feature, threshold): prefix sums over the bins
 //                 give every threshold's left/right class counts; FP64
 //                 NormalizedInformationGainScore (score.h:45-216) in the
 //                 reference's operation order; per-feature best / second best.
@@ -23,6 +23,7 @@
 //                      <=>  bin(q) := #{k : thr[k] < q} <= rank[t]
 // with NaN responses in bin T (always right), so left(t, c) is the prefix sum
 // of the bins up to rank[t].
+#include <algorithm>
 #include <cfloat>
 
 #include "cf_internal.h"
@@ -238,70 +239,151 @@ __device__ double nigScore(int C, const uint32_t* L, const uint32_t* R, const ui
     return clamp01((2 * ig) / (Hs + Hc));
 }
 
-template<int CM>
+// nigScore of the split that sends L[c] of the node's A[c] samples left, with the terms that the node's
+// thresholds share: classProb[c] = A[c] / total, entropyOf(total) and Hc.  The totals are integers, exact in
+// double however they are summed.  A caller's class counts below the bins' wrap as nigScore's do.
+__device__ __forceinline__ double splitScore(int C, const uint32_t* L, const uint32_t* A, const double* classProb,
+        double totalEntropy, double classEntropy) {
+    double totalLeft = 0, totalRight = 0, total = 0;
+    for (int c = 0; c < C; c++) {
+        totalLeft += static_cast<double>(L[c]);
+        totalRight += static_cast<double>(A[c] - L[c]);
+        total += static_cast<double>(A[c]);
+    }
+    const bool wraps = totalLeft + totalRight != total;
+    total = totalLeft + totalRight;
+    const double leftProb = totalLeft / total;
+    const double rightProb = totalRight / total;
+    double score = 0;
+    for (int c = 0; c < C; c++) {
+        const uint32_t l = L[c], r = A[c] - l;
+        const double prob = wraps ? static_cast<double>(A[c]) / total : classProb[c];
+        if (l > 0) {
+            const double p = static_cast<double>(l) / total;
+            score = __dadd_rn(score, __dmul_rn(p, log2(p / (leftProb * prob))));
+        }
+        if (r > 0) {
+            const double p = static_cast<double>(r) / total;
+            score = __dadd_rn(score, __dmul_rn(p, log2(p / (rightProb * prob))));
+        }
+    }
+    const double ig = clamp01(score);
+    if (ig == 0) return 0;
+    double Ht = totalEntropy, Hc = classEntropy;
+    if (wraps) {
+        Ht = entropyOf(total);
+        Hc = 0;
+        for (int c = 0; c < C; c++) {
+            if (A[c] > 0) Hc += entropyOf(static_cast<double>(A[c]));
+        }
+        Hc -= Ht;
+        Hc /= total;
+    }
+    const double Hs = (entropyOf(totalLeft) + entropyOf(totalRight) - Ht) / total;
+    return clamp01((2 * ig) / (Hs + Hc));
+}
+
+// Scores of a workgroup's features of one slot, a thread per (feature, threshold), and the features'
+// summaries.  The features' bins come into LDS in one run and become prefix sums there, so that threshold t's
+// left counts are row rank[t].  Bound by the double divisions and logarithms: what all thresholds of a node
+// share (the class probabilities, the entropies of the classes and of the total, 7 of 19 logarithms with 5
+// classes) is formed once per workgroup, by the same operations as nigScore.  A thread per feature that walked
+// its thresholds took 96 us for one node of 1000 features x 20 thresholds (now 10) and 866 us for 206 nodes x
+// 4000 x 32 (now 709).
+struct ScoreShape {
+    int feats;      // features of a workgroup
+    size_t lds;     // their bins (and prefix sums), the class probabilities, the scores
+};
+static ScoreShape scoreShape(int T, int C) {
+    ScoreShape s;
+    const int words = (T + 1) * C;
+    s.feats = std::max(1, std::min({256 / T, 64, 8192 / words}));
+    s.lds = (static_cast<size_t>(s.feats) * T + C + 2) * sizeof(double) + static_cast<size_t>(C) * sizeof(uint32_t) +
+            static_cast<size_t>(s.feats) * words * sizeof(uint32_t);
+    return s;
+}
+
 __global__ void __launch_bounds__(256) k_scores(const uint32_t* __restrict__ G, const uint32_t* __restrict__ nodeHist,
-        const int* __restrict__ slotTree, int numSlots, const uint16_t* __restrict__ rank,
-        const uint16_t* __restrict__ order, int F, int T, int C, FeatSummary* __restrict__ summ,
-        double* __restrict__ allScores, int onlySlot, int fOffset, int Fb) {
+        const int* __restrict__ slotTree, const uint16_t* __restrict__ rank, int F, int T, int C, int feats, int blocks,
+        FeatSummary* __restrict__ summ, double* __restrict__ allScores, int onlySlot, int fOffset, int Fb) {
+    extern __shared__ double scoreLds[];
+    double* scores = scoreLds;                    // [feats][T]
+    double* classProb = scores + feats * T;       // [C]
+    double* terms = classProb + C;                // entropyOf(total), Hc
+    uint32_t* A = reinterpret_cast<uint32_t*>(terms + 2);   // [C]
+    uint32_t* pre = A + C;                        // [feats][T + 1][C]
     // G holds Fb features per slot starting at feature fOffset
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    int slot, j;
-    if (onlySlot >= 0) {
-        slot = onlySlot;
-        j = gid;
-        if (j >= Fb) return;
-    } else {
-        if (gid >= numSlots * Fb) return;
-        slot = gid / Fb;
-        j = gid % Fb;
+    const int slot = onlySlot >= 0 ? onlySlot : static_cast<int>(blockIdx.x) / blocks;
+    const int j0 = (static_cast<int>(blockIdx.x) % blocks) * feats;
+    const int nf = min(feats, min(Fb - j0, F - fOffset - j0));
+    if (nf <= 0) return;
+    const int tid = threadIdx.x, words = (T + 1) * C;
+    const uint32_t* g = G + (static_cast<size_t>(slot) * Fb + j0) * words;
+    for (int i = tid; i < nf * words; i += 256) pre[i] = g[i];
+    if (tid < 64) {
+        // total of the node, exact in double; lane c: class c, lane C: the total
+        double total = 0;
+        for (int c = 0; c < C; c++) total += static_cast<double>(nodeHist[static_cast<size_t>(slot) * C + c]);
+        const uint32_t a = tid < C ? nodeHist[static_cast<size_t>(slot) * C + tid] : 0u;
+        const double e = entropyOf(tid < C ? static_cast<double>(a) : total);
+        if (tid < C) {
+            A[tid] = a;
+            classProb[tid] = static_cast<double>(a) / total;
+        }
+        double Hc = 0;
+        for (int c = 0; c < C; c++) {
+            const double ec = __shfl(e, c, 64);
+            if (__shfl(a, c, 64) > 0u) Hc += ec;
+        }
+        const double et = __shfl(e, C, 64);
+        Hc -= et;
+        if (tid == 0) {
+            terms[0] = et;
+            terms[1] = Hc / total;
+        }
     }
-    const int f = fOffset + j;
-    if (f >= F) return;
-    const int tree = slotTree[slot];
-    uint32_t A[CM], run[CM];
-#pragma unroll
-    for (int c = 0; c < CM; c++) {
-        A[c] = (c < C) ? nodeHist[static_cast<size_t>(slot) * C + c] : 0u;
-        run[c] = 0;
+    __syncthreads();
+    for (int i = tid; i < nf * C; i += 256) {
+        uint32_t* row = pre + (i / C) * words + i % C;
+        uint32_t run = 0;
+#pragma unroll 8
+        for (int b = 0; b <= T; b++) {
+            run += row[b * C];
+            row[b * C] = run;
+        }
     }
-    const size_t tf = static_cast<size_t>(tree) * F + f;
-    const uint32_t* g = G + (static_cast<size_t>(slot) * Fb + j) * (T + 1) * C;
-    const uint16_t* rk = rank + tf * T;
-    const uint16_t* od = order + tf * T;
-    double best = -DBL_MAX, second = -DBL_MAX;
-    int bestT = 0x7fffffff;
-    int b = 0;
-    for (int k = 0; k < T; k++) {
-        const int t = od[k];
-        const int r = rk[t];
-        while (b <= r) {
-#pragma unroll
-            for (int c = 0; c < CM; c++) {
-                if (c < C) run[c] += g[b * C + c];
+    __syncthreads();
+    const size_t row0 = static_cast<size_t>(slotTree[slot]) * F + fOffset + j0;
+    for (int i = tid; i < nf * T; i += 256) {
+        const int fi = i / T, t = i - fi * T;
+        const uint32_t* left = pre + fi * words + rank[(row0 + fi) * T + t] * C;
+        const double sc = splitScore(C, left, A, classProb, terms[0], terms[1]);
+        scores[i] = sc;
+        if (allScores) {
+            allScores[(static_cast<size_t>(onlySlot >= 0 ? 0 : slot) * T + t) * F + fOffset + j0 + fi] = sc;
+        }
+    }
+    __syncthreads();
+    if (tid < nf) {
+        double best = -DBL_MAX, second = -DBL_MAX;
+        int bestT = 0x7fffffff;
+        for (int t = 0; t < T; t++) {
+            const double sc = scores[tid * T + t];
+            if (sc > best) {
+                second = best;
+                best = sc;
+                bestT = t;
+            } else if (sc < best && sc > second) {
+                second = sc;
             }
-            b++;
         }
-        uint32_t right[CM];
-#pragma unroll
-        for (int c = 0; c < CM; c++) right[c] = A[c] - run[c];
-        const double sc = nigScore<CM>(C, run, right, A);
-        if (allScores) allScores[(static_cast<size_t>(onlySlot >= 0 ? 0 : slot) * T + t) * F + f] = sc;
-        if (sc > best) {
-            second = best;
-            best = sc;
-            bestT = t;
-        } else if (sc == best) {
-            bestT = min(bestT, t);
-        } else if (sc > second) {
-            second = sc;
-        }
+        FeatSummary s;
+        s.best = best;
+        s.second = second;
+        s.thresh = bestT;
+        s.pad = 0;
+        summ[static_cast<size_t>(slot) * F + fOffset + j0 + tid] = s;
     }
-    FeatSummary s;
-    s.best = best;
-    s.second = second;
-    s.thresh = bestT;
-    s.pad = 0;
-    summ[static_cast<size_t>(slot) * F + f] = s;
 }
 
 // scores[T][F] of one node straight from counters [F][T][C][2]
@@ -511,16 +593,13 @@ void launchEvalHistograms(hipStream_t s, const ImageSet& imgs, const cf_sample* 
 void launchScores(hipStream_t s, const uint32_t* G, const uint32_t* nodeHist, const int* slotTree, int numSlots,
         const FeatTables& tabs, int C, FeatSummary* summ, double* allScores, int onlySlot, int fOffset, int Fb) {
     if (Fb < 0) Fb = tabs.F;
-    const int threads = onlySlot >= 0 ? Fb : numSlots * Fb;
-    if (threads == 0) return;
-    const dim3 grid((threads + 255) / 256);
-    if (C <= 8) {
-        hipLaunchKernelGGL(k_scores<8>, grid, dim3(256), 0, s, G, nodeHist, slotTree, numSlots, tabs.rank.get(),
-                tabs.order.get(), tabs.F, tabs.T, C, summ, allScores, onlySlot, fOffset, Fb);
-    } else {
-        hipLaunchKernelGGL(k_scores<kMaxClasses>, grid, dim3(256), 0, s, G, nodeHist, slotTree, numSlots,
-                tabs.rank.get(), tabs.order.get(), tabs.F, tabs.T, C, summ, allScores, onlySlot, fOffset, Fb);
-    }
+    const int slots = onlySlot >= 0 ? 1 : numSlots;
+    if (slots == 0 || Fb <= 0) return;
+    const ScoreShape shape = scoreShape(tabs.T, C);
+    const int blocks = (Fb + shape.feats - 1) / shape.feats;
+    allowLds(reinterpret_cast<const void*>(&k_scores), shape.lds);
+    hipLaunchKernelGGL(k_scores, dim3(static_cast<unsigned>(slots) * blocks), dim3(256), shape.lds, s, G, nodeHist,
+            slotTree, tabs.rank.get(), tabs.F, tabs.T, C, shape.feats, blocks, summ, allScores, onlySlot, fOffset, Fb);
 }
 
 void launchReduce(hipStream_t s, const FeatSummary* summ, int numSlots, int F, NodeBest* best) {

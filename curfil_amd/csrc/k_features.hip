@@ -589,28 +589,18 @@ __global__ void __launch_bounds__(kAdvanceLanes) k_fg_advance(const FeatGenJob* 
     }
 }
 
-// Place of threshold t among its feature's T: rank = #{k : th[k] < th[t]}, and its position in the order by
-// (value, index), NaN after every number, so that the order is a permutation whatever the table holds (the
-// callers refuse NaN thresholds).  A sample with float key q goes left at threshold t iff q <= th[t] iff
-// #{k : th[k] < q} <= rank[t].
-__device__ __forceinline__ int2 thresholdPlace(const float* __restrict__ th, int T, int t) {
+// #{k : th[k] < th[t]} of threshold t among its feature's T.  A sample with float key q goes left at threshold
+// t iff q <= th[t] iff #{k : th[k] < q} is at most that.
+__device__ __forceinline__ uint16_t thresholdRank(const float* __restrict__ th, int T, int t) {
     const float v = th[t];
-    const bool vNan = v != v;
-    int r = 0, pos = 0;
+    int r = 0;
 #pragma unroll 8
-    for (int k = 0; k < T; k++) {
-        const float u = th[k];
-        const bool uNan = u != u;
-        const bool below = vNan ? !uNan : u < v;
-        const bool same = vNan ? uNan : u == v;
-        r += (u < v) ? 1 : 0;
-        pos += (below || (same && k < t)) ? 1 : 0;
-    }
-    return make_int2(r, pos);
+    for (int k = 0; k < T; k++) r += (th[k] < v) ? 1 : 0;
+    return static_cast<uint16_t>(r);
 }
 
 // Stable sort of each job's F features by key (rank = #smaller keys + #equal keys earlier), scattering the
-// features and their threshold tables: values, ranks, order, the rows padded to TM with +inf that pass 1
+// features and their threshold tables: values, ranks, the rows padded to TM with +inf that pass 1
 // compares against (a NaN threshold becomes +inf and -0 becomes +0; neither changes any comparison
 // th < q), and, where asked for, the reference's layouts.  The keys start with (type, channel1, channel2), so
 // the sorted order also groups the features by the planes they read.
@@ -621,7 +611,7 @@ __device__ __forceinline__ int2 thresholdPlace(const float* __restrict__ th, int
 constexpr int kSortFeat = 64;
 __global__ void __launch_bounds__(256) k_fg_sort(const int* __restrict__ keys, const FeatRec* __restrict__ inFeat,
         const float* __restrict__ inThr, int F, int T, int TM, FeatRec* __restrict__ feat, float* __restrict__ thrFT,
-        uint16_t* __restrict__ rank, uint16_t* __restrict__ order, float* __restrict__ thrPad,
+        uint16_t* __restrict__ rank, float* __restrict__ thrPad,
         float* __restrict__ thrTF, int8_t* __restrict__ soa) {
     extern __shared__ int sk[];
     __shared__ int part[4][kSortFeat];
@@ -658,11 +648,9 @@ __global__ void __launch_bounds__(256) k_fg_sort(const int* __restrict__ keys, c
         const int l = e / T, t = e - l * T, dst = part[0][l];
         const float* th = inThr + (jobF + i0 + l) * T;
         const float v = th[t];
-        const int2 place = thresholdPlace(th, T, t);
         const size_t row = (jobF + dst) * T;
         thrFT[row + t] = v;
-        rank[row + t] = static_cast<uint16_t>(place.x);
-        order[row + place.y] = static_cast<uint16_t>(t);
+        rank[row + t] = thresholdRank(th, T, t);
         if (TM > 0) thrPad[(jobF + dst) * TM + t] = (v != v) ? __builtin_inff() : v + 0.0f;
         if (thrTF) thrTF[(static_cast<size_t>(blockIdx.y) * T + t) * F + dst] = v;
     }
@@ -688,16 +676,13 @@ __global__ void __launch_bounds__(256) k_tables_from_reference(const int8_t* __r
     for (int t = 0; t < T; t++) thrFT[static_cast<size_t>(i) * T + t] = thrTF[(static_cast<size_t>(job) * T + t) * F + f];
 }
 
-// rank[t] and the order of every feature's thresholds, one lane per threshold.
+// The ranks of every feature's thresholds, one lane per threshold.
 __global__ void __launch_bounds__(256) k_threshold_ranks(const float* __restrict__ thrFT, int total, int T,
-        uint16_t* __restrict__ rank, uint16_t* __restrict__ order) {
+        uint16_t* __restrict__ rank) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= static_cast<size_t>(total) * T) return;
     const size_t row = i / T * T;
-    const int t = static_cast<int>(i - row);
-    const int2 place = thresholdPlace(thrFT + row, T, t);
-    rank[i] = static_cast<uint16_t>(place.x);
-    order[row + place.y] = static_cast<uint16_t>(t);
+    rank[i] = thresholdRank(thrFT + row, T, static_cast<int>(i - row));
 }
 
 void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJob* jobsDev, int numJobs, int F,
@@ -720,7 +705,6 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
         tabs.soa.resize(static_cast<size_t>(numJobs) * F * kFeatParams);
     }
     tabs.rank.resize(static_cast<size_t>(numJobs) * F * T);
-    tabs.order.resize(static_cast<size_t>(numJobs) * F * T);
     const int TM = T <= kMaxBinThresholds ? binThresholdWidth(T) : 0;
     tabs.thrPad.resize(static_cast<size_t>(numJobs) * F * TM);
     tabs.err.resize(1);
@@ -792,7 +776,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
         }
         hipLaunchKernelGGL(k_fg_sort, dim3((F + kSortFeat - 1) / kSortFeat, numJobs), dim3(256), F * sizeof(int), s,
                 tabs.unsortedKey.get(), tabs.unsortedFeat.get(), tabs.unsortedThr.get(), F, T, TM, tabs.feat.get(),
-                tabs.thrFT.get(), tabs.rank.get(), tabs.order.get(), tabs.thrPad.get(),
+                tabs.thrFT.get(), tabs.rank.get(), tabs.thrPad.get(),
                 referenceLayouts ? tabs.thrTF.get() : nullptr, referenceLayouts ? tabs.soa.get() : nullptr);
         CF_HIP(hipMemcpyAsync(states.data(), dWalk, numJobs * sizeof(WalkState), hipMemcpyDeviceToHost, s));
         CF_HIP(hipMemcpyAsync(&errHost, tabs.err.get(), sizeof(int), hipMemcpyDeviceToHost, s));
@@ -826,13 +810,12 @@ void launchPrepareTables(hipStream_t s, int trees, int F, int T, FeatTables& tab
     tabs.feat.resize(static_cast<size_t>(trees) * F);
     tabs.thrFT.resize(static_cast<size_t>(trees) * F * T);
     tabs.rank.resize(static_cast<size_t>(trees) * F * T);
-    tabs.order.resize(static_cast<size_t>(trees) * F * T);
     const int total = trees * F;
     hipLaunchKernelGGL(k_tables_from_reference, dim3((total + 255) / 256), dim3(256), 0, s, tabs.soa.get(),
             tabs.thrTF.get(), trees, F, T, tabs.feat.get(), tabs.thrFT.get());
     const size_t thresholds = static_cast<size_t>(total) * T;
     hipLaunchKernelGGL(k_threshold_ranks, dim3(static_cast<unsigned>((thresholds + 255) / 256)), dim3(256), 0, s,
-            tabs.thrFT.get(), total, T, tabs.rank.get(), tabs.order.get());
+            tabs.thrFT.get(), total, T, tabs.rank.get());
 }
 
 }  // namespace cf
