@@ -117,7 +117,8 @@ void singleNodeBins(cf_ctx* ctx, cf_images* im, const cf_sample* samples, int n,
     dS.resize(std::max(n, 1));
     CF_HIP(hipMemcpyAsync(dS.get(), samples, static_cast<size_t>(n) * sizeof(cf_sample), hipMemcpyHostToDevice, ctx->stream));
     std::vector<Chunk> chunks;
-    for (int b = 0; b < n; b += 4096) chunks.push_back(Chunk{0, 0, b, std::min(4096, n - b)});
+    const int per = evalChunkSamples(static_cast<size_t>(n), tabs.F);
+    for (int b = 0; b < n; b += per) chunks.push_back(Chunk{0, 0, b, std::min(per, n - b)});
     dC.resize(std::max<size_t>(chunks.size(), 1));
     if (!chunks.empty()) {
         CF_HIP(hipMemcpyAsync(dC.get(), chunks.data(), chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, ctx->stream));

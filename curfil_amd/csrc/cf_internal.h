@@ -162,7 +162,7 @@ struct FeatTables {
     DevBuf<float> thrFT;       // thresholds feature-major [trees*F][T]
     DevBuf<float> thrTF;       // thresholds threshold-major [trees][T][F] (reference layout)
     DevBuf<uint16_t> rank;     // rank[tf*T + t] = #{k : thr[k] < thr[t]} within the feature
-    DevBuf<float> thrPad;      // thresholds padded with +inf to binThresholdWidth(T), for pass 1 [trees*F][width]
+    DevBuf<float> thrPad;      // thresholds padded with +inf to binThresholdWidth(T), for the evaluation kernels [trees*F][width]
     DevBuf<int8_t> soa;        // [trees][11][F] (reference SoA layout)
     // candidate / unsorted staging
     DevBuf<FeatRec> cand;
@@ -205,7 +205,9 @@ struct FeatSummary {
     int pad;
 };
 
-// histogram bins G[slot][F][T+1][C] (interval histograms)
+// histogram bins G[slot][F][T+1][C] (interval histograms) of the chunks' samples; evalChunkSamples: the chunk
+// size for a launch over so many samples
+int evalChunkSamples(size_t samples, int F);
 void launchEvalHistograms(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk* chunks,
         int numChunks, const FeatTables& tabs, int C, uint32_t* G);
 
@@ -270,7 +272,7 @@ const EvalShape& evalShape(int i);
 // CURFIL_TUNE_FILE keeps the choices between runs.
 int evalTunerChoose(int TM, size_t entries, bool* measure);
 void evalTunerRecord(int TM, size_t entries, int shape, double ms, double responses);
-// padded threshold width of the bin kernel for T thresholds
+// padded threshold width of the evaluation kernels for T thresholds
 int binThresholdWidth(int T);
 // G[slot][ng * 16][T + 1][C] from the bin rows of the chunks' samples
 // (samples still set to Both also count their flipped row at flipOffset)

@@ -357,11 +357,11 @@ void allowLds(const void* kernel, size_t bytes) {
 }
 
 int binThresholdWidth(int T) {
-    static const int widths[] = {8, 12, 16, 20, 24, 32, 64, kMaxBinThresholds};
+    static const int widths[] = {8, 12, 16, 20, 24, 32, 64, kMaxThresholds};
     for (int w : widths) {
         if (T <= w) return w;
     }
-    throw Error(CF_ERR_ARG, "too many thresholds for 8-bit bins");
+    throw Error(CF_ERR_ARG, "too many thresholds (max 256)");
 }
 
 void launchLevelKeys(hipStream_t s, const cf_sample* samples, int begin, int n, uint32_t keyBase, uint32_t keyMul,
@@ -456,7 +456,7 @@ static void launchEvalBinsShape(hipStream_t s, int TM, size_t lds, const ImageSe
         case 24: CF_EVAL_BINS(24); break;
         case 32: CF_EVAL_BINS(32); break;
         case 64: CF_EVAL_BINS(64); break;
-        default: CF_EVAL_BINS(kMaxBinThresholds); break;
+        default: CF_EVAL_BINS(kMaxThresholds); break;
     }
 #undef CF_EVAL_BINS
 }

@@ -25,16 +25,17 @@
 // of the bins up to rank[t].
 #include <algorithm>
 #include <cfloat>
+#include <type_traits>
 
 #include "cf_internal.h"
 
 namespace cf {
 
 constexpr int kEvalThreads = 256;
-constexpr int kFeatTile = 16;
-constexpr int kSamplesPerThread = 4;   // samples held in registers per pass
-constexpr int kPass = kEvalThreads * kSamplesPerThread;
-constexpr int kXcds = 8;                  // MI355X: 8 XCDs, workgroups dispatched round-robin
+constexpr int kEvalStep = 4;           // features whose corner gathers are issued together
+constexpr int kEvalTile = 16;          // features of a workgroup
+constexpr int kEvalSmallTile = 4;      // the same where there are few workgroups
+constexpr int kXcds = 8;               // MI355X: 8 XCDs, workgroups dispatched round-robin
 
 // One training pixel held in registers for the feature loop.
 struct RegSample {
@@ -44,137 +45,128 @@ struct RegSample {
     int lab;       // label | flip << 8 | (invalid depth) << 10;  < 0: empty slot
 };
 
-// Interval of q among the T thresholds (thresholds held in registers; the
-// loop bound is a compile-time constant so the compare chain unrolls).
+// #{t : th[t] < q} over a row padded with +inf, T for NaN.
 template<int TM>
 __device__ __forceinline__ int binOf(float q, const float (&th)[TM], int T) {
-    if (__builtin_isnan(q)) return T;
-    int b = 0;
+    uint32_t b = 0;
 #pragma unroll
-    for (int t = 0; t < TM; t++) b += (t < T && th[t] < q) ? 1 : 0;
-    return b;
+    for (int t = 0; t < TM; t++) b += (th[t] < q) ? 1u : 0u;
+    return (q != q) ? T : static_cast<int>(b);
 }
 
 // All images of a set share W x H and are stored back to back, so a sample's
 // integrals are found from its image index.
 //
 // Work mapping: workgroups are dispatched round-robin over the 8 XCDs, each
-// with its own L2.  Workgroup L runs on XCD L % 8; the j-th workgroup of an
-// XCD takes feature tile j % tiles of chunk (j / tiles) * 8 + L % 8, so an XCD
-// sweeps all feature tiles of one chunk (one image region) before the next
-// and keeps that image's integrals cache-resident.
+// with its own L2.  With many chunks (perXcd), workgroup L runs on XCD L % 8 and
+// the j-th workgroup of an XCD takes feature tile j % tiles of chunk
+// (j / tiles) * 8 + L % 8, so an XCD sweeps all feature tiles of one chunk (one
+// image region) before the next and keeps that image's integrals
+// cache-resident.  With few, that leaves XCDs idle (a single chunk ran on one of
+// them): the tiles of a chunk go to all XCDs in turn.
+//
+// A lane holds one sample and issues the gathers of kEvalStep features before the
+// first response is formed: a small node is bound by their latency, and four
+// samples of one feature per lane left three quarters of the lanes of a
+// 256-sample chunk idle.
 template<int TM>
 __global__ void __launch_bounds__(kEvalThreads) k_eval_hist(const float* __restrict__ colBase,
         const int2* __restrict__ depBase, int W, int H, const cf_sample* __restrict__ samples,
-        const Chunk* __restrict__ chunks, int numChunks, int tiles, const FeatRec* __restrict__ feat,
-        const float* __restrict__ thrFT, int F, int T, int C, uint32_t* __restrict__ G) {
+        const Chunk* __restrict__ chunks, int numChunks, int tile, int tiles, int perXcd, const FeatRec* __restrict__ feat,
+        const float* __restrict__ thrPad, int F, int T, int C, uint32_t* __restrict__ G) {
     extern __shared__ uint32_t h[];
-    const int xcd = blockIdx.x % kXcds;
-    const int j = blockIdx.x / kXcds;
-    const int chunkIdx = (j / tiles) * kXcds + xcd;
+    int chunkIdx, tileIdx;
+    if (perXcd) {
+        const int j = blockIdx.x / kXcds;
+        chunkIdx = (j / tiles) * kXcds + blockIdx.x % kXcds;
+        tileIdx = j % tiles;
+    } else {
+        chunkIdx = blockIdx.x / tiles;
+        tileIdx = blockIdx.x % tiles;
+    }
     if (chunkIdx >= numChunks) return;
     const Chunk ch = chunks[chunkIdx];
-    const int f0 = (j % tiles) * kFeatTile;
-    const int nf = min(kFeatTile, F - f0);
+    const int f0 = tileIdx * tile;
+    const int nf = min(tile, F - f0);
     const int binsPerF = (T + 1) * C;
     const int nb = nf * binsPerF;
     const size_t plane = static_cast<size_t>(W) * H;
     for (int k = threadIdx.x; k < nb; k += kEvalThreads) h[k] = 0;
     __syncthreads();
     const FeatRec* fp = feat + static_cast<size_t>(ch.tree) * F + f0;
-    const float* tp = thrFT + (static_cast<size_t>(ch.tree) * F + f0) * T;
-    for (int base = 0; base < ch.count; base += kPass) {
-        RegSample rs[kSamplesPerThread];
-#pragma unroll
-        for (int k = 0; k < kSamplesPerThread; k++) {
-            const int i = base + k * kEvalThreads + threadIdx.x;
-            // lanes past the chunk's end gather (unused) corners at index 0
-            // of image 0, so every field must hold an in-range value
-            rs[k].lab = -1;
-            rs[k].img = 0;
-            rs[k].xy = 0;
-            rs[k].rinv = 0.0;
-            if (i < ch.count) {
-                const cf_sample s = samples[ch.begin + i];
-                const bool valid = s.depth_mm > 0;
-                rs[k].rinv = valid ? depthReciprocal(depthToFloat(s.depth_mm)) : 0.0;
-                rs[k].img = static_cast<int>(s.image);
-                rs[k].xy = s.x | (s.y << 16);
-                rs[k].lab = s.label | (s.flip << 8) | ((valid ? 0 : 1) << 10);
-            }
+    const float* tp = thrPad + (static_cast<size_t>(ch.tree) * F + f0) * TM;
+    for (int base = 0; base < ch.count; base += kEvalThreads) {
+        RegSample rs;
+        const int i = base + threadIdx.x;
+        rs.lab = -1;
+        rs.img = 0;
+        rs.xy = 0;
+        rs.rinv = 0.0;
+        if (i < ch.count) {
+            const cf_sample s = samples[ch.begin + i];
+            const bool valid = s.depth_mm > 0;
+            rs.rinv = valid ? depthReciprocal(depthToFloat(s.depth_mm)) : 0.0;
+            rs.img = static_cast<int>(s.image);
+            rs.xy = s.x | (s.y << 16);
+            rs.lab = s.label | (s.flip << 8) | ((valid ? 0 : 1) << 10);
         }
-        for (int fi = 0; fi < nf; fi++) {
-            const Feat fr = loadFeat(fp + fi);
-            float th[TM];
-            const float* tf = tp + static_cast<size_t>(fi) * T;
+        const int2* dep = depBase + static_cast<size_t>(rs.img) * plane;
+        const float* col = colBase + static_cast<size_t>(rs.img) * 3 * plane;
+        const bool live = rs.lab >= 0, valid = live && (rs.lab >> 10) == 0;
+        // orientation 0: the sample's own (Both: unflipped); 1: the flipped evaluation of Both samples
+        auto evaluate = [&](bool on, bool flip) {
+            for (int fi = 0; fi < nf; fi += kEvalStep) {
+                Feat fr[kEvalStep];
+                int2 cv[kEvalStep][8];   // depth corners, or colour corners' bits in .x
+                bool ok[kEvalStep];
 #pragma unroll
-            for (int t = 0; t < TM; t++) th[t] = (t < T) ? tf[t] : 0.0f;
-            const int hoff = fi * binsPerF;
-            // flipped responses of flip=Both samples take the generic path below
-            if (fr.type == T_DEPTH) {
-                int2 cv[kSamplesPerThread][8];
-                bool ok[kSamplesPerThread];
-#pragma unroll
-                for (int k = 0; k < kSamplesPerThread; k++) {
-                    const int lab = rs[k].lab;
+                for (int j = 0; j < kEvalStep; j++) {
+                    // past a partial tile's end (uniform): the tile's last feature, not counted
+                    fr[j] = loadFeat(fp + min(fi + j, nf - 1));
                     int idx[8];
-                    ok[k] = lab >= 0 && (lab >> 10) == 0 &&
-                            responseCorners(fr, rs[k].xy & 0xffff, rs[k].xy >> 16, W, H, rs[k].rinv,
-                                    ((lab >> 8) & 3) == 1, idx);
-                    const int2* dep = depBase + static_cast<size_t>(rs[k].img) * plane;
+                    ok[j] = on && valid && fi + j < nf &&
+                            responseCorners(fr[j], rs.xy & 0xffff, rs.xy >> 16, W, H, rs.rinv, flip, idx);
+                    if (ok[j]) {
+                        if (fr[j].type == T_DEPTH) {
 #pragma unroll
-                    for (int c = 0; c < 8; c++) cv[k][c] = dep[ok[k] ? idx[c] : 0];
+                            for (int c = 0; c < 8; c++) cv[j][c] = planeAt(dep, idx[c]);
+                        } else {
+                            const float* colA = col + static_cast<size_t>(fr[j].c1) * plane;
+                            const float* colB = col + static_cast<size_t>(fr[j].c2) * plane;
+#pragma unroll
+                            for (int c = 0; c < 4; c++) cv[j][c].x = __float_as_int(planeAt(colA, idx[c]));
+#pragma unroll
+                            for (int c = 4; c < 8; c++) cv[j][c].x = __float_as_int(planeAt(colB, idx[c]));
+                        }
+                    }
                 }
 #pragma unroll
-                for (int k = 0; k < kSamplesPerThread; k++) {
-                    const int lab = rs[k].lab;
-                    if (lab < 0) continue;
+                for (int j = 0; j < kEvalStep; j++) {
+                    if (fi + j >= nf) break;
+                    float th[TM];
+                    const float* tf = tp + static_cast<size_t>(fi + j) * TM;
+#pragma unroll
+                    for (int t = 0; t < TM; t++) th[t] = tf[t];
                     int b = T;
-                    if (ok[k]) b = binOf<TM>(roundUpToFloat(depthResponseFromCorners(cv[k])), th, T);
-                    atomicAdd(&h[hoff + b * C + (lab & 0xff)], 1u);
-                }
-            } else {
-                float cv[kSamplesPerThread][8];
-                bool ok[kSamplesPerThread];
+                    if (ok[j]) {
+                        double r;
+                        if (fr[j].type == T_DEPTH) {
+                            r = depthResponseFromCorners(cv[j]);
+                        } else {
+                            float c8[8];
 #pragma unroll
-                for (int k = 0; k < kSamplesPerThread; k++) {
-                    const int lab = rs[k].lab;
-                    int idx[8];
-                    ok[k] = lab >= 0 && (lab >> 10) == 0 &&
-                            responseCorners(fr, rs[k].xy & 0xffff, rs[k].xy >> 16, W, H, rs[k].rinv,
-                                    ((lab >> 8) & 3) == 1, idx);
-                    const float* colA = colBase + static_cast<size_t>(rs[k].img) * 3 * plane + fr.c1 * plane;
-                    const float* colB = colBase + static_cast<size_t>(rs[k].img) * 3 * plane + fr.c2 * plane;
-#pragma unroll
-                    for (int c = 0; c < 4; c++) cv[k][c] = colA[ok[k] ? idx[c] : 0];
-#pragma unroll
-                    for (int c = 4; c < 8; c++) cv[k][c] = colB[ok[k] ? idx[c] : 0];
-                }
-#pragma unroll
-                for (int k = 0; k < kSamplesPerThread; k++) {
-                    const int lab = rs[k].lab;
-                    if (lab < 0) continue;
-                    int b = T;
-                    if (ok[k]) b = binOf<TM>(roundUpToFloat(colorResponseFromCorners(cv[k])), th, T);
-                    atomicAdd(&h[hoff + b * C + (lab & 0xff)], 1u);
+                            for (int c = 0; c < 8; c++) c8[c] = __int_as_float(cv[j][c].x);
+                            r = colorResponseFromCorners(c8);
+                        }
+                        b = binOf<TM>(roundUpToFloat(r), th, T);
+                    }
+                    if (on) atomicAdd(&h[(fi + j) * binsPerF + b * C + (rs.lab & 0xff)], 1u);
                 }
             }
-            // the second (flipped) response of samples with flip setting Both
-#pragma unroll
-            for (int k = 0; k < kSamplesPerThread; k++) {
-                const int lab = rs[k].lab;
-                if (lab < 0 || ((lab >> 8) & 3) != 2) continue;
-                int b = T;
-                if ((lab >> 10) == 0) {
-                    const float* col = colBase + static_cast<size_t>(rs[k].img) * 3 * plane;
-                    const int2* dep = depBase + static_cast<size_t>(rs[k].img) * plane;
-                    const double r = featureResponseR(col, dep, W, H, fr, rs[k].xy & 0xffff, rs[k].xy >> 16,
-                            rs[k].rinv, true);
-                    b = binOf<TM>(roundUpToFloat(r), th, T);
-                }
-                atomicAdd(&h[hoff + b * C + (lab & 0xff)], 1u);
-            }
-        }
+        };
+        evaluate(live, ((rs.lab >> 8) & 3) == 1);
+        const bool both = live && ((rs.lab >> 8) & 3) == 2;
+        if (__any(both)) evaluate(both, true);
     }
     __syncthreads();
     uint32_t* g = G + (static_cast<size_t>(ch.slot) * F + f0) * binsPerF;
@@ -555,38 +547,43 @@ __global__ void __launch_bounds__(256) k_responses_paired(const DevImage* __rest
     out[i] = featureResponse(imgs[s.image], loadFeat(feats + i), s.x, s.y, s.depth_mm, s.flip == 1);
 }
 
+// Chunks of at least 256 samples (one per lane) and at most 4096 (over which the zeroing and flushing of a
+// workgroup's histograms no longer shows), of a size that gives about 2048 workgroups: 8 per CU.
+int evalChunkSamples(size_t samples, int F) {
+    const size_t tiles = (static_cast<size_t>(F) + kEvalTile - 1) / kEvalTile;
+    int c = 256;
+    while (c < 4096 && samples * tiles > static_cast<size_t>(c) * 4096) c *= 2;
+    return c;
+}
+
 void launchEvalHistograms(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk* chunks,
         int numChunks, const FeatTables& tabs, int C, uint32_t* G) {
     if (numChunks == 0) return;
-    const int tiles = (tabs.F + kFeatTile - 1) / kFeatTile;
-    const size_t lds = static_cast<size_t>(kFeatTile) * (tabs.T + 1) * C * sizeof(uint32_t);
-    const int groups = (numChunks + kXcds - 1) / kXcds;
-    const dim3 grid(groups * kXcds * tiles), block(kEvalThreads);
-    const void* kernel = tabs.T <= 8 ? reinterpret_cast<const void*>(&k_eval_hist<8>)
-            : tabs.T <= 16 ? reinterpret_cast<const void*>(&k_eval_hist<16>)
-            : tabs.T <= 24 ? reinterpret_cast<const void*>(&k_eval_hist<24>)
-            : tabs.T <= 32 ? reinterpret_cast<const void*>(&k_eval_hist<32>)
-            : tabs.T <= 64 ? reinterpret_cast<const void*>(&k_eval_hist<64>)
-            : reinterpret_cast<const void*>(&k_eval_hist<kMaxThresholds>);
-    allowLds(kernel, lds);
-    if (tabs.T <= 8) {
-        hipLaunchKernelGGL(k_eval_hist<8>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples,
-                chunks, numChunks, tiles, tabs.feat.get(), tabs.thrFT.get(), tabs.F, tabs.T, C, G);
-    } else if (tabs.T <= 16) {
-        hipLaunchKernelGGL(k_eval_hist<16>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples,
-                chunks, numChunks, tiles, tabs.feat.get(), tabs.thrFT.get(), tabs.F, tabs.T, C, G);
-    } else if (tabs.T <= 24) {
-        hipLaunchKernelGGL(k_eval_hist<24>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples,
-                chunks, numChunks, tiles, tabs.feat.get(), tabs.thrFT.get(), tabs.F, tabs.T, C, G);
-    } else if (tabs.T <= 32) {
-        hipLaunchKernelGGL(k_eval_hist<32>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples,
-                chunks, numChunks, tiles, tabs.feat.get(), tabs.thrFT.get(), tabs.F, tabs.T, C, G);
-    } else if (tabs.T <= 64) {
-        hipLaunchKernelGGL(k_eval_hist<64>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples,
-                chunks, numChunks, tiles, tabs.feat.get(), tabs.thrFT.get(), tabs.F, tabs.T, C, G);
-    } else {
-        hipLaunchKernelGGL(k_eval_hist<kMaxThresholds>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples,
-                chunks, numChunks, tiles, tabs.feat.get(), tabs.thrFT.get(), tabs.F, tabs.T, C, G);
+    // under two workgroups per CU with full tiles: tiles of one step
+    const int tile = static_cast<int64_t>(numChunks) * ((tabs.F + kEvalTile - 1) / kEvalTile) < 512 ? kEvalSmallTile : kEvalTile;
+    const int tiles = (tabs.F + tile - 1) / tile;
+    const int perXcd = numChunks >= 8 * kXcds;   // fewer chunks would not spread evenly over the XCDs
+    const size_t lds = static_cast<size_t>(tile) * (tabs.T + 1) * C * sizeof(uint32_t);
+    const int64_t blocks = static_cast<int64_t>(perXcd ? (numChunks + kXcds - 1) / kXcds * kXcds : numChunks) * tiles;
+    if (blocks > INT32_MAX) throw Error(CF_ERR_UNSUPPORTED, "too many samples in one evaluation launch");
+    const dim3 grid(static_cast<unsigned>(blocks)), block(kEvalThreads);
+    auto launch = [&](auto tm) {
+        constexpr int TM = decltype(tm)::value;
+        // the limit is that of a full tile, whatever the tile
+        const size_t full = static_cast<size_t>(kEvalTile) * (tabs.T + 1) * C * sizeof(uint32_t);
+        allowLds(reinterpret_cast<const void*>(&k_eval_hist<TM>), full);
+        hipLaunchKernelGGL(k_eval_hist<TM>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples, chunks,
+                numChunks, tile, tiles, perXcd, tabs.feat.get(), tabs.thrPad.get(), tabs.F, tabs.T, C, G);
+    };
+    switch (binThresholdWidth(tabs.T)) {
+        case 8: launch(std::integral_constant<int, 8>{}); break;
+        case 12: launch(std::integral_constant<int, 12>{}); break;
+        case 16: launch(std::integral_constant<int, 16>{}); break;
+        case 20: launch(std::integral_constant<int, 20>{}); break;
+        case 24: launch(std::integral_constant<int, 24>{}); break;
+        case 32: launch(std::integral_constant<int, 32>{}); break;
+        case 64: launch(std::integral_constant<int, 64>{}); break;
+        default: launch(std::integral_constant<int, kMaxThresholds>{}); break;
     }
 }
 

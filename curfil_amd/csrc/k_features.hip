@@ -600,8 +600,8 @@ __device__ __forceinline__ uint16_t thresholdRank(const float* __restrict__ th, 
 }
 
 // Stable sort of each job's F features by key (rank = #smaller keys + #equal keys earlier), scattering the
-// features and their threshold tables: values, ranks, the rows padded to TM with +inf that pass 1
-// compares against (a NaN threshold becomes +inf and -0 becomes +0; neither changes any comparison
+// features and their threshold tables: values, ranks, the rows padded to TM with +inf that the
+// evaluation kernels compare against (a NaN threshold becomes +inf and -0 becomes +0; neither changes any comparison
 // th < q), and, where asked for, the reference's layouts.  The keys start with (type, channel1, channel2), so
 // the sorted order also groups the features by the planes they read.
 //
@@ -651,10 +651,10 @@ __global__ void __launch_bounds__(256) k_fg_sort(const int* __restrict__ keys, c
         const size_t row = (jobF + dst) * T;
         thrFT[row + t] = v;
         rank[row + t] = thresholdRank(th, T, t);
-        if (TM > 0) thrPad[(jobF + dst) * TM + t] = (v != v) ? __builtin_inff() : v + 0.0f;
+        thrPad[(jobF + dst) * TM + t] = (v != v) ? __builtin_inff() : v + 0.0f;
         if (thrTF) thrTF[(static_cast<size_t>(blockIdx.y) * T + t) * F + dst] = v;
     }
-    const int padT = max(0, TM - T);
+    const int padT = TM - T;
     for (int e = threadIdx.x; e < nf * padT; e += 256) {
         const int l = e / padT;
         thrPad[(jobF + part[0][l]) * TM + T + (e - l * padT)] = __builtin_inff();
@@ -676,13 +676,17 @@ __global__ void __launch_bounds__(256) k_tables_from_reference(const int8_t* __r
     for (int t = 0; t < T; t++) thrFT[static_cast<size_t>(i) * T + t] = thrTF[(static_cast<size_t>(job) * T + t) * F + f];
 }
 
-// The ranks of every feature's thresholds, one lane per threshold.
-__global__ void __launch_bounds__(256) k_threshold_ranks(const float* __restrict__ thrFT, int total, int T,
-        uint16_t* __restrict__ rank) {
+// The ranks and the padded rows of every feature's thresholds, one lane per entry of a padded row.
+__global__ void __launch_bounds__(256) k_threshold_ranks(const float* __restrict__ thrFT, int total, int T, int TM,
+        uint16_t* __restrict__ rank, float* __restrict__ thrPad) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= static_cast<size_t>(total) * T) return;
-    const size_t row = i / T * T;
-    rank[i] = thresholdRank(thrFT + row, T, static_cast<int>(i - row));
+    if (i >= static_cast<size_t>(total) * TM) return;
+    const size_t f = i / TM;
+    const int t = static_cast<int>(i - f * TM);
+    const float* th = thrFT + f * T;
+    const float v = t < T ? th[t] : __builtin_inff();
+    thrPad[i] = (v != v) ? __builtin_inff() : v + 0.0f;
+    if (t < T) rank[f * T + t] = thresholdRank(th, T, t);
 }
 
 void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJob* jobsDev, int numJobs, int F,
@@ -705,7 +709,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
         tabs.soa.resize(static_cast<size_t>(numJobs) * F * kFeatParams);
     }
     tabs.rank.resize(static_cast<size_t>(numJobs) * F * T);
-    const int TM = T <= kMaxBinThresholds ? binThresholdWidth(T) : 0;
+    const int TM = binThresholdWidth(T);
     tabs.thrPad.resize(static_cast<size_t>(numJobs) * F * TM);
     tabs.err.resize(1);
     CF_HIP(hipMemsetAsync(tabs.err.get(), 0, sizeof(int), s));
@@ -813,9 +817,11 @@ void launchPrepareTables(hipStream_t s, int trees, int F, int T, FeatTables& tab
     const int total = trees * F;
     hipLaunchKernelGGL(k_tables_from_reference, dim3((total + 255) / 256), dim3(256), 0, s, tabs.soa.get(),
             tabs.thrTF.get(), trees, F, T, tabs.feat.get(), tabs.thrFT.get());
-    const size_t thresholds = static_cast<size_t>(total) * T;
-    hipLaunchKernelGGL(k_threshold_ranks, dim3(static_cast<unsigned>((thresholds + 255) / 256)), dim3(256), 0, s,
-            tabs.thrFT.get(), total, T, tabs.rank.get());
+    const int TM = binThresholdWidth(T);
+    tabs.thrPad.resize(static_cast<size_t>(total) * TM);
+    const size_t entries = static_cast<size_t>(total) * TM;
+    hipLaunchKernelGGL(k_threshold_ranks, dim3(static_cast<unsigned>((entries + 255) / 256)), dim3(256), 0, s,
+            tabs.thrFT.get(), total, T, TM, tabs.rank.get(), tabs.thrPad.get());
 }
 
 }  // namespace cf

@@ -113,6 +113,11 @@ struct LevelNode {
     int chunkBegin, chunkEnd;
 };
 
+// a node's samples in chunks of at most `per` for slot `slot` of a direct evaluation
+void appendChunks(std::vector<Chunk>& out, const LevelNode& ln, int slot, int per) {
+    for (int b = 0; b < ln.count; b += per) out.push_back(Chunk{slot, ln.active, ln.begin + b, std::min(per, ln.count - b)});
+}
+
 // Device time of the work enqueued between begin() and end() on the stream.  The events are read by
 // flush(), called where the host waits for the stream anyway, so timing adds no host waits between
 // the kernels of a level.
@@ -376,9 +381,11 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
         // ---- evaluation
         auto evalSlots = [&](int s0, int s1) {
             const int ns = s1 - s0;
-            const int c0 = nodes[s0].chunkBegin, c1 = nodes[s1 - 1].chunkEnd;
-            std::vector<Chunk> bc(chunks.begin() + c0, chunks.begin() + c1);
-            for (auto& c : bc) c.slot -= s0;
+            size_t slotSamples = 0;
+            for (int i = s0; i < s1; i++) slotSamples += nodes[i].count;
+            const int per = evalChunkSamples(slotSamples, F);
+            std::vector<Chunk> bc;
+            for (int i = s0; i < s1; i++) appendChunks(bc, nodes[i], i - s0, per);
             std::vector<uint32_t> nh(static_cast<size_t>(ns) * C);
             std::vector<int> st(ns);
             for (int i = 0; i < ns; i++) {
@@ -429,13 +436,12 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 std::vector<Chunk> bc;
                 std::vector<uint32_t> nh(static_cast<size_t>(ns) * C);
                 std::vector<int> st(ns);
+                size_t flaggedSamples = 0;
+                for (int k = 0; k < ns; k++) flaggedSamples += nodes[flagged[a + k]].count;
+                const int per = evalChunkSamples(flaggedSamples, F);
                 for (int k = 0; k < ns; k++) {
                     const LevelNode& ln = nodes[flagged[a + k]];
-                    for (int c = ln.chunkBegin; c < ln.chunkEnd; c++) {
-                        Chunk ch = chunks[c];
-                        ch.slot = k;
-                        bc.push_back(ch);
-                    }
+                    appendChunks(bc, ln, k, per);
                     std::memcpy(&nh[static_cast<size_t>(k) * C],
                             &out[active[ln.active].job].hist[static_cast<size_t>(ln.node) * C], C * sizeof(uint32_t));
                     st[k] = ln.active;
