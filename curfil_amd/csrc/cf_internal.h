@@ -227,23 +227,25 @@ struct BinBlock {
     int count;
     int image;   // the image of every sample in the block
 };
-// keys ((image * keyMul + keyBase) << yBits | y) and values (level index) of one tree's level segment;
+// keys ((image * keyMul + keyBase) << placeBits | the sample's place in the image, below levelPlaces) and
+// values (level index) of one tree's level segment;
 // with flipN > 0 also the flipped evaluation of every Both sample at flipN + index (value |
 // kFlipEntry), and segment absentKey for the other samples there
 constexpr uint32_t kFlipEntry = 0x80000000u;
 void launchLevelKeys(hipStream_t s, const cf_sample* samples, int begin, int n, uint32_t keyBase, uint32_t keyMul,
-        uint32_t* keys, uint32_t* vals, int flipN, uint32_t absentKey, int yBits);
+        uint32_t* keys, uint32_t* vals, int flipN, uint32_t absentKey, int placeBits, int H);
+int levelPlaces(int W, int H);
 // label per level index, bit 7 set for samples still set to Both (counted in both orientations)
 void launchLevelLabels(hipStream_t s, const cf_sample* samples, int n, uint8_t* labels);
-// Counting sort of n level entries by key (< levelSortBuckets(numSegs, yBits)): out = the values in key
-// order (input order inside every segment bucket of up to 64 entries), starts[seg] = first position of segment seg (key >> yBits) or -1 if it is empty, and
-// starts[numSegs] = the number of entries with a key below numSegs << yBits.  count and cursor hold
+// Counting sort of n level entries by key (< levelSortBuckets(numSegs, placeBits)): out = the values in key
+// order (input order inside every segment bucket of up to 64 entries), starts[seg] = first position of segment seg (key >> placeBits) or -1 if it is empty, and
+// starts[numSegs] = the number of entries with a key below numSegs << placeBits.  count and cursor hold
 // levelSortBuckets entries, blockSum levelSortScanBlocks.
-size_t levelSortBuckets(int numSegs, int yBits);
+size_t levelSortBuckets(int numSegs, int placeBits);
 // p[0 .. n) = v by a kernel (usable inside a captured graph, where memset nodes are avoided)
 void launchFillU32(hipStream_t s, uint32_t* p, size_t n, uint32_t v);
-size_t levelSortScanBlocks(int numSegs, int yBits);
-void levelCountingSort(hipStream_t s, const uint32_t* keys, const uint32_t* vals, int n, int numSegs, int yBits,
+size_t levelSortScanBlocks(int numSegs, int placeBits);
+void levelCountingSort(hipStream_t s, const uint32_t* keys, const uint32_t* vals, int n, int numSegs, int placeBits,
         uint32_t* count, uint32_t* cursor, uint32_t* blockSum, uint32_t* out, int* starts);
 // Work list of pass 1 for ngb feature groups, built on the device.  The items are ordered by image group
 // (segment i: its blocks segFirst[i] .. + segCount[i], segPrefix[i] blocks before them), feature group and

@@ -1,7 +1,7 @@
 // Image-major order of a batched level: a counting sort of the level
-// entries by their key ((tree, image) segment << yBits | row).
+// entries by their key ((image, tree) segment << placeBits | place).
 //
-// The keys are small integers (segments x rows: 4000 x 480 buckets for 5
+// The keys are small integers (segments x places: 4000 x 600 buckets for 5
 // trees over 800 frames of 640x480), so one counting pass replaces a radix
 // sort:
 //   k_sort_count    counts the entries of every bucket (global atomics);
@@ -16,12 +16,12 @@
 //                   one lane per bucket;
 //   k_sort_starts   the first position of every (tree, image) segment.
 // Buckets hold a few entries on average (one sample per 77 pixels per tree
-// at the benchmark's sampling density; a bucket holds at most the entries of
-// one row of one segment), so the result is the stable sort by key.  Longer
+// at the benchmark's sampling density, and 512 pixels per bucket), so the
+// result is the stable sort by key.  Longer
 // buckets, and the bucket past the segments that collects the flipped
 // entries of samples that are not Both (up to one per sample, never
 // evaluated), keep their arrival order: the order inside a bucket only
-// decides which lanes of pass 1 evaluate which samples of one row, never a
+// decides which lanes of pass 1 evaluate which samples of one place, never a
 // result, since every bin row is stored at its entry's level index.
 #include "cf_internal.h"
 
@@ -134,16 +134,16 @@ __global__ void __launch_bounds__(256) k_sort_settle(const uint32_t* __restrict_
 // starts[seg] = first position of segment seg, or -1 if it is empty.  After the scatter, a bucket's
 // first position is cursor - count.
 __global__ void __launch_bounds__(256) k_sort_starts(const uint32_t* __restrict__ count,
-        const uint32_t* __restrict__ cursor, int numSegs, int yBits, int* __restrict__ starts) {
+        const uint32_t* __restrict__ cursor, int numSegs, int placeBits, int* __restrict__ starts) {
     const int seg = blockIdx.x * blockDim.x + threadIdx.x;
     if (seg > numSegs) return;
-    const size_t b0 = static_cast<size_t>(seg) << yBits;
+    const size_t b0 = static_cast<size_t>(seg) << placeBits;
     const uint32_t first = cursor[b0] - count[b0];
     if (seg == numSegs) {
         starts[seg] = static_cast<int>(first);
         return;
     }
-    const size_t b1 = static_cast<size_t>(seg + 1) << yBits;
+    const size_t b1 = static_cast<size_t>(seg + 1) << placeBits;
     const uint32_t next = cursor[b1] - count[b1];
     starts[seg] = next > first ? static_cast<int>(first) : -1;
 }
@@ -157,15 +157,15 @@ void launchFillU32(hipStream_t s, uint32_t* p, size_t n, uint32_t v) {
     hipLaunchKernelGGL(k_fill_u32, dim3(blocksFor(n, 256)), dim3(256), 0, s, p, n, v);
 }
 
-size_t levelSortBuckets(int numSegs, int yBits) {
+size_t levelSortBuckets(int numSegs, int placeBits) {
     // the segments, one past the last for the flipped evaluations of samples that are not Both, and
     // the empty bucket after them that k_sort_starts reads
-    return (static_cast<size_t>(numSegs) + 2) << yBits;
+    return (static_cast<size_t>(numSegs) + 2) << placeBits;
 }
 
-void levelCountingSort(hipStream_t s, const uint32_t* keys, const uint32_t* vals, int n, int numSegs, int yBits,
+void levelCountingSort(hipStream_t s, const uint32_t* keys, const uint32_t* vals, int n, int numSegs, int placeBits,
         uint32_t* count, uint32_t* cursor, uint32_t* blockSum, uint32_t* out, int* starts) {
-    const size_t buckets = levelSortBuckets(numSegs, yBits);
+    const size_t buckets = levelSortBuckets(numSegs, placeBits);
     if (buckets > (static_cast<size_t>(1) << 28)) throw Error(CF_ERR_UNSUPPORTED, "too many level segments to sort");
     const int nb = static_cast<int>(blocksFor(buckets, kScanBlock));
     hipLaunchKernelGGL(k_fill_u32, dim3(blocksFor(buckets, 256)), dim3(256), 0, s, count, buckets, 0u);
@@ -176,16 +176,16 @@ void levelCountingSort(hipStream_t s, const uint32_t* keys, const uint32_t* vals
     if (n > 0) {
         hipLaunchKernelGGL(k_sort_scatter, dim3(blocksFor(n, 256)), dim3(256), 0, s, keys, vals, n, cursor, out);
         // the segments' buckets only: the bucket past them holds the flipped entries of samples that are not Both
-        const size_t segBuckets = static_cast<size_t>(numSegs) << yBits;
+        const size_t segBuckets = static_cast<size_t>(numSegs) << placeBits;
         hipLaunchKernelGGL(k_sort_settle, dim3(blocksFor(segBuckets, 256)), dim3(256), 0, s, count, cursor, segBuckets,
                 out);
     }
     hipLaunchKernelGGL(k_sort_starts, dim3(blocksFor(static_cast<size_t>(numSegs) + 1, 256)), dim3(256), 0, s,
-            count, cursor, numSegs, yBits, starts);
+            count, cursor, numSegs, placeBits, starts);
 }
 
-size_t levelSortScanBlocks(int numSegs, int yBits) {
-    return (levelSortBuckets(numSegs, yBits) + kScanBlock - 1) / kScanBlock;
+size_t levelSortScanBlocks(int numSegs, int placeBits) {
+    return (levelSortBuckets(numSegs, placeBits) + kScanBlock - 1) / kScanBlock;
 }
 
 }  // namespace cf

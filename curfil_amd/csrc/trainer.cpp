@@ -474,7 +474,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
         auto evalTwoPass = [&]() {
             int N = 0;
             for (int a = 0; a < numActive; a++) N = std::max(N, active[a].begin + active[a].n);
-            // image-major order of the level: (tree, image, row) keys, counting sort of level indices.
+            // image-major order of the level: (image, tree, place) keys, counting sort of level indices.
             // With Both samples a second entry per level index evaluates it flipped; the entries of samples
             // that are not Both get the key one past the last (tree, image) and sort to the end.
             const int M = anyBoth ? 2 * N : N;
@@ -484,23 +484,23 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             dLab8.resize(N);
             const uint64_t keyRange = static_cast<uint64_t>(numActive) * static_cast<uint64_t>(images->count);
             if (keyRange >= (1ull << 27)) throw Error(CF_ERR_UNSUPPORTED, "too many (tree, image) segments in one level");
-            // within a segment, samples ordered by row while the buckets stay below 2^26 (CURFIL_ROW_ORDER=0: off)
-            int yBits = 0;
-            while ((1 << yBits) < images->H) yBits++;
+            // within a segment, samples ordered by place while the buckets stay below 2^26 (CURFIL_ROW_ORDER=0: off)
+            int placeBits = 0;
+            while ((1 << placeBits) < levelPlaces(images->W, images->H)) placeBits++;
             const char* rowOrder = std::getenv("CURFIL_ROW_ORDER");
-            if (((keyRange + 2) << yBits) > (1ull << 26) || (rowOrder && std::strcmp(rowOrder, "0") == 0)) yBits = 0;
+            if (((keyRange + 2) << placeBits) > (1ull << 26) || (rowOrder && std::strcmp(rowOrder, "0") == 0)) placeBits = 0;
             // segments (image, tree) in image-major order: the trees' segments of one image are adjacent
             for (int a = 0; a < numActive; a++) {
                 launchLevelKeys(s, level[cur].get(), active[a].begin, active[a].n, static_cast<uint32_t>(a),
                         static_cast<uint32_t>(numActive), dKeys.get(), dVals.get(), anyBoth ? N : 0,
-                        static_cast<uint32_t>(keyRange), yBits);
+                        static_cast<uint32_t>(keyRange), placeBits, images->H);
             }
             const int numKeys = static_cast<int>(keyRange);
-            dSortCount.resize(levelSortBuckets(numKeys, yBits));
-            dSortCursor.resize(levelSortBuckets(numKeys, yBits));
-            dSortBlocks.resize(levelSortScanBlocks(numKeys, yBits));
+            dSortCount.resize(levelSortBuckets(numKeys, placeBits));
+            dSortCursor.resize(levelSortBuckets(numKeys, placeBits));
+            dSortBlocks.resize(levelSortScanBlocks(numKeys, placeBits));
             dStarts.resize(numKeys + 1);
-            levelCountingSort(s, dKeys.get(), dVals.get(), M, numKeys, yBits, dSortCount.get(), dSortCursor.get(),
+            levelCountingSort(s, dKeys.get(), dVals.get(), M, numKeys, placeBits, dSortCount.get(), dSortCursor.get(),
                     dSortBlocks.get(), dPerm.get(), dStarts.get());
             launchLevelLabels(s, level[cur].get(), N, dLab8.get());
             // (image, tree) segments of the sorted order -> blocks of <= kBinBlockSamples samples within a segment;
