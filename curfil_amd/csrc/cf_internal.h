@@ -260,7 +260,7 @@ void launchBuildWork(hipStream_t s, const int* segFirst, const int* segCount, co
 void launchEvalBins(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const uint32_t* perm,
         const BinBlock* blocks, const int2* work, int numWork, int g0,
         const FeatTables& tabs, int N, uint4* bins, size_t flipOffset, int shape);
-// A launch shape of pass 1: lanes per workgroup, samples per lane (a workgroup's block holds
+// A launch shape of pass 1: lanes per workgroup, samples of its block per lane (the block holds
 // lanes * perLane samples), features whose corner gathers are issued together, workgroups per CU (held
 // by an LDS reservation).
 struct EvalShape {

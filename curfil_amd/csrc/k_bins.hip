@@ -3,11 +3,10 @@
 //   k_eval_bins   pass 1, image-major: the level's samples ordered by
 //                 (image, tree, place) are cut into blocks of <= 256 within
 //                 each (image, tree) segment; one workgroup per
-//                 (block, group of 16 features), one sample per lane,
-//                 computes every response's interval among the feature's
-//                 thresholds (the bin used by the interval histograms) and
-//                 stores the 16 bins of a sample as one 16-byte row,
-//                 bins[group][level index].
+//                 (block, group of 16 features) computes every response's
+//                 interval among the feature's thresholds (the bin used by the
+//                 interval histograms) and stores the 16 bins of a sample as
+//                 one 16-byte row, bins[group][level index].
 //   k_hist_bins   pass 2, node-major: one workgroup per (node chunk, group)
 //                 streams the chunk's bin rows and labels into LDS interval
 //                 histograms and adds them to the node's global bins.
@@ -23,15 +22,17 @@
 // trees' workgroups of one feature group read the same planes of one image
 // and an XCD's L2 holds them.
 //
-// Pass 1 is bound by the vector memory path (L1 -> L2 requests times their
-// latency, about 70 in flight per CU), not by arithmetic or HBM.  Two
-// workgroups of four waves per CU, each lane with its one sample's 8 corner
-// loads in flight, beat every configuration with more samples in flight
-// (more samples per lane, more waves, larger blocks): with 256-sample blocks
-// the workgroups an XCD runs at once cover a few feature groups of a
-// segment rather than many, the planes they read fit the XCD's L2 (1.3%
-// misses instead of 3.8%) and requests return sooner.  The launch reserves
-// LDS the kernel does not use to hold the CU at two workgroups.
+// Pass 1 is bound by the vector memory path (the L1's misses in flight, about
+// 60 of 64 per CU, times the L2's latency of 150 cycles under this load), not by
+// arithmetic or HBM; its lookups are not far behind (0.94 per CU and cycle).
+// What counts is lines fetched per response: 3.33 with samples ordered by row,
+// 3.06 in strips, 2.76 with the waves of a workgroup on the same samples.  Eight
+// waves per CU, each lane with one sample's 8 corner loads in flight, beat
+// configurations with more in flight: the blocks an XCD runs at once cover a few
+// feature groups of a segment, the planes they read fit the XCD's L2 (0.5%
+// misses) and requests return sooner.  The launch reserves LDS the kernel does
+// not use to hold the CU at the shape's workgroups.
+#include <algorithm>
 #include <map>
 #include <mutex>
 
@@ -59,15 +60,6 @@ __device__ __forceinline__ int binOfT(float q, const float (&th)[TM], int T) {
 }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// Shifts a sample's 16-byte bin row right by one byte and inserts b as the
-// last byte: after 16 inserts the first inserted bin is byte 0.
-__device__ __forceinline__ void pushBin(uint32_t (&w)[4], uint32_t b) {
-    w[0] = (w[0] >> 8) | (w[1] << 24);
-    w[1] = (w[1] >> 8) | (w[2] << 24);
-    w[2] = (w[2] >> 8) | (w[3] << 24);
-    w[3] = (w[3] >> 8) | (b << 24);
-}
 
 // The 8 corners of one (sample, feature) response: depth corners as {sum, count}, colour corners'
 // float bits in .x.  Returns false (and issues no load) when the sample has no valid depth or a box
@@ -112,16 +104,27 @@ __device__ __forceinline__ uint32_t binFromCorners(const Feat& fr, bool ok, cons
 
 }  // namespace
 
-// Pass 1 with the launch shape <LANES lanes per workgroup, SPL samples per
-// lane, FPS features whose corner gathers are issued together>: a workgroup
-// covers one block of LANES * SPL samples.
-template<int TM, int LANES, int SPL, int FPS>
-__global__ void __launch_bounds__(LANES) k_eval_bins(const float* __restrict__ colBase,
+// A workgroup's block in LDS: its samples, their bin rows in the making, their level indices.
+constexpr int kBlockSampleBytes = sizeof(BinSample) + kBinGroup + sizeof(int);
+
+// Pass 1 with the launch shape <WAVES waves, FPS features whose corner gathers are issued together>.  A workgroup
+// covers one block of samples and a group of 16 features.  All its waves take the same 64 samples at a time,
+// wave w the features w, w + WAVES, ... of the group: neighbouring features of the table read the same plane with
+// nearly the same row offset, so the waves' corners fall on the same lines of a small patch, and a line that one
+// wave brought into the L1 serves the others.  (Waves with samples of their own and the same feature share
+// nothing: XX.)  A wave's features and thresholds are uniform and stay in scalar registers over the block.
+template<int TM, int WAVES, int FPS>
+__global__ void __launch_bounds__(WAVES * 64) k_eval_bins(const float* __restrict__ colBase,
         const int2* __restrict__ depBase, int W, int H, const cf_sample* __restrict__ samples,
         const uint32_t* __restrict__ perm, const BinBlock* __restrict__ blocks, const int2* __restrict__ work,
         int g0, const FeatRec* __restrict__ feat, const float* __restrict__ thrPad, int F, int T, int N,
-        uint4* __restrict__ bins, size_t flipOffset) {
-    static_assert(kBinGroup % FPS == 0, "features per step divide the group");
+        uint4* __restrict__ bins, size_t flipOffset, int blockMax) {
+    constexpr int kPerWave = kBinGroup / WAVES;
+    static_assert(kPerWave % FPS == 0, "features per step divide a wave's features");
+    extern __shared__ uint4 blockLds[];
+    BinSample* smp = reinterpret_cast<BinSample*>(blockLds);                  // [blockMax]
+    uint8_t* rows = reinterpret_cast<uint8_t*>(smp + blockMax);               // [blockMax][16]
+    int* outIdx = reinterpret_cast<int*>(rows + blockMax * kBinGroup);        // [blockMax]
     // work[blockIdx] = (sample block, feature group within the batch); the
     // XCDs' lists are interleaved (workgroup w runs on XCD w % 8) so each XCD
     // sweeps one image (the segments of all trees) for every group of the
@@ -140,90 +143,64 @@ __global__ void __launch_bounds__(LANES) k_eval_bins(const float* __restrict__ c
     const int2* dep = depBase + static_cast<size_t>(bb.image) * plane;
     const float* col = colBase + static_cast<size_t>(bb.image) * 3 * plane;
 
+    const int count64 = (bb.count + 63) & ~63;
+    for (int i = threadIdx.x; i < count64; i += WAVES * 64) {
+        // empty lanes keep in-range fields (they issue no gathers)
+        BinSample b{0.0, 0, -1};
+        if (i < bb.count) {
+            const uint32_t v = perm[bb.begin + i];
+            const int s = static_cast<int>(v & ~kFlipEntry);
+            const cf_sample x = samples[s];
+            const bool valid = x.depth_mm > 0;
+            // a flip entry evaluates a Both sample flipped; other entries in the sample's own
+            // orientation (Both: unflipped); bit 12 selects the flipped bin rows
+            const bool flipEntry = (v & kFlipEntry) != 0;
+            outIdx[i] = s;
+            b.rinv = valid ? depthReciprocal(depthToFloat(x.depth_mm)) : 0.0;
+            b.xy = x.x | (x.y << 16);
+            b.lab = ((flipEntry ? 1 : x.flip) << 8) | ((valid ? 0 : 1) << 10) | (flipEntry ? 1 << 12 : 0);
+        }
+        smp[i] = b;
+    }
+    __syncthreads();
+
     const int pos0 = (g0 + g) * kBinGroup;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6), lane = threadIdx.x & 63;
+    for (int f0 = 0; f0 < kPerWave; f0 += FPS) {
+        Feat fr[FPS];
+        float th[FPS][TM];
+        int pos[FPS];
+#pragma unroll
+        for (int j = 0; j < FPS; j++) {
+            pos[j] = wave + (f0 + j) * WAVES;
+            // past the table's end (uniform): the last feature again, its bins are not read
+            const size_t tp = static_cast<size_t>(bb.tree) * F + min(pos0 + pos[j], F - 1);
+            fr[j] = loadFeat(feat + tp);
+#pragma unroll
+            for (int t = 0; t < TM; t++) th[j][t] = thrPad[tp * TM + t];
+        }
+        for (int base = 0; base < bb.count; base += 64) {
+            const BinSample rs = smp[base + lane];
+            int2 cv[FPS][8];
+            bool ok[FPS];
+            // the gathers of FPS features are all issued before any response is formed
+#pragma unroll
+            for (int j = 0; j < FPS; j++) ok[j] = gatherCorners(fr[j], rs, col, dep, W, H, plane, cv[j]);
+#pragma unroll
+            for (int j = 0; j < FPS; j++) {
+                rows[(base + lane) * kBinGroup + pos[j]] =
+                        static_cast<uint8_t>(binFromCorners<TM>(fr[j], ok[j], cv[j], th[j], T));
+            }
+        }
+    }
+    __syncthreads();
     uint4* out = bins + static_cast<size_t>(g) * N;
     uint4* outFlip = bins + flipOffset + static_cast<size_t>(g) * N;
-    for (int base = 0; base < bb.count; base += LANES * SPL) {
-        BinSample rs[SPL];
-        int outIdx[SPL];
-#pragma unroll
-        for (int k = 0; k < SPL; k++) {
-            const int i = base + k * LANES + threadIdx.x;
-            // empty lanes keep in-range fields (they issue no gathers)
-            rs[k].lab = -1;
-            rs[k].xy = 0;
-            rs[k].rinv = 0.0;
-            outIdx[k] = -1;
-            if (i < bb.count) {
-                const uint32_t v = perm[bb.begin + i];
-                const int s = static_cast<int>(v & ~kFlipEntry);
-                const cf_sample x = samples[s];
-                const bool valid = x.depth_mm > 0;
-                // a flip entry evaluates a Both sample flipped; other entries in the sample's own
-                // orientation (Both: unflipped); bit 12 selects the flipped bin rows
-                const bool flipEntry = (v & kFlipEntry) != 0;
-                outIdx[k] = s;
-                rs[k].rinv = valid ? depthReciprocal(depthToFloat(x.depth_mm)) : 0.0;
-                rs[k].xy = x.x | (x.y << 16);
-                rs[k].lab = ((flipEntry ? 1 : x.flip) << 8) | ((valid ? 0 : 1) << 10) | (flipEntry ? 1 << 12 : 0);
-            }
-        }
-        uint32_t row[SPL][4];
-#pragma unroll
-        for (int k = 0; k < SPL; k++) row[k][0] = row[k][1] = row[k][2] = row[k][3] = 0u;
-
-        // thresholds are uniform (scalar loads): with few of them in flight they are loaded together with
-        // the features, before the gathers
-        constexpr bool kThFirst = FPS * TM <= 64;
-        for (int fi = 0; fi < kBinGroup; fi += FPS) {
-            Feat fr[FPS];
-            bool live[FPS];
-            int2 cv[FPS][SPL][8];
-            bool ok[FPS][SPL];
-            float th[kThFirst ? FPS : 1][TM];
-            // the gathers of FPS features x SPL samples are all issued before any response is formed
-#pragma unroll
-            for (int j = 0; j < FPS; j++) {
-                const size_t tp = static_cast<size_t>(bb.tree) * F + pos0 + fi + j;
-                live[j] = pos0 + fi + j < F;   // uniform: the last group of the table may be partial
-                fr[j] = live[j] ? loadFeat(feat + tp) : Feat{};
-                if (kThFirst && live[j]) {
-#pragma unroll
-                    for (int t = 0; t < TM; t++) th[kThFirst ? j : 0][t] = thrPad[tp * TM + t];
-                }
-#pragma unroll
-                for (int k = 0; k < SPL; k++) {
-                    ok[j][k] = live[j] && gatherCorners(fr[j], rs[k], col, dep, W, H, plane, cv[j][k]);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < FPS; j++) {
-                if (!live[j]) {
-#pragma unroll
-                    for (int k = 0; k < SPL; k++) pushBin(row[k], 0u);
-                    continue;
-                }
-                const int tj = kThFirst ? j : 0;
-                if (!kThFirst) {
-                    const size_t tp = static_cast<size_t>(bb.tree) * F + pos0 + fi + j;
-#pragma unroll
-                    for (int t = 0; t < TM; t++) th[tj][t] = thrPad[tp * TM + t];
-                }
-#pragma unroll
-                for (int k = 0; k < SPL; k++) {
-                    pushBin(row[k], binFromCorners<TM>(fr[j], ok[j][k], cv[j][k], th[tj], T));
-                }
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < SPL; k++) {
-            if (outIdx[k] >= 0) {
-                // rows are read once, by pass 2: streaming stores keep them from evicting image planes from L2
-                uint4* o = (rs[k].lab & (1 << 12)) ? outFlip : out;
-                const u32x4 v = {row[k][0], row[k][1], row[k][2], row[k][3]};
-                __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(o + outIdx[k]));
-            }
-        }
+    for (int i = threadIdx.x; i < bb.count; i += WAVES * 64) {
+        // rows are read once, by pass 2: streaming stores keep them from evicting image planes from L2
+        const u32x4 v = reinterpret_cast<const u32x4*>(rows)[i];
+        uint4* o = (smp[i].lab & (1 << 12)) ? outFlip : out;
+        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(o + outIdx[i]));
     }
 }
 
@@ -400,23 +377,17 @@ void launchLevelLabels(hipStream_t s, const cf_sample* samples, int n, uint8_t* 
     hipLaunchKernelGGL(k_level_labels, dim3((n + 255) / 256), dim3(256), 0, s, samples, n, labels);
 }
 
-// Launch shapes of pass 1 the tuner chooses from.  Shape 0 is the default:
-// two workgroups of four waves per CU, one sample per lane, one feature's
-// gathers at a time (the fastest of a manual sweep on the full-frame
-// workload).  The others trade samples in flight per CU (waves, samples per
-// lane, workgroups per CU) against L2 working set, and issue two features'
-// gathers together.
+// Launch shapes of pass 1 the tuner chooses from: {lanes, samples of a block per lane, features whose gathers
+// are issued together, workgroups per CU}.  Shape 0 is the default.  On large levels the shapes with two
+// workgroups are within 1% of each other and ahead (21 frames, 3 trees, 2000 x 20: 93.2, 92.2, 91.6, 96.5, 99.2 ms
+// of pass 1 a training in this order); on small ones with wide threshold rows the last two are (13 flipped
+// frames of 320x240, 2 trees, 500 x 50: 3.5, 3.9, 4.0, 3.0, 2.95 ms).
 constexpr EvalShape kEvalShapes[] = {
     {256, 1, 1, 2},
     {256, 1, 2, 2},
-    {256, 1, 1, 3},
-    {128, 1, 1, 4},
-    {128, 2, 1, 2},
-    {256, 2, 1, 1},
-    {512, 1, 1, 1},
-    {128, 1, 2, 4},
-    {128, 1, 4, 4},
     {256, 1, 4, 2},
+    {256, 1, 1, 3},
+    {256, 1, 1, 4},
 };
 constexpr int kNumEvalShapes = static_cast<int>(sizeof(kEvalShapes) / sizeof(kEvalShapes[0]));
 static_assert(kNumEvalShapes <= 16, "TrainStats counts launches of at most 16 shapes");
@@ -449,15 +420,16 @@ static size_t evalBinsLdsBytes(int w) {
     return bytes[{dev, w}] = b;
 }
 
-template<int LANES, int SPL, int FPS>
+template<int WAVES, int FPS>
 static void launchEvalBinsShape(hipStream_t s, int TM, size_t lds, const ImageSet& imgs, const cf_sample* samples,
-        const uint32_t* perm, const BinBlock* blocks, const int2* work, int numWork, int g0,
-        const FeatTables& tabs, int N, uint4* bins, size_t flipOffset) {
-    const dim3 grid(static_cast<unsigned>(numWork)), block(LANES);
+        const uint32_t* perm, const BinBlock* blocks, const int2* work, int numWork, int g0, const FeatTables& tabs,
+        int N, uint4* bins, size_t flipOffset, int blockMax) {
+    const dim3 grid(static_cast<unsigned>(numWork)), block(WAVES * 64);
 #define CF_EVAL_BINS(TMV)                                                                                        \
-    allowLds(reinterpret_cast<const void*>(&k_eval_bins<TMV, LANES, SPL, FPS>), lds);                            \
-    hipLaunchKernelGGL((k_eval_bins<TMV, LANES, SPL, FPS>), grid, block, lds, s, imgs.col, imgs.dep, imgs.W,     \
-            imgs.H, samples, perm, blocks, work, g0, tabs.feat.get(), tabs.thrPad.get(), tabs.F, tabs.T, N, bins, flipOffset)
+    allowLds(reinterpret_cast<const void*>(&k_eval_bins<TMV, WAVES, FPS>), lds);                                 \
+    hipLaunchKernelGGL((k_eval_bins<TMV, WAVES, FPS>), grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H,  \
+            samples, perm, blocks, work, g0, tabs.feat.get(), tabs.thrPad.get(), tabs.F, tabs.T, N, bins,         \
+            flipOffset, blockMax)
     switch (TM) {
         case 8: CF_EVAL_BINS(8); break;
         case 12: CF_EVAL_BINS(12); break;
@@ -472,26 +444,24 @@ static void launchEvalBinsShape(hipStream_t s, int TM, size_t lds, const ImageSe
 }
 
 void launchEvalBins(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const uint32_t* perm,
-        const BinBlock* blocks, const int2* work, int numWork, int g0, const FeatTables& tabs, int N, uint4* bins, size_t flipOffset, int shape) {
+        const BinBlock* blocks, const int2* work, int numWork, int g0,
+        const FeatTables& tabs, int N, uint4* bins, size_t flipOffset, int shape) {
     if (numWork == 0) return;
     const int TM = binThresholdWidth(tabs.T);
     const EvalShape& sh = evalShape(shape);
-    const size_t lds = evalBinsLdsBytes(sh.wgPerCu);
-#define CF_SHAPE(L, S, F)                                                                                         \
-    if (sh.lanes == L && sh.perLane == S && sh.featPerStep == F) {                                               \
-        launchEvalBinsShape<L, S, F>(s, TM, lds, imgs, samples, perm, blocks, work, numWork, g0, tabs, \
-                N, bins, flipOffset);                                                                            \
+    const int blockMax = sh.lanes * sh.perLane;
+    const size_t lds = std::max(evalBinsLdsBytes(sh.wgPerCu), static_cast<size_t>(blockMax) * kBlockSampleBytes);
+#define CF_SHAPE(L, F)                                                                                            \
+    if (sh.lanes == L && sh.featPerStep == F) {                                                                  \
+        launchEvalBinsShape<L / 64, F>(s, TM, lds, imgs, samples, perm, blocks, work, numWork, g0, tabs, N, bins,  \
+                flipOffset, blockMax);                                                                           \
         return;                                                                                                  \
     }
-    CF_SHAPE(256, 1, 1)
-    CF_SHAPE(256, 1, 2)
-    CF_SHAPE(128, 1, 1)
-    CF_SHAPE(128, 2, 1)
-    CF_SHAPE(256, 2, 1)
-    CF_SHAPE(512, 1, 1)
-    CF_SHAPE(128, 1, 2)
-    CF_SHAPE(128, 1, 4)
-    CF_SHAPE(256, 1, 4)
+    CF_SHAPE(128, 1)
+    CF_SHAPE(128, 2)
+    CF_SHAPE(256, 1)
+    CF_SHAPE(256, 2)
+    CF_SHAPE(256, 4)
 #undef CF_SHAPE
     throw Error(CF_ERR_RUNTIME, "pass-1 launch shape without a kernel");
 }
