@@ -90,6 +90,13 @@ void checkFeaturesSoA(const int8_t* soa, int F) {
     }
 }
 
+// The context's tables for a call on one node: the memory is kept, nothing of an earlier call is read.
+FeatTables& nodeTables(cf_ctx* ctx) {
+    if (!ctx->nodeTables) ctx->nodeTables = std::make_shared<FeatTables>();
+    ctx->nodeTables->meanDraws = 0;
+    return *ctx->nodeTables;
+}
+
 void uploadFeaturesSoA(cf_ctx* ctx, FeatTables& tabs, const int8_t* soa, const float* thrTF, int F, int T) {
     tabs.soa.resize(static_cast<size_t>(F) * kFeatParams);
     tabs.thrTF.resize(static_cast<size_t>(F) * T);
@@ -265,6 +272,8 @@ int cf_ctx_destroy(cf_ctx* ctx) {
     ctx->scratch0.release();
     ctx->scratch1.release();
     ctx->scratch2.release();
+    ctx->trainWorkspace.reset();
+    ctx->nodeTables.reset();
     for (hipEvent_t e : ctx->launchDone) (void)hipEventDestroy(e);
     for (hipEvent_t e : ctx->copyDone) (void)hipEventDestroy(e);
     if (ctx->hostStage) (void)hipHostFree(ctx->hostStage);
@@ -494,12 +503,11 @@ int cf_generate_features(cf_ctx* ctx, cf_images* im, const cf_sample* samples, i
         DevBuf<cf_sample> dS(n);
         CF_HIP(hipMemcpyAsync(dS.get(), samples, static_cast<size_t>(n) * sizeof(cf_sample), hipMemcpyHostToDevice,
                 ctx->stream));
-        FeatGenJob j{dS.get(), n, seed, 0, 0};
+        FeatGenJob j{dS.get(), n, seed, 0};
         DevBuf<FeatGenJob> dJ(1);
         CF_HIP(hipMemcpyAsync(dJ.get(), &j, sizeof(j), hipMemcpyHostToDevice, ctx->stream));
-        FeatTables tabs;
-        launchFeatureGeneration(ctx->stream, im->set(), dJ.get(), 1, F, T, boxRadius, regionSize, useDepth, &seed, tabs,
-                true);
+        FeatTables& tabs = nodeTables(ctx);
+        launchFeatureGeneration(ctx->stream, im->set(), dJ.get(), 1, F, T, boxRadius, regionSize, useDepth, tabs, true);
         CF_HIP(hipMemcpyAsync(featuresOut, tabs.soa.get(), static_cast<size_t>(F) * kFeatParams, hipMemcpyDeviceToHost,
                 ctx->stream));
         CF_HIP(hipMemcpyAsync(thresholdsOut, tabs.thrTF.get(), static_cast<size_t>(F) * T * sizeof(float),
@@ -562,7 +570,7 @@ int cf_node_counters(cf_ctx* ctx, cf_images* im, const cf_sample* samples, int n
         require(n > 0 && F > 0 && T > 0 && C > 0 && C <= kMaxClasses, "invalid sizes");
         checkSamples(im, samples, n);
         for (int i = 0; i < n; i++) require(samples[i].label < C, "sample label >= number of classes");
-        FeatTables tabs;
+        FeatTables& tabs = nodeTables(ctx);
         uploadFeaturesSoA(ctx, tabs, features, thresholds, F, T);
         DevBuf<cf_sample> dS;
         DevBuf<Chunk> dC;
@@ -584,7 +592,7 @@ int cf_node_best_split(cf_ctx* ctx, cf_images* im, const cf_sample* samples, int
         require(n > 0 && F > 0 && T > 0 && C > 0 && C <= kMaxClasses, "invalid sizes");
         checkSamples(im, samples, n);
         for (int i = 0; i < n; i++) require(samples[i].label < C, "sample label >= number of classes");
-        FeatTables tabs;
+        FeatTables& tabs = nodeTables(ctx);
         uploadFeaturesSoA(ctx, tabs, features, thresholds, F, T);
         DevBuf<cf_sample> dS;
         DevBuf<Chunk> dC;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -73,11 +74,44 @@ public:
     T* get() const { return p_; }
     size_t size() const { return n_; }
     size_t bytes() const { return n_ * sizeof(T); }
+    size_t capacityBytes() const { return cap_ * sizeof(T); }
 
 private:
     T* p_ = nullptr;
     size_t n_ = 0, cap_ = 0;
 };
+
+// Owning page-locked host buffer.
+class PinnedBuf {
+public:
+    PinnedBuf() = default;
+    ~PinnedBuf() { release(); }
+    PinnedBuf(const PinnedBuf&) = delete;
+    PinnedBuf& operator=(const PinnedBuf&) = delete;
+    // grows (never shrinks) the allocation; contents are not preserved
+    uint8_t* resize(size_t n) {
+        if (n > cap_) {
+            release();
+            CF_HIP(hipHostMalloc(reinterpret_cast<void**>(&p_), n, hipHostMallocDefault));
+            cap_ = n;
+        }
+        return p_;
+    }
+    void release() {
+        if (p_) (void)hipHostFree(p_);
+        p_ = nullptr;
+        cap_ = 0;
+    }
+    uint8_t* get() const { return p_; }
+    size_t capacityBytes() const { return cap_; }
+
+private:
+    uint8_t* p_ = nullptr;
+    size_t cap_ = 0;
+};
+
+struct TrainWorkspace;   // trainer.cpp
+struct FeatTables;
 
 // Uniform-size image set: image i's planes start at col + i*3*W*H and dep + i*W*H.
 struct ImageSet {
@@ -101,6 +135,10 @@ struct cf_ctx {
     bool profiling = false;
     // scratch buffers reused across calls
     cf::DevBuf<uint8_t> scratch0, scratch1, scratch2;
+    // device and page-locked memory of training calls, kept between them (bounded: trainer.cpp)
+    std::shared_ptr<cf::TrainWorkspace> trainWorkspace;
+    // feature tables of the calls on one node (at most about 60 MB)
+    std::shared_ptr<cf::FeatTables> nodeTables;
 };
 
 struct cf_images {
@@ -133,7 +171,6 @@ struct FeatGenJob {
     int n;                    // number of samples
     int seed;                 // seed of the level's RandomSource
     int outOffset;            // feature slot offset (tree * F)
-    int pad;
 };
 
 // A feature generation job's place in its candidates and its stream of sample-index draws (absolute draw
@@ -169,16 +206,15 @@ struct FeatTables {
     DevBuf<FeatRec> unsortedFeat;
     DevBuf<float> unsortedThr;
     DevBuf<int> unsortedKey;
-    DevBuf<int> err;
     // the walk over the draws (k_features.hip)
     DevBuf<uint8_t> walkSpace;
+    PinnedBuf walkHost;
     float meanDraws = 0;       // draws per candidate in the last generation (0: none yet)
     int trees = 0, F = 0, T = 0;
 };
 
 void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJob* jobsDev, int numJobs,
-        int F, int T, int boxRadius, int regionSize, int useDepth, const int* seedsHost, FeatTables& tabs,
-        bool referenceLayouts = false);
+        int F, int T, int boxRadius, int regionSize, int useDepth, FeatTables& tabs, bool referenceLayouts = false);
 // thresholds given in reference layout [trees][T][F] + features SoA [trees][11][F] -> tables
 void launchPrepareTables(hipStream_t s, int trees, int F, int T, FeatTables& tabs);
 
@@ -277,9 +313,9 @@ void evalTunerRecord(int TM, size_t entries, int shape, double ms, double respon
 // padded threshold width of the evaluation kernels for T thresholds
 int binThresholdWidth(int T);
 // G[slot][ng * 16][T + 1][C] from the bin rows of the chunks' samples
-// (samples still set to Both also count their flipped row at flipOffset)
+// (samples still set to Both also count their flipped row at flipOffset; the chunks' slots count from slotBase)
 void launchHistBins(hipStream_t s, const uint4* bins, const uint8_t* labels, const Chunk* chunks, int numChunks,
-        int g0, int ng, const FeatTables& tabs, int C, int N, uint32_t* G, size_t flipOffset = 0);
+        int slotBase, int g0, int ng, const FeatTables& tabs, int C, int N, uint32_t* G, size_t flipOffset = 0);
 // Scores and per-feature summaries of the slots' histograms.  With allScores, also every score:
 // allScores[T][F] of slot onlySlot alone, or allScores[slot][T][F] of all slots (onlySlot < 0).
 void launchScores(hipStream_t s, const uint32_t* G, const uint32_t* nodeHist, const int* slotTree, int numSlots,

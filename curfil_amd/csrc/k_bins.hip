@@ -211,8 +211,8 @@ __global__ void __launch_bounds__(WAVES * 64) k_eval_bins(const float* __restric
 // and at most 4 lanes can hit one address (all lanes counting one feature, as
 // for samples of an almost pure node, would collide on few bins).
 __global__ void __launch_bounds__(256) k_hist_bins(const uint4* __restrict__ bins, const uint8_t* __restrict__ labels,
-        const Chunk* __restrict__ chunks, int g0, int ng, int F, int T, int C, int N, uint32_t* __restrict__ G,
-        size_t flipOffset) {
+        const Chunk* __restrict__ chunks, int slotBase, int g0, int ng, int F, int T, int C, int N,
+        uint32_t* __restrict__ G, size_t flipOffset) {
     extern __shared__ uint32_t h[];
     const int chunkIdx = blockIdx.x / ng;
     const int g = blockIdx.x % ng;
@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(256) k_hist_bins(const uint4* __restrict__ bin
         }
     }
     __syncthreads();
-    uint32_t* out = G + (static_cast<size_t>(ch.slot) * ng + g) * kBinGroup * binsPerF;
+    uint32_t* out = G + (static_cast<size_t>(ch.slot - slotBase) * ng + g) * kBinGroup * binsPerF;
     for (int k = threadIdx.x; k < nb; k += 256) {
         const uint32_t v = h[k];
         if (v) atomicAdd(&out[k], v);
@@ -467,12 +467,12 @@ void launchEvalBins(hipStream_t s, const ImageSet& imgs, const cf_sample* sample
 }
 
 void launchHistBins(hipStream_t s, const uint4* bins, const uint8_t* labels, const Chunk* chunks, int numChunks,
-        int g0, int ng, const FeatTables& tabs, int C, int N, uint32_t* G, size_t flipOffset) {
+        int slotBase, int g0, int ng, const FeatTables& tabs, int C, int N, uint32_t* G, size_t flipOffset) {
     if (numChunks == 0 || ng == 0) return;
     const size_t lds = static_cast<size_t>(kBinGroup) * (tabs.T + 1) * C * sizeof(uint32_t);
     allowLds(reinterpret_cast<const void*>(&k_hist_bins), lds);
     hipLaunchKernelGGL(k_hist_bins, dim3(static_cast<unsigned>(numChunks) * ng), dim3(256), lds, s, bins, labels,
-            chunks, g0, ng, tabs.F, tabs.T, C, N, G, flipOffset);
+            chunks, slotBase, g0, ng, tabs.F, tabs.T, C, N, G, flipOffset);
 }
 
 }  // namespace cf

@@ -26,6 +26,7 @@
 // one workgroup per tree that evaluated 16 candidates a round on its own CU
 // took 15.2 ms, bound by that CU's gathers.
 #include <algorithm>
+#include <cstring>
 
 #include "cf_internal.h"
 #include "cf_rng.h"
@@ -42,7 +43,7 @@ constexpr int kPrefixDraws = 24;   // engine outputs available to one feature sa
 // g++ on x86-64 evaluates the two getNext() calls of `Offset(rgen.getNext(),
 // rgen.getNext())` right to left, so the second coordinate is drawn first
 // (pinned by the reference's golden feature hash).
-__global__ void __launch_bounds__(256) k_fg_candidates(const int* __restrict__ seeds, int numCand, int first, int count,
+__global__ void __launch_bounds__(256) k_fg_candidates(const FeatGenJob* __restrict__ jobs, int numCand, int first, int count,
         int boxRadius, int regionSize, int useDepth, FeatRec* __restrict__ cand, int* __restrict__ err) {
     constexpr int kStride = kPrefixDraws + 1;
     __shared__ uint32_t outputs[256 * kStride];
@@ -50,7 +51,7 @@ __global__ void __launch_bounds__(256) k_fg_candidates(const int* __restrict__ s
     {
         const int k = first + blockIdx.x * 64 + static_cast<int>(threadIdx.x >> 2);
         uint32_t out[kPrefixDraws];
-        mtPrefix<kPrefixDraws>(static_cast<uint32_t>(seeds[job] + 1 + 4 * k + static_cast<int>(threadIdx.x & 3)), out);
+        mtPrefix<kPrefixDraws>(static_cast<uint32_t>(jobs[job].seed + 1 + 4 * k + static_cast<int>(threadIdx.x & 3)), out);
 #pragma unroll
         for (int i = 0; i < kPrefixDraws; i++) outputs[threadIdx.x * kStride + i] = out[i];
     }
@@ -690,7 +691,7 @@ __global__ void __launch_bounds__(256) k_threshold_ranks(const float* __restrict
 }
 
 void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJob* jobsDev, int numJobs, int F,
-        int T, int boxRadius, int regionSize, int useDepth, const int* seedsHost, FeatTables& tabs, bool referenceLayouts) {
+        int T, int boxRadius, int regionSize, int useDepth, FeatTables& tabs, bool referenceLayouts) {
     if (T > kMaxThresholds) throw Error(CF_ERR_ARG, "too many thresholds (max 256)");
     if (F > 8192) throw Error(CF_ERR_ARG, "too many features (max 8192)");
     if (boxRadius > 127 || regionSize > 127) throw Error(CF_ERR_ARG, "boxRadius/regionSize must fit int8");
@@ -711,8 +712,6 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     tabs.rank.resize(static_cast<size_t>(numJobs) * F * T);
     const int TM = binThresholdWidth(T);
     tabs.thrPad.resize(static_cast<size_t>(numJobs) * F * TM);
-    tabs.err.resize(1);
-    CF_HIP(hipMemsetAsync(tabs.err.get(), 0, sizeof(int), s));
     const int band = bandDraws(T);
     const int m = std::min(kRoundTable / band, kRoundCandMax);   // candidates of a round
     int ring = 1 << 14;
@@ -726,14 +725,15 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
         bytes += (b + 255) & ~static_cast<size_t>(255);
         return at;
     };
-    const size_t oSeeds = part(n * sizeof(int)), oWalk = part(n * sizeof(WalkState)), oMt = part(n * 624 * sizeof(uint32_t)),
+    const size_t oWalk = part(n * sizeof(WalkState) + sizeof(int)), oMt = part(n * 624 * sizeof(uint32_t)),
             oRaw = part(n * maxSteps * 256 * sizeof(uint32_t)), oMasks = part(n * maxSteps * 4 * sizeof(uint64_t)),
             oRecs = part(n * ring * sizeof(DrawRec)), oResp = part(perRound * sizeof(float)),
             oNext = part(perRound * sizeof(uint16_t)), oBands = part(n * m * sizeof(int4));
     tabs.walkSpace.resize(bytes);
     uint8_t* space = tabs.walkSpace.get();
-    int* dSeeds = reinterpret_cast<int*>(space + oSeeds);
     WalkState* dWalk = reinterpret_cast<WalkState*>(space + oWalk);
+    int* dErr = reinterpret_cast<int*>(dWalk + numJobs);   // read back with the states
+    CF_HIP(hipMemsetAsync(dErr, 0, sizeof(int), s));
     uint32_t* dMt = reinterpret_cast<uint32_t*>(space + oMt);
     uint32_t* dRaw = reinterpret_cast<uint32_t*>(space + oRaw);
     unsigned long long* dMasks = reinterpret_cast<unsigned long long*>(space + oMasks);
@@ -741,17 +741,19 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     float* dResp = reinterpret_cast<float*>(space + oResp);
     uint16_t* dNext = reinterpret_cast<uint16_t*>(space + oNext);
     int4* dBands = reinterpret_cast<int4*>(space + oBands);
-    CF_HIP(hipMemcpyAsync(dSeeds, seedsHost, numJobs * sizeof(int), hipMemcpyHostToDevice, s));
     // a candidate in twenty or fewer is rejected on ordinary frames: the rest are drawn if they are needed
     auto drawCandidates = [&](int first, int count) {
         if (count > 0) {
-            hipLaunchKernelGGL(k_fg_candidates, dim3((count + 63) / 64, numJobs), dim3(256), 0, s, dSeeds, numCand, first,
-                    count, boxRadius, regionSize, useDepth, tabs.cand.get(), tabs.err.get());
+            hipLaunchKernelGGL(k_fg_candidates, dim3((count + 63) / 64, numJobs), dim3(256), 0, s, jobsDev, numCand, first,
+                    count, boxRadius, regionSize, useDepth, tabs.cand.get(), dErr);
         }
     };
     int drawn = std::min(numCand, F + F / 8 + 64);
     drawCandidates(0, drawn);
-    std::vector<WalkState> states(numJobs);
+    const size_t stateBytes = n * sizeof(WalkState) + sizeof(int);
+    uint8_t* host = tabs.walkHost.resize(stateBytes);
+    std::memset(host, 0, stateBytes);
+    const WalkState* states = reinterpret_cast<const WalkState*>(host);
     int errHost = 0;
     // draws of a candidate: the mean of these tables' last generation (the level before), or 5/4 T
     const float guess = tabs.meanDraws > 0 ? tabs.meanDraws : 1.25f * T;
@@ -760,7 +762,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     // more, they and the sort are enqueued again.
     for (bool fresh = true, more = true; more; fresh = false) {
         int missing = 0;
-        for (const WalkState& st : states) missing = std::max(missing, st.done ? 0 : F - st.generated);
+        for (int j = 0; j < numJobs; j++) missing = std::max(missing, states[j].done ? 0 : F - states[j].generated);
         // (without a table before this one to go by, the first rounds are short: a candidate's mean use is
         // only guessed)
         const int rounds = std::min(64, missing / std::max(1, m * 9 / 10) + (fresh && tabs.meanDraws > 0 ? 2 : 4));
@@ -782,13 +784,13 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
                 tabs.unsortedKey.get(), tabs.unsortedFeat.get(), tabs.unsortedThr.get(), F, T, TM, tabs.feat.get(),
                 tabs.thrFT.get(), tabs.rank.get(), tabs.thrPad.get(),
                 referenceLayouts ? tabs.thrTF.get() : nullptr, referenceLayouts ? tabs.soa.get() : nullptr);
-        CF_HIP(hipMemcpyAsync(states.data(), dWalk, numJobs * sizeof(WalkState), hipMemcpyDeviceToHost, s));
-        CF_HIP(hipMemcpyAsync(&errHost, tabs.err.get(), sizeof(int), hipMemcpyDeviceToHost, s));
+        CF_HIP(hipMemcpyAsync(host, dWalk, stateBytes, hipMemcpyDeviceToHost, s));
         CF_HIP(hipStreamSynchronize(s));
+        std::memcpy(&errHost, host + n * sizeof(WalkState), sizeof(int));
         more = false;
-        for (const WalkState& st : states) {
-            if (st.err != 0 && errHost == 0) errHost = st.err;
-            more = more || !st.done;
+        for (int j = 0; j < numJobs; j++) {
+            if (states[j].err != 0 && errHost == 0) errHost = states[j].err;
+            more = more || !states[j].done;
         }
         if (errHost != 0) break;
         if (more && drawn < numCand) {
@@ -797,9 +799,9 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
         }
     }
     double draws = 0, cands = 0;
-    for (const WalkState& st : states) {
-        draws += st.drawsDone;
-        cands += st.candsDone;
+    for (int j = 0; j < numJobs; j++) {
+        draws += states[j].drawsDone;
+        cands += states[j].candsDone;
     }
     tabs.meanDraws = cands > 0 ? static_cast<float>(draws / cands) : 0.0f;
     if (errHost == 1) throw Error(CF_ERR_RUNTIME, "failed to generate random features. max loops exceeded");

@@ -24,6 +24,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 
 #include "cf_host.h"
 
@@ -44,8 +45,9 @@ struct ActiveTree {
 // The pass-1 blocks of one block size at the current level, and the work list of a batch size.
 struct BlockSet {
     int level = -1;        // level the blocks were built for
-    DevBuf<BinBlock> blocks;
-    DevBuf<int> segInfo;   // per image group: first block, block count, blocks before it
+    // in the level's staged tables
+    const BinBlock* dBlocks = nullptr;
+    const int* dSegInfo = nullptr;   // per image group: first block, block count, blocks before it
     int numSegs = 0, numBlocks = 0;
     DevBuf<int2> work;
     int workGroups = -1;   // feature groups the work list was built for
@@ -209,6 +211,122 @@ bool isPure(const uint32_t* h, int C) {
     return nz == 1;
 }
 
+// Small host tables on their way to the device: put() copies one into page-locked memory and returns where it
+// will lie on the device, flush() enqueues the copies (one per block, in practice one).  reset() when the
+// copies and the kernels that read them are done.
+class StageArena {
+public:
+    void reset() {
+        if (blocks_.size() > 1) {   // one block of the size that was needed
+            size_t n = 0;
+            for (const auto& b : blocks_) n += b->cap;
+            blocks_.clear();
+            addBlock(n);
+        }
+        for (auto& b : blocks_) b->used = b->flushed = 0;
+    }
+    template<class V>
+    V* put(const V* p, size_t n) {
+        const size_t bytes = (n * sizeof(V) + 255) & ~static_cast<size_t>(255);
+        if (blocks_.empty() || blocks_.back()->used + bytes > blocks_.back()->cap) addBlock(bytes);
+        Block& b = *blocks_.back();
+        V* d = reinterpret_cast<V*>(b.dev.get() + b.used);
+        if (n > 0) std::memcpy(b.host.get() + b.used, p, n * sizeof(V));
+        b.used += bytes;
+        return d;
+    }
+    template<class V>
+    V* put(const std::vector<V>& v) { return put(v.data(), v.size()); }
+    void flush(hipStream_t s) {
+        for (auto& b : blocks_) {
+            if (b->used == b->flushed) continue;
+            CF_HIP(hipMemcpyAsync(b->dev.get() + b->flushed, b->host.get() + b->flushed, b->used - b->flushed,
+                    hipMemcpyHostToDevice, s));
+            b->flushed = b->used;
+        }
+    }
+    void release() { blocks_.clear(); }
+    size_t capacityBytes() const {
+        size_t n = 0;
+        for (const auto& b : blocks_) n += b->cap;
+        return n;
+    }
+
+private:
+    struct Block {
+        PinnedBuf host;
+        DevBuf<uint8_t> dev;
+        size_t cap = 0, used = 0, flushed = 0;
+    };
+    void addBlock(size_t bytes) {
+        auto b = std::make_unique<Block>();
+        b->cap = std::max<size_t>(bytes, 256 * 1024);
+        b->host.resize(b->cap);
+        b->dev.resize(b->cap);
+        blocks_.push_back(std::move(b));
+    }
+    std::vector<std::unique_ptr<Block>> blocks_;
+};
+
+}  // namespace
+
+// What a training call allocates.  It stays with the context for the next call (hipMalloc and hipFree took 7.6
+// of 22 ms of a small training: 13 flipped frames of 320x240, 2 trees, 500 x 50), under the context's mutex, on
+// the context's stream; contents never carry over.  After a call the buffers over kKeepBytes in all are given
+// back, the largest first; the rest with the context.
+struct TrainWorkspace {
+    static constexpr size_t kKeepBytes = size_t{1} << 30;
+    DevBuf<cf_sample> level[2];
+    DevBuf<uint8_t> dir;
+    FeatTables tabs;
+    DevBuf<int2> graphWork[2];   // work lists of a captured level: full and last feature-group batch
+    DevBuf<uint32_t> G;
+    DevBuf<FeatSummary> summ, repSumm;
+    DevBuf<double> allScores;
+    DevBuf<NodeBest> repBest;
+    DevBuf<uint32_t> keys, vals, perm, sortCount, sortCursor, sortBlocks;
+    DevBuf<uint8_t> lab8;
+    std::map<int, BlockSet> blockSets;   // by pass-1 block size
+    DevBuf<int> starts;
+    DevBuf<uint4> bins;
+    DevBuf<uint8_t> results;     // a level's argmax, split records, chunk counts and left histograms
+    PinnedBuf hostResults, hostStarts;
+    StageArena arena[2];         // by level parity
+
+    template<class Fn>
+    void each(Fn&& fn) {
+        fn(level[0]); fn(level[1]); fn(dir); fn(graphWork[0]); fn(graphWork[1]); fn(G); fn(summ); fn(repSumm);
+        fn(allScores); fn(repBest); fn(keys); fn(vals); fn(perm); fn(sortCount); fn(sortCursor); fn(sortBlocks);
+        fn(lab8); fn(starts); fn(bins); fn(results); fn(hostResults); fn(hostStarts); fn(arena[0]); fn(arena[1]);
+        fn(tabs.feat); fn(tabs.thrFT); fn(tabs.thrTF); fn(tabs.rank); fn(tabs.thrPad); fn(tabs.soa); fn(tabs.cand);
+        fn(tabs.unsortedFeat); fn(tabs.unsortedThr); fn(tabs.unsortedKey); fn(tabs.walkSpace); fn(tabs.walkHost);
+        for (auto& kv : blockSets) fn(kv.second.work);
+    }
+    void trim() {
+        for (;;) {
+            size_t sum = 0, most = 0;
+            each([&](auto& b) {
+                sum += b.capacityBytes();
+                most = std::max(most, b.capacityBytes());
+            });
+            if (sum <= kKeepBytes) return;
+            each([&](auto& b) {
+                if (b.capacityBytes() == most) b.release();
+            });
+        }
+    }
+};
+
+namespace {
+// the workspace of one call, trimmed at its end (also when the call throws: after its enqueued work)
+struct WorkspaceUse {
+    TrainWorkspace& ws;
+    hipStream_t s;
+    ~WorkspaceUse() {
+        (void)hipStreamSynchronize(s);
+        ws.trim();
+    }
+};
 }  // namespace
 
 void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int C, std::vector<TreeJob>& jobs,
@@ -232,10 +350,14 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
     // a Both sample splits at most once into a NoFlip sample and a Flip copy, which
     // never split again: a level holds at most twice the root samples
     const size_t capacity = std::max<size_t>(anyBoth ? 2 * total : total, 1);
-    DevBuf<cf_sample> level[2];
+    if (!ctx->trainWorkspace) ctx->trainWorkspace = std::make_shared<TrainWorkspace>();
+    TrainWorkspace& ws = *ctx->trainWorkspace;
+    WorkspaceUse use{ws, s};
+    DevBuf<cf_sample>* level = ws.level;
     level[0].resize(capacity);
     level[1].resize(capacity);
-    DevBuf<uint8_t> dir(capacity);
+    DevBuf<uint8_t>& dir = ws.dir;
+    dir.resize(capacity);
 
     std::vector<ActiveTree> active;
     {
@@ -280,33 +402,22 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
     const bool twoPass = mode == CF_MODE_BATCHED && T <= kMaxBinThresholds &&
             std::getenv("CURFIL_EVAL_DIRECT") == nullptr;
 
-    FeatTables tabs;
-    DevBuf<FeatGenJob> dJobs;
-    DevBuf<Chunk> dChunks;
-    DevBuf<int2> dGraphWork[2];   // work lists of a captured level: full and last feature-group batch
-    DevBuf<uint32_t> dNodeHist;
-    DevBuf<int> dSlotTree;
-    DevBuf<uint32_t> dG;
-    DevBuf<FeatSummary> dSumm;
-    DevBuf<NodeBest> dBest;
-    DevBuf<double> dAllScores;
-    DevBuf<SplitRec> dSplits;
-    DevBuf<NodeBest> dBestAll;
-    DevBuf<int> dNodeTree;
-    DevBuf<int2> dChunkCounts;
-    DevBuf<uint32_t> dLeftHist;
-    DevBuf<int2> dDst;
-    DevBuf<uint32_t> dKeys, dVals, dPerm, dSortCount, dSortCursor, dSortBlocks;
-    DevBuf<uint8_t> dLab8;
-    std::map<int, BlockSet> blockSets;   // by pass-1 block size
+    FeatTables& tabs = ws.tabs;
+    tabs.meanDraws = 0;
+    DevBuf<int2>* dGraphWork = ws.graphWork;
+    DevBuf<uint32_t>& dG = ws.G;
+    DevBuf<FeatSummary>& dSumm = ws.summ;
+    DevBuf<FeatSummary>& dRepSumm = ws.repSumm;
+    DevBuf<double>& dAllScores = ws.allScores;
+    DevBuf<NodeBest>& dRepBest = ws.repBest;
+    DevBuf<uint32_t>&dKeys = ws.keys, &dVals = ws.vals, &dPerm = ws.perm, &dSortCount = ws.sortCount,
+            &dSortCursor = ws.sortCursor, &dSortBlocks = ws.sortBlocks;
+    DevBuf<uint8_t>& dLab8 = ws.lab8;
+    std::map<int, BlockSet>& blockSets = ws.blockSets;
     EventPair tuneEvents;
     const hipEvent_t tuneStart = tuneEvents.a, tuneEnd = tuneEvents.b;
-    DevBuf<uint32_t> dRepHist;
-    DevBuf<int> dRepTree;
-    DevBuf<FeatSummary> dRepSumm;
-    DevBuf<NodeBest> dRepBest;
-    DevBuf<int> dStarts;
-    DevBuf<uint4> dBins;
+    DevBuf<int>& dStarts = ws.starts;
+    DevBuf<uint4>& dBins = ws.bins;
     const size_t binsBudget = binsBudgetBytes();
     // CURFIL_LEVEL_GRAPH=1: levels whose pass-1 shape is settled run as one captured graph.  Off by default:
     // once a graph has been instantiated the HIP runtime holds one of the process's hardware queues
@@ -327,28 +438,22 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
         if (levelNr == cfg.max_depth) break;
         stats.levels++;
         const int numActive = static_cast<int>(active.size());
-        // ---- feature generation, one job per tree
-        std::vector<int> seeds(numActive);
+        // the level before the last has been read back, and with it everything that its tables fed
+        StageArena& up = ws.arena[levelNr & 1];
+        up.reset();
+        // ---- feature generation jobs, one per tree
         std::vector<FeatGenJob> fj(numActive);
         for (int a = 0; a < numActive; a++) {
-            seeds[a] = jobs[active[a].job].rs.uniformSampler(0xFFFFFF).next();
             fj[a].samples = level[cur].get() + active[a].begin;
             fj[a].n = active[a].n;
-            fj[a].seed = seeds[a];
+            fj[a].seed = jobs[active[a].job].rs.uniformSampler(0xFFFFFF).next();
             fj[a].outOffset = a * F;
-            fj[a].pad = 0;
         }
-        dJobs.resize(numActive);
-        CF_HIP(hipMemcpyAsync(dJobs.get(), fj.data(), numActive * sizeof(FeatGenJob), hipMemcpyHostToDevice, s));
-        timer.begin();
-        launchFeatureGeneration(s, images->set(), dJobs.get(), numActive, F, T, cfg.box_radius, cfg.region_size,
-                cfg.use_depth_images, seeds.data(), tabs);
-        timer.end(stats.featGenMs);
-
         // ---- nodes and chunks of the level (slot = position in `nodes`)
         std::vector<LevelNode> nodes;
         std::vector<Chunk> chunks;
-        std::vector<int> chunkSlotTree;
+        std::vector<uint32_t> nodeHist;   // class histograms and trees of the level's nodes
+        std::vector<int> nodeTree;
         for (int a = 0; a < numActive; a++) {
             int off = active[a].begin;
             for (size_t k = 0; k < active[a].nodes.size(); k++) {
@@ -358,25 +463,84 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 ln.begin = off;
                 ln.count = active[a].counts[k];
                 ln.chunkBegin = static_cast<int>(chunks.size());
-                for (int b = 0; b < ln.count; b += kChunk) {
-                    Chunk c;
-                    c.slot = static_cast<int>(nodes.size());
-                    c.tree = a;
-                    c.begin = off + b;
-                    c.count = std::min(kChunk, ln.count - b);
-                    chunks.push_back(c);
-                }
+                appendChunks(chunks, ln, static_cast<int>(nodes.size()), kChunk);
                 ln.chunkEnd = static_cast<int>(chunks.size());
                 off += ln.count;
                 nodes.push_back(ln);
+                const uint32_t* h = &out[active[a].job].hist[static_cast<size_t>(ln.node) * C];
+                nodeHist.insert(nodeHist.end(), h, h + C);
+                nodeTree.push_back(a);
                 stats.evaluations += static_cast<double>(ln.count) * F * T;
                 stats.responses += static_cast<double>(ln.count) * F;
                 stats.nodes += 1;
             }
         }
+        const FeatGenJob* dJobs = up.put(fj);
+        const Chunk* dChunks = up.put(chunks);
+        const uint32_t* dNodeHist = up.put(nodeHist);
+        const int* dNodeTree = up.put(nodeTree);
+        up.flush(s);
         const int numNodes = static_cast<int>(nodes.size());
-        std::vector<NodeBest> best(numNodes);
+        const int numChunks = static_cast<int>(chunks.size());
         const double evalMsBefore = stats.evalKernelMs;
+        // what the host reads of a level, in one buffer: split record and argmax per node, left and right
+        // entries per chunk, left class histogram per node
+        const size_t splitsAt = 0, bestAt = splitsAt + numNodes * sizeof(SplitRec),
+                countsAt = bestAt + numNodes * sizeof(NodeBest), histAt = countsAt + numChunks * sizeof(int2),
+                resultBytes = histAt + static_cast<size_t>(numNodes) * C * sizeof(uint32_t);
+        static_assert(sizeof(SplitRec) % 8 == 0 && sizeof(NodeBest) % 8 == 0, "alignment of the parts that follow");
+        ws.results.resize(resultBytes + 16);
+        NodeBest* dBest = reinterpret_cast<NodeBest*>(ws.results.get() + bestAt);
+        SplitRec* dSplits = reinterpret_cast<SplitRec*>(ws.results.get() + splitsAt);
+        int2* dChunkCounts = reinterpret_cast<int2*>(ws.results.get() + countsAt);
+        uint32_t* dLeftHist = reinterpret_cast<uint32_t*>(ws.results.get() + histAt);
+        uint8_t* hostResults = ws.hostResults.resize(resultBytes + 16);
+        NodeBest* best = reinterpret_cast<NodeBest*>(hostResults + bestAt);
+
+        // image-major order of a level that is evaluated in two passes; the segments' starts are read at the
+        // feature generation's wait
+        int N = 0, M = 0, numKeys = 0;
+        auto sortLevel = [&]() {
+            for (int a = 0; a < numActive; a++) N = std::max(N, active[a].begin + active[a].n);
+            // image-major order of the level: (image, tree, place) keys, counting sort of level indices.
+            // With Both samples a second entry per level index evaluates it flipped; the entries of samples
+            // that are not Both get the key one past the last (tree, image) and sort to the end.
+            M = anyBoth ? 2 * N : N;
+            dKeys.resize(M);
+            dVals.resize(M);
+            dPerm.resize(M);
+            dLab8.resize(N);
+            const uint64_t keyRange = static_cast<uint64_t>(numActive) * static_cast<uint64_t>(images->count);
+            if (keyRange >= (1ull << 27)) throw Error(CF_ERR_UNSUPPORTED, "too many (tree, image) segments in one level");
+            // within a segment, samples ordered by place while the buckets stay below 2^26 (CURFIL_ROW_ORDER=0: off)
+            int placeBits = 0;
+            while ((1 << placeBits) < levelPlaces(images->W, images->H)) placeBits++;
+            const char* rowOrder = std::getenv("CURFIL_ROW_ORDER");
+            if (((keyRange + 2) << placeBits) > (1ull << 26) || (rowOrder && std::strcmp(rowOrder, "0") == 0)) placeBits = 0;
+            // segments (image, tree) in image-major order: the trees' segments of one image are adjacent
+            for (int a = 0; a < numActive; a++) {
+                launchLevelKeys(s, level[cur].get(), active[a].begin, active[a].n, static_cast<uint32_t>(a),
+                        static_cast<uint32_t>(numActive), dKeys.get(), dVals.get(), anyBoth ? N : 0,
+                        static_cast<uint32_t>(keyRange), placeBits, images->H);
+            }
+            numKeys = static_cast<int>(keyRange);
+            dSortCount.resize(levelSortBuckets(numKeys, placeBits));
+            dSortCursor.resize(levelSortBuckets(numKeys, placeBits));
+            dSortBlocks.resize(levelSortScanBlocks(numKeys, placeBits));
+            dStarts.resize(numKeys + 1);
+            levelCountingSort(s, dKeys.get(), dVals.get(), M, numKeys, placeBits, dSortCount.get(), dSortCursor.get(),
+                    dSortBlocks.get(), dPerm.get(), dStarts.get());
+            launchLevelLabels(s, level[cur].get(), N, dLab8.get());
+            int* hostStarts = reinterpret_cast<int*>(ws.hostStarts.resize((static_cast<size_t>(numKeys) + 1) * sizeof(int)));
+            CF_HIP(hipMemcpyAsync(hostStarts, dStarts.get(), (static_cast<size_t>(numKeys) + 1) * sizeof(int),
+                    hipMemcpyDeviceToHost, s));
+        };
+        if (twoPass) sortLevel();
+
+        timer.begin();
+        launchFeatureGeneration(s, images->set(), dJobs, numActive, F, T, cfg.box_radius, cfg.region_size,
+                cfg.use_depth_images, tabs);
+        timer.end(stats.featGenMs);
 
         // ---- evaluation
         auto evalSlots = [&](int s0, int s1) {
@@ -386,45 +550,29 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             const int per = evalChunkSamples(slotSamples, F);
             std::vector<Chunk> bc;
             for (int i = s0; i < s1; i++) appendChunks(bc, nodes[i], i - s0, per);
-            std::vector<uint32_t> nh(static_cast<size_t>(ns) * C);
-            std::vector<int> st(ns);
-            for (int i = 0; i < ns; i++) {
-                const LevelNode& ln = nodes[s0 + i];
-                std::memcpy(&nh[static_cast<size_t>(i) * C], &out[active[ln.active].job].hist[static_cast<size_t>(ln.node) * C],
-                        C * sizeof(uint32_t));
-                st[i] = ln.active;
-            }
-            dChunks.resize(bc.size());
-            dNodeHist.resize(nh.size());
-            dSlotTree.resize(ns);
+            const Chunk* dEval = up.put(bc);
+            up.flush(s);
+            const uint32_t* slotHist = dNodeHist + static_cast<size_t>(s0) * C;
             dG.resize(static_cast<size_t>(ns) * perSlot);
             dSumm.resize(static_cast<size_t>(ns) * F);
-            dBest.resize(ns);
-            CF_HIP(hipMemcpyAsync(dChunks.get(), bc.data(), bc.size() * sizeof(Chunk), hipMemcpyHostToDevice, s));
-            CF_HIP(hipMemcpyAsync(dNodeHist.get(), nh.data(), nh.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-            CF_HIP(hipMemcpyAsync(dSlotTree.get(), st.data(), ns * sizeof(int), hipMemcpyHostToDevice, s));
             CF_HIP(hipMemsetAsync(dG.get(), 0, static_cast<size_t>(ns) * perSlot * sizeof(uint32_t), s));
             timer.begin();
-            launchEvalHistograms(s, images->set(), level[cur].get(), dChunks.get(), static_cast<int>(bc.size()),
-                    tabs, C, dG.get());
+            launchEvalHistograms(s, images->set(), level[cur].get(), dEval, static_cast<int>(bc.size()), tabs, C, dG.get());
             timer.end(stats.evalKernelMs);
             stats.evalLaunches += 1;
             timer.begin();
-            launchScores(s, dG.get(), dNodeHist.get(), dSlotTree.get(), ns, tabs, C, dSumm.get(), nullptr, -1);
-            launchReduce(s, dSumm.get(), ns, F, dBest.get());
+            launchScores(s, dG.get(), slotHist, dNodeTree + s0, ns, tabs, C, dSumm.get(), nullptr, -1);
+            launchReduce(s, dSumm.get(), ns, F, dBest + s0);
             timer.end(stats.scoreMs);
-            CF_HIP(hipMemcpyAsync(&best[s0], dBest.get(), ns * sizeof(NodeBest), hipMemcpyDeviceToHost, s));
+            CF_HIP(hipMemcpyAsync(&best[s0], dBest + s0, ns * sizeof(NodeBest), hipMemcpyDeviceToHost, s));
             CF_HIP(hipStreamSynchronize(s));
             timer.flush();
             for (int i = 0; i < ns; i++) {
                 if (!best[s0 + i].flag) continue;
                 // near-tie band: replay the reference's sequential scan for this node
                 dAllScores.resize(static_cast<size_t>(T) * F);
-                launchScores(s, dG.get(), dNodeHist.get(), dSlotTree.get(), ns, tabs, C, dSumm.get(), dAllScores.get(), i);
-                launchSequentialArgmax(s, dAllScores.get(), T, F, dBest.get() + i);
-                CF_HIP(hipMemcpyAsync(&best[s0 + i], dBest.get() + i, sizeof(NodeBest), hipMemcpyDeviceToHost, s));
-                CF_HIP(hipStreamSynchronize(s));
-                timer.flush();
+                launchScores(s, dG.get(), slotHist, dNodeTree + s0, ns, tabs, C, dSumm.get(), dAllScores.get(), i);
+                launchSequentialArgmax(s, dAllScores.get(), T, F, dBest + s0 + i);
                 stats.replays++;
             }
         };
@@ -446,68 +594,31 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                             &out[active[ln.active].job].hist[static_cast<size_t>(ln.node) * C], C * sizeof(uint32_t));
                     st[k] = ln.active;
                 }
-                dChunks.resize(bc.size());
+                const Chunk* dRepChunks = up.put(bc);
+                const uint32_t* dRepHist = up.put(nh);
+                const int* dRepTree = up.put(st);
+                up.flush(s);
                 dG.resize(static_cast<size_t>(ns) * perSlot);
                 dAllScores.resize(static_cast<size_t>(ns) * T * F);
-                dRepHist.resize(nh.size());
-                dRepTree.resize(ns);
                 dRepSumm.resize(static_cast<size_t>(ns) * F);
                 dRepBest.resize(ns);
-                CF_HIP(hipMemcpyAsync(dChunks.get(), bc.data(), bc.size() * sizeof(Chunk), hipMemcpyHostToDevice, s));
-                CF_HIP(hipMemcpyAsync(dRepHist.get(), nh.data(), nh.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-                CF_HIP(hipMemcpyAsync(dRepTree.get(), st.data(), ns * sizeof(int), hipMemcpyHostToDevice, s));
                 CF_HIP(hipMemsetAsync(dG.get(), 0, static_cast<size_t>(ns) * perSlot * sizeof(uint32_t), s));
-                launchEvalHistograms(s, images->set(), level[cur].get(), dChunks.get(), static_cast<int>(bc.size()),
-                        tabs, C, dG.get());
-                launchScores(s, dG.get(), dRepHist.get(), dRepTree.get(), ns, tabs, C, dRepSumm.get(), dAllScores.get(),
-                        -1);
+                launchEvalHistograms(s, images->set(), level[cur].get(), dRepChunks, static_cast<int>(bc.size()), tabs, C,
+                        dG.get());
+                launchScores(s, dG.get(), dRepHist, dRepTree, ns, tabs, C, dRepSumm.get(), dAllScores.get(), -1);
                 launchSequentialArgmax(s, dAllScores.get(), T, F, dRepBest.get(), ns);
-                std::vector<NodeBest> rb(ns);
-                CF_HIP(hipMemcpyAsync(rb.data(), dRepBest.get(), ns * sizeof(NodeBest), hipMemcpyDeviceToHost, s));
-                CF_HIP(hipStreamSynchronize(s));
-                timer.flush();
-                for (int k = 0; k < ns; k++) best[flagged[a + k]] = rb[k];
+                for (int k = 0; k < ns; k++) {
+                    CF_HIP(hipMemcpyAsync(dBest + flagged[a + k], dRepBest.get() + k, sizeof(NodeBest),
+                            hipMemcpyDeviceToDevice, s));
+                }
                 stats.replays += ns;
                 a += ns;
             }
         };
         auto evalTwoPass = [&]() {
-            int N = 0;
-            for (int a = 0; a < numActive; a++) N = std::max(N, active[a].begin + active[a].n);
-            // image-major order of the level: (image, tree, place) keys, counting sort of level indices.
-            // With Both samples a second entry per level index evaluates it flipped; the entries of samples
-            // that are not Both get the key one past the last (tree, image) and sort to the end.
-            const int M = anyBoth ? 2 * N : N;
-            dKeys.resize(M);
-            dVals.resize(M);
-            dPerm.resize(M);
-            dLab8.resize(N);
-            const uint64_t keyRange = static_cast<uint64_t>(numActive) * static_cast<uint64_t>(images->count);
-            if (keyRange >= (1ull << 27)) throw Error(CF_ERR_UNSUPPORTED, "too many (tree, image) segments in one level");
-            // within a segment, samples ordered by place while the buckets stay below 2^26 (CURFIL_ROW_ORDER=0: off)
-            int placeBits = 0;
-            while ((1 << placeBits) < levelPlaces(images->W, images->H)) placeBits++;
-            const char* rowOrder = std::getenv("CURFIL_ROW_ORDER");
-            if (((keyRange + 2) << placeBits) > (1ull << 26) || (rowOrder && std::strcmp(rowOrder, "0") == 0)) placeBits = 0;
-            // segments (image, tree) in image-major order: the trees' segments of one image are adjacent
-            for (int a = 0; a < numActive; a++) {
-                launchLevelKeys(s, level[cur].get(), active[a].begin, active[a].n, static_cast<uint32_t>(a),
-                        static_cast<uint32_t>(numActive), dKeys.get(), dVals.get(), anyBoth ? N : 0,
-                        static_cast<uint32_t>(keyRange), placeBits, images->H);
-            }
-            const int numKeys = static_cast<int>(keyRange);
-            dSortCount.resize(levelSortBuckets(numKeys, placeBits));
-            dSortCursor.resize(levelSortBuckets(numKeys, placeBits));
-            dSortBlocks.resize(levelSortScanBlocks(numKeys, placeBits));
-            dStarts.resize(numKeys + 1);
-            levelCountingSort(s, dKeys.get(), dVals.get(), M, numKeys, placeBits, dSortCount.get(), dSortCursor.get(),
-                    dSortBlocks.get(), dPerm.get(), dStarts.get());
-            launchLevelLabels(s, level[cur].get(), N, dLab8.get());
             // (image, tree) segments of the sorted order -> blocks of <= kBinBlockSamples samples within a segment;
             // the segments of one image form a group of consecutive blocks
-            std::vector<int> starts(numKeys + 1);
-            CF_HIP(hipMemcpyAsync(starts.data(), dStarts.get(), (numKeys + 1) * sizeof(int), hipMemcpyDeviceToHost, s));
-            CF_HIP(hipStreamSynchronize(s));
+            int* starts = reinterpret_cast<int*>(ws.hostStarts.get());
             timer.flush();
             if (starts[numKeys] < 0) starts[numKeys] = M;   // the end of the last segment
             // blocks of one pass-1 block size: consecutive runs of <= blockSamples entries within a (image, tree)
@@ -542,11 +653,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                     }
                     k = k2;
                 }
-                bs.blocks.resize(std::max<size_t>(blocks.size(), 1));
-                if (!blocks.empty()) {
-                    CF_HIP(hipMemcpyAsync(bs.blocks.get(), blocks.data(), blocks.size() * sizeof(BinBlock),
-                            hipMemcpyHostToDevice, s));
-                }
+                bs.dBlocks = up.put(blocks);
                 bs.numSegs = static_cast<int>(segBlocks.size());
                 bs.numBlocks = static_cast<int>(blocks.size());
                 std::vector<int> segInfo(3 * static_cast<size_t>(bs.numSegs), 0);
@@ -556,9 +663,8 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                     segInfo[2 * static_cast<size_t>(bs.numSegs) + i] = before;
                     before += segBlocks[i].second;
                 }
-                bs.segInfo.resize(std::max<size_t>(segInfo.size(), 1));
-                CF_HIP(hipMemcpyAsync(bs.segInfo.get(), segInfo.data(), segInfo.size() * sizeof(int),
-                        hipMemcpyHostToDevice, s));
+                bs.dSegInfo = up.put(segInfo);
+                up.flush(s);
                 return bs;
             };
             // the work list of a batch of ngb feature groups into `work`; returns its length
@@ -566,7 +672,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 const int numWork = buildWorkLength(bs.numBlocks, ngb);
                 work.resize(std::max<size_t>(static_cast<size_t>(numWork), 1));
                 const int ns = bs.numSegs;
-                launchBuildWork(s, bs.segInfo.get(), bs.segInfo.get() + ns, bs.segInfo.get() + 2 * ns, ns, bs.numBlocks, ngb,
+                launchBuildWork(s, bs.dSegInfo, bs.dSegInfo + ns, bs.dSegInfo + 2 * ns, ns, bs.numBlocks, ngb,
                         work.get());
                 return numWork;
             };
@@ -575,21 +681,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 bs.workGroups = ngb;
                 bs.numWork = buildWork(bs, ngb, bs.work);
             };
-            // node histograms and trees of the whole level
-            std::vector<uint32_t> nh(static_cast<size_t>(numNodes) * C);
-            std::vector<int> st(numNodes);
-            for (int i = 0; i < numNodes; i++) {
-                const LevelNode& ln = nodes[i];
-                std::memcpy(&nh[static_cast<size_t>(i) * C],
-                        &out[active[ln.active].job].hist[static_cast<size_t>(ln.node) * C], C * sizeof(uint32_t));
-                st[i] = ln.active;
-            }
-            dNodeHist.resize(nh.size());
-            dSlotTree.resize(numNodes);
             dSumm.resize(static_cast<size_t>(numNodes) * F);
-            dBest.resize(numNodes);
-            CF_HIP(hipMemcpyAsync(dNodeHist.get(), nh.data(), nh.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-            CF_HIP(hipMemcpyAsync(dSlotTree.get(), st.data(), numNodes * sizeof(int), hipMemcpyHostToDevice, s));
             // feature groups in batches that fit the bin-row budget; node slots in batches that fit the histogram budget
             const int groupsTotal = (F + kBinGroup - 1) / kBinGroup;
             // a group's rows: one per level index, and a second (flipped) one with Both samples
@@ -628,8 +720,6 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 const int numWorkLast = lastNgb == ng ? numWorkFull : buildWork(bs, lastNgb, dGraphWork[1]);
                 bs.workGroups = -1;
                 std::vector<Batch> batches;
-                std::vector<Chunk> allChunks;
-                std::vector<size_t> chunkOff;   // per (batch, slot batch), in order
                 size_t maxG = 1;
                 for (int g0 = 0; g0 < groupsTotal; g0 += ng) {
                     const int ngb = std::min(ng, groupsTotal - g0);
@@ -637,27 +727,15 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                             slotBatches(ngb)};
                     const size_t perSlotB = static_cast<size_t>(ngb) * kBinGroup * (T + 1) * C;
                     for (const auto& sb : b.slots) {
-                        chunkOff.push_back(allChunks.size());
-                        for (int c = nodes[sb.first].chunkBegin; c < nodes[sb.second - 1].chunkEnd; c++) {
-                            Chunk ch = chunks[c];
-                            ch.slot -= sb.first;
-                            allChunks.push_back(ch);
-                        }
                         maxG = std::max(maxG, static_cast<size_t>(sb.second - sb.first) * perSlotB);
                     }
                     batches.push_back(std::move(b));
                 }
-                dChunks.resize(std::max<size_t>(allChunks.size(), 1));
-                CF_HIP(hipMemcpyAsync(dChunks.get(), allChunks.data(), allChunks.size() * sizeof(Chunk),
-                        hipMemcpyHostToDevice, s));
                 dG.resize(maxG);
-                CF_HIP(hipStreamSynchronize(s));   // allChunks is read by the copy; nothing host-side in the capture
-                timer.flush();
                 graph.beginCapture();
-                size_t k = 0;
                 for (const Batch& b : batches) {
                     timer.begin();
-                    launchEvalBins(s, images->set(), level[cur].get(), dPerm.get(), bs.blocks.get(), b.work->get(),
+                    launchEvalBins(s, images->set(), level[cur].get(), dPerm.get(), bs.dBlocks, b.work->get(),
                             b.numWork, b.g0, tabs, N, dBins.get(), flipOffset, levelShape);
                     timer.end(stats.evalKernelMs);
                     stats.evalLaunches += 1;
@@ -669,19 +747,18 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                         const int nc = nodes[sb.second - 1].chunkEnd - nodes[s0].chunkBegin;
                         launchFillU32(s, dG.get(), static_cast<size_t>(ns) * perSlotB, 0u);
                         timer.begin();
-                        launchHistBins(s, dBins.get(), dLab8.get(), dChunks.get() + chunkOff[k], nc, b.g0, b.ngb, tabs,
-                                C, N, dG.get(), flipOffset);
+                        launchHistBins(s, dBins.get(), dLab8.get(), dChunks + nodes[s0].chunkBegin, nc, s0, b.g0, b.ngb,
+                                tabs, C, N, dG.get(), flipOffset);
                         timer.end(stats.histMs);
                         timer.begin();
-                        launchScores(s, dG.get(), dNodeHist.get() + static_cast<size_t>(s0) * C, dSlotTree.get() + s0,
-                                ns, tabs, C, dSumm.get() + static_cast<size_t>(s0) * F, nullptr, -1, b.g0 * kBinGroup,
+                        launchScores(s, dG.get(), dNodeHist + static_cast<size_t>(s0) * C, dNodeTree + s0, ns, tabs, C,
+                                dSumm.get() + static_cast<size_t>(s0) * F, nullptr, -1, b.g0 * kBinGroup,
                                 b.ngb * kBinGroup);
                         timer.end(stats.scoreMs);
-                        k++;
                     }
                 }
                 timer.begin();
-                launchReduce(s, dSumm.get(), numNodes, F, dBest.get());
+                launchReduce(s, dSumm.get(), numNodes, F, dBest);
                 timer.end(stats.scoreMs);
                 graph.launch();
                 stats.levelGraphs += 1;
@@ -695,7 +772,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 workFor(bs, ngb);
                 if (measure) CF_HIP(hipEventRecord(tuneStart, s));
                 timer.begin();
-                launchEvalBins(s, images->set(), level[cur].get(), dPerm.get(), bs.blocks.get(), bs.work.get(),
+                launchEvalBins(s, images->set(), level[cur].get(), dPerm.get(), bs.dBlocks, bs.work.get(),
                         bs.numWork, g0, tabs, N, dBins.get(), flipOffset, shape);
                 timer.end(stats.evalKernelMs);
                 if (measure) {
@@ -715,18 +792,15 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 for (int s0 = 0; s0 < numNodes;) {
                     const int s1 = std::min(numNodes, s0 + maxSlotsB);
                     const int ns = s1 - s0;
-                    std::vector<Chunk> bc(chunks.begin() + nodes[s0].chunkBegin, chunks.begin() + nodes[s1 - 1].chunkEnd);
-                    for (auto& c : bc) c.slot -= s0;
-                    dChunks.resize(bc.size());
+                    const int nc = nodes[s1 - 1].chunkEnd - nodes[s0].chunkBegin;
                     dG.resize(static_cast<size_t>(ns) * perSlotB);
-                    CF_HIP(hipMemcpyAsync(dChunks.get(), bc.data(), bc.size() * sizeof(Chunk), hipMemcpyHostToDevice, s));
                     CF_HIP(hipMemsetAsync(dG.get(), 0, static_cast<size_t>(ns) * perSlotB * sizeof(uint32_t), s));
                     timer.begin();
-                    launchHistBins(s, dBins.get(), dLab8.get(), dChunks.get(), static_cast<int>(bc.size()), g0, ngb, tabs,
-                            C, N, dG.get(), flipOffset);
+                    launchHistBins(s, dBins.get(), dLab8.get(), dChunks + nodes[s0].chunkBegin, nc, s0, g0, ngb, tabs, C, N,
+                            dG.get(), flipOffset);
                     timer.end(stats.histMs);
                     timer.begin();
-                    launchScores(s, dG.get(), dNodeHist.get() + static_cast<size_t>(s0) * C, dSlotTree.get() + s0, ns,
+                    launchScores(s, dG.get(), dNodeHist + static_cast<size_t>(s0) * C, dNodeTree + s0, ns,
                             tabs, C, dSumm.get() + static_cast<size_t>(s0) * F, nullptr, -1, g0 * kBinGroup,
                             ngb * kBinGroup);
                     timer.end(stats.scoreMs);
@@ -735,17 +809,9 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             }
             if (!graph.launched()) {
                 timer.begin();
-                launchReduce(s, dSumm.get(), numNodes, F, dBest.get());
+                launchReduce(s, dSumm.get(), numNodes, F, dBest);
                 timer.end(stats.scoreMs);
             }
-            CF_HIP(hipMemcpyAsync(best.data(), dBest.get(), numNodes * sizeof(NodeBest), hipMemcpyDeviceToHost, s));
-            CF_HIP(hipStreamSynchronize(s));
-            timer.flush();
-            std::vector<int> flagged;
-            for (int i = 0; i < numNodes; i++) {
-                if (best[i].flag) flagged.push_back(i);
-            }
-            replayNodes(flagged);
         };
         if (mode == CF_MODE_PLAIN) {
             for (int i = 0; i < numNodes; i++) evalSlots(i, i + 1);
@@ -767,33 +833,30 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                     levelSamples * F / ((stats.evalKernelMs - evalMsBefore) * 1e-3));
         }
 
-        // ---- split records, built on the device from the argmax and the level's feature tables
-        std::vector<int> nodeTree(numNodes);
-        for (int i = 0; i < numNodes; i++) nodeTree[i] = nodes[i].active;
-        dSplits.resize(numNodes);
-        dBestAll.resize(numNodes);
-        dNodeTree.resize(numNodes);
-        dChunkCounts.resize(chunks.size());
-        dLeftHist.resize(static_cast<size_t>(numNodes) * C);
-        dChunks.resize(chunks.size());
-        CF_HIP(hipMemcpyAsync(dBestAll.get(), best.data(), numNodes * sizeof(NodeBest), hipMemcpyHostToDevice, s));
-        CF_HIP(hipMemcpyAsync(dNodeTree.get(), nodeTree.data(), numNodes * sizeof(int), hipMemcpyHostToDevice, s));
-        launchSplitRecords(s, dBestAll.get(), dNodeTree.get(), numNodes, tabs, dSplits.get());
-        CF_HIP(hipMemcpyAsync(dChunks.get(), chunks.data(), chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, s));
-        CF_HIP(hipMemsetAsync(dLeftHist.get(), 0, static_cast<size_t>(numNodes) * C * sizeof(uint32_t), s));
-        timer.begin();
-        launchPartitionDirections(s, images->desc.get(), level[cur].get(), dChunks.get(), static_cast<int>(chunks.size()),
-                dSplits.get(), C, dir.get(), dChunkCounts.get(), dLeftHist.get());
-        timer.end(stats.partitionMs);
-        std::vector<int2> chunkCounts(chunks.size());   // left and right entries per chunk
-        std::vector<uint32_t> leftHist(static_cast<size_t>(numNodes) * C);
-        std::vector<SplitRec> splits(numNodes);
-        CF_HIP(hipMemcpyAsync(chunkCounts.data(), dChunkCounts.get(), chunks.size() * sizeof(int2), hipMemcpyDeviceToHost,
-                s));
-        CF_HIP(hipMemcpyAsync(leftHist.data(), dLeftHist.get(), leftHist.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        CF_HIP(hipMemcpyAsync(splits.data(), dSplits.get(), numNodes * sizeof(SplitRec), hipMemcpyDeviceToHost, s));
-        CF_HIP(hipStreamSynchronize(s));
-        timer.flush();
+        // ---- split records, built on the device from the argmax and the level's feature tables, and the samples'
+        // directions; the level's one read-back.  Nodes of a two-pass level whose argmax has to be replayed show
+        // up in it: they are replayed, and the records and directions made again.
+        for (bool again = twoPass;; again = false) {
+            launchSplitRecords(s, dBest, dNodeTree, numNodes, tabs, dSplits);
+            CF_HIP(hipMemsetAsync(dLeftHist, 0, static_cast<size_t>(numNodes) * C * sizeof(uint32_t), s));
+            timer.begin();
+            launchPartitionDirections(s, images->desc.get(), level[cur].get(), dChunks, numChunks, dSplits, C, dir.get(),
+                    dChunkCounts, dLeftHist);
+            timer.end(stats.partitionMs);
+            CF_HIP(hipMemcpyAsync(hostResults, ws.results.get(), resultBytes, hipMemcpyDeviceToHost, s));
+            CF_HIP(hipStreamSynchronize(s));
+            timer.flush();
+            if (!again) break;
+            std::vector<int> flagged;
+            for (int i = 0; i < numNodes; i++) {
+                if (best[i].flag) flagged.push_back(i);
+            }
+            if (flagged.empty()) break;
+            replayNodes(flagged);
+        }
+        const SplitRec* splits = reinterpret_cast<const SplitRec*>(hostResults + splitsAt);
+        const int2* chunkCounts = reinterpret_cast<const int2*>(hostResults + countsAt);
+        const uint32_t* leftHist = reinterpret_cast<const uint32_t*>(hostResults + histAt);
 
         // ---- tree growth on the host, next frontier and sample destinations
         std::vector<int2> dst(chunks.size(), make_int2(-1, -1));
@@ -870,17 +933,13 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             if (!na.nodes.empty()) next.push_back(std::move(na));
         }
         if (nextOff > 0) {
-            dDst.resize(dst.size());
-            CF_HIP(hipMemcpyAsync(dDst.get(), dst.data(), dst.size() * sizeof(int2), hipMemcpyHostToDevice, s));
+            const int2* dDst = up.put(dst);
+            up.flush(s);
             timer.begin();
-            launchPartitionScatter(s, level[cur].get(), dChunks.get(), static_cast<int>(chunks.size()), dir.get(),
-                    dDst.get(), level[1 - cur].get());
+            launchPartitionScatter(s, level[cur].get(), dChunks, numChunks, dir.get(), dDst, level[1 - cur].get());
             timer.end(stats.partitionMs);
             cur = 1 - cur;
         }
-        // the host vectors handed to the copies above live until here
-        CF_HIP(hipStreamSynchronize(s));
-        timer.flush();
         active.swap(next);
     }
     CF_HIP(hipStreamSynchronize(s));
