@@ -273,10 +273,10 @@ void launchLevelKeys(hipStream_t s, const cf_sample* samples, int begin, int n, 
 int levelPlaces(int W, int H);
 // label per level index, bit 7 set for samples still set to Both (counted in both orientations)
 void launchLevelLabels(hipStream_t s, const cf_sample* samples, int n, uint8_t* labels);
-// Counting sort of n level entries by key (< levelSortBuckets(numSegs, placeBits)): out = the values in key
-// order (input order inside every segment bucket of up to 64 entries), starts[seg] = first position of segment seg (key >> placeBits) or -1 if it is empty, and
-// starts[numSegs] = the number of entries with a key below numSegs << placeBits.  count and cursor hold
-// levelSortBuckets entries, blockSum levelSortScanBlocks.
+// Counting sort of the n level entries with a key below numSegs << placeBits (the others are not placed): out =
+// their values in key order, starts[seg] = first position of segment seg (key >> placeBits) or -1 if it is
+// empty, starts[numSegs] = the number of placed entries.  count and cursor hold levelSortBuckets entries,
+// blockSum levelSortScanBlocks.
 size_t levelSortBuckets(int numSegs, int placeBits);
 // p[0 .. n) = v by a kernel (usable inside a captured graph, where memset nodes are avoided)
 void launchFillU32(hipStream_t s, uint32_t* p, size_t n, uint32_t v);

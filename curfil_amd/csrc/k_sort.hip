@@ -9,20 +9,15 @@
 //                   scan of the block totals, the block offsets added);
 //   k_sort_scatter  places every entry at its bucket's cursor (atomic, so
 //                   the order inside a bucket follows arrival);
-//   k_sort_settle   restores the input order inside every segment bucket of
-//                   at most kSettleMax entries by sorting its values (the
-//                   entries' level indices, with kFlipEntry on the flipped
-//                   evaluations that follow all plain entries in the input),
-//                   one lane per bucket;
-//   k_sort_starts   the first position of every (tree, image) segment.
-// Buckets hold a few entries on average (one sample per 77 pixels per tree
-// at the benchmark's sampling density, and 512 pixels per bucket), so the
-// result is the stable sort by key.  Longer
-// buckets, and the bucket past the segments that collects the flipped
-// entries of samples that are not Both (up to one per sample, never
-// evaluated), keep their arrival order: the order inside a bucket only
-// decides which lanes of pass 1 evaluate which samples of one place, never a
-// result, since every bin row is stored at its entry's level index.
+//   k_sort_starts   the first position of every (image, tree) segment.
+// The order inside a bucket (the samples of one place of a segment, seven on
+// average at one sample per 77 pixels) only decides which lanes of pass 1
+// evaluate which of them, never a result, since every bin row is stored at its
+// entry's level index.  (Putting the buckets back into input order took 131 us
+// of a level of 4 small frames, where they are longest.)  Entries with a key
+// past the segments, the flipped evaluations of samples that are not Both, are
+// not placed: nothing reads them, and the atomics of one shared bucket took
+// 2 x 135 us of a level of 13 flipped frames.
 #include "cf_internal.h"
 
 namespace cf {
@@ -30,17 +25,16 @@ namespace cf {
 namespace {
 
 constexpr int kScanBlock = 1024;   // counts scanned per workgroup (256 lanes x 4)
-constexpr uint32_t kSettleMax = 64;   // longest bucket put back into input order
 
 __global__ void __launch_bounds__(256) k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
 }
 
-__global__ void __launch_bounds__(256) k_sort_count(const uint32_t* __restrict__ keys, int n,
+__global__ void __launch_bounds__(256) k_sort_count(const uint32_t* __restrict__ keys, int n, uint32_t keyEnd,
         uint32_t* __restrict__ count) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) atomicAdd(&count[keys[i]], 1u);
+    if (i < n && keys[i] < keyEnd) atomicAdd(&count[keys[i]], 1u);
 }
 
 // Exclusive scan of kScanBlock counts per workgroup into `start`, the workgroup's total into blockSum.
@@ -107,28 +101,10 @@ __global__ void __launch_bounds__(256) k_scan_add(uint32_t* __restrict__ start, 
 
 // cursor[b] starts at bucket b's first position and ends one past its last.
 __global__ void __launch_bounds__(256) k_sort_scatter(const uint32_t* __restrict__ keys,
-        const uint32_t* __restrict__ vals, int n, uint32_t* __restrict__ cursor, uint32_t* __restrict__ out) {
+        const uint32_t* __restrict__ vals, int n, uint32_t keyEnd, uint32_t* __restrict__ cursor,
+        uint32_t* __restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[atomicAdd(&cursor[keys[i]], 1u)] = vals[i];
-}
-
-// One lane per segment bucket of 2..kSettleMax entries: insertion sort of its values.
-__global__ void __launch_bounds__(256) k_sort_settle(const uint32_t* __restrict__ count,
-        const uint32_t* __restrict__ cursor, size_t buckets, uint32_t* __restrict__ out) {
-    const size_t b = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (b >= buckets) return;
-    const uint32_t c = count[b];
-    if (c < 2 || c > kSettleMax) return;
-    const uint32_t e = cursor[b], s = e - c;
-    for (uint32_t i = s + 1; i < e; i++) {
-        const uint32_t v = out[i];
-        uint32_t j = i;
-        while (j > s && out[j - 1] > v) {
-            out[j] = out[j - 1];
-            j--;
-        }
-        out[j] = v;
-    }
+    if (i < n && keys[i] < keyEnd) out[atomicAdd(&cursor[keys[i]], 1u)] = vals[i];
 }
 
 // starts[seg] = first position of segment seg, or -1 if it is empty.  After the scatter, a bucket's
@@ -169,16 +145,13 @@ void levelCountingSort(hipStream_t s, const uint32_t* keys, const uint32_t* vals
     if (buckets > (static_cast<size_t>(1) << 28)) throw Error(CF_ERR_UNSUPPORTED, "too many level segments to sort");
     const int nb = static_cast<int>(blocksFor(buckets, kScanBlock));
     hipLaunchKernelGGL(k_fill_u32, dim3(blocksFor(buckets, 256)), dim3(256), 0, s, count, buckets, 0u);
-    if (n > 0) hipLaunchKernelGGL(k_sort_count, dim3(blocksFor(n, 256)), dim3(256), 0, s, keys, n, count);
+    const uint32_t keyEnd = static_cast<uint32_t>(numSegs) << placeBits;
+    if (n > 0) hipLaunchKernelGGL(k_sort_count, dim3(blocksFor(n, 256)), dim3(256), 0, s, keys, n, keyEnd, count);
     hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(256), 0, s, count, buckets, cursor, blockSum);
     hipLaunchKernelGGL(k_scan_totals, dim3(1), dim3(256), 0, s, blockSum, nb);
     hipLaunchKernelGGL(k_scan_add, dim3(blocksFor(buckets, 256)), dim3(256), 0, s, cursor, buckets, blockSum);
     if (n > 0) {
-        hipLaunchKernelGGL(k_sort_scatter, dim3(blocksFor(n, 256)), dim3(256), 0, s, keys, vals, n, cursor, out);
-        // the segments' buckets only: the bucket past them holds the flipped entries of samples that are not Both
-        const size_t segBuckets = static_cast<size_t>(numSegs) << placeBits;
-        hipLaunchKernelGGL(k_sort_settle, dim3(blocksFor(segBuckets, 256)), dim3(256), 0, s, count, cursor, segBuckets,
-                out);
+        hipLaunchKernelGGL(k_sort_scatter, dim3(blocksFor(n, 256)), dim3(256), 0, s, keys, vals, n, keyEnd, cursor, out);
     }
     hipLaunchKernelGGL(k_sort_starts, dim3(blocksFor(static_cast<size_t>(numSegs) + 1, 256)), dim3(256), 0, s,
             count, cursor, numSegs, placeBits, starts);
