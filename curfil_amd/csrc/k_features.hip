@@ -22,7 +22,7 @@
 //                 candidates' thresholds.
 // The bands only decide how far a round gets, never which draws a candidate
 // uses.  Per level of 5 trees with F = 4000, T = 32 on 50 frames of 640x480 the
-// walk takes 1.7 ms (about 40 rounds of 112 candidates: 15 us + 18 us each);
+// walk takes 1.6 ms (about 40 rounds of 112 candidates: 15 us + 18 us each);
 // one workgroup per tree that evaluated 16 candidates a round on its own CU
 // took 15.2 ms, bound by that CU's gathers.
 #include <algorithm>
@@ -274,21 +274,28 @@ __device__ __forceinline__ int nthBit(unsigned long long w, int n) {
 }
 
 constexpr int kBandMax = 2048;            // draws of the widest band
-constexpr int kRoundTable = 28672;        // table entries of a round (two bytes each, in the walker's LDS)
-constexpr int kRoundCandMax = 224;        // candidates of a round (kRoundTable / the narrowest band)
+constexpr int kRoundCandMax = 224;        // candidates of a round
 constexpr int kAdvanceLanes = 1024;
 constexpr int kGroup = 8;                 // consecutive candidates that k_fg_advance composes
 constexpr uint16_t kOpen = 0x8000;        // the candidate does not end inside its band
 constexpr uint16_t kAccept = 0x4000;      // it ends with its T-th threshold (else rejected)
 
 // Band of a round for T thresholds: a power of two of at least 8 T draws.  A candidate uses about 1.25 T
-// draws with a spread of T / 8, so the start of the round's j-th candidate is known to about sqrt(j) T / 8;
-// with 28672 / band candidates a round that is covered to its end (measured on 640x480 frames: T = 32,
-// 112 candidates, starts within 80 draws of the mean in nine rounds of ten).
+// draws with a spread of T / 8, so the start of the round's j-th candidate is known to about sqrt(j) T / 8:
+// 112 candidates are covered to their end (measured on 640x480 frames: T = 32, starts within 80 draws of the
+// mean in nine rounds of ten).  Rounds of twice as many with bands of 256 draws often ended early and cost twice
+// as much each (21 frames, 3 trees, 2000 x 20: 117.3 against 116.1 ms a training).
 static int bandDraws(int T) {
     int b = 128;
     while (b < 8 * T && b < kBandMax) b *= 2;
     return b;
+}
+
+// Candidates of a round: 224 with the narrowest band, else 112 as far as their tables (two bytes an entry) fit
+// the walker's LDS with the composed ones, and no more than a small feature table can need.
+static int roundCandidates(int band, int F) {
+    const int most = std::max(28672 / band, std::min(112, 57344 / band));
+    return std::min(most, (F + F / 8 + 2 * kGroup) / kGroup * kGroup);
 }
 
 // One candidate of a round on its band (see the head of this file).  Bound by the latency of the corner
@@ -713,7 +720,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     const int TM = binThresholdWidth(T);
     tabs.thrPad.resize(static_cast<size_t>(numJobs) * F * TM);
     const int band = bandDraws(T);
-    const int m = std::min(kRoundTable / band, kRoundCandMax);   // candidates of a round
+    const int m = roundCandidates(band, F);
     int ring = 1 << 14;
     while (ring < (1 << 19) && ring < 2.0 * F * T) ring *= 2;
     const int maxSteps = ring / kMtStep + 1;
