@@ -381,7 +381,7 @@ struct FrameJob {
 };
 // the shape of a launch over jobs: the tree-split kernel for few pixels, and the launch's tiles
 struct ClassifyPlan {
-    bool split = false;
+    int splitWaves = 0;   // waves that share a tile's trees, 0: one thread per pixel
     int totalTiles = 0;
 };
 // chooses the shape by the jobs' pixels (the tree-split kernel up to splitMaxPixels) and sets their firstTile

@@ -367,9 +367,9 @@ __global__ void __launch_bounds__(256) k_classify_jobs(const FrameJob* __restric
 
 // Few pixels (a single frame, a few small frames): with one thread per pixel most SIMDs hold a single
 // wave, and a wave's time is its walk of all trees one after another.  Here a workgroup takes one 16 x 4
-// tile and its waves walk the trees t = w, w + kSplitWaves, ... (w the wave); the leaf numbers meet in
+// tile and its waves walk the trees t = w, w + waves, ... (w the wave); the leaf numbers meet in
 // LDS and wave 0 adds the posteriors in tree order, the same float sums as one thread walking all trees.
-constexpr int kSplitWaves = 4;
+constexpr int kSplitWavesMax = 8;
 
 __host__ __device__ __forceinline__ int splitTiles(int W, int rows) {
     return ((W + kTileW - 1) / kTileW) * ((rows + kTileH - 1) / kTileH);
@@ -390,7 +390,7 @@ __device__ __forceinline__ void classifyTileSplit(const DevImage& im, int tile, 
         int32_t depth;
         const bool depthOk = pixelDepthAt(im, x, y, depth);
         const double rinv = depthOk ? depthReciprocal(depthToFloat(depth)) : 0.0;
-        for (int t = wave; t < T; t += kSplitWaves) {
+        for (int t = wave; t < T; t += static_cast<int>(blockDim.x >> 6)) {
             leafLds[t * 64 + lane] = walkTree(im, x, y, depthOk, rinv, forest, forest.treeRoot[t]);
         }
     }
@@ -410,7 +410,7 @@ __device__ __forceinline__ void classifyTileSplit(const DevImage& im, int tile, 
 }
 
 template<int CM>
-__global__ void __launch_bounds__(256) k_classify_split(const DevImage* __restrict__ imgs,
+__global__ void __launch_bounds__(64 * kSplitWavesMax) k_classify_split(const DevImage* __restrict__ imgs,
         const int* __restrict__ frameIdx, int numFrames, int W, int H, DevForest forest, float* __restrict__ probs,
         uint8_t* __restrict__ labels) {
     ClassifyTile tile;
@@ -423,8 +423,8 @@ __global__ void __launch_bounds__(256) k_classify_split(const DevImage* __restri
 }
 
 template<int CM>
-__global__ void __launch_bounds__(256) k_classify_jobs_split(const FrameJob* __restrict__ jobs, int numJobs,
-        int totalTiles, DevForest forest) {
+__global__ void __launch_bounds__(64 * kSplitWavesMax) k_classify_jobs_split(
+        const FrameJob* __restrict__ jobs, int numJobs, int totalTiles, DevForest forest) {
     ClassifyTile tile;
     if (!classifyTile(totalTiles, 1, tile)) return;
     const int j = tile.block;
@@ -448,7 +448,7 @@ void dispatchClasses(int C, Launch&& launch) {
 
 // Launches of at most kSplitPixels pixels (CURFIL_CLASSIFY_SPLIT_MPIX overrides it, read once per process
 // for single and batched predictions and when a serving loop is created; 0: never) split each
-// tile's trees over the waves of a workgroup, given at least kSplitWaves trees and at most 128 (their
+// tile's trees over the waves of a workgroup, given at least two trees and at most 128 (their
 // leaf numbers, 256 bytes per tree, fill the workgroup's LDS).  Measured with 10 trees of depth 20: one
 // 640x480 frame 0.80 against 0.89 ms to the host; 64 frames (19.7 Mpix) 2.7% slower split.  The bound
 // covers every launch of the serving loop (at most 1.25 Mpix), which served the 320x240 / 640x480 /
@@ -460,8 +460,21 @@ double classifySplitPixels() {
     const char* e = std::getenv("CURFIL_CLASSIFY_SPLIT_MPIX");
     return e ? std::atof(e) * 1e6 : kSplitPixels;
 }
-static bool splitLaunch(double pixels, double maxPx, const DevForest& forest) {
-    return pixels <= maxPx && forest.numTrees >= kSplitWaves && forest.numTrees <= kSplitMaxTrees;
+
+// The waves of a workgroup that share a tile's trees in a launch of so many pixels, 0: the launch is not
+// split.  Four at most once they alone keep the SIMDs busy (more of them wait for wave 0 and hold their
+// registers); a smaller launch is as fast as its longest wave, so there each wave takes one tree, or two of
+// more than eight.  Microseconds with 1 (as fast as the unsplit kernel) / 4 / 5 / 7 / 10 waves, depth 16:
+// 160x120, 10 trees 147 / 67 / 58 / 58 / 54; 320x240, 10 trees 173 / 99 / 93 / 98 / 97, 7 trees 128 / 75 /
+// 77 / 73; 640x480, 10 trees 305 / 266 / 272 / 277 / 283; 1280x960, 10 trees 971 / 928 / 1003 / 1073 / 1103.
+// Three waves for 3 trees against one: 160x120 58 -> 36, 320x240 68 -> 45, 640x480 111 -> 100, 1280x960
+// 320 -> 300.
+constexpr double kSplitFewPixels = 131072;
+static int splitWaves(double pixels, double maxPx, const DevForest& forest) {
+    const int T = forest.numTrees;
+    if (pixels > maxPx || T < 2 || T > kSplitMaxTrees) return 0;
+    if (pixels > kSplitFewPixels) return std::min(T, 4);
+    return T <= kSplitWavesMax ? T : std::min((T + 1) / 2, kSplitWavesMax);
 }
 static size_t splitLds(const DevForest& forest) {
     return static_cast<size_t>(forest.numTrees) * 64 * sizeof(int);
@@ -471,11 +484,11 @@ void launchClassify(hipStream_t s, const DevImage* imgs, const int* frameIdx, in
         const DevForest& forest, float* probs, uint8_t* labels) {
     static const double maxPx = classifySplitPixels();   // once per process
     const double pixels = static_cast<double>(numFrames) * W * H;
-    if (splitLaunch(pixels, maxPx, forest)) {
+    if (const int waves = splitWaves(pixels, maxPx, forest)) {
         const dim3 grid = classifyGrid(splitTiles(W, H), numFrames);
         dispatchClasses(forest.C, [&](auto cm) {
-            hipLaunchKernelGGL(k_classify_split<decltype(cm)::value>, grid, dim3(64 * kSplitWaves), splitLds(forest),
-                    s, imgs, frameIdx, numFrames, W, H, forest, probs, labels);
+            hipLaunchKernelGGL(k_classify_split<decltype(cm)::value>, grid, dim3(64 * waves), splitLds(forest), s,
+                    imgs, frameIdx, numFrames, W, H, forest, probs, labels);
         });
         return;
     }
@@ -490,11 +503,11 @@ ClassifyPlan planClassifyJobs(FrameJob* jobs, int numJobs, const DevForest& fore
     double pixels = 0;
     for (int i = 0; i < numJobs; i++) pixels += static_cast<double>(jobs[i].im.W) * (jobs[i].rowEnd - jobs[i].rowBegin);
     ClassifyPlan plan;
-    plan.split = splitLaunch(pixels, splitMaxPixels, forest);
+    plan.splitWaves = splitWaves(pixels, splitMaxPixels, forest);
     int tiles = 0;
     for (int i = 0; i < numJobs; i++) {
         const int rows = jobs[i].rowEnd - jobs[i].rowBegin;
-        const int t = plan.split ? splitTiles(jobs[i].im.W, rows) : tileBlocks(jobs[i].im.W, rows);
+        const int t = plan.splitWaves ? splitTiles(jobs[i].im.W, rows) : tileBlocks(jobs[i].im.W, rows);
         if (tiles > INT32_MAX - t) throw Error(CF_ERR_UNSUPPORTED, "too many pixels in one launch");
         jobs[i].firstTile = tiles;
         tiles += t;
@@ -508,8 +521,8 @@ void launchClassifyJobs(hipStream_t s, const FrameJob* jobs, int numJobs, const 
     if (numJobs == 0) return;
     const dim3 grid = classifyGrid(plan.totalTiles, 1);
     dispatchClasses(forest.C, [&](auto cm) {
-        if (plan.split) {
-            hipLaunchKernelGGL(k_classify_jobs_split<decltype(cm)::value>, grid, dim3(64 * kSplitWaves),
+        if (plan.splitWaves) {
+            hipLaunchKernelGGL(k_classify_jobs_split<decltype(cm)::value>, grid, dim3(64 * plan.splitWaves),
                     splitLds(forest), s, jobs, numJobs, plan.totalTiles, forest);
         } else {
             hipLaunchKernelGGL(k_classify_jobs<decltype(cm)::value>, grid, dim3(256), 0, s, jobs, numJobs,
