@@ -277,8 +277,12 @@ constexpr int kBandMax = 2048;            // draws of the widest band
 constexpr int kRoundCandMax = 224;        // candidates of a round
 constexpr int kAdvanceLanes = 1024;
 constexpr int kGroup = 8;                 // consecutive candidates that k_fg_advance composes
-constexpr uint16_t kOpen = 0x8000;        // the candidate does not end inside its band
-constexpr uint16_t kAccept = 0x4000;      // it ends with its T-th threshold (else rejected)
+// What a candidate started at a draw of its band comes to, 16 bits: kAccept if it ends with its T-th threshold
+// (else rejected) and, in the value bits, the place of its successor's first draw in the successor's band; with
+// kLeave, that draw lies outside the successor's band and the value is where the candidate ends in its own;
+// kOpen: it does not end inside its band.
+constexpr uint16_t kOpen = 0x8000, kAccept = 0x4000, kLeave = 0x1000, kPlace = 0x0fff;
+static_assert(kBandMax <= kPlace, "places and ends of a band fit the value bits");
 
 // Band of a round for T thresholds: a power of two of at least 8 T draws.  A candidate uses about 1.25 T
 // draws with a spread of T / 8, so the start of the round's j-th candidate is known to about sqrt(j) T / 8:
@@ -298,24 +302,38 @@ static int roundCandidates(int band, int F) {
     return std::min(most, (F + F / 8 + 2 * kGroup) / kGroup * kGroup);
 }
 
+// The band of a round's candidate j, in draws from the walk's next one: around j times the draws that a candidate
+// has used so far, wider the later the candidate.  The round and the walk over its tables both form it, in
+// operations that no compilation contracts.
+struct RoundBand {
+    int lo, width;
+};
+__device__ __forceinline__ RoundBand roundBand(const WalkState& st, int j, int T, int band, int numCand, int drawn) {
+    const float avg = __fdiv_rn(__fadd_rn(static_cast<float>(st.drawsDone), __fmul_rn(16.0f, st.guess)),
+            __fadd_rn(static_cast<float>(st.candsDone), 16.0f));
+    const float dev = __fadd_rn(8.0f, __fmul_rn(__fmul_rn(0.19f, avg), __fsqrt_rn(static_cast<float>(j))));
+    RoundBand b;
+    b.lo = j == 0 ? 0 : max(j * minDraws(T), static_cast<int>(__fsub_rn(__fmul_rn(static_cast<float>(j), avg), dev)));
+    b.width = j == 0 ? band
+                     : min(band, static_cast<int>(__fadd_rn(__fmul_rn(2.0f, dev), __fmul_rn(1.25f, avg))) + 8);
+    b.width = max(0, min(b.width, st.tail - st.head - b.lo));
+    if (st.k + j >= min(drawn, numCand)) b.width = 0;   // not drawn yet, or past the last: the walk stops here
+    return b;
+}
+
 // One candidate of a round on its band (see the head of this file).  Bound by the latency of the corner
 // gathers, which the round's candidates x trees workgroups overlap on all CUs.
 __global__ void __launch_bounds__(256) k_fg_round(const WalkState* __restrict__ states, ImageSet imgs,
         const FeatRec* __restrict__ cand, int numCand, int drawn, int T, int ring, int band, const DrawRec* __restrict__ recs,
-        float* __restrict__ resp, uint16_t* __restrict__ next, int4* __restrict__ bands) {
+        float* __restrict__ resp, uint16_t* __restrict__ next, int2* __restrict__ firsts) {
     constexpr int kWords = kBandMax / 64;
     __shared__ unsigned long long finite[kWords], rejects[kWords];   // not NaN; tenth NaN of a run
     const WalkState st = states[blockIdx.y];
     const int j = blockIdx.x;
     if (st.done || st.k + j >= numCand) return;
     const size_t row = static_cast<size_t>(blockIdx.y) * gridDim.x + j;
-    // the band: around j times the draws that a candidate has used so far, wider the later the candidate
-    const float avg = (st.drawsDone + 16.0f * st.guess) / (st.candsDone + 16.0f);
-    const float dev = 8.0f + 0.19f * avg * sqrtf(static_cast<float>(j));
-    const int lo = j == 0 ? 0 : max(j * minDraws(T), static_cast<int>(j * avg - dev));
-    int width = j == 0 ? band : min(band, static_cast<int>(2.0f * dev + 1.25f * avg) + 8);
-    width = max(0, min(width, st.tail - st.head - lo));
-    if (st.k + j >= drawn) width = 0;   // not drawn yet: the walk stops here
+    const RoundBand own = roundBand(st, j, T, band, numCand, drawn), after = roundBand(st, j + 1, T, band, numCand, drawn);
+    const int lo = own.lo, width = own.width;
     const Feat f = loadFeat(cand + static_cast<size_t>(blockIdx.y) * numCand + st.k + j);
     const DrawRec* rec = recs + static_cast<size_t>(blockIdx.y) * ring;
     const size_t plane = static_cast<size_t>(imgs.W) * imgs.H;
@@ -401,18 +419,20 @@ __global__ void __launch_bounds__(256) k_fg_round(const WalkState* __restrict__ 
             }
             need -= c;
         }
-        next[row * band + i] = static_cast<uint16_t>(how | end);
+        if (how != kOpen) {
+            const int place = lo + end - after.lo;
+            how |= place >= 0 && place < after.width ? place : (kLeave | end);
+        }
+        next[row * band + i] = how;
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && j == 0) {
         // the band's finite draws and the NaN draws after the last of them, for a candidate that runs past it
         int found = 0, last = -1;
-        if (j == 0) {
-            for (int w = 0; w < words; w++) {
-                found += __popcll(finite[w]);
-                if (finite[w]) last = w * 64 + 63 - __clzll(finite[w]);
-            }
+        for (int w = 0; w < words; w++) {
+            found += __popcll(finite[w]);
+            if (finite[w]) last = w * 64 + 63 - __clzll(finite[w]);
         }
-        bands[row] = make_int4(lo, width, found, width - 1 - last);
+        firsts[blockIdx.y] = make_int2(found, width - 1 - last);
     }
 }
 
@@ -426,104 +446,154 @@ struct WalkStep {
 // Follows the candidates of a round through their tables, from the state's next draw and candidate on.  The
 // round ends at the first candidate that starts outside its band or does not end inside it; the round's first
 // candidate, which starts at its band's first draw, then carries its thresholds and tries into the next.
-// Bound by the chain of dependent LDS reads, about 0.2 us each.  The chain is shortened by composing the
-// tables of kGroup consecutive candidates for every start of the first's band, all in parallel: the walk then
-// takes a read per group, and the groups it passed are expanded in parallel (F = 4000, T = 32: 18 us a launch,
-// 32 us with a read per candidate).
+// Bound by the chain of dependent LDS reads.  The chain is shortened by composing the tables of kGroup
+// consecutive candidates for every start of the first's band, all in parallel: the walk then takes a read per
+// group, checks all groups at once, and the groups it passed are expanded in parallel.  An entry is the place of
+// the next entry to read, so that a step of a chain is one read and two operations (with the draw's number in
+// the entry, and each candidate's band read beside it to find the place: F = 4000, T = 32 18 us a launch, of
+// them 6.6 composing and 3.8 walking; now 11, 2.3 and 1.9).
 __global__ void __launch_bounds__(kAdvanceLanes) k_fg_advance(const FeatGenJob* __restrict__ jobs,
-        WalkState* __restrict__ states, const FeatRec* __restrict__ cand, int numCand, int F, int T, int band, int m,
-        const float* __restrict__ resp, const uint16_t* __restrict__ next, const int4* __restrict__ bands,
-        FeatRec* __restrict__ outFeat, float* __restrict__ outThr, int* __restrict__ outKey) {
-    // uint16 [m][band], then per group of kGroup candidates uint32 [band]: the end of the group's last
-    // candidate (20 bits), its accepted candidates << 20, or kGroupStop if the walk ends inside the group
+        WalkState* __restrict__ states, const FeatRec* __restrict__ cand, int numCand, int drawn, int F, int T,
+        int band, int m, const float* __restrict__ resp, const uint16_t* __restrict__ next,
+        const int2* __restrict__ firsts, FeatRec* __restrict__ outFeat, float* __restrict__ outThr,
+        int* __restrict__ outKey) {
+    // uint16 [m][band], then per group of kGroup candidates uint32 [band]: the place after the group's last
+    // candidate, its accepted candidates << 16, or kGroupStop if the walk leaves the bands inside the group
     extern __shared__ uint4 tableWords[];
-    __shared__ int4 bd[kRoundCandMax];
+    __shared__ RoundBand bd[kRoundCandMax + 1];
     __shared__ WalkStep steps[kRoundCandMax];
     __shared__ int groupStart[kRoundCandMax / kGroup], groupGen[kRoundCandMax / kGroup];   // start -1: not passed whole
     constexpr uint32_t kGroupStop = 0xffffffffu;
-    const WalkState st = states[blockIdx.x];
-    if (st.done) return;
+    constexpr int kHold = 4;   // table words loaded while the state is
     const int tid = threadIdx.x, lane = tid & 63;
     const size_t row0 = static_cast<size_t>(blockIdx.x) * m;
     const uint4* src = reinterpret_cast<const uint4*>(next + row0 * band);
     const int words = m * band / 8, groups = m / kGroup;
-    for (int i = tid; i < words; i += kAdvanceLanes) tableWords[i] = src[i];
-    for (int i = tid; i < m; i += kAdvanceLanes) {
-        // rows of candidates past the last are never written: empty bands
-        bd[i] = st.k + i < numCand ? bands[row0 + i] : make_int4(0, 0, 0, 0);
-        steps[i].st = 2;
+    uint4 hold[kHold];
+#pragma unroll
+    for (int u = 0; u < kHold; u++) hold[u] = src[min(tid + u * kAdvanceLanes, words - 1)];
+    const WalkState st = states[blockIdx.x];
+#pragma unroll
+    for (int u = 0; u < kHold; u++) __asm__ volatile("" : : "v"(hold[u].x), "v"(hold[u].y), "v"(hold[u].z), "v"(hold[u].w));
+    if (st.done) return;
+#pragma unroll
+    for (int u = 0; u < kHold; u++) {
+        if (tid + u * kAdvanceLanes < words) tableWords[tid + u * kAdvanceLanes] = hold[u];
+    }
+    for (int i = tid + kHold * kAdvanceLanes; i < words; i += kAdvanceLanes) tableWords[i] = src[i];
+    for (int i = tid; i <= m; i += kAdvanceLanes) {
+        bd[i] = roundBand(st, i, T, band, numCand, drawn);
+        if (i < m) steps[i].st = 2;
     }
     for (int i = tid; i < groups; i += kAdvanceLanes) groupStart[i] = -1;
     __syncthreads();
     const uint16_t* table = reinterpret_cast<const uint16_t*>(tableWords);
     uint32_t* composed = reinterpret_cast<uint32_t*>(tableWords + words);
-    for (int i = tid; i < groups * band; i += kAdvanceLanes) {
-        const int g = i / band, j0 = g * kGroup;
-        uint32_t accepted = 0;
-        int p = bd[j0].x + (i - g * band);
-        bool whole = true;
-        for (int q = 0; whole && q < kGroup; q++) {
-            const int lo = bd[j0 + q].x, at = p - lo;
-            whole = at >= 0 && at < bd[j0 + q].y;
-            if (whole) {
-                const int e = table[(j0 + q) * band + at];
-                whole = (e & kOpen) == 0;
-                accepted += (e & kAccept) ? 1u : 0u;
-                p = lo + (e & (kAccept - 1));
+    constexpr int kChains = 4;   // chains that a lane follows together
+    const int bandShift = 31 - __clz(band);
+    for (int i0 = tid; i0 < groups * band; i0 += kAdvanceLanes * kChains) {
+        const uint16_t* row[kChains];
+        int at[kChains];
+        uint32_t seen[kChains], accepted[kChains];
+#pragma unroll
+        for (int u = 0; u < kChains; u++) {
+            const int i = i0 + u * kAdvanceLanes, g = min(i >> bandShift, groups - 1);
+            row[u] = table + ((g * kGroup) << bandShift);
+            at[u] = i & (band - 1);
+            // (rows hold entries up to their band's width only)
+            seen[u] = at[u] < bd[g * kGroup].width ? 0u : kOpen;
+            if (seen[u]) at[u] = 0;
+            accepted[u] = 0;
+        }
+#pragma unroll
+        for (int q = 0; q < kGroup; q++) {
+            uint32_t e[kChains];
+#pragma unroll
+            for (int u = 0; u < kChains; u++) e[u] = row[u][(q << bandShift) + at[u]];
+#pragma unroll
+            for (int u = 0; u < kChains; u++) {
+                seen[u] |= e[u];
+                accepted[u] += e[u] & kAccept;
+                at[u] = seen[u] & (kOpen | kLeave) ? 0 : static_cast<int>(e[u] & kPlace);
             }
         }
-        composed[i] = whole && p < (1 << 20) ? static_cast<uint32_t>(p) | (accepted << 20) : kGroupStop;
+#pragma unroll
+        for (int u = 0; u < kChains; u++) {
+            const int i = i0 + u * kAdvanceLanes;
+            if (i < groups * band) {
+                composed[i] = seen[u] & (kOpen | kLeave) ? kGroupStop
+                                                         : static_cast<uint32_t>(at[u]) | (accepted[u] / kAccept << 16);
+            }
+        }
     }
     __syncthreads();
     const int outOffset = jobs[blockIdx.x].outOffset;
     if (tid < 64) {
-        // wave 0, all lanes in step: the walk's state is uniform
-        int p = 0, j = 0, gen = st.generated, err = 0;
-        bool open = false, stop = false;
-        while (j < m && !stop) {
-            // a whole group, unless the features or candidates may run out in it
-            const int g = j / kGroup;
-            if (j % kGroup == 0 && gen + kGroup < F && st.k + j + kGroup < 3 * F && g < groups) {
-                const int lo = __builtin_amdgcn_readfirstlane(bd[j].x), at = p - lo;
-                if (at >= 0 && at < __builtin_amdgcn_readfirstlane(bd[j].y)) {
-                    const uint32_t c = __builtin_amdgcn_readfirstlane(composed[g * band + at]);
-                    if (c != kGroupStop) {
-                        if (lane == 0) {
-                            groupStart[g] = p;
-                            groupGen[g] = gen;
-                        }
-                        p = static_cast<int>(c & ((1u << 20) - 1u));
-                        gen += static_cast<int>(c >> 20);
-                        j += kGroup;
-                        continue;
-                    }
-                }
+        // wave 0: the groups that are passed whole.  Lane g keeps where group g starts and what it accepts; past a
+        // stop the reads go on at place 0 and count for nothing.
+        int start = 0, at = 0;
+        uint32_t mine = kGroupStop;
+        bool inside = bd[0].width > 0;
+        for (int g = 0; g < groups; g++) {
+            const uint32_t c = composed[(g << bandShift) + at];
+            if (lane == g) {
+                start = at;
+                mine = inside ? c : kGroupStop;
             }
+            inside = inside && c != kGroupStop;
+            at = inside ? static_cast<int>(c & kPlace) : 0;
+        }
+        // features accepted before group `lane`: a group counts only if the features and candidates cannot run
+        // out in it
+        int before = mine == kGroupStop ? 0 : static_cast<int>(mine >> 16);
+        const int own = before;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(before, d, 64);
+            if (lane >= d) before += o;
+        }
+        before += st.generated - own;
+        const bool pass = mine != kGroupStop && before + kGroup < F && st.k + (lane + 1) * kGroup < 3 * F;
+        const unsigned long long fails = __ballot(!pass);
+        const int passed = fails ? __builtin_ctzll(fails) : 64;   // lanes past the groups fail
+        if (lane < passed) {
+            groupStart[lane] = start;
+            groupGen[lane] = before;
+        }
+        // the candidates one by one from there on, all lanes in step: the walk's state is uniform
+        int j = passed * kGroup, gen = __shfl(before, passed, 64), err = 0;
+        at = 0;
+        if (passed > 0) at = static_cast<int>(__shfl(mine, passed - 1, 64) & kPlace);
+        j = __builtin_amdgcn_readfirstlane(j);
+        gen = __builtin_amdgcn_readfirstlane(gen);
+        at = __builtin_amdgcn_readfirstlane(at);
+        int left = j > 0 || bd[0].width > 0 ? -1 : 0;   // the draw at which the walk left the bands
+        bool open = false;
+        while (j < m) {
             // `--maxLoops <= 0` with maxLoops = 3F, checked right after sampling candidate k
             if (gen >= F || st.k + j + 1 >= 3 * F) {
                 err = gen < F;
                 break;
             }
-            const int lo = __builtin_amdgcn_readfirstlane(bd[j].x), width = __builtin_amdgcn_readfirstlane(bd[j].y);
-            const int at = p - lo;
-            if (at < 0 || at >= width) break;   // its first draw was not evaluated: the next round starts here
-            const int e = __builtin_amdgcn_readfirstlane(table[j * band + at]);
+            if (left >= 0) break;   // its first draw was not evaluated: the next round starts here
+            const int e = __builtin_amdgcn_readfirstlane(table[(j << bandShift) + at]);
+            const int p = bd[j].lo + at;
             if (e & kOpen) {
                 open = j == 0;
-                if (open) {
-                    if (lane == 0) steps[0] = WalkStep{0, p, width, st.t, outOffset + gen};
-                    p = width;
-                }
+                left = open ? bd[0].width : p;
+                if (open && lane == 0) steps[0] = WalkStep{0, p, left, st.t, outOffset + gen};
                 break;
             }
-            const int end = lo + (e & (kAccept - 1));
+            const int value = e & kPlace;
+            const int end = e & kLeave ? bd[j].lo + value : bd[j + 1].lo + value;
+            if (e & kLeave) left = end;
+            at = value;
             if (e & kAccept) {
                 if (lane == 0) steps[j] = WalkStep{1, p, end, j == 0 ? st.t : 0, outOffset + gen};
                 gen++;
             }
-            p = end;
             j++;
         }
+        const int p = left >= 0 ? left : bd[j].lo + at;
         if (lane == 0) {
             WalkState ns = st;
             ns.head = st.head + p;
@@ -532,9 +602,10 @@ __global__ void __launch_bounds__(kAdvanceLanes) k_fg_advance(const FeatGenJob* 
             ns.err = err;
             ns.done = gen >= F || err != 0;
             if (open) {   // its draws count once it has ended
+                const int2 first = firsts[blockIdx.x];
                 ns.openDraws = st.openDraws + p;
-                ns.t = st.t + bd[0].z;
-                ns.tries = bd[0].z > 0 ? 10 - bd[0].w : st.tries - bd[0].w;
+                ns.t = st.t + first.x;
+                ns.tries = first.x > 0 ? 10 - first.y : st.tries - first.y;
             } else if (j > 0) {
                 ns.drawsDone = st.drawsDone + st.openDraws + p;
                 ns.candsDone = st.candsDone + j;
@@ -547,13 +618,13 @@ __global__ void __launch_bounds__(kAdvanceLanes) k_fg_advance(const FeatGenJob* 
     }
     __syncthreads();
     if (tid < groups && groupStart[tid] >= 0) {
-        int p = groupStart[tid], slot = outOffset + groupGen[tid];
+        int at = groupStart[tid], slot = outOffset + groupGen[tid];
         for (int j = tid * kGroup; j < tid * kGroup + kGroup; j++) {
-            const int lo = bd[j].x;
-            const int e = table[j * band + (p - lo)];
-            const int end = lo + (e & (kAccept - 1));
-            if (e & kAccept) steps[j] = WalkStep{1, p, end, j == 0 ? st.t : 0, slot++};
-            p = end;
+            const int e = table[(j << bandShift) + at], after = e & kPlace;
+            if (e & kAccept) {
+                steps[j] = WalkStep{1, bd[j].lo + at, bd[j + 1].lo + after, j == 0 ? st.t : 0, slot++};
+            }
+            at = after;
         }
     }
     __syncthreads();
@@ -575,7 +646,7 @@ __global__ void __launch_bounds__(kAdvanceLanes) k_fg_advance(const FeatGenJob* 
             v[u] = __builtin_nanf("");
             if (j < m && steps[j].st != 2) {
                 const int i = steps[j].begin + lane;
-                if (i < steps[j].end) v[u] = resp[(row0 + j) * band + (i - bd[j].x)];
+                if (i < steps[j].end) v[u] = resp[(row0 + j) * band + (i - bd[j].lo)];
             }
         }
 #pragma unroll
@@ -591,7 +662,7 @@ __global__ void __launch_bounds__(kAdvanceLanes) k_fg_advance(const FeatGenJob* 
                 to += __popcll(fm);
                 i0 += 64;
                 if (i0 >= ws.end) break;
-                cur = i0 + lane < ws.end ? resp[(row0 + j) * band + (i0 + lane - bd[j].x)] : __builtin_nanf("");
+                cur = i0 + lane < ws.end ? resp[(row0 + j) * band + (i0 + lane - bd[j].lo)] : __builtin_nanf("");
             }
         }
     }
@@ -735,7 +806,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     const size_t oWalk = part(n * sizeof(WalkState) + sizeof(int)), oMt = part(n * 624 * sizeof(uint32_t)),
             oRaw = part(n * maxSteps * 256 * sizeof(uint32_t)), oMasks = part(n * maxSteps * 4 * sizeof(uint64_t)),
             oRecs = part(n * ring * sizeof(DrawRec)), oResp = part(perRound * sizeof(float)),
-            oNext = part(perRound * sizeof(uint16_t)), oBands = part(n * m * sizeof(int4));
+            oNext = part(perRound * sizeof(uint16_t)), oFirsts = part(n * sizeof(int2));
     tabs.walkSpace.resize(bytes);
     uint8_t* space = tabs.walkSpace.get();
     WalkState* dWalk = reinterpret_cast<WalkState*>(space + oWalk);
@@ -747,7 +818,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     DrawRec* dRecs = reinterpret_cast<DrawRec*>(space + oRecs);
     float* dResp = reinterpret_cast<float*>(space + oResp);
     uint16_t* dNext = reinterpret_cast<uint16_t*>(space + oNext);
-    int4* dBands = reinterpret_cast<int4*>(space + oBands);
+    int2* dFirsts = reinterpret_cast<int2*>(space + oFirsts);
     // a candidate in twenty or fewer is rejected on ordinary frames: the rest are drawn if they are needed
     auto drawCandidates = [&](int first, int count) {
         if (count > 0) {
@@ -782,10 +853,10 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
         allowLds(reinterpret_cast<const void*>(&k_fg_advance), lds);
         for (int r = 0; r < rounds; r++) {
             hipLaunchKernelGGL(k_fg_round, dim3(m, numJobs), dim3(std::min(band, 256)), 0, s, dWalk, imgs,
-                    tabs.cand.get(), numCand, drawn, T, ring, band, dRecs, dResp, dNext, dBands);
+                    tabs.cand.get(), numCand, drawn, T, ring, band, dRecs, dResp, dNext, dFirsts);
             hipLaunchKernelGGL(k_fg_advance, dim3(numJobs), dim3(kAdvanceLanes), lds, s, jobsDev, dWalk,
-                    tabs.cand.get(), numCand, F, T, band, m, dResp, dNext, dBands, tabs.unsortedFeat.get(),
-                    tabs.unsortedThr.get(), tabs.unsortedKey.get());
+                    tabs.cand.get(), numCand, drawn, F, T, band, m, dResp, dNext, dFirsts,
+                    tabs.unsortedFeat.get(), tabs.unsortedThr.get(), tabs.unsortedKey.get());
         }
         hipLaunchKernelGGL(k_fg_sort, dim3((F + kSortFeat - 1) / kSortFeat, numJobs), dim3(256), F * sizeof(int), s,
                 tabs.unsortedKey.get(), tabs.unsortedFeat.get(), tabs.unsortedThr.get(), F, T, TM, tabs.feat.get(),
