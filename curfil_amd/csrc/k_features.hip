@@ -8,8 +8,8 @@
 // RandomSource(seed) hands seed to the sample-index sampler and seeds
 // seed+1+4k .. seed+4+4k to candidate k's four samplers (type, offset,
 // region, channel).  Candidates are therefore independent and are drawn in
-// parallel (k_fg_candidates), and so is the stream of sample-index draws
-// (k_fg_draws, k_fg_records).  Thresholds consume that one stream in order, and
+// parallel, and so is the stream of sample-index draws (k_fg_draws,
+// k_fg_records).  Thresholds consume that one stream in order, and
 // how many draws a candidate consumes depends on which responses are NaN, so a
 // candidate's first draw is known only after its predecessor's last.  That
 // chain is taken in rounds of two launches:
@@ -43,21 +43,23 @@ constexpr int kPrefixDraws = 24;   // engine outputs available to one feature sa
 // g++ on x86-64 evaluates the two getNext() calls of `Offset(rgen.getNext(),
 // rgen.getNext())` right to left, so the second coordinate is drawn first
 // (pinned by the reference's golden feature hash).
-__global__ void __launch_bounds__(256) k_fg_candidates(const FeatGenJob* __restrict__ jobs, int numCand, int first, int count,
-        int boxRadius, int regionSize, int useDepth, FeatRec* __restrict__ cand, int* __restrict__ err) {
+constexpr int kCandBlock = 64;   // candidates of a workgroup (its first 256 lanes)
+__device__ __forceinline__ void drawCandidates(const FeatGenJob* __restrict__ jobs, int job, int block, int numCand,
+        int first, int count, int boxRadius, int regionSize, int useDepth, FeatRec* __restrict__ cand,
+        int* __restrict__ err) {
     constexpr int kStride = kPrefixDraws + 1;
-    __shared__ uint32_t outputs[256 * kStride];
-    const int job = blockIdx.y;
+    __shared__ uint32_t outputs[4 * kCandBlock * kStride];
+    if (threadIdx.x >= 4 * kCandBlock) return;
     {
-        const int k = first + blockIdx.x * 64 + static_cast<int>(threadIdx.x >> 2);
+        const int k = first + block * kCandBlock + static_cast<int>(threadIdx.x >> 2);
         uint32_t out[kPrefixDraws];
         mtPrefix<kPrefixDraws>(static_cast<uint32_t>(jobs[job].seed + 1 + 4 * k + static_cast<int>(threadIdx.x & 3)), out);
 #pragma unroll
         for (int i = 0; i < kPrefixDraws; i++) outputs[threadIdx.x * kStride + i] = out[i];
     }
     __syncthreads();
-    const int k = first + blockIdx.x * 64 + threadIdx.x;
-    if (threadIdx.x >= 64 || k >= first + count) return;
+    const int k = first + block * kCandBlock + threadIdx.x;
+    if (threadIdx.x >= kCandBlock || k >= first + count) return;
     const uint32_t* mine = outputs + threadIdx.x * 4 * kStride;   // samplers: type, offset, region, channel
     FeatRec f;
 #pragma unroll
@@ -131,19 +133,31 @@ __device__ __forceinline__ int featureSortKey(const FeatRec& f) {
 __host__ __device__ __forceinline__ int minDraws(int T) { return T < 10 ? T : 10; }
 
 // The next words of each job's index generator: as many as the features still missing are expected to
-// take, tempered, and per wave the mask of those that uniform_int accepts.  MT19937 as the recurrence
-// x[n + 624] = mix(x[n], x[n + 1], x[n + 397]), 227 words a step (no word of a step depends on another) in
-// an LDS ring with one barrier a step.  One workgroup per job: bound by the latency of a step.  uniform_int
-// accepts a word w iff w / bucket <= range, that is iff w < bucket (range + 1).
+// take, tempered, and per wave the mask of those that uniform_int accepts; and, in the workgroups past the
+// first, the job's next candidates, which wait for nothing of it.  MT19937 as the recurrence x[n + 624] =
+// mix(x[n], x[n + 1], x[n + 397]) in an LDS ring: no word of the 227 after the last depends on another, and a
+// lane's word 227 further on needs its own word and older ones, so four waves make two such steps per barrier
+// while eight others temper, test and store the two before.  Bound by the latency of a step, after the 624
+// dependent ones that seed the generator (with one step a barrier and all of it in the same four waves, and the
+// candidates in a launch of their own: 59 + 13 us for 2000 features x 20 thresholds, 12 + 12 for 100 x 10; now
+// 50 and 14).  uniform_int accepts a word w iff w / bucket <= range, that is iff w < bucket (range + 1).
 constexpr int kMtStep = 227;
 constexpr int kMtRing = 2048;
-__global__ void __launch_bounds__(256) k_fg_draws(const FeatGenJob* __restrict__ jobs, int F, int T, int ring,
+constexpr int kDrawLanes = 768;
+__global__ void __launch_bounds__(kDrawLanes) k_fg_draws(const FeatGenJob* __restrict__ jobs, int F, int T, int ring,
         int fresh, float guess, WalkState* __restrict__ states, uint32_t* __restrict__ mtState, uint32_t* __restrict__ raw,
-        unsigned long long* __restrict__ masks, int maxSteps) {
+        unsigned long long* __restrict__ masks, int maxSteps, int numCand, int first, int count, int boxRadius,
+        int regionSize, int useDepth, FeatRec* __restrict__ cand, int* __restrict__ err) {
     __shared__ uint32_t x[kMtRing];
-    __shared__ int counts[4];
-    const FeatGenJob job = jobs[blockIdx.x];
-    WalkState st = states[blockIdx.x];
+    __shared__ int counts[kDrawLanes / 64];
+    const int jobIdx = blockIdx.y;
+    if (blockIdx.x > 0) {
+        drawCandidates(jobs, jobIdx, static_cast<int>(blockIdx.x) - 1, numCand, first, count, boxRadius, regionSize,
+                useDepth, cand, err);
+        return;
+    }
+    const FeatGenJob job = jobs[jobIdx];
+    WalkState st = states[jobIdx];
     if (fresh) {
         st = WalkState{};
         st.tries = 10;
@@ -152,9 +166,9 @@ __global__ void __launch_bounds__(256) k_fg_draws(const FeatGenJob* __restrict__
     if (st.done) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const UniformIntParams up = uniformIntParams(0, job.n - 1);
-    uint32_t* saved = mtState + static_cast<size_t>(blockIdx.x) * 624;
+    uint32_t* saved = mtState + static_cast<size_t>(jobIdx) * 624;
     if (!fresh) {
-        for (int i = tid; i < 624; i += 256) x[i] = saved[i];
+        for (int i = tid; i < 624; i += kDrawLanes) x[i] = saved[i];
     } else if (tid == 0) {
         uint32_t v = static_cast<uint32_t>(job.seed);
         x[0] = v;
@@ -176,36 +190,49 @@ __global__ void __launch_bounds__(256) k_fg_draws(const FeatGenJob* __restrict__
         // at least half of the words are accepted, so the ring (at most ring - 512 ahead of the walk before
         // this, and no more than `missing` words over that) never overruns
         steps = min(maxSteps, min(static_cast<int>(missing / share), ring - 512 - (st.tail - st.head)) / kMtStep + (missing > 0 ? 1 : 0));
-        uint32_t* out = raw + static_cast<size_t>(blockIdx.x) * maxSteps * 256;
-        unsigned long long* mk = masks + static_cast<size_t>(blockIdx.x) * maxSteps * 4;
-        int base = 0;
+        uint32_t* out = raw + static_cast<size_t>(jobIdx) * maxSteps * 256;
+        unsigned long long* mk = masks + static_cast<size_t>(jobIdx) * maxSteps * 4;
         made = 0;
-        for (int s = 0; s < steps; s++) {
-            bool acc = false;
-            if (tid < kMtStep) {
-                const int i = base + tid;
-                const uint32_t w = mtMix(x[i & (kMtRing - 1)], x[(i + 1) & (kMtRing - 1)], x[(i + 397) & (kMtRing - 1)]);
-                x[(i + 624) & (kMtRing - 1)] = w;
-                const uint32_t v = mtTemper(w);
-                acc = v < limit;
-                out[s * 256 + tid] = v;
+        // lanes 0 .. 255 make steps s and s + 1, lanes 256 .. 511 and 512 .. 767 test steps s - 2 and s - 1
+        const int half = tid >> 8, i = tid & 255;
+        for (int s = 0; s < steps + 2; s += 2) {
+            const int base = s * kMtStep + i;
+            if (half == 0) {
+                if (s < steps && i < kMtStep) {
+                    const uint32_t a0 = x[base & (kMtRing - 1)], a1 = x[(base + 1) & (kMtRing - 1)];
+                    const uint32_t b0 = x[(base + kMtStep) & (kMtRing - 1)], b1 = x[(base + kMtStep + 1) & (kMtRing - 1)];
+                    const uint32_t w0 = mtMix(a0, a1, x[(base + 397) & (kMtRing - 1)]);
+                    x[(base + 624) & (kMtRing - 1)] = w0;
+                    x[(base + kMtStep + 624) & (kMtRing - 1)] = mtMix(b0, b1, w0);
+                }
+            } else {
+                const int step = s - 3 + half;
+                if (step >= 0 && step < steps) {
+                    bool acc = false;
+                    if (i < kMtStep) {
+                        const uint32_t v = mtTemper(x[(base + 624 - (3 - half) * kMtStep) & (kMtRing - 1)]);
+                        acc = v < limit;
+                        out[step * 256 + i] = v;
+                    }
+                    const unsigned long long mask = __ballot(acc);
+                    if (lane == 0) mk[step * 4 + (wave & 3)] = mask;
+                    made += __popcll(mask);
+                }
             }
-            const unsigned long long mask = __ballot(acc);
-            if (lane == 0) mk[s * 4 + wave] = mask;
-            made += __popcll(mask);
-            base += kMtStep;
             __syncthreads();
         }
+        const int base = steps * kMtStep;
         if (lane == 0) counts[wave] = made;
         __syncthreads();
-        made = counts[0] + counts[1] + counts[2] + counts[3];
-        for (int i = tid; i < 624; i += 256) saved[i] = x[(base + i) & (kMtRing - 1)];
+        made = 0;
+        for (int w = 4; w < kDrawLanes / 64; w++) made += counts[w];
+        for (int i = tid; i < 624; i += kDrawLanes) saved[i] = x[(base + i) & (kMtRing - 1)];
     }
     if (tid == 0) {
         st.recorded = st.tail;
         st.tail += made;
         st.steps = steps;
-        states[blockIdx.x] = st;
+        states[jobIdx] = st;
     }
 }
 
@@ -820,14 +847,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     uint16_t* dNext = reinterpret_cast<uint16_t*>(space + oNext);
     int2* dFirsts = reinterpret_cast<int2*>(space + oFirsts);
     // a candidate in twenty or fewer is rejected on ordinary frames: the rest are drawn if they are needed
-    auto drawCandidates = [&](int first, int count) {
-        if (count > 0) {
-            hipLaunchKernelGGL(k_fg_candidates, dim3((count + 63) / 64, numJobs), dim3(256), 0, s, jobsDev, numCand, first,
-                    count, boxRadius, regionSize, useDepth, tabs.cand.get(), dErr);
-        }
-    };
-    int drawn = std::min(numCand, F + F / 8 + 64);
-    drawCandidates(0, drawn);
+    int drawnBefore = 0, drawn = std::min(numCand, F + F / 8 + 64);
     const size_t stateBytes = n * sizeof(WalkState) + sizeof(int);
     uint8_t* host = tabs.walkHost.resize(stateBytes);
     std::memset(host, 0, stateBytes);
@@ -844,8 +864,11 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
         // (without a table before this one to go by, the first rounds are short: a candidate's mean use is
         // only guessed)
         const int rounds = std::min(64, missing / std::max(1, m * 9 / 10) + (fresh && tabs.meanDraws > 0 ? 2 : 4));
-        hipLaunchKernelGGL(k_fg_draws, dim3(numJobs), dim3(256), 0, s, jobsDev, F, T, ring, fresh ? 1 : 0, guess,
-                dWalk, dMt, dRaw, dMasks, maxSteps);
+        const int candBlocks = (drawn - drawnBefore + kCandBlock - 1) / kCandBlock;
+        hipLaunchKernelGGL(k_fg_draws, dim3(1 + candBlocks, numJobs), dim3(kDrawLanes), 0, s, jobsDev, F, T, ring,
+                fresh ? 1 : 0, guess, dWalk, dMt, dRaw, dMasks, maxSteps, numCand, drawnBefore, drawn - drawnBefore,
+                boxRadius, regionSize, useDepth, tabs.cand.get(), dErr);
+        drawnBefore = drawn;
         const int steps = static_cast<int>(std::min<double>(maxSteps, 1.4 * missing * T / kMtStep + 12));
         hipLaunchKernelGGL(k_fg_records, dim3(steps, numJobs), dim3(256), 0, s, jobsDev, dWalk, ring, dRaw,
                 dMasks, maxSteps, dRecs);
@@ -871,10 +894,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
             more = more || !states[j].done;
         }
         if (errHost != 0) break;
-        if (more && drawn < numCand) {
-            drawCandidates(drawn, numCand - drawn);
-            drawn = numCand;
-        }
+        if (more) drawn = numCand;
     }
     double draws = 0, cands = 0;
     for (int j = 0; j < numJobs; j++) {
