@@ -333,13 +333,15 @@ void launchResponsesPaired(hipStream_t s, const DevImage* imgs, const cf_sample*
         double* out);
 
 // Partition
-// split record of node i from best[i] and the feature table of tree nodeTree[i]
-void launchSplitRecords(hipStream_t s, const NodeBest* best, const int* nodeTree, int numNodes, const FeatTables& tabs,
-        SplitRec* out);
-void launchPartitionDirections(hipStream_t s, const DevImage* imgs, const cf_sample* samples, const Chunk* chunks,
-        int numChunks, const SplitRec* splits, int C, uint8_t* dir, int2* chunkCounts, uint32_t* leftHist);
-void launchPartitionScatter(hipStream_t s, const cf_sample* samples, const Chunk* chunks, int numChunks,
-        const uint8_t* dir, const int2* dst, cf_sample* out);
+// the parts that a level's chunks are cut into, of partLen places each (the last may be shorter, or empty)
+int partitionParts(int numChunks);
+// the split records of the level's nodes from their argmax, every sample's direction, the left and right entries
+// of every chunk's parts
+void launchPartitionDirections(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk* chunks,
+        int numChunks, int parts, int partLen, const NodeBest* best, const int* nodeTree, const FeatTables& tabs, int C,
+        SplitRec* splits, uint8_t* dir, int2* partCounts, uint32_t* leftHist);
+void launchPartitionScatter(hipStream_t s, const cf_sample* samples, const Chunk* chunks, int numChunks, int parts,
+        int partLen, const uint8_t* dir, const int2* partCounts, const int2* dst, cf_sample* out);
 
 // Prediction
 //

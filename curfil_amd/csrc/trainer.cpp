@@ -484,15 +484,16 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
         const int numChunks = static_cast<int>(chunks.size());
         const double evalMsBefore = stats.evalKernelMs;
         // what the host reads of a level, in one buffer: split record and argmax per node, left and right
-        // entries per chunk, left class histogram per node
+        // entries per part of a chunk, left class histogram per node
+        const int parts = partitionParts(numChunks), partLen = (kChunk + parts - 1) / parts;
         const size_t splitsAt = 0, bestAt = splitsAt + numNodes * sizeof(SplitRec),
-                countsAt = bestAt + numNodes * sizeof(NodeBest), histAt = countsAt + numChunks * sizeof(int2),
+                countsAt = bestAt + numNodes * sizeof(NodeBest), histAt = countsAt + static_cast<size_t>(numChunks) * parts * sizeof(int2),
                 resultBytes = histAt + static_cast<size_t>(numNodes) * C * sizeof(uint32_t);
         static_assert(sizeof(SplitRec) % 8 == 0 && sizeof(NodeBest) % 8 == 0, "alignment of the parts that follow");
         ws.results.resize(resultBytes + 16);
         NodeBest* dBest = reinterpret_cast<NodeBest*>(ws.results.get() + bestAt);
         SplitRec* dSplits = reinterpret_cast<SplitRec*>(ws.results.get() + splitsAt);
-        int2* dChunkCounts = reinterpret_cast<int2*>(ws.results.get() + countsAt);
+        int2* dPartCounts = reinterpret_cast<int2*>(ws.results.get() + countsAt);
         uint32_t* dLeftHist = reinterpret_cast<uint32_t*>(ws.results.get() + histAt);
         uint8_t* hostResults = ws.hostResults.resize(resultBytes + 16);
         NodeBest* best = reinterpret_cast<NodeBest*>(hostResults + bestAt);
@@ -837,11 +838,10 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
         // directions; the level's one read-back.  Nodes of a two-pass level whose argmax has to be replayed show
         // up in it: they are replayed, and the records and directions made again.
         for (bool again = twoPass;; again = false) {
-            launchSplitRecords(s, dBest, dNodeTree, numNodes, tabs, dSplits);
             CF_HIP(hipMemsetAsync(dLeftHist, 0, static_cast<size_t>(numNodes) * C * sizeof(uint32_t), s));
             timer.begin();
-            launchPartitionDirections(s, images->desc.get(), level[cur].get(), dChunks, numChunks, dSplits, C, dir.get(),
-                    dChunkCounts, dLeftHist);
+            launchPartitionDirections(s, images->set(), level[cur].get(), dChunks, numChunks, parts, partLen, dBest,
+                    dNodeTree, tabs, C, dSplits, dir.get(), dPartCounts, dLeftHist);
             timer.end(stats.partitionMs);
             CF_HIP(hipMemcpyAsync(hostResults, ws.results.get(), resultBytes, hipMemcpyDeviceToHost, s));
             CF_HIP(hipStreamSynchronize(s));
@@ -855,7 +855,15 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             replayNodes(flagged);
         }
         const SplitRec* splits = reinterpret_cast<const SplitRec*>(hostResults + splitsAt);
-        const int2* chunkCounts = reinterpret_cast<const int2*>(hostResults + countsAt);
+        int2* chunkCounts = reinterpret_cast<int2*>(hostResults + countsAt);   // of the parts, then of the chunks
+        for (int c = 0; c < numChunks; c++) {
+            int2 sum = make_int2(0, 0);
+            for (int q = 0; q < parts; q++) {
+                sum.x += chunkCounts[c * parts + q].x;
+                sum.y += chunkCounts[c * parts + q].y;
+            }
+            chunkCounts[c] = sum;
+        }
         const uint32_t* leftHist = reinterpret_cast<const uint32_t*>(hostResults + histAt);
 
         // ---- tree growth on the host, next frontier and sample destinations
@@ -936,7 +944,8 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             const int2* dDst = up.put(dst);
             up.flush(s);
             timer.begin();
-            launchPartitionScatter(s, level[cur].get(), dChunks, numChunks, dir.get(), dDst, level[1 - cur].get());
+            launchPartitionScatter(s, level[cur].get(), dChunks, numChunks, parts, partLen, dir.get(), dPartCounts, dDst,
+                    level[1 - cur].get());
             timer.end(stats.partitionMs);
             cur = 1 - cur;
         }

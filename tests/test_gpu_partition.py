@@ -1,0 +1,46 @@
+"""GPU training against the oracle where a level's samples are cut into chunks and parts of chunks."""
+import numpy as np
+import pytest
+
+import curfil_amd as cf
+import oracle as orc
+from helpers import random_samples, random_u8_dataset
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def frames(ctx):
+    rgb, depth, labels = random_u8_dataset(3, 160, 120, seed=8)
+    im = cf.Images(ctx, 3, 160, 120)
+    for i in range(3):
+        im.set_rgbd_u8(i, rgb[i], depth[i])
+    return depth, labels, im, orc.Dataset.from_u8(rgb, depth, labels)
+
+
+# a part of 512 samples, one less and one more; a whole chunk of 4096 and its neighbours; the numbers of chunks past which
+# they are cut into 4, 2 and no parts instead of 8
+@pytest.mark.parametrize("n", [511, 512, 513, 4095, 4096, 4097, 4096 * 128 + 1, 4096 * 256 + 1, 4096 * 512 + 1])
+@pytest.mark.parametrize("flip", [False, True])
+@pytest.mark.parametrize("mode", [cf.MODE_BATCHED, cf.MODE_PLAIN])
+def test_partition_edges_match_oracle(ctx, frames, n, flip, mode):
+    depth, labels, im, ds = frames
+    rng = np.random.default_rng(n)
+    s = random_samples(rng, n, 3, 160, 120, depth.astype(np.int32), labels=labels)
+    s["label"] = rng.integers(0, 5, n)
+    s["flip"] = 2 if flip else 0
+    s = s[s["depth_mm"] > 0]
+    s = np.resize(s, n)
+    params = dict(randomSeed=99, samplesPerImage=1, featureCount=3, minSampleCount=2, maxDepth=4, boxRadius=20,
+                  regionSize=6, thresholds=2, horizontalFlipping=flip)
+    forest = cf.RandomForestImage.train_tree_from_samples(ctx, im, cf.TrainingConfiguration(**params), 0, 5, 99, s,
+                                                          mode=mode)
+    nodes, hist = forest.tree(0)
+    on, oh = ds.train_tree(orc.config(**params), 0, 5, 99, s)
+    assert len(nodes) == len(on) > 1
+    inner = on["is_leaf"] == 0
+    for name in ("id", "level", "parent", "left", "right", "num_samples", "is_leaf"):
+        assert np.array_equal(nodes[name], on[name]), name
+    for name in ("feature", "threshold"):
+        assert np.array_equal(nodes[name][inner], on[name][inner]), name
+    assert np.array_equal(hist, oh)
