@@ -219,6 +219,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
 void launchPrepareTables(hipStream_t s, int trees, int F, int T, FeatTables& tabs);
 
 // Evaluation work item: a chunk of one node's samples.
+constexpr int kChunk = 4096;   // samples of a batched level's chunks
 struct Chunk {
     int slot;   // node slot within the launch batch
     int tree;   // tree index (feature table)

@@ -7,9 +7,9 @@
 //                 interval among the feature's thresholds (the bin used by the
 //                 interval histograms) and stores the 16 bins of a sample as
 //                 one 16-byte row, bins[group][level index].
-//   k_hist_bins   pass 2, node-major: one workgroup per (node chunk, group)
-//                 streams the chunk's bin rows and labels into LDS interval
-//                 histograms and adds them to the node's global bins.
+//   k_hist_bins   pass 2, node-major: one workgroup per (part of a node
+//                 chunk, group) streams the part's bin rows and labels into LDS
+//                 interval histograms and adds them to the node's global bins.
 //
 // Counting is order-independent, so the histograms equal those of the direct
 // path (k_eval_hist), whose single kernel gathers the integrals in node order:
@@ -204,60 +204,81 @@ __global__ void __launch_bounds__(WAVES * 64) k_eval_bins(const float* __restric
     }
 }
 
-// Pass 2: interval histograms of (node chunk, feature group) from the bin rows.
-// G holds the batch's groups: G[slot][ng * 16][T + 1][C].  Lane l counts
-// feature l % 16 of sample l / 16, so one LDS atomic instruction covers 4
-// samples x 16 features: the 16 features' histograms lie in different banks
-// and at most 4 lanes can hit one address (all lanes counting one feature, as
-// for samples of an almost pure node, would collide on few bins).
+// Pass 2: interval histograms of (part of a node chunk, feature group) from the bin rows.
+// G holds the batch's groups: G[slot][ng * 16][T + 1][C].  Bound by the LDS atomics and the instructions that
+// form their addresses: a lane takes four features of a sample in one word, 16 samples a wave, and its features in
+// an order rotated by the sample, so that one LDS atomic instruction covers 4 samples of each of the 16
+// features: their histograms lie in different banks and at most 4 lanes can hit one address (all lanes counting
+// one feature, as for samples of an almost pure node, would collide on few bins).  Features past the table's last
+// hold anything in the rows; they are counted into histograms that nothing reads.  Of the LDS cycles, 70% of
+// the time, a third are banks met twice and a third equal addresses (samples of one class in one bin).
+// One feature of a sample a lane took a byte load and three times the instructions for each atomic, and a
+// chunk was not cut into parts: 13 flipped frames, 500 x 50 108 us a level (now 36); 4 small frames 19 (5); 21
+// frames, 3 trees, 2000 x 20 199 (151); 50 frames, 5 trees, 4000 x 32 1562 (1245).
 __global__ void __launch_bounds__(256) k_hist_bins(const uint4* __restrict__ bins, const uint8_t* __restrict__ labels,
-        const Chunk* __restrict__ chunks, int slotBase, int g0, int ng, int F, int T, int C, int N,
-        uint32_t* __restrict__ G, size_t flipOffset) {
+        const Chunk* __restrict__ chunks, int parts, int partLen, int slotBase, int g0, int ng, int F, int T, int C,
+        int N, uint32_t* __restrict__ G, size_t flipOffset) {
     extern __shared__ uint32_t h[];
-    const int chunkIdx = blockIdx.x / ng;
+    const int partIdx = blockIdx.x / ng;
     const int g = blockIdx.x % ng;
-    const Chunk ch = chunks[chunkIdx];
+    Chunk ch = chunks[partIdx / parts];
+    const int from = partIdx % parts * partLen;
+    ch.begin += from;
+    ch.count = min(ch.count - from, partLen);
+    if (ch.count <= 0) return;
     const int nf = min(kBinGroup, F - (g0 + g) * kBinGroup);
     const int binsPerF = (T + 1) * C;
-    const int nb = nf * binsPerF;
-    for (int k = threadIdx.x; k < nb; k += 256) h[k] = 0;
+    for (int k = threadIdx.x; k < kBinGroup * binsPerF; k += 256) h[k] = 0;
     __syncthreads();
-    const int fi = threadIdx.x & (kBinGroup - 1);
-    const int sub = threadIdx.x >> 4;   // 16 samples per pass of the workgroup
-    const uint8_t* row = reinterpret_cast<const uint8_t*>(bins + static_cast<size_t>(g) * N + ch.begin);
-    const uint8_t* rowFlip = reinterpret_cast<const uint8_t*>(bins + flipOffset + static_cast<size_t>(g) * N + ch.begin);
+    constexpr int kWords = kBinGroup / 4;   // words of a row, lanes of a sample
+    const int word = threadIdx.x % kWords;
+    const int sub = threadIdx.x / kWords;   // 64 samples per pass of the workgroup
+    const size_t row0 = static_cast<size_t>(g) * N + ch.begin;
+    const uint32_t* row = reinterpret_cast<const uint32_t*>(bins + row0) + word;
+    const uint32_t* rowFlip = reinterpret_cast<const uint32_t*>(bins + flipOffset + row0) + word;
     const uint8_t* lab = labels + ch.begin;
-    uint32_t* hf = h + fi * binsPerF;
-    if (fi < nf) {
-        constexpr int kUnroll = 16;   // bins loaded ahead of their atomics (8: 4% slower, 4: 19% slower)
-        for (int base = 0; base < ch.count; base += 16 * kUnroll) {
-            int b[kUnroll], l[kUnroll];
+    int shift[4];
+    uint32_t* hf[4];
 #pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                const int i = base + u * 16 + sub;
-                l[u] = -1;
-                if (i < ch.count) {
-                    b[u] = row[static_cast<size_t>(i) * kBinGroup + fi];
-                    l[u] = lab[i];
-                }
+    for (int k = 0; k < 4; k++) {
+        const int byte = (k + sub) & 3;
+        shift[k] = 8 * byte;
+        hf[k] = h + (word * 4 + byte) * binsPerF;
+    }
+    // bins are 0..T; the clamp keeps the LDS index inside the histogram whatever a row holds
+    auto count = [&](uint32_t v, int label) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int bin = min(static_cast<int>((v >> shift[k]) & 0xffu), T);
+            atomicAdd(&hf[k][bin * C + label], 1u);
+        }
+    };
+    constexpr int kUnroll = 8;   // words loaded ahead of their atomics
+    constexpr int kPass = 256 / kWords;
+    for (int base = 0; base < ch.count; base += kPass * kUnroll) {
+        uint32_t v[kUnroll];
+        int l[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; u++) {
+            const int i = base + u * kPass + sub;
+            l[u] = -1;
+            if (i < ch.count) {
+                v[u] = row[static_cast<size_t>(i) * kWords];
+                l[u] = lab[i];
             }
+        }
 #pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                // bins are 0..T; the clamp keeps the LDS index inside the histogram whatever a row holds
-                if (l[u] >= 0) {
-                    atomicAdd(&hf[min(b[u], T) * C + (l[u] & 0x7f)], 1u);
-                    if (l[u] & 0x80) {   // still Both: its flipped evaluation counts too
-                        const int i = base + u * 16 + sub;
-                        atomicAdd(&hf[min(static_cast<int>(rowFlip[static_cast<size_t>(i) * kBinGroup + fi]), T) * C +
-                                (l[u] & 0x7f)], 1u);
-                    }
-                }
+        for (int u = 0; u < kUnroll; u++) {
+            if (l[u] >= 0) {
+                count(v[u], l[u] & 0x7f);
+                // still Both: its flipped evaluation counts too
+                if (l[u] & 0x80) count(rowFlip[static_cast<size_t>(base + u * kPass + sub) * kWords], l[u] & 0x7f);
             }
         }
     }
     __syncthreads();
     uint32_t* out = G + (static_cast<size_t>(ch.slot - slotBase) * ng + g) * kBinGroup * binsPerF;
-    for (int k = threadIdx.x; k < nb; k += 256) {
+    for (int k = threadIdx.x; k < nf * binsPerF; k += 256) {
         const uint32_t v = h[k];
         if (v) atomicAdd(&out[k], v);
     }
@@ -471,8 +492,12 @@ void launchHistBins(hipStream_t s, const uint4* bins, const uint8_t* labels, con
     if (numChunks == 0 || ng == 0) return;
     const size_t lds = static_cast<size_t>(kBinGroup) * (tabs.T + 1) * C * sizeof(uint32_t);
     allowLds(reinterpret_cast<const void*>(&k_hist_bins), lds);
-    hipLaunchKernelGGL(k_hist_bins, dim3(static_cast<unsigned>(numChunks) * ng), dim3(256), lds, s, bins, labels,
-            chunks, slotBase, g0, ng, tabs.F, tabs.T, C, N, G, flipOffset);
+    // few chunks and groups: chunks cut into parts while that gives at most 2048 workgroups
+    int parts = 1;
+    while (parts < 8 && static_cast<int64_t>(2) * parts * numChunks * ng <= 2048) parts *= 2;
+    const int partLen = (kChunk + parts - 1) / parts;
+    hipLaunchKernelGGL(k_hist_bins, dim3(static_cast<unsigned>(numChunks) * parts * ng), dim3(256), lds, s, bins, labels,
+            chunks, parts, partLen, slotBase, g0, ng, tabs.F, tabs.T, C, N, G, flipOffset);
 }
 
 }  // namespace cf

@@ -32,8 +32,6 @@ namespace cf {
 
 namespace {
 
-constexpr int kChunk = 4096;
-
 struct ActiveTree {
     int job;                  // index into jobs / out
     int idNode;               // last assigned node id
