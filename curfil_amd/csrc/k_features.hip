@@ -711,59 +711,57 @@ __device__ __forceinline__ uint16_t thresholdRank(const float* __restrict__ th, 
 // th < q), and, where asked for, the reference's layouts.  The keys start with (type, channel1, channel2), so
 // the sorted order also groups the features by the planes they read.
 //
-// A workgroup ranks kSortFeat features: lane l of each wave takes feature l and a quarter of the keys, which
-// lie in LDS (one feature per lane over all keys, and a lane per feature for the threshold tables, took
-// 136 + 218 us for 5 x 4000 features with 32 thresholds).
-constexpr int kSortFeat = 64;
-__global__ void __launch_bounds__(256) k_fg_sort(const int* __restrict__ keys, const FeatRec* __restrict__ inFeat,
-        const float* __restrict__ inThr, int F, int T, int TM, FeatRec* __restrict__ feat, float* __restrict__ thrFT,
-        uint16_t* __restrict__ rank, float* __restrict__ thrPad,
+// A workgroup ranks kSortFeat features against all keys, which lie in LDS, 16 lanes a feature, and the features'
+// thresholds against one another, in LDS too.  Bound by those reads: 12 us for 3 x 2000
+// features with 20 thresholds, 9.5 for 2 x 500 with 50 (21 and 29 with 64 features a workgroup, a lane a feature,
+// thresholds read from memory).
+constexpr int kSortFeat = 16, kSortLanes = 16;   // features of a workgroup, lanes of a feature
+__global__ void __launch_bounds__(kSortFeat * kSortLanes) k_fg_sort(const int* __restrict__ keys,
+        const FeatRec* __restrict__ inFeat, const float* __restrict__ inThr, int F, int T, int TM,
+        FeatRec* __restrict__ feat, float* __restrict__ thrFT, uint16_t* __restrict__ rank, float* __restrict__ thrPad,
         float* __restrict__ thrTF, int8_t* __restrict__ soa) {
-    extern __shared__ int sk[];
-    __shared__ int part[4][kSortFeat];
+    extern __shared__ int sk[];                       // [F] keys
+    float* th = reinterpret_cast<float*>(sk + F);     // [kSortFeat][T]
+    __shared__ int place[kSortFeat];
+    constexpr int kLanes = kSortFeat * kSortLanes;
     const size_t jobF = static_cast<size_t>(blockIdx.y) * F;
-    for (int i = threadIdx.x; i < F; i += 256) sk[i] = keys[jobF + i];
+    const int i0 = blockIdx.x * kSortFeat, nf = min(kSortFeat, F - i0);
+    for (int i = threadIdx.x; i < F; i += kLanes) sk[i] = keys[jobF + i];
+    for (int e = threadIdx.x; e < nf * T; e += kLanes) th[e] = inThr[(jobF + i0) * T + e];
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int i0 = blockIdx.x * kSortFeat, i = i0 + lane;
-    {
-        const int ki = i < F ? sk[i] : 0;
-        const int a = static_cast<int>(static_cast<int64_t>(F) * wave / 4), b = static_cast<int>(static_cast<int64_t>(F) * (wave + 1) / 4);
-        const int m1 = min(max(a, i0), b), m2 = min(max(a, i0 + kSortFeat), b);   // [m1, m2): the workgroup's own
+    const int own = threadIdx.x / kSortLanes, sub = threadIdx.x % kSortLanes;
+    if (own < nf) {
+        const int i = i0 + own, ki = sk[i];
         int r = 0;
 #pragma unroll 8
-        for (int j = a; j < m1; j++) r += sk[j] <= ki ? 1 : 0;
-        for (int j = m1; j < m2; j++) r += (sk[j] < ki || (sk[j] == ki && j < i)) ? 1 : 0;
-#pragma unroll 8
-        for (int j = m2; j < b; j++) r += sk[j] < ki ? 1 : 0;
-        part[wave][lane] = r;
-    }
-    __syncthreads();
-    const int nf = min(kSortFeat, F - i0);
-    if (threadIdx.x < nf) {
-        const int r = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
-        part[0][lane] = r;
-        const FeatRec fr = inFeat[jobF + i];
-        feat[jobF + r] = fr;
-        if (soa) {
-            for (int p = 0; p < kFeatParams; p++) soa[(static_cast<size_t>(blockIdx.y) * kFeatParams + p) * F + r] = fr.p[p];
+        for (int j = sub; j < F; j += kSortLanes) r += (sk[j] < ki || (sk[j] == ki && j < i)) ? 1 : 0;
+#pragma unroll
+        for (int o = kSortLanes / 2; o > 0; o >>= 1) r += __shfl_xor(r, o, kSortLanes);
+        if (sub == 0) {
+            place[own] = r;
+            const FeatRec fr = inFeat[jobF + i];
+            feat[jobF + r] = fr;
+            if (soa) {
+                for (int p = 0; p < kFeatParams; p++) {
+                    soa[(static_cast<size_t>(blockIdx.y) * kFeatParams + p) * F + r] = fr.p[p];
+                }
+            }
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < nf * T; e += 256) {
-        const int l = e / T, t = e - l * T, dst = part[0][l];
-        const float* th = inThr + (jobF + i0 + l) * T;
-        const float v = th[t];
+    for (int e = threadIdx.x; e < nf * T; e += kLanes) {
+        const int l = e / T, t = e - l * T, dst = place[l];
+        const float v = th[e];
         const size_t row = (jobF + dst) * T;
         thrFT[row + t] = v;
-        rank[row + t] = thresholdRank(th, T, t);
+        rank[row + t] = thresholdRank(th + l * T, T, t);
         thrPad[(jobF + dst) * TM + t] = (v != v) ? __builtin_inff() : v + 0.0f;
         if (thrTF) thrTF[(static_cast<size_t>(blockIdx.y) * T + t) * F + dst] = v;
     }
     const int padT = TM - T;
-    for (int e = threadIdx.x; e < nf * padT; e += 256) {
+    for (int e = threadIdx.x; e < nf * padT; e += kLanes) {
         const int l = e / padT;
-        thrPad[(jobF + part[0][l]) * TM + T + (e - l * padT)] = __builtin_inff();
+        thrPad[(jobF + place[l]) * TM + T + (e - l * padT)] = __builtin_inff();
     }
 }
 
@@ -874,6 +872,7 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
                 dMasks, maxSteps, dRecs);
         const size_t lds = static_cast<size_t>(m) * band * 2 + static_cast<size_t>(m / kGroup) * band * 4;
         allowLds(reinterpret_cast<const void*>(&k_fg_advance), lds);
+        const size_t sortLds = F * sizeof(int) + kSortFeat * T * sizeof(float);   // 48 KiB at most
         for (int r = 0; r < rounds; r++) {
             hipLaunchKernelGGL(k_fg_round, dim3(m, numJobs), dim3(std::min(band, 256)), 0, s, dWalk, imgs,
                     tabs.cand.get(), numCand, drawn, T, ring, band, dRecs, dResp, dNext, dFirsts);
@@ -881,7 +880,8 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
                     tabs.cand.get(), numCand, drawn, F, T, band, m, dResp, dNext, dFirsts,
                     tabs.unsortedFeat.get(), tabs.unsortedThr.get(), tabs.unsortedKey.get());
         }
-        hipLaunchKernelGGL(k_fg_sort, dim3((F + kSortFeat - 1) / kSortFeat, numJobs), dim3(256), F * sizeof(int), s,
+        hipLaunchKernelGGL(k_fg_sort, dim3((F + kSortFeat - 1) / kSortFeat, numJobs), dim3(kSortFeat * kSortLanes),
+                sortLds, s,
                 tabs.unsortedKey.get(), tabs.unsortedFeat.get(), tabs.unsortedThr.get(), F, T, TM, tabs.feat.get(),
                 tabs.thrFT.get(), tabs.rank.get(), tabs.thrPad.get(),
                 referenceLayouts ? tabs.thrTF.get() : nullptr, referenceLayouts ? tabs.soa.get() : nullptr);
