@@ -247,6 +247,11 @@ struct FeatSummary {
 int evalChunkSamples(size_t samples, int F);
 void launchEvalHistograms(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk* chunks,
         int numChunks, const FeatTables& tabs, int C, uint32_t* G);
+// the same for one node, its chunks of evalChunkSamples formed from the whole (node.slot 0).  With summ, for a node
+// that evalScoresNode tells to be scored where it is counted: its features' summaries instead of its bins.
+bool evalScoresNode(int count, int F, int T, int C);
+void launchEvalNode(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk& node,
+        const FeatTables& tabs, int C, uint32_t* G, const uint32_t* nodeHist = nullptr, FeatSummary* summ = nullptr);
 
 // ---- two-pass level evaluation (k_bins.hip)
 // LDS a workgroup may use on the current device (MI355X: 160 KB); kernels whose

@@ -27,7 +27,7 @@
 #include <cfloat>
 #include <type_traits>
 
-#include "cf_internal.h"
+#include "cf_score.h"
 
 namespace cf {
 
@@ -54,6 +54,14 @@ __device__ __forceinline__ int binOf(float q, const float (&th)[TM], int T) {
     return (q != q) ? T : static_cast<int>(b);
 }
 
+// What a workgroup that counts a node completely needs to score it: the node's class counts, the tables' ranks, the
+// node's summaries (null: it does not).
+struct NodeScoring {
+    const uint32_t* hist = nullptr;
+    const uint16_t* rank = nullptr;
+    FeatSummary* summ = nullptr;
+};
+
 // All images of a set share W x H and are stored back to back, so a sample's
 // integrals are found from its image index.
 //
@@ -78,14 +86,22 @@ __device__ __forceinline__ int binOf(float q, const float (&th)[TM], int T) {
 template<int TM>
 __global__ void __launch_bounds__(kEvalThreads) k_eval_hist(const float* __restrict__ colBase,
         const int2* __restrict__ depBase, int W, int H, const cf_sample* __restrict__ samples,
-        const Chunk* __restrict__ chunks, int numChunks, int tile, int tiles, const FeatRec* __restrict__ feat,
-        const float* __restrict__ thrPad, int F, int T, int C, uint32_t* __restrict__ G) {
-    extern __shared__ uint32_t h[];
+        const Chunk* __restrict__ chunks, Chunk node, int chunkLen, int numChunks, int tile, int tiles,
+        const FeatRec* __restrict__ feat, const float* __restrict__ thrPad, int F, int T, int C,
+        uint32_t* __restrict__ G, NodeScoring scoring) {
+    extern __shared__ double evalLds[];   // scoreFeatures' part where the tile is scored, the bins
+    uint32_t* h = reinterpret_cast<uint32_t*>(evalLds) + (scoring.summ ? scoreLdsBytes(tile, T, C) / sizeof(uint32_t) : 0);
     const int total = numChunks * tiles, per = (total + kXcds - 1) / kXcds;
     const int item = static_cast<int>(blockIdx.x % kXcds) * per + static_cast<int>(blockIdx.x / kXcds);
     if (item >= total) return;
     const int chunkIdx = item / tiles, tileIdx = item - chunkIdx * tiles;
-    const Chunk ch = chunks[chunkIdx];
+    Chunk ch = node;
+    if (chunks) {
+        ch = chunks[chunkIdx];
+    } else {
+        ch.begin += chunkIdx * chunkLen;
+        ch.count = min(chunkLen, ch.count - chunkIdx * chunkLen);
+    }
     const int f0 = tileIdx * tile;
     const int nf = min(tile, F - f0);
     const int binsPerF = (T + 1) * C;
@@ -173,24 +189,16 @@ __global__ void __launch_bounds__(kEvalThreads) k_eval_hist(const float* __restr
         if (__any(both)) evaluate(both, true);
     }
     __syncthreads();
+    if (scoring.summ) {
+        scoreFeatures(h, nf, F, T, C, scoring.hist, scoring.rank + (static_cast<size_t>(ch.tree) * F + f0) * T, evalLds,
+                scoring.summ + f0, nullptr);
+        return;
+    }
     uint32_t* g = G + (static_cast<size_t>(ch.slot) * F + f0) * binsPerF;
     for (int k = threadIdx.x; k < nb; k += kEvalThreads) {
         const uint32_t v = h[k];
         if (v) atomicAdd(&g[k], v);
     }
-}
-
-// NormalizedInformationGainScore::calculateScore (score.h:191-215) over
-// InformationGainScore::calculateScore (score.h:87-139); the operation order
-// follows the reference so host and device round identically apart from log2.
-__device__ __forceinline__ double entropyOf(double p) {
-    if (p == 0.0) return 0.0;
-    return -p * log2(p);
-}
-__device__ __forceinline__ double clamp01(double s) {
-    if (s > 1.0) return 1.0;
-    if (s < 0.0) return 0.0;
-    return s;
 }
 
 template<int CM>
@@ -235,67 +243,18 @@ __device__ double nigScore(int C, const uint32_t* L, const uint32_t* R, const ui
     return clamp01((2 * ig) / (Hs + Hc));
 }
 
-// nigScore of the split that sends L[c] of the node's A[c] samples left, with the terms that the node's
-// thresholds share: classProb[c] = A[c] / total, entropyOf(total) and Hc.  The totals are integers, exact in
-// double however they are summed.  A caller's class counts below the bins' wrap as nigScore's do.
-__device__ __forceinline__ double splitScore(int C, const uint32_t* L, const uint32_t* A, const double* classProb,
-        double totalEntropy, double classEntropy) {
-    double totalLeft = 0, totalRight = 0, total = 0;
-    for (int c = 0; c < C; c++) {
-        totalLeft += static_cast<double>(L[c]);
-        totalRight += static_cast<double>(A[c] - L[c]);
-        total += static_cast<double>(A[c]);
-    }
-    const bool wraps = totalLeft + totalRight != total;
-    total = totalLeft + totalRight;
-    const double leftProb = totalLeft / total;
-    const double rightProb = totalRight / total;
-    double score = 0;
-    for (int c = 0; c < C; c++) {
-        const uint32_t l = L[c], r = A[c] - l;
-        const double prob = wraps ? static_cast<double>(A[c]) / total : classProb[c];
-        if (l > 0) {
-            const double p = static_cast<double>(l) / total;
-            score = __dadd_rn(score, __dmul_rn(p, log2(p / (leftProb * prob))));
-        }
-        if (r > 0) {
-            const double p = static_cast<double>(r) / total;
-            score = __dadd_rn(score, __dmul_rn(p, log2(p / (rightProb * prob))));
-        }
-    }
-    const double ig = clamp01(score);
-    if (ig == 0) return 0;
-    double Ht = totalEntropy, Hc = classEntropy;
-    if (wraps) {
-        Ht = entropyOf(total);
-        Hc = 0;
-        for (int c = 0; c < C; c++) {
-            if (A[c] > 0) Hc += entropyOf(static_cast<double>(A[c]));
-        }
-        Hc -= Ht;
-        Hc /= total;
-    }
-    const double Hs = (entropyOf(totalLeft) + entropyOf(totalRight) - Ht) / total;
-    return clamp01((2 * ig) / (Hs + Hc));
-}
-
-// Scores of a workgroup's features of one slot, a thread per (feature, threshold), and the features'
-// summaries.  The features' bins come into LDS in one run and become prefix sums there, so that threshold t's
-// left counts are row rank[t].  Bound by the double divisions and logarithms: what all thresholds of a node
-// share (the class probabilities, the entropies of the classes and of the total, 7 of 19 logarithms with 5
-// classes) is formed once per workgroup, by the same operations as nigScore.  A thread per feature that walked
-// its thresholds took 96 us for one node of 1000 features x 20 thresholds (now 10) and 866 us for 206 nodes x
-// 4000 x 32 (now 709).
+// Scores of a workgroup's features of one slot from their bins, which come into LDS in one run.  Bound by the
+// double divisions and logarithms.  A thread per feature that walked its thresholds took 96 us for one node of
+// 1000 features x 20 thresholds (now 10) and 866 us for 206 nodes x 4000 x 32 (now 709).
 struct ScoreShape {
     int feats;      // features of a workgroup
-    size_t lds;     // their bins (and prefix sums), the class probabilities, the scores
+    size_t lds;     // their bins (and prefix sums) and scoreFeatures' own
 };
 static ScoreShape scoreShape(int T, int C) {
     ScoreShape s;
     const int words = (T + 1) * C;
     s.feats = std::max(1, std::min({256 / T, 64, 8192 / words}));
-    s.lds = (static_cast<size_t>(s.feats) * T + C + 2) * sizeof(double) + static_cast<size_t>(C) * sizeof(uint32_t) +
-            static_cast<size_t>(s.feats) * words * sizeof(uint32_t);
+    s.lds = scoreLdsBytes(s.feats, T, C) + static_cast<size_t>(s.feats) * words * sizeof(uint32_t);
     return s;
 }
 
@@ -303,11 +262,7 @@ __global__ void __launch_bounds__(256) k_scores(const uint32_t* __restrict__ G, 
         const int* __restrict__ slotTree, const uint16_t* __restrict__ rank, int F, int T, int C, int feats, int blocks,
         FeatSummary* __restrict__ summ, double* __restrict__ allScores, int onlySlot, int fOffset, int Fb) {
     extern __shared__ double scoreLds[];
-    double* scores = scoreLds;                    // [feats][T]
-    double* classProb = scores + feats * T;       // [C]
-    double* terms = classProb + C;                // entropyOf(total), Hc
-    uint32_t* A = reinterpret_cast<uint32_t*>(terms + 2);   // [C]
-    uint32_t* pre = A + C;                        // [feats][T + 1][C]
+    uint32_t* pre = reinterpret_cast<uint32_t*>(scoreLds) + scoreLdsBytes(feats, T, C) / sizeof(uint32_t);   // [feats][T + 1][C]
     // G holds Fb features per slot starting at feature fOffset
     const int slot = onlySlot >= 0 ? onlySlot : static_cast<int>(blockIdx.x) / blocks;
     const int j0 = (static_cast<int>(blockIdx.x) % blocks) * feats;
@@ -316,70 +271,11 @@ __global__ void __launch_bounds__(256) k_scores(const uint32_t* __restrict__ G, 
     const int tid = threadIdx.x, words = (T + 1) * C;
     const uint32_t* g = G + (static_cast<size_t>(slot) * Fb + j0) * words;
     for (int i = tid; i < nf * words; i += 256) pre[i] = g[i];
-    if (tid < 64) {
-        // total of the node, exact in double; lane c: class c, lane C: the total
-        double total = 0;
-        for (int c = 0; c < C; c++) total += static_cast<double>(nodeHist[static_cast<size_t>(slot) * C + c]);
-        const uint32_t a = tid < C ? nodeHist[static_cast<size_t>(slot) * C + tid] : 0u;
-        const double e = entropyOf(tid < C ? static_cast<double>(a) : total);
-        if (tid < C) {
-            A[tid] = a;
-            classProb[tid] = static_cast<double>(a) / total;
-        }
-        double Hc = 0;
-        for (int c = 0; c < C; c++) {
-            const double ec = __shfl(e, c, 64);
-            if (__shfl(a, c, 64) > 0u) Hc += ec;
-        }
-        const double et = __shfl(e, C, 64);
-        Hc -= et;
-        if (tid == 0) {
-            terms[0] = et;
-            terms[1] = Hc / total;
-        }
-    }
     __syncthreads();
-    for (int i = tid; i < nf * C; i += 256) {
-        uint32_t* row = pre + (i / C) * words + i % C;
-        uint32_t run = 0;
-#pragma unroll 8
-        for (int b = 0; b <= T; b++) {
-            run += row[b * C];
-            row[b * C] = run;
-        }
-    }
-    __syncthreads();
-    const size_t row0 = static_cast<size_t>(slotTree[slot]) * F + fOffset + j0;
-    for (int i = tid; i < nf * T; i += 256) {
-        const int fi = i / T, t = i - fi * T;
-        const uint32_t* left = pre + fi * words + rank[(row0 + fi) * T + t] * C;
-        const double sc = splitScore(C, left, A, classProb, terms[0], terms[1]);
-        scores[i] = sc;
-        if (allScores) {
-            allScores[(static_cast<size_t>(onlySlot >= 0 ? 0 : slot) * T + t) * F + fOffset + j0 + fi] = sc;
-        }
-    }
-    __syncthreads();
-    if (tid < nf) {
-        double best = -DBL_MAX, second = -DBL_MAX;
-        int bestT = 0x7fffffff;
-        for (int t = 0; t < T; t++) {
-            const double sc = scores[tid * T + t];
-            if (sc > best) {
-                second = best;
-                best = sc;
-                bestT = t;
-            } else if (sc < best && sc > second) {
-                second = sc;
-            }
-        }
-        FeatSummary s;
-        s.best = best;
-        s.second = second;
-        s.thresh = bestT;
-        s.pad = 0;
-        summ[static_cast<size_t>(slot) * F + fOffset + j0 + tid] = s;
-    }
+    scoreFeatures(pre, nf, F, T, C, nodeHist + static_cast<size_t>(slot) * C,
+            rank + (static_cast<size_t>(slotTree[slot]) * F + fOffset + j0) * T, scoreLds,
+            summ + static_cast<size_t>(slot) * F + fOffset + j0,
+            allScores ? allScores + (onlySlot >= 0 ? 0 : static_cast<size_t>(slot) * T * F) + fOffset + j0 : nullptr);
 }
 
 // scores[T][F] of one node straight from counters [F][T][C][2]
@@ -587,13 +483,15 @@ int evalChunkSamples(size_t samples, int F) {
     return c;
 }
 
-void launchEvalHistograms(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk* chunks,
-        int numChunks, const FeatTables& tabs, int C, uint32_t* G) {
+static void launchEval(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk* chunks,
+        const Chunk& node, int chunkLen, int numChunks, const FeatTables& tabs, int C, uint32_t* G,
+        const NodeScoring& scoring) {
     if (numChunks == 0) return;
     // under two workgroups per CU with full tiles: tiles of one step
     const int tile = static_cast<int64_t>(numChunks) * ((tabs.F + kEvalTile - 1) / kEvalTile) < 512 ? kEvalSmallTile : kEvalTile;
     const int tiles = (tabs.F + tile - 1) / tile;
-    const size_t lds = static_cast<size_t>(tile) * (tabs.T + 1) * C * sizeof(uint32_t);
+    const size_t lds = static_cast<size_t>(tile) * (tabs.T + 1) * C * sizeof(uint32_t) +
+            (scoring.summ ? scoreLdsBytes(tile, tabs.T, C) : 0);
     const int64_t blocks = (static_cast<int64_t>(numChunks) * tiles + kXcds - 1) / kXcds * kXcds;
     if (blocks > INT32_MAX) throw Error(CF_ERR_UNSUPPORTED, "too many samples in one evaluation launch");
     const dim3 grid(static_cast<unsigned>(blocks)), block(kEvalThreads);
@@ -601,9 +499,9 @@ void launchEvalHistograms(hipStream_t s, const ImageSet& imgs, const cf_sample* 
         constexpr int TM = decltype(tm)::value;
         // the limit is that of a full tile, whatever the tile
         const size_t full = static_cast<size_t>(kEvalTile) * (tabs.T + 1) * C * sizeof(uint32_t);
-        allowLds(reinterpret_cast<const void*>(&k_eval_hist<TM>), full);
-        hipLaunchKernelGGL(k_eval_hist<TM>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples, chunks,
-                numChunks, tile, tiles, tabs.feat.get(), tabs.thrPad.get(), tabs.F, tabs.T, C, G);
+        allowLds(reinterpret_cast<const void*>(&k_eval_hist<TM>), std::max(full, lds));
+        hipLaunchKernelGGL(k_eval_hist<TM>, grid, block, lds, s, imgs.col, imgs.dep, imgs.W, imgs.H, samples, chunks, node,
+                chunkLen, numChunks, tile, tiles, tabs.feat.get(), tabs.thrPad.get(), tabs.F, tabs.T, C, G, scoring);
     };
     switch (binThresholdWidth(tabs.T)) {
         case 8: launch(std::integral_constant<int, 8>{}); break;
@@ -615,6 +513,29 @@ void launchEvalHistograms(hipStream_t s, const ImageSet& imgs, const cf_sample* 
         case 64: launch(std::integral_constant<int, 64>{}); break;
         default: launch(std::integral_constant<int, kMaxThresholds>{}); break;
     }
+}
+
+void launchEvalHistograms(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk* chunks,
+        int numChunks, const FeatTables& tabs, int C, uint32_t* G) {
+    launchEval(s, imgs, samples, chunks, Chunk{}, 0, numChunks, tabs, C, G, NodeScoring{});
+}
+
+// A node of few samples is taken as one chunk and scored by the workgroups that count it: no histogram is cleared,
+// added to and read again, and there is no second launch.  Where the line lies: 117 nodes of 8 frames, 1000 x 20, half
+// of them below 256 samples, took 10.7 ms without, 10.4 up to 256, 10.2 up to 512, 1024 and 2048 (with more samples the
+// single chunk leaves CUs idle for as long as the second launch takes).
+constexpr int kScoredSamples = 512;
+bool evalScoresNode(int count, int F, int T, int C) {
+    const int tile = (F + kEvalTile - 1) / kEvalTile < 512 ? kEvalSmallTile : kEvalTile;
+    return count <= kScoredSamples &&
+            static_cast<size_t>(tile) * (T + 1) * C * sizeof(uint32_t) + scoreLdsBytes(tile, T, C) <= kScoreFusedLds;
+}
+
+void launchEvalNode(hipStream_t s, const ImageSet& imgs, const cf_sample* samples, const Chunk& node,
+        const FeatTables& tabs, int C, uint32_t* G, const uint32_t* nodeHist, FeatSummary* summ) {
+    const int chunkLen = summ ? std::max(node.count, 1) : evalChunkSamples(node.count, tabs.F);
+    launchEval(s, imgs, samples, nullptr, node, chunkLen, (node.count + chunkLen - 1) / chunkLen, tabs, C, G,
+            NodeScoring{nodeHist, tabs.rank.get(), summ});
 }
 
 void launchScores(hipStream_t s, const uint32_t* G, const uint32_t* nodeHist, const int* slotTree, int numSlots,

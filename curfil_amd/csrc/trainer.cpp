@@ -544,23 +544,37 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
         // ---- evaluation
         auto evalSlots = [&](int s0, int s1) {
             const int ns = s1 - s0;
-            size_t slotSamples = 0;
-            for (int i = s0; i < s1; i++) slotSamples += nodes[i].count;
-            const int per = evalChunkSamples(slotSamples, F);
-            std::vector<Chunk> bc;
-            for (int i = s0; i < s1; i++) appendChunks(bc, nodes[i], i - s0, per);
-            const Chunk* dEval = up.put(bc);
-            up.flush(s);
             const uint32_t* slotHist = dNodeHist + static_cast<size_t>(s0) * C;
             dG.resize(static_cast<size_t>(ns) * perSlot);
             dSumm.resize(static_cast<size_t>(ns) * F);
-            CF_HIP(hipMemsetAsync(dG.get(), 0, static_cast<size_t>(ns) * perSlot * sizeof(uint32_t), s));
+            const Chunk node{0, nodes[s0].active, nodes[s0].begin, nodes[s0].count};
+            const bool scored = ns == 1 && evalScoresNode(node.count, F, T, C);
+            auto histograms = [&]() {
+                CF_HIP(hipMemsetAsync(dG.get(), 0, static_cast<size_t>(ns) * perSlot * sizeof(uint32_t), s));
+                if (ns == 1) {
+                    launchEvalNode(s, images->set(), level[cur].get(), node, tabs, C, dG.get());
+                    return;
+                }
+                size_t slotSamples = 0;
+                for (int i = s0; i < s1; i++) slotSamples += nodes[i].count;
+                const int per = evalChunkSamples(slotSamples, F);
+                std::vector<Chunk> bc;
+                for (int i = s0; i < s1; i++) appendChunks(bc, nodes[i], i - s0, per);
+                const Chunk* dEval = up.put(bc);
+                up.flush(s);
+                launchEvalHistograms(s, images->set(), level[cur].get(), dEval, static_cast<int>(bc.size()), tabs, C,
+                        dG.get());
+            };
             timer.begin();
-            launchEvalHistograms(s, images->set(), level[cur].get(), dEval, static_cast<int>(bc.size()), tabs, C, dG.get());
+            if (scored) {
+                launchEvalNode(s, images->set(), level[cur].get(), node, tabs, C, nullptr, slotHist, dSumm.get());
+            } else {
+                histograms();
+            }
             timer.end(stats.evalKernelMs);
             stats.evalLaunches += 1;
             timer.begin();
-            launchScores(s, dG.get(), slotHist, dNodeTree + s0, ns, tabs, C, dSumm.get(), nullptr, -1);
+            if (!scored) launchScores(s, dG.get(), slotHist, dNodeTree + s0, ns, tabs, C, dSumm.get(), nullptr, -1);
             launchReduce(s, dSumm.get(), ns, F, dBest + s0);
             timer.end(stats.scoreMs);
             CF_HIP(hipMemcpyAsync(&best[s0], dBest + s0, ns * sizeof(NodeBest), hipMemcpyDeviceToHost, s));
@@ -570,6 +584,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 if (!best[s0 + i].flag) continue;
                 // near-tie band: replay the reference's sequential scan for this node
                 dAllScores.resize(static_cast<size_t>(T) * F);
+                if (scored) histograms();
                 launchScores(s, dG.get(), slotHist, dNodeTree + s0, ns, tabs, C, dSumm.get(), dAllScores.get(), i);
                 launchSequentialArgmax(s, dAllScores.get(), T, F, dBest + s0 + i);
                 stats.replays++;
