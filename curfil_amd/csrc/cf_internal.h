@@ -321,12 +321,19 @@ int binThresholdWidth(int T);
 // G[slot][ng * 16][T + 1][C] from the bin rows of the chunks' samples
 // (samples still set to Both also count their flipped row at flipOffset; the chunks' slots count from slotBase)
 void launchHistBins(hipStream_t s, const uint4* bins, const uint8_t* labels, const Chunk* chunks, int numChunks,
-        int slotBase, int g0, int ng, const FeatTables& tabs, int C, int N, uint32_t* G, size_t flipOffset = 0);
+        int slotBase, int g0, int ng, const FeatTables& tabs, int C, int N, uint32_t* G, size_t flipOffset,
+        const uint32_t* nodeHist, FeatSummary* summ);
+// Whether launchHistBins over so many chunks may score the nodes of a single chunk where it counts them (with the
+// level's nodeHist and summ given, which start at slot 0; their G stays as it is)
+bool histScoresNodes(int numChunks, int ng, int T, int C);
+// clears the perSlot words of each listed slot in G, which starts at slotBase
+void launchClearSlots(hipStream_t s, uint32_t* G, const int* slots, int numSlots, int slotBase, size_t perSlot);
 // Scores and per-feature summaries of the slots' histograms.  With allScores, also every score:
-// allScores[T][F] of slot onlySlot alone, or allScores[slot][T][F] of all slots (onlySlot < 0).
+// allScores[T][F] of slot onlySlot alone, or allScores[slot][T][F] of all slots (onlySlot < 0).  With `listed`, only
+// the numSlots slots listed[i] - listBase.
 void launchScores(hipStream_t s, const uint32_t* G, const uint32_t* nodeHist, const int* slotTree, int numSlots,
         const FeatTables& tabs, int C, FeatSummary* summ, double* allScores, int onlySlot, int fOffset = 0,
-        int Fb = -1);
+        int Fb = -1, const int* listed = nullptr, int listBase = 0);
 void launchScoresFromCounters(hipStream_t s, const uint32_t* counters, const uint32_t* hist, int F, int T, int C,
         double* scores);
 void launchReduce(hipStream_t s, const FeatSummary* summ, int numSlots, int F, NodeBest* best);

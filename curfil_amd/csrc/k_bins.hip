@@ -10,6 +10,11 @@
 //   k_hist_bins   pass 2, node-major: one workgroup per (part of a node
 //                 chunk, group) streams the part's bin rows and labels into LDS
 //                 interval histograms and adds them to the node's global bins.
+//                 Nodes of a single chunk are scored from LDS there and then;
+//                 only the others' bins go through memory to k_scores (50
+//                 frames, 5 trees, 4000 x 32: 47 ms of clears, histograms and
+//                 scores per training, 40 with this; 21 frames, 3 trees,
+//                 2000 x 20: 5.25 and 4.7).
 //
 // Counting is order-independent, so the histograms equal those of the direct
 // path (k_eval_hist), whose single kernel gathers the integrals in node order:
@@ -36,7 +41,7 @@
 #include <map>
 #include <mutex>
 
-#include "cf_internal.h"
+#include "cf_score.h"
 
 namespace cf {
 
@@ -204,6 +209,14 @@ __global__ void __launch_bounds__(WAVES * 64) k_eval_bins(const float* __restric
     }
 }
 
+// What pass 2 needs to score the nodes of a single chunk where it counts them, by slot of the level: their class
+// counts, the tables' ranks, their summaries (null: it does not).
+struct LevelScoring {
+    const uint32_t* hist;
+    const uint16_t* rank;
+    FeatSummary* summ;
+};
+
 // Pass 2: interval histograms of (part of a node chunk, feature group) from the bin rows.
 // G holds the batch's groups: G[slot][ng * 16][T + 1][C].  Bound by the LDS atomics and the instructions that
 // form their addresses: a lane takes four features of a sample in one word, 16 samples a wave, and its features in
@@ -216,9 +229,11 @@ __global__ void __launch_bounds__(WAVES * 64) k_eval_bins(const float* __restric
 // chunk was not cut into parts: 13 flipped frames, 500 x 50 108 us a level (now 36); 4 small frames 19 (5); 21
 // frames, 3 trees, 2000 x 20 199 (151); 50 frames, 5 trees, 4000 x 32 1562 (1245).
 __global__ void __launch_bounds__(256) k_hist_bins(const uint4* __restrict__ bins, const uint8_t* __restrict__ labels,
-        const Chunk* __restrict__ chunks, int parts, int partLen, int slotBase, int g0, int ng, int F, int T, int C,
-        int N, uint32_t* __restrict__ G, size_t flipOffset) {
-    extern __shared__ uint32_t h[];
+        const Chunk* __restrict__ chunks, int numChunks, int parts, int partLen, int slotBase, int g0, int ng, int F,
+        int T, int C, int N, uint32_t* __restrict__ G, size_t flipOffset, LevelScoring scoring) {
+    extern __shared__ double histLds[];   // scoreFeatures' part where nodes are scored, the bins
+    uint32_t* h = reinterpret_cast<uint32_t*>(histLds) +
+            (scoring.summ ? scoreLdsBytes(kBinGroup, T, C) / sizeof(uint32_t) : 0);
     const int partIdx = blockIdx.x / ng;
     const int g = blockIdx.x % ng;
     Chunk ch = chunks[partIdx / parts];
@@ -277,6 +292,15 @@ __global__ void __launch_bounds__(256) k_hist_bins(const uint4* __restrict__ bin
         }
     }
     __syncthreads();
+    const int chunk = partIdx / parts;
+    if (scoring.summ && (chunk == 0 || chunks[chunk - 1].slot != ch.slot) &&
+            (chunk == numChunks - 1 || chunks[chunk + 1].slot != ch.slot)) {
+        const int f0 = (g0 + g) * kBinGroup;
+        scoreFeatures(h, nf, F, T, C, scoring.hist + static_cast<size_t>(ch.slot) * C,
+                scoring.rank + (static_cast<size_t>(ch.tree) * F + f0) * T, histLds,
+                scoring.summ + static_cast<size_t>(ch.slot) * F + f0, nullptr);
+        return;
+    }
     uint32_t* out = G + (static_cast<size_t>(ch.slot - slotBase) * ng + g) * kBinGroup * binsPerF;
     for (int k = threadIdx.x; k < nf * binsPerF; k += 256) {
         const uint32_t v = h[k];
@@ -487,17 +511,44 @@ void launchEvalBins(hipStream_t s, const ImageSet& imgs, const cf_sample* sample
     throw Error(CF_ERR_RUNTIME, "pass-1 launch shape without a kernel");
 }
 
-void launchHistBins(hipStream_t s, const uint4* bins, const uint8_t* labels, const Chunk* chunks, int numChunks,
-        int slotBase, int g0, int ng, const FeatTables& tabs, int C, int N, uint32_t* G, size_t flipOffset) {
-    if (numChunks == 0 || ng == 0) return;
-    const size_t lds = static_cast<size_t>(kBinGroup) * (tabs.T + 1) * C * sizeof(uint32_t);
-    allowLds(reinterpret_cast<const void*>(&k_hist_bins), lds);
-    // few chunks and groups: chunks cut into parts while that gives at most 2048 workgroups
+// The histograms of the listed slots, cleared.
+__global__ void __launch_bounds__(256) k_clear_slots(uint4* __restrict__ G, const int* __restrict__ slots, int slotBase,
+        int words) {
+    uint4* g = G + static_cast<size_t>(slots[blockIdx.y] - slotBase) * words;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < words) g[i] = make_uint4(0, 0, 0, 0);
+}
+
+void launchClearSlots(hipStream_t s, uint32_t* G, const int* slots, int numSlots, int slotBase, size_t perSlot) {
+    if (numSlots == 0) return;
+    const int words = static_cast<int>(perSlot / 4);
+    hipLaunchKernelGGL(k_clear_slots, dim3((words + 255) / 256, numSlots), dim3(256), 0, s, reinterpret_cast<uint4*>(G),
+            slots, slotBase, words);
+}
+
+// few chunks and groups: chunks cut into parts while that gives at most 2048 workgroups
+static int histParts(int numChunks, int ng) {
     int parts = 1;
     while (parts < 8 && static_cast<int64_t>(2) * parts * numChunks * ng <= 2048) parts *= 2;
-    const int partLen = (kChunk + parts - 1) / parts;
+    return parts;
+}
+
+bool histScoresNodes(int numChunks, int ng, int T, int C) {
+    return histParts(numChunks, ng) == 1 &&
+            static_cast<size_t>(kBinGroup) * (T + 1) * C * sizeof(uint32_t) + scoreLdsBytes(kBinGroup, T, C) <= kScoreFusedLds;
+}
+
+void launchHistBins(hipStream_t s, const uint4* bins, const uint8_t* labels, const Chunk* chunks, int numChunks,
+        int slotBase, int g0, int ng, const FeatTables& tabs, int C, int N, uint32_t* G, size_t flipOffset,
+        const uint32_t* nodeHist, FeatSummary* summ) {
+    if (numChunks == 0 || ng == 0) return;
+    const size_t bytes = static_cast<size_t>(kBinGroup) * (tabs.T + 1) * C * sizeof(uint32_t);
+    const size_t lds = bytes + (summ ? scoreLdsBytes(kBinGroup, tabs.T, C) : 0);
+    allowLds(reinterpret_cast<const void*>(&k_hist_bins), std::max(bytes, lds));
+    const int parts = histParts(numChunks, ng), partLen = (kChunk + parts - 1) / parts;
     hipLaunchKernelGGL(k_hist_bins, dim3(static_cast<unsigned>(numChunks) * parts * ng), dim3(256), lds, s, bins, labels,
-            chunks, parts, partLen, slotBase, g0, ng, tabs.F, tabs.T, C, N, G, flipOffset);
+            chunks, numChunks, parts, partLen, slotBase, g0, ng, tabs.F, tabs.T, C, N, G, flipOffset,
+            LevelScoring{nodeHist, tabs.rank.get(), summ});
 }
 
 }  // namespace cf

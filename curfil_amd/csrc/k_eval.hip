@@ -260,11 +260,13 @@ static ScoreShape scoreShape(int T, int C) {
 
 __global__ void __launch_bounds__(256) k_scores(const uint32_t* __restrict__ G, const uint32_t* __restrict__ nodeHist,
         const int* __restrict__ slotTree, const uint16_t* __restrict__ rank, int F, int T, int C, int feats, int blocks,
-        FeatSummary* __restrict__ summ, double* __restrict__ allScores, int onlySlot, int fOffset, int Fb) {
+        FeatSummary* __restrict__ summ, double* __restrict__ allScores, int onlySlot, int fOffset, int Fb,
+        const int* __restrict__ listed, int listBase) {
     extern __shared__ double scoreLds[];
     uint32_t* pre = reinterpret_cast<uint32_t*>(scoreLds) + scoreLdsBytes(feats, T, C) / sizeof(uint32_t);   // [feats][T + 1][C]
     // G holds Fb features per slot starting at feature fOffset
-    const int slot = onlySlot >= 0 ? onlySlot : static_cast<int>(blockIdx.x) / blocks;
+    const int at = static_cast<int>(blockIdx.x) / blocks;
+    const int slot = onlySlot >= 0 ? onlySlot : (listed ? listed[at] - listBase : at);
     const int j0 = (static_cast<int>(blockIdx.x) % blocks) * feats;
     const int nf = min(feats, min(Fb - j0, F - fOffset - j0));
     if (nf <= 0) return;
@@ -539,7 +541,8 @@ void launchEvalNode(hipStream_t s, const ImageSet& imgs, const cf_sample* sample
 }
 
 void launchScores(hipStream_t s, const uint32_t* G, const uint32_t* nodeHist, const int* slotTree, int numSlots,
-        const FeatTables& tabs, int C, FeatSummary* summ, double* allScores, int onlySlot, int fOffset, int Fb) {
+        const FeatTables& tabs, int C, FeatSummary* summ, double* allScores, int onlySlot, int fOffset, int Fb,
+        const int* listed, int listBase) {
     if (Fb < 0) Fb = tabs.F;
     const int slots = onlySlot >= 0 ? 1 : numSlots;
     if (slots == 0 || Fb <= 0) return;
@@ -547,7 +550,8 @@ void launchScores(hipStream_t s, const uint32_t* G, const uint32_t* nodeHist, co
     const int blocks = (Fb + shape.feats - 1) / shape.feats;
     allowLds(reinterpret_cast<const void*>(&k_scores), shape.lds);
     hipLaunchKernelGGL(k_scores, dim3(static_cast<unsigned>(slots) * blocks), dim3(256), shape.lds, s, G, nodeHist,
-            slotTree, tabs.rank.get(), tabs.F, tabs.T, C, shape.feats, blocks, summ, allScores, onlySlot, fOffset, Fb);
+            slotTree, tabs.rank.get(), tabs.F, tabs.T, C, shape.feats, blocks, summ, allScores, onlySlot, fOffset, Fb,
+            listed, listBase);
 }
 
 void launchReduce(hipStream_t s, const FeatSummary* summ, int numSlots, int F, NodeBest* best) {

@@ -452,6 +452,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
         std::vector<Chunk> chunks;
         std::vector<uint32_t> nodeHist;   // class histograms and trees of the level's nodes
         std::vector<int> nodeTree;
+        std::vector<int> multiSlots;      // the nodes of more than one chunk
         for (int a = 0; a < numActive; a++) {
             int off = active[a].begin;
             for (size_t k = 0; k < active[a].nodes.size(); k++) {
@@ -468,6 +469,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 const uint32_t* h = &out[active[a].job].hist[static_cast<size_t>(ln.node) * C];
                 nodeHist.insert(nodeHist.end(), h, h + C);
                 nodeTree.push_back(a);
+                if (ln.chunkEnd - ln.chunkBegin > 1) multiSlots.push_back(static_cast<int>(nodes.size()) - 1);
                 stats.evaluations += static_cast<double>(ln.count) * F * T;
                 stats.responses += static_cast<double>(ln.count) * F;
                 stats.nodes += 1;
@@ -477,6 +479,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
         const Chunk* dChunks = up.put(chunks);
         const uint32_t* dNodeHist = up.put(nodeHist);
         const int* dNodeTree = up.put(nodeTree);
+        const int* dMulti = up.put(multiSlots);
         up.flush(s);
         const int numNodes = static_cast<int>(nodes.size());
         const int numChunks = static_cast<int>(chunks.size());
@@ -715,6 +718,31 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 for (int s0 = 0; s0 < numNodes; s0 += maxSlots) out.emplace_back(s0, std::min(numNodes, s0 + maxSlots));
                 return out;
             };
+            // pass 2 and the scores of the slots [s0, s1) for the feature groups [g0, g0 + ngb): nodes of a single chunk
+            // are scored where they are counted, the others' histograms cleared, added to and read
+            auto countAndScore = [&](int s0, int s1, int g0, int ngb) {
+                const int nc = nodes[s1 - 1].chunkEnd - nodes[s0].chunkBegin;
+                const size_t perSlotB = static_cast<size_t>(ngb) * kBinGroup * (T + 1) * C;
+                const bool scored = histScoresNodes(nc, ngb, T, C);
+                int ns = s1 - s0;
+                const int* listed = nullptr;
+                if (scored) {
+                    const auto m0 = std::lower_bound(multiSlots.begin(), multiSlots.end(), s0);
+                    listed = dMulti + (m0 - multiSlots.begin());
+                    ns = static_cast<int>(std::lower_bound(m0, multiSlots.end(), s1) - m0);
+                    launchClearSlots(s, dG.get(), listed, ns, s0, perSlotB);
+                } else {
+                    launchFillU32(s, dG.get(), ns * perSlotB, 0u);
+                }
+                timer.begin();
+                launchHistBins(s, dBins.get(), dLab8.get(), dChunks + nodes[s0].chunkBegin, nc, s0, g0, ngb, tabs, C, N,
+                        dG.get(), flipOffset, scored ? dNodeHist : nullptr, scored ? dSumm.get() : nullptr);
+                timer.end(stats.histMs);
+                timer.begin();
+                launchScores(s, dG.get(), dNodeHist + static_cast<size_t>(s0) * C, dNodeTree + s0, ns, tabs, C,
+                        dSumm.get() + static_cast<size_t>(s0) * F, nullptr, -1, g0 * kBinGroup, ngb * kBinGroup, listed, s0);
+                timer.end(stats.scoreMs);
+            };
             LevelGraph graph(s);
             if (!tuning && levelGraphs) {
                 // The shape is settled: the level's evaluation (every batch's pass 1; per node-slot batch the
@@ -755,21 +783,7 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                     stats.evalLaunches += 1;
                     stats.shapeLaunches[levelShape] += 1;
                     stats.slotBatchesMax = std::max(stats.slotBatchesMax, static_cast<int>(b.slots.size()));
-                    const size_t perSlotB = static_cast<size_t>(b.ngb) * kBinGroup * (T + 1) * C;
-                    for (const auto& sb : b.slots) {
-                        const int s0 = sb.first, ns = sb.second - sb.first;
-                        const int nc = nodes[sb.second - 1].chunkEnd - nodes[s0].chunkBegin;
-                        launchFillU32(s, dG.get(), static_cast<size_t>(ns) * perSlotB, 0u);
-                        timer.begin();
-                        launchHistBins(s, dBins.get(), dLab8.get(), dChunks + nodes[s0].chunkBegin, nc, s0, b.g0, b.ngb,
-                                tabs, C, N, dG.get(), flipOffset);
-                        timer.end(stats.histMs);
-                        timer.begin();
-                        launchScores(s, dG.get(), dNodeHist + static_cast<size_t>(s0) * C, dNodeTree + s0, ns, tabs, C,
-                                dSumm.get() + static_cast<size_t>(s0) * F, nullptr, -1, b.g0 * kBinGroup,
-                                b.ngb * kBinGroup);
-                        timer.end(stats.scoreMs);
-                    }
+                    for (const auto& sb : b.slots) countAndScore(sb.first, sb.second, b.g0, b.ngb);
                 }
                 timer.begin();
                 launchReduce(s, dSumm.get(), numNodes, F, dBest);
@@ -805,19 +819,8 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
                 stats.slotBatchesMax = std::max(stats.slotBatchesMax, (numNodes + maxSlotsB - 1) / maxSlotsB);
                 for (int s0 = 0; s0 < numNodes;) {
                     const int s1 = std::min(numNodes, s0 + maxSlotsB);
-                    const int ns = s1 - s0;
-                    const int nc = nodes[s1 - 1].chunkEnd - nodes[s0].chunkBegin;
-                    dG.resize(static_cast<size_t>(ns) * perSlotB);
-                    CF_HIP(hipMemsetAsync(dG.get(), 0, static_cast<size_t>(ns) * perSlotB * sizeof(uint32_t), s));
-                    timer.begin();
-                    launchHistBins(s, dBins.get(), dLab8.get(), dChunks + nodes[s0].chunkBegin, nc, s0, g0, ngb, tabs, C, N,
-                            dG.get(), flipOffset);
-                    timer.end(stats.histMs);
-                    timer.begin();
-                    launchScores(s, dG.get(), dNodeHist + static_cast<size_t>(s0) * C, dNodeTree + s0, ns,
-                            tabs, C, dSumm.get() + static_cast<size_t>(s0) * F, nullptr, -1, g0 * kBinGroup,
-                            ngb * kBinGroup);
-                    timer.end(stats.scoreMs);
+                    dG.resize(static_cast<size_t>(s1 - s0) * perSlotB);
+                    countAndScore(s0, s1, g0, ngb);
                     s0 = s1;
                 }
             }
