@@ -44,3 +44,29 @@ def test_partition_edges_match_oracle(ctx, frames, n, flip, mode):
     for name in ("feature", "threshold"):
         assert np.array_equal(nodes[name][inner], on[name][inner]), name
     assert np.array_equal(hist, oh)
+
+
+# levels that hold both nodes of several chunks and nodes of one, which are scored where they are counted, with a
+# broken last group of features; histograms too large for that (30 thresholds, 32 classes)
+@pytest.mark.parametrize("T,C,flip", [(6, 5, False), (6, 5, True), (30, 32, False)])
+def test_scored_where_counted_matches_oracle(ctx, frames, T, C, flip):
+    depth, labels, im, ds = frames
+    rng = np.random.default_rng(T)
+    s = random_samples(rng, 24000, 3, 160, 120, depth.astype(np.int32), labels=labels)
+    s["label"] = (s["x"] // 20 + 2 * (s["y"] // 30)) % C
+    s["flip"] = 2 if flip else 0
+    s = s[s["depth_mm"] > 0][:12000]
+    params = dict(randomSeed=99, samplesPerImage=1, featureCount=2100, minSampleCount=20, maxDepth=7, boxRadius=20,
+                  regionSize=6, thresholds=T, horizontalFlipping=flip)
+    forest = cf.RandomForestImage.train_tree_from_samples(ctx, im, cf.TrainingConfiguration(**params), 0, C, 99, s,
+                                                          mode=cf.MODE_BATCHED)
+    nodes, hist = forest.tree(0)
+    on, oh = ds.train_tree(orc.config(**params), 0, C, 99, s)
+    assert len(nodes) == len(on) > 20
+    inner = on["is_leaf"] == 0
+    for name in ("id", "level", "parent", "left", "right", "num_samples", "is_leaf"):
+        assert np.array_equal(nodes[name], on[name]), name
+    for name in ("feature", "threshold"):
+        assert np.array_equal(nodes[name][inner], on[name][inner]), name
+    assert np.abs(nodes["score"][inner] - on["score"][inner]).max() <= 4e-16
+    assert np.array_equal(hist, oh)
