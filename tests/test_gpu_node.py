@@ -41,3 +41,27 @@ def test_node_counters_and_split_edges(ctx, frames, n, F, T, C):
     bf, bt, bs = orc.argmax(sc)
     assert abs(score - bs) <= 4e-16
     assert (f, t) == (bf, bt)
+
+
+# windows of 64 scores and segments of them, one score more and less; scans that take every score, none after the
+# first, a few, and steps around the 1e-13 below which a larger score is not taken
+@pytest.mark.parametrize("F,T", [(1, 1), (63, 1), (64, 1), (65, 1), (1024, 1), (1025, 1), (73, 15), (400, 50), (1200, 60)])
+@pytest.mark.parametrize("order", ["random", "ascending", "descending", "equal", "ties", "steps"])
+def test_argmax_scan_edges(ctx, F, T, order):
+    rng = np.random.default_rng(F * T)
+    n = F * T
+    scores = rng.random(n)
+    if order == "ascending":
+        scores = np.sort(scores)
+    elif order == "descending":
+        scores = np.sort(scores)[::-1].copy()
+    elif order == "equal":
+        scores[:] = 0.25
+    elif order == "ties":
+        scores = 0.5 + rng.integers(0, 40, n) * 0.3e-13
+    elif order == "steps":
+        scores = 0.5 + np.arange(n) * rng.choice([0.2e-13, 0.6e-13, 1.1e-13], n)
+    scores = scores.reshape(T, F)
+    f, t, best = cf.argmax_scores(ctx, scores)
+    bf, bt, bb = orc.argmax(scores)
+    assert (f, t) == (bf, bt) and best == bb
