@@ -18,6 +18,7 @@
 // CURFIL_TUNE_ROUNDS=r sets the ratios per shape, and
 // CURFIL_TUNE_FILE=path loads finished keys from a file and writes them back
 // when a key finishes.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <fstream>
@@ -163,8 +164,10 @@ private:
         const char* pin = std::getenv("CURFIL_EVAL_SHAPE");
         if (!pin || !*pin) return -1;
         const int v = std::atoi(pin);
-        if (v < 0 || v >= numEvalShapes()) throw Error(CF_ERR_ARG, "CURFIL_EVAL_SHAPE out of range");
-        return v;
+        // numbers 5 to 9 were shapes of an earlier kernel (every shape gives the same bins): the default takes their place
+        constexpr int kNumbers = 10;
+        if (v < 0 || v >= std::max(kNumbers, numEvalShapes())) throw Error(CF_ERR_ARG, "CURFIL_EVAL_SHAPE out of range");
+        return v < numEvalShapes() ? v : 0;
     }
 
     // CURFIL_TUNE_SMALL=1: levels and launches of any size are tuned and timed (for tests on small workloads)
