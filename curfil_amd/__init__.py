@@ -982,7 +982,7 @@ def synth_forest(ctx, images, depth_mm, trees=10, depth=20, classes=5, seed=4711
 
 
 def eval_shape_info(shape):
-    """(lanes, samples per lane, features per step, workgroups per CU) of a pass-1 launch shape, or None."""
+    """(lanes, samples of a block per lane, features per step, workgroups per CU) of a pass-1 launch shape, or None."""
     v = [ctypes.c_int() for _ in range(4)]
     if lib.cf_eval_shape_info(shape, *[ctypes.byref(x) for x in v]) != CF_OK:
         return None

@@ -12,7 +12,8 @@
 //   k_scores      one thread per (node, feature, threshold): prefix sums over the bins
 //                 give every threshold's left/right class counts; FP64
 //                 NormalizedInformationGainScore (score.h:45-216) in the
-//                 reference's operation order; per-feature best / second best.
+//                 reference's operation order; per-feature best / second best
+//                 (scoreFeatures; small nodes are scored by k_eval_hist itself).
 //   k_reduce      per node: the reference's threshold-major sequential argmax
 //                 with its 1e-13 tie rule (random_tree_image.cpp:445-457,
 //                 random_tree.cpp:36-52) as max + first occurrence, valid

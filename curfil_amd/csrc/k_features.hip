@@ -15,14 +15,15 @@
 // chain is taken in rounds of two launches:
 //   k_fg_round    a workgroup per candidate evaluates it on a band of draws
 //                 around its expected first draw and, from the finite bits,
-//                 tabulates for every start in the band where the candidate
-//                 would end and whether it would be accepted;
+//                 tabulates for every start in the band where in the next
+//                 candidate's band that one would start, and whether the
+//                 candidate would be accepted;
 //   k_fg_advance  a workgroup per tree follows the chain through the tables
-//                 (one LDS read per candidate) and writes the accepted
-//                 candidates' thresholds.
+//                 (one LDS read per eight candidates, whose tables it has
+//                 composed) and writes the accepted candidates' thresholds.
 // The bands only decide how far a round gets, never which draws a candidate
 // uses.  Per level of 5 trees with F = 4000, T = 32 on 50 frames of 640x480 the
-// walk takes 1.6 ms (about 40 rounds of 112 candidates: 15 us + 18 us each);
+// walk takes 1.1 ms (about 40 rounds of 112 candidates: 15 us + 11 us each);
 // one workgroup per tree that evaluated 16 candidates a round on its own CU
 // took 15.2 ms, bound by that CU's gathers.
 #include <algorithm>

@@ -203,7 +203,7 @@ int cf_forest_profile(const cf_forest* forest, double* out, int n);
 /* Launch shapes of the batched levels' response kernel and their tuner (no
  * counterpart in the reference, whose kernels have fixed shapes,
  * random_tree_image_gpu.cu:2034-2065, 2095-2108).  A shape: lanes per
- * workgroup, samples per lane, features whose gathers are issued together,
+ * workgroup, samples of a block per lane, features whose gathers are issued together,
  * workgroups per CU.  Every shape gives the same histograms; the tuner times
  * them on the first launches of each (threshold width, level size class),
  * each shape's launch right after a launch of shape 0, and keeps the shape
