@@ -513,17 +513,17 @@ void launchEvalBins(hipStream_t s, const ImageSet& imgs, const cf_sample* sample
 
 // The histograms of the listed slots, cleared.
 __global__ void __launch_bounds__(256) k_clear_slots(uint4* __restrict__ G, const int* __restrict__ slots, int slotBase,
-        int words) {
-    uint4* g = G + static_cast<size_t>(slots[blockIdx.y] - slotBase) * words;
-    const int i = blockIdx.x * 256 + threadIdx.x;
+        int words, int blocks) {
+    uint4* g = G + static_cast<size_t>(slots[blockIdx.x / blocks] - slotBase) * words;
+    const int i = static_cast<int>(blockIdx.x % blocks) * 256 + threadIdx.x;
     if (i < words) g[i] = make_uint4(0, 0, 0, 0);
 }
 
 void launchClearSlots(hipStream_t s, uint32_t* G, const int* slots, int numSlots, int slotBase, size_t perSlot) {
     if (numSlots == 0) return;
-    const int words = static_cast<int>(perSlot / 4);
-    hipLaunchKernelGGL(k_clear_slots, dim3((words + 255) / 256, numSlots), dim3(256), 0, s, reinterpret_cast<uint4*>(G),
-            slots, slotBase, words);
+    const int words = static_cast<int>(perSlot / 4), blocks = (words + 255) / 256;
+    hipLaunchKernelGGL(k_clear_slots, dim3(static_cast<unsigned>(blocks) * numSlots), dim3(256), 0, s,
+            reinterpret_cast<uint4*>(G), slots, slotBase, words, blocks);
 }
 
 // few chunks and groups: chunks cut into parts while that gives at most 2048 workgroups
