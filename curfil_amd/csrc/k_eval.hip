@@ -492,23 +492,32 @@ __global__ void __launch_bounds__(64 * kSeqWaves) k_seq_argmax(const double* __r
     }
 }
 
-// counters[F][T][C][2] of one node (slot 0) from its bins.
+// counters[F][T][C][2] of one node (slot 0) from its bins: a workgroup's features come into LDS and become prefix
+// sums there, then a lane writes a (threshold, class)'s two counters (a lane per threshold that summed its bins
+// from memory: 20 us for 500 x 50 with 5 classes; now 5.8).
 __global__ void __launch_bounds__(256) k_counters_from_bins(const uint32_t* __restrict__ G,
-        const uint16_t* __restrict__ rank, int F, int T, int C, uint32_t* __restrict__ counters) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= F * T) return;
-    const int f = i / T, t = i % T;
-    const uint32_t* g = G + static_cast<size_t>(f) * (T + 1) * C;
-    const int r = rank[static_cast<size_t>(f) * T + t];
-    for (int c = 0; c < C; c++) {
-        uint32_t left = 0, total = 0;
+        const uint16_t* __restrict__ rank, int F, int T, int C, int feats, uint32_t* __restrict__ counters) {
+    extern __shared__ uint32_t pre[];   // [feats][T + 1][C]
+    const int f0 = blockIdx.x * feats, nf = min(feats, F - f0), words = (T + 1) * C;
+    const uint32_t* g = G + static_cast<size_t>(f0) * words;
+    for (int i = threadIdx.x; i < nf * words; i += 256) pre[i] = g[i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < nf * C; i += 256) {
+        uint32_t* row = pre + (i / C) * words + i % C;
+        uint32_t run = 0;
+#pragma unroll 8
         for (int b = 0; b <= T; b++) {
-            const uint32_t v = g[b * C + c];
-            total += v;
-            if (b <= r) left += v;
+            run += row[b * C];
+            row[b * C] = run;
         }
-        counters[((static_cast<size_t>(f) * T + t) * C + c) * 2 + 0] = left;
-        counters[((static_cast<size_t>(f) * T + t) * C + c) * 2 + 1] = total - left;
+    }
+    __syncthreads();
+    uint2* out = reinterpret_cast<uint2*>(counters) + static_cast<size_t>(f0) * T * C;
+    for (int i = threadIdx.x; i < nf * T * C; i += 256) {
+        const int ft = i / C, c = i - ft * C, fi = ft / T;
+        const uint32_t* p = pre + fi * words + c;
+        const uint32_t left = p[rank[static_cast<size_t>(f0) * T + ft] * C];
+        out[i] = make_uint2(left, p[T * C] - left);
     }
 }
 
@@ -620,9 +629,10 @@ void launchSequentialArgmax(hipStream_t s, const double* scores, int T, int F, N
 }
 
 void launchCountersFromBins(hipStream_t s, const uint32_t* G, const FeatTables& tabs, int C, uint32_t* counters) {
-    const int n = tabs.F * tabs.T;
-    hipLaunchKernelGGL(k_counters_from_bins, dim3((n + 255) / 256), dim3(256), 0, s, G, tabs.rank.get(), tabs.F,
-            tabs.T, C, counters);
+    const int words = (tabs.T + 1) * C, feats = std::max(1, std::min(4, 8192 / words));
+    const size_t lds = static_cast<size_t>(feats) * words * sizeof(uint32_t);
+    hipLaunchKernelGGL(k_counters_from_bins, dim3((tabs.F + feats - 1) / feats), dim3(256), lds, s, G, tabs.rank.get(),
+            tabs.F, tabs.T, C, feats, counters);
 }
 
 void launchResponses(hipStream_t s, const DevImage* imgs, const cf_sample* samples, int n, const FeatRec* feats,
