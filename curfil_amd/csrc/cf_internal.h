@@ -18,6 +18,11 @@ namespace cf {
 // its own L2.
 constexpr int kNumXcds = 8;
 
+// Workgroups of 256 lanes in one launch over node histograms: a grid of 2^32 work-items or more is refused, and
+// a histogram budget of 16 GiB (CURFIL_EVAL_BUDGET_MB) holds 2^32 words, so these launches loop or are cut above
+// this number (the fill of the default budget's 2 GiB takes one pass).
+constexpr unsigned kMaxLaunchBlocks = 1u << 21;
+
 // Thrown inside the library, turned into a status at the C ABI.
 struct Error : std::runtime_error {
     int code;

@@ -522,8 +522,12 @@ __global__ void __launch_bounds__(256) k_clear_slots(uint4* __restrict__ G, cons
 void launchClearSlots(hipStream_t s, uint32_t* G, const int* slots, int numSlots, int slotBase, size_t perSlot) {
     if (numSlots == 0) return;
     const int words = static_cast<int>(perSlot / 4), blocks = (words + 255) / 256;
-    hipLaunchKernelGGL(k_clear_slots, dim3(static_cast<unsigned>(blocks) * numSlots), dim3(256), 0, s,
-            reinterpret_cast<uint4*>(G), slots, slotBase, words, blocks);
+    const int most = std::max(1, static_cast<int>(kMaxLaunchBlocks / blocks));
+    for (int i = 0; i < numSlots; i += most) {
+        const int n = std::min(most, numSlots - i);
+        hipLaunchKernelGGL(k_clear_slots, dim3(static_cast<unsigned>(blocks) * n), dim3(256), 0, s,
+                reinterpret_cast<uint4*>(G), slots + i, slotBase, words, blocks);
+    }
 }
 
 // few chunks and groups: chunks cut into parts while that gives at most 2048 workgroups

@@ -261,12 +261,12 @@ static ScoreShape scoreShape(int T, int C) {
 
 __global__ void __launch_bounds__(256) k_scores(const uint32_t* __restrict__ G, const uint32_t* __restrict__ nodeHist,
         const int* __restrict__ slotTree, const uint16_t* __restrict__ rank, int F, int T, int C, int feats, int blocks,
-        FeatSummary* __restrict__ summ, double* __restrict__ allScores, int onlySlot, int fOffset, int Fb,
+        int first, FeatSummary* __restrict__ summ, double* __restrict__ allScores, int onlySlot, int fOffset, int Fb,
         const int* __restrict__ listed, int listBase) {
     extern __shared__ double scoreLds[];
     uint32_t* pre = reinterpret_cast<uint32_t*>(scoreLds) + scoreLdsBytes(feats, T, C) / sizeof(uint32_t);   // [feats][T + 1][C]
     // G holds Fb features per slot starting at feature fOffset
-    const int at = static_cast<int>(blockIdx.x) / blocks;
+    const int at = first + static_cast<int>(blockIdx.x) / blocks;
     const int slot = onlySlot >= 0 ? onlySlot : (listed ? listed[at] - listBase : at);
     const int j0 = (static_cast<int>(blockIdx.x) % blocks) * feats;
     const int nf = min(feats, min(Fb - j0, F - fOffset - j0));
@@ -613,9 +613,13 @@ void launchScores(hipStream_t s, const uint32_t* G, const uint32_t* nodeHist, co
     const ScoreShape shape = scoreShape(tabs.T, C);
     const int blocks = (Fb + shape.feats - 1) / shape.feats;
     allowLds(reinterpret_cast<const void*>(&k_scores), shape.lds);
-    hipLaunchKernelGGL(k_scores, dim3(static_cast<unsigned>(slots) * blocks), dim3(256), shape.lds, s, G, nodeHist,
-            slotTree, tabs.rank.get(), tabs.F, tabs.T, C, shape.feats, blocks, summ, allScores, onlySlot, fOffset, Fb,
-            listed, listBase);
+    const int most = std::max(1, static_cast<int>(kMaxLaunchBlocks / blocks));
+    for (int i = 0; i < slots; i += most) {
+        const int n = std::min(most, slots - i);
+        hipLaunchKernelGGL(k_scores, dim3(static_cast<unsigned>(n) * blocks), dim3(256), shape.lds, s, G, nodeHist,
+                slotTree, tabs.rank.get(), tabs.F, tabs.T, C, shape.feats, blocks, i, summ, allScores, onlySlot, fOffset,
+                Fb, listed, listBase);
+    }
 }
 
 void launchReduce(hipStream_t s, const FeatSummary* summ, int numSlots, int F, NodeBest* best) {

@@ -18,6 +18,8 @@
 // past the segments, the flipped evaluations of samples that are not Both, are
 // not placed: nothing reads them, and the atomics of one shared bucket took
 // 2 x 135 us of a level of 13 flipped frames.
+#include <algorithm>
+
 #include "cf_internal.h"
 
 namespace cf {
@@ -27,8 +29,8 @@ namespace {
 constexpr int kScanBlock = 1024;   // counts scanned per workgroup (256 lanes x 4)
 
 __global__ void __launch_bounds__(256) k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+    const size_t step = static_cast<size_t>(gridDim.x) * blockDim.x;
+    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += step) p[i] = v;
 }
 
 __global__ void __launch_bounds__(256) k_sort_count(const uint32_t* __restrict__ keys, int n, uint32_t keyEnd,
@@ -130,7 +132,8 @@ inline unsigned blocksFor(size_t n, int per) { return static_cast<unsigned>((n +
 
 void launchFillU32(hipStream_t s, uint32_t* p, size_t n, uint32_t v) {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_fill_u32, dim3(blocksFor(n, 256)), dim3(256), 0, s, p, n, v);
+    const size_t blocks = std::min<size_t>((n + 255) / 256, kMaxLaunchBlocks);
+    hipLaunchKernelGGL(k_fill_u32, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, p, n, v);
 }
 
 size_t levelSortBuckets(int numSegs, int placeBits) {
