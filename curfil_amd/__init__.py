@@ -10,6 +10,7 @@ counters of calculateFeatureResponsesAndHistograms.  All compute runs in the
 HIP library; importing this package fails if the library is not built.
 """
 import ctypes
+import functools
 import os
 
 import numpy as np
@@ -155,9 +156,20 @@ class Context:
             raise CurfilError(st, f"cf_ctx_create(device={device}) failed")
         self.h = h
         self._children = weakref.WeakSet()
+        # id of a child -> (rank, release of its native handle): when the context and its children are collected
+        # together their finalizers run in any order and the weak references are already gone
+        self._handles = {}
 
-    def _adopt(self, obj):
+    def _adopt(self, obj, release, rank=1):
+        """`obj` holds a native handle of this context; `release` gives it back (and does not refer to obj)."""
         self._children.add(obj)
+        self._handles[id(obj)] = (rank, release)
+
+    def _release(self, obj):
+        """Gives a child's handle back, unless the context has done so."""
+        rank_release = self._handles.pop(id(obj), None)
+        if rank_release:
+            rank_release[1]()
 
     def check(self, st):
         if st != CF_OK:
@@ -175,6 +187,9 @@ class Context:
             children = sorted(self._children, key=lambda c: 0 if isinstance(c, Server) else 1)
             for child in children:
                 child.close()
+            for _, release in sorted(self._handles.values(), key=lambda r: r[0]):
+                release()
+            self._handles.clear()
             lib.cf_ctx_destroy(self.h)
             self.h = None
 
@@ -195,7 +210,7 @@ class Images:
             h = ctypes.c_void_p()
             ctx.check(lib.cf_images_create(ctx.h, count, width, height, ctypes.byref(h)))
         self.h = h
-        ctx._adopt(self)
+        ctx._adopt(self, functools.partial(lib.cf_images_destroy, h))
 
     def set_rgbd_u8_padded(self, index, rgb, depth):
         """an image smaller than the set, padded as loadImages pads integrated images"""
@@ -231,7 +246,7 @@ class Images:
 
     def close(self):
         if self.h:
-            lib.cf_images_destroy(self.h)
+            self.ctx._release(self)
             self.h = None
 
     def __del__(self):
@@ -374,7 +389,7 @@ class RandomForestImage:
     def __init__(self, ctx, h):
         self.ctx, self.h = ctx, h
         if ctx is not None:
-            ctx._adopt(self)
+            ctx._adopt(self, functools.partial(lib.cf_forest_destroy, h))
 
     def _check(self, st):
         _check(self.ctx, st)
@@ -384,7 +399,7 @@ class RandomForestImage:
         that predicts with it; the library binds it at its first device call as well."""
         if self.ctx is None:
             self.ctx = ctx
-            ctx._adopt(self)
+            ctx._adopt(self, functools.partial(lib.cf_forest_destroy, self.h))
         elif self.ctx is not ctx:
             raise ValueError("forest belongs to another context")
         return self
@@ -574,7 +589,10 @@ class RandomForestImage:
 
     def close(self):
         if self.h:
-            lib.cf_forest_destroy(self.h)
+            if self.ctx is not None:
+                self.ctx._release(self)
+            else:
+                lib.cf_forest_destroy(self.h)
             self.h = None
 
     def __del__(self):
@@ -820,7 +838,7 @@ class DeviceBuffer:
         p = ctypes.c_void_p()
         ctx.check(lib.cf_device_alloc(ctx.h, nbytes, ctypes.byref(p)))
         self.ptr = p.value
-        ctx._adopt(self)
+        ctx._adopt(self, functools.partial(lib.cf_device_free, ctx.h, ctypes.c_void_p(self.ptr)))
 
     def to_host(self, dtype, shape):
         out = np.empty(shape, dtype)
@@ -830,7 +848,7 @@ class DeviceBuffer:
 
     def close(self):
         if getattr(self, "ptr", None):
-            lib.cf_device_free(self.ctx.h, ctypes.c_void_p(self.ptr))
+            self.ctx._release(self)
             self.ptr = None
 
     def __del__(self):
@@ -873,7 +891,7 @@ class Server:
         ctx.check(lib.cf_server_create(ctx.h, forest.h, float(budget_mb), max_batch, ctypes.byref(h)))
         self.h = h
         self.sizes = {}
-        ctx._adopt(self)
+        ctx._adopt(self, functools.partial(lib.cf_server_destroy, h), rank=0)
 
     def submit(self, rgb, depth):
         rgb = np.ascontiguousarray(rgb, np.uint8)
@@ -907,7 +925,7 @@ class Server:
 
     def close(self):
         if getattr(self, "h", None):
-            lib.cf_server_destroy(self.h)
+            self.ctx._release(self)
             self.h = None
 
     def __del__(self):

@@ -70,3 +70,55 @@ def test_context_without_device_fails_cleanly():
         pytest.skip("a device is present")
     h = ctypes.c_void_p()
     assert cf.lib.cf_ctx_create(0, ctypes.byref(h)) != cf.CF_OK
+
+
+class _RecordingLibrary:
+    """Stands in for the native library: hands out handles and records the calls that release them."""
+
+    def __init__(self):
+        self.released, self.handles = [], 0
+
+    def __getattr__(self, name):
+        def call(*args):
+            if name.endswith(("_destroy", "_free")):
+                self.released.append((name, getattr(args[-1], "value", args[-1])))
+            for a in args:
+                if hasattr(a, "_obj"):
+                    self.handles += 1
+                    a._obj.value = self.handles
+            return cf.CF_OK
+        return call
+
+
+@pytest.mark.parametrize("how", ["collected", "closed", "children first"])
+def test_handles_are_released_before_their_context(monkeypatch, how):
+    """A context and what lives on it that become garbage together (a cycle, or a script's globals at exit)
+    are finalized in any order, their weak references already cleared: the native handles still go before
+    the context's, the serving loop first, each once."""
+    import ctypes
+    import gc
+    lib = _RecordingLibrary()
+    monkeypatch.setattr(cf, "lib", lib)
+    ctx = cf.Context(0)
+    images = cf.Images(ctx, 1, 8, 8)
+    forest = cf.RandomForestImage(None, ctypes.c_void_p(77))
+    buffer = cf.DeviceBuffer(ctx, 64)
+    server = cf.Server(ctx, forest)
+    if how == "collected":
+        cycle = [ctx, images, forest, buffer, server]
+        cycle.append(cycle)
+        del cycle
+    elif how == "closed":
+        ctx.close()
+        assert images.h is None and forest.h is None and server.h is None
+    else:
+        server.close()
+        forest.close()
+        images.close()
+    del ctx, images, forest, buffer, server
+    gc.collect()
+    names = [n for n, _ in lib.released]
+    assert sorted(names) == ["cf_ctx_destroy", "cf_device_free", "cf_forest_destroy", "cf_images_destroy",
+                             "cf_server_destroy"]
+    assert names[0] == "cf_server_destroy" and names[-1] == "cf_ctx_destroy"
+    assert ("cf_forest_destroy", 77) in lib.released
