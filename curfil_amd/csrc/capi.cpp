@@ -90,12 +90,27 @@ void checkFeaturesSoA(const int8_t* soa, int F) {
     }
 }
 
-// The context's tables for a call on one node: the memory is kept, nothing of an earlier call is read.
-FeatTables& nodeTables(cf_ctx* ctx) {
-    if (!ctx->nodeTables) ctx->nodeTables = std::make_shared<FeatTables>();
-    ctx->nodeTables->meanDraws = 0;
-    return *ctx->nodeTables;
-}
+// The context's tables for a call on one node: nothing of an earlier call is read, and the memory is kept for the
+// next one while it is at most kKeepBytes (the largest table that can be generated, 8192 features x 256 thresholds,
+// takes 47 MiB; given features are not limited in number).  Given back here after the call, also when it throws.
+struct NodeTables {
+    static constexpr size_t kKeepBytes = size_t{64} << 20;
+    cf_ctx* ctx;
+    explicit NodeTables(cf_ctx* c) : ctx(c) {
+        if (!ctx->nodeTables) ctx->nodeTables = std::make_shared<FeatTables>();
+        ctx->nodeTables->meanDraws = 0;
+    }
+    ~NodeTables() {
+        size_t sum = 0;
+        ctx->nodeTables->each([&](auto& b) { sum += b.capacityBytes(); });
+        if (sum <= kKeepBytes) return;
+        (void)hipStreamSynchronize(ctx->stream);
+        ctx->nodeTables.reset();
+    }
+    NodeTables(const NodeTables&) = delete;
+    NodeTables& operator=(const NodeTables&) = delete;
+    FeatTables& get() const { return *ctx->nodeTables; }
+};
 
 void uploadFeaturesSoA(cf_ctx* ctx, FeatTables& tabs, const int8_t* soa, const float* thrTF, int F, int T) {
     tabs.soa.resize(static_cast<size_t>(F) * kFeatParams);
@@ -506,7 +521,8 @@ int cf_generate_features(cf_ctx* ctx, cf_images* im, const cf_sample* samples, i
         FeatGenJob j{dS.get(), n, seed, 0};
         DevBuf<FeatGenJob> dJ(1);
         CF_HIP(hipMemcpyAsync(dJ.get(), &j, sizeof(j), hipMemcpyHostToDevice, ctx->stream));
-        FeatTables& tabs = nodeTables(ctx);
+        const NodeTables kept(ctx);
+        FeatTables& tabs = kept.get();
         launchFeatureGeneration(ctx->stream, im->set(), dJ.get(), 1, F, T, boxRadius, regionSize, useDepth, tabs, true);
         CF_HIP(hipMemcpyAsync(featuresOut, tabs.soa.get(), static_cast<size_t>(F) * kFeatParams, hipMemcpyDeviceToHost,
                 ctx->stream));
@@ -570,7 +586,8 @@ int cf_node_counters(cf_ctx* ctx, cf_images* im, const cf_sample* samples, int n
         require(n > 0 && F > 0 && T > 0 && C > 0 && C <= kMaxClasses, "invalid sizes");
         checkSamples(im, samples, n);
         for (int i = 0; i < n; i++) require(samples[i].label < C, "sample label >= number of classes");
-        FeatTables& tabs = nodeTables(ctx);
+        const NodeTables kept(ctx);
+        FeatTables& tabs = kept.get();
         uploadFeaturesSoA(ctx, tabs, features, thresholds, F, T);
         DevBuf<cf_sample> dS;
         DevBuf<Chunk> dC;
@@ -592,7 +609,8 @@ int cf_node_best_split(cf_ctx* ctx, cf_images* im, const cf_sample* samples, int
         require(n > 0 && F > 0 && T > 0 && C > 0 && C <= kMaxClasses, "invalid sizes");
         checkSamples(im, samples, n);
         for (int i = 0; i < n; i++) require(samples[i].label < C, "sample label >= number of classes");
-        FeatTables& tabs = nodeTables(ctx);
+        const NodeTables kept(ctx);
+        FeatTables& tabs = kept.get();
         uploadFeaturesSoA(ctx, tabs, features, thresholds, F, T);
         DevBuf<cf_sample> dS;
         DevBuf<Chunk> dC;

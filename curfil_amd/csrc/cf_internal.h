@@ -142,7 +142,7 @@ struct cf_ctx {
     cf::DevBuf<uint8_t> scratch0, scratch1, scratch2;
     // device and page-locked memory of training calls, kept between them (bounded: trainer.cpp)
     std::shared_ptr<cf::TrainWorkspace> trainWorkspace;
-    // feature tables of the calls on one node (at most about 60 MB)
+    // feature tables of the calls on one node, kept between them up to 64 MiB (NodeTables, capi.cpp)
     std::shared_ptr<cf::FeatTables> nodeTables;
 };
 
@@ -216,6 +216,12 @@ struct FeatTables {
     PinnedBuf walkHost;
     float meanDraws = 0;       // draws per candidate in the last generation (0: none yet)
     int trees = 0, F = 0, T = 0;
+
+    template<class Fn>
+    void each(Fn&& fn) {
+        fn(feat); fn(thrFT); fn(thrTF); fn(rank); fn(thrPad); fn(soa); fn(cand); fn(unsortedFeat); fn(unsortedThr);
+        fn(unsortedKey); fn(walkSpace); fn(walkHost);
+    }
 };
 
 void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJob* jobsDev, int numJobs,

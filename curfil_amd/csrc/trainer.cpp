@@ -296,8 +296,7 @@ struct TrainWorkspace {
         fn(level[0]); fn(level[1]); fn(dir); fn(graphWork[0]); fn(graphWork[1]); fn(G); fn(summ); fn(repSumm);
         fn(allScores); fn(repBest); fn(keys); fn(vals); fn(perm); fn(sortCount); fn(sortCursor); fn(sortBlocks);
         fn(lab8); fn(starts); fn(bins); fn(results); fn(hostResults); fn(hostStarts); fn(arena[0]); fn(arena[1]);
-        fn(tabs.feat); fn(tabs.thrFT); fn(tabs.thrTF); fn(tabs.rank); fn(tabs.thrPad); fn(tabs.soa); fn(tabs.cand);
-        fn(tabs.unsortedFeat); fn(tabs.unsortedThr); fn(tabs.unsortedKey); fn(tabs.walkSpace); fn(tabs.walkHost);
+        tabs.each(fn);
         for (auto& kv : blockSets) fn(kv.second.work);
     }
     void trim() {

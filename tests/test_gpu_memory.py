@@ -1,10 +1,25 @@
-"""Sizes of device memory: histograms past 2^32 words."""
+"""Sizes of device memory: histograms past 2^32 words, what a context keeps between calls."""
+import ctypes
+import time
+
 import numpy as np
 import pytest
 
 import curfil_amd as cf
+from helpers import random_features, random_samples, random_u8_dataset
 
 pytestmark = pytest.mark.gpu
+
+
+def _free_bytes(ctx):
+    """free device memory, from the HIP runtime that the library has loaded; the driver returns freed memory a
+    millisecond or so after hipFree"""
+    ctx.synchronize()
+    time.sleep(0.25)
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
 
 
 def test_histograms_past_2_32_words(ctx, monkeypatch):
@@ -29,4 +44,39 @@ def test_histograms_past_2_32_words(ctx, monkeypatch):
         nodes += int(((wn["level"] == 7) & (wn["num_samples"] >= 2) & ((wh > 0).sum(1) > 1)).sum())
     assert nodes * 8192 * 256 * 10 > 1 << 32
     assert want.profile()["slot_batches_max"] > 1 and got.profile()["slot_batches_max"] == 1
+    im.close()
+
+
+@pytest.mark.parametrize("call", ["counters", "best split", "refused"])
+def test_tables_of_a_large_node_call_are_given_back(ctx, call):
+    """The features of a single-node call are not limited in number: its tables (here 340 MiB) stay with the
+    context up to 64 MiB only, also when the call is refused after its buffers were made."""
+    rgb, depth, _ = random_u8_dataset(1, 64, 48, seed=5)
+    im = cf.Images(ctx, 1, 64, 48)
+    im.set_rgbd_u8(0, rgb[0], depth[0])
+    rng = np.random.default_rng(2)
+    s = random_samples(rng, 40, 1, 64, 48, depth.astype(np.int32))
+    s["depth_mm"] = np.where(s["depth_mm"] > 0, s["depth_mm"], -1)
+    s["label"] = rng.integers(0, 2, 40)
+    hist = np.bincount(s["label"], minlength=2).astype(np.uint32)
+
+    def run(F, T, bad=False):
+        feats = random_features(rng, F, box_radius=10)
+        thr = rng.normal(0, 200, (T, F)).astype(np.float32)
+        if bad:
+            thr[0, 0] = np.nan
+        if call == "counters":
+            cf.node_counters(ctx, im, s, feats, thr, 2)
+        else:
+            cf.node_best_split(ctx, im, s, feats, thr, 2, hist)
+
+    run(10, 8)
+    before = _free_bytes(ctx)
+    if call == "refused":
+        with pytest.raises(cf.CurfilError):
+            run(4000000, 16, bad=True)
+    else:
+        run(400000, 64)
+    assert before - _free_bytes(ctx) <= 80 << 20
+    run(10, 8)
     im.close()
