@@ -80,3 +80,41 @@ def test_tables_of_a_large_node_call_are_given_back(ctx, call):
     assert before - _free_bytes(ctx) <= 80 << 20
     run(10, 8)
     im.close()
+
+
+def test_workspace_of_a_large_training_is_trimmed_and_used_again(ctx):
+    """A training whose workspace passes 1 GiB (a level of more than 50 nodes of 8192 features x 65 bins x 10 classes
+    in its histograms alone) leaves at most that with the context; the next trainings on it, a small one and the
+    same again, give the same trees as the first and as another context."""
+    rgb, depth, labels = cf.synth_dataset(4, 160, 120, sites=60, classes=9, zero_frac=0.05, seed0=4711)
+    rng = np.random.default_rng(3)
+    labels = np.where(rng.random(labels.shape) < 0.3, rng.integers(0, 10, labels.shape), labels).astype(np.uint8)
+    im = cf.Images(ctx, 4, 160, 120)
+    for i in range(4):
+        im.set_rgbd_u8(i, rgb[i], depth[i])
+        im.set_labels(i, labels[i])
+
+    def train(c, images, features, thresholds):
+        cfg = cf.TrainingConfiguration(4711, 6000, features, 2, 6, 30, 8, thresholds)
+        f = cf.RandomForestImage.train(c, images, cfg, 4, 10, cf.MODE_BATCHED)
+        out = [f.tree(t) for t in range(4)]
+        f.close()
+        return out
+
+    before = _free_bytes(ctx)
+    own = cf.Context(0)
+    im2 = cf.Images(own, 4, 160, 120)
+    for i in range(4):
+        im2.set_rgbd_u8(i, rgb[i], depth[i])
+        im2.set_labels(i, labels[i])
+    first = train(own, im2, 8192, 64)
+    level = sum(int(((n["level"] == 5) & (n["num_samples"] >= 2) & ((h > 0).sum(1) > 1)).sum()) for n, h in first)
+    assert level * 8192 * 65 * 10 * 4 > 1 << 30
+    assert before - _free_bytes(own) <= (1 << 30) + (256 << 20)   # the images, the stream and the call's scratch beside it
+    small = train(own, im2, 40, 10)
+    again = train(own, im2, 8192, 64)
+    want = train(ctx, im, 40, 10)
+    for a, b in list(zip(first, again)) + list(zip(small, want)):
+        assert a[0].tobytes() == b[0].tobytes() and np.array_equal(a[1], b[1])
+    own.close()
+    im.close()
