@@ -194,7 +194,10 @@ private:
         return k;
     }
 
-    // file lines: "TM class shape"
+    // file lines: "TM class lanes perLane featPerStep wgPerCu kernel".  A shape is kept by what it is, not by its place
+    // in the list, together with the kernel that it was timed on: a line of another list or kernel (or "TM class
+    // shape", as earlier builds wrote) settles nothing and its key is tuned again.
+    static constexpr int kKernel = 2;   // 1: waves with samples of their own; 2: the waves share their samples
     void load() {
         if (loaded_ || file_.empty()) return;
         loaded_ = true;
@@ -202,9 +205,15 @@ private:
         std::string line;
         while (std::getline(in, line)) {
             std::istringstream ls(line);
-            int tm = 0, cls = 0, shape = -1;
-            if (!(ls >> tm >> cls >> shape) || shape < 0 || shape >= numEvalShapes()) continue;
-            state(tm, cls).best = shape;
+            int tm = 0, cls = 0, kernel = 0;
+            EvalShape sh{};
+            if (!(ls >> tm >> cls >> sh.lanes >> sh.perLane >> sh.featPerStep >> sh.wgPerCu >> kernel) || kernel != kKernel) continue;
+            for (int i = 0; i < numEvalShapes(); i++) {
+                const EvalShape& e = evalShape(i);
+                if (e.lanes == sh.lanes && e.perLane == sh.perLane && e.featPerStep == sh.featPerStep && e.wgPerCu == sh.wgPerCu) {
+                    state(tm, cls).best = i;
+                }
+            }
         }
     }
 
@@ -212,7 +221,10 @@ private:
         if (file_.empty()) return;
         std::ofstream o(file_, std::ios::trunc);
         for (auto& kv : keys_) {
-            if (kv.second.best >= 0) o << kv.first.first << ' ' << kv.first.second << ' ' << kv.second.best << '\n';
+            if (kv.second.best < 0) continue;
+            const EvalShape& e = evalShape(kv.second.best);
+            o << kv.first.first << ' ' << kv.first.second << ' ' << e.lanes << ' ' << e.perLane << ' ' << e.featPerStep << ' '
+              << e.wgPerCu << ' ' << kKernel << '\n';
         }
     }
 

@@ -122,3 +122,50 @@ def test_handles_are_released_before_their_context(monkeypatch, how):
                              "cf_server_destroy"]
     assert names[0] == "cf_server_destroy" and names[-1] == "cf_ctx_destroy"
     assert ("cf_forest_destroy", 77) in lib.released
+
+
+_TUNER_SCRIPT = """
+import ctypes, os, sys
+import curfil_amd as cf
+choose = cf.lib._ZN2cf15evalTunerChooseEimPb
+choose.argtypes = [ctypes.c_int, ctypes.c_size_t, ctypes.POINTER(ctypes.c_bool)]
+record = cf.lib._ZN2cf15evalTunerRecordEimidd
+record.argtypes = [ctypes.c_int, ctypes.c_size_t, ctypes.c_int, ctypes.c_double, ctypes.c_double]
+record.restype = None
+measure = ctypes.c_bool()
+shape = choose(32, 1 << 24, ctypes.byref(measure))
+print(shape, int(measure.value))
+fastest = int(sys.argv[1])
+while fastest >= 0 and measure.value:
+    record(32, 1 << 24, shape, 1.0 if shape == fastest else 2.0, 1e9)
+    shape = choose(32, 1 << 24, ctypes.byref(measure))
+print(shape)
+"""
+
+
+def _tuner(path, fastest=-1):
+    """First choice (shape, whether it is to be timed) and last for a large level of 32 thresholds in a process of
+    its own, which times launches until its key is settled if `fastest` names a shape."""
+    import subprocess
+    import sys
+    env = dict(os.environ, CURFIL_TUNE_FILE=str(path), CURFIL_TUNE_ROUNDS="1", PYTHONPATH=ROOT)
+    for name in ("CURFIL_EVAL_SHAPE", "CURFIL_TUNE"):
+        env.pop(name, None)
+    out = subprocess.run([sys.executable, "-c", _TUNER_SCRIPT, str(fastest)], env=env, cwd=ROOT, check=True,
+                         capture_output=True, text=True).stdout.split()
+    return int(out[0]), int(out[1]), int(out[2])
+
+
+def test_tune_file_of_another_build_is_tuned_again(tmp_path):
+    """A tune file names a launch shape by what it is and the kernel it was measured on; lines that do not (an
+    earlier build's shape numbers) or that name another kernel are not taken as choices."""
+    path = tmp_path / "tuning.txt"
+    path.write_text("32 2 4\n20 2 1\n")
+    assert _tuner(path)[:2] == (0, 1)
+    # what this build settles is read back as settled
+    assert _tuner(path, fastest=2)[2] == 2
+    assert _tuner(path)[:2] == (2, 0)
+    line = [v.split() for v in path.read_text().splitlines() if v.startswith("32 2 ")][-1]
+    assert tuple(int(v) for v in line[2:6]) == cf.eval_shape_info(2)
+    path.write_text(" ".join(line[:-1] + [str(int(line[-1]) - 1)]) + "\n")
+    assert _tuner(path)[:2] == (0, 1)
