@@ -280,14 +280,17 @@ struct BinBlock {
     int count;
     int image;   // the image of every sample in the block
 };
-// keys ((image * keyMul + keyBase) << placeBits | the sample's place in the image, below levelPlaces) and
-// values (level index) of one tree's level segment;
+// keys ((image * keyMul + keyBase) << placeBits | the sample's place in the image, below levelPlaces, >> placeShift)
+// and values (level index) of one tree's level segment;
 // with flipN > 0 also the flipped evaluation of every Both sample at flipN + index (value |
 // kFlipEntry), and segment absentKey for the other samples there
 constexpr uint32_t kFlipEntry = 0x80000000u;
 void launchLevelKeys(hipStream_t s, const cf_sample* samples, int begin, int n, uint32_t keyBase, uint32_t keyMul,
-        uint32_t* keys, uint32_t* vals, int flipN, uint32_t absentKey, int placeBits, int H);
+        uint32_t* keys, uint32_t* vals, int flipN, uint32_t absentKey, int placeBits, int placeShift, int H);
 int levelPlaces(int W, int H);
+// Bits of a place in the keys of so many segments, and in *shift the low bits that are dropped from the place:
+// as many as the buckets have to be fewer than 2^26 (their counts are cleared and scanned at every level).
+int levelPlaceBits(uint64_t segments, int places, int* shift);
 // label per level index, bit 7 set for samples still set to Both (counted in both orientations)
 void launchLevelLabels(hipStream_t s, const cf_sample* samples, int n, uint8_t* labels);
 // Counting sort of the n level entries with a key below numSegs << placeBits (the others are not placed): out =

@@ -321,14 +321,27 @@ int levelPlaces(int W, int H) {
     return ((W + kStripWidth - 1) / kStripWidth) * ((H + kStripRows - 1) / kStripRows);
 }
 
+// Past 2^26 buckets a place loses low bits (steps of 8, 16 ... rows of a strip) rather than all of them: 50 frames of
+// 640x480, 5 trees, 1000 x 32 take 131 ms of pass 1 with whole places, 132, 133, 136, 140 with 1, 2, 3, 4 bits
+// dropped, 153 with 8, 163 with none kept.  Whole places fit 65534 (image, tree) segments of 640x480.
+int levelPlaceBits(uint64_t segments, int places, int* shift) {
+    constexpr uint64_t kMaxBuckets = 1ull << 26;
+    int bits = 0;
+    while ((1 << bits) < places) bits++;
+    int kept = bits;
+    while (kept > 0 && ((segments + 2) << kept) > kMaxBuckets) kept--;
+    *shift = bits - kept;
+    return kept;
+}
+
 // Sort keys (segment << placeBits | place) and values (level index) of one tree's level segment.
 __global__ void __launch_bounds__(256) k_level_keys(const cf_sample* __restrict__ samples, int begin, int n,
         uint32_t keyBase, uint32_t keyMul, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, int flipN,
-        uint32_t absentKey, int placeBits, int stripPlaces) {
+        uint32_t absentKey, int placeBits, int placeShift, int stripPlaces) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const cf_sample x = samples[begin + i];
-    const uint32_t place = placeBits > 0 ? (x.x / kStripWidth) * stripPlaces + x.y / kStripRows : 0u;
+    const uint32_t place = placeBits > 0 ? ((x.x / kStripWidth) * stripPlaces + x.y / kStripRows) >> placeShift : 0u;
     const uint32_t seg = static_cast<uint32_t>(x.image) * keyMul + keyBase;
     keys[begin + i] = (seg << placeBits) | place;
     vals[begin + i] = static_cast<uint32_t>(begin + i);
@@ -397,10 +410,10 @@ int binThresholdWidth(int T) {
 }
 
 void launchLevelKeys(hipStream_t s, const cf_sample* samples, int begin, int n, uint32_t keyBase, uint32_t keyMul,
-        uint32_t* keys, uint32_t* vals, int flipN, uint32_t absentKey, int placeBits, int H) {
+        uint32_t* keys, uint32_t* vals, int flipN, uint32_t absentKey, int placeBits, int placeShift, int H) {
     if (n == 0) return;
     hipLaunchKernelGGL(k_level_keys, dim3((n + 255) / 256), dim3(256), 0, s, samples, begin, n, keyBase, keyMul, keys,
-            vals, flipN, absentKey, placeBits, (H + kStripRows - 1) / kStripRows);
+            vals, flipN, absentKey, placeBits, placeShift, (H + kStripRows - 1) / kStripRows);
 }
 
 int buildWorkLength(int blocks, int ngb) {

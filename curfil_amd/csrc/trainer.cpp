@@ -513,16 +513,17 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             dLab8.resize(N);
             const uint64_t keyRange = static_cast<uint64_t>(numActive) * static_cast<uint64_t>(images->count);
             if (keyRange >= (1ull << 27)) throw Error(CF_ERR_UNSUPPORTED, "too many (tree, image) segments in one level");
-            // within a segment, samples ordered by place while the buckets stay below 2^26 (CURFIL_ROW_ORDER=0: off)
-            int placeBits = 0;
-            while ((1 << placeBits) < levelPlaces(images->W, images->H)) placeBits++;
+            // within a segment, samples ordered by place, as finely as the number of segments allows
+            // (CURFIL_ROW_ORDER=0: not at all)
+            int placeShift = 0;
+            int placeBits = levelPlaceBits(keyRange, levelPlaces(images->W, images->H), &placeShift);
             const char* rowOrder = std::getenv("CURFIL_ROW_ORDER");
-            if (((keyRange + 2) << placeBits) > (1ull << 26) || (rowOrder && std::strcmp(rowOrder, "0") == 0)) placeBits = 0;
+            if (rowOrder && std::strcmp(rowOrder, "0") == 0) placeBits = 0;
             // segments (image, tree) in image-major order: the trees' segments of one image are adjacent
             for (int a = 0; a < numActive; a++) {
                 launchLevelKeys(s, level[cur].get(), active[a].begin, active[a].n, static_cast<uint32_t>(a),
                         static_cast<uint32_t>(numActive), dKeys.get(), dVals.get(), anyBoth ? N : 0,
-                        static_cast<uint32_t>(keyRange), placeBits, images->H);
+                        static_cast<uint32_t>(keyRange), placeBits, placeShift, images->H);
             }
             numKeys = static_cast<int>(keyRange);
             dSortCount.resize(levelSortBuckets(numKeys, placeBits));

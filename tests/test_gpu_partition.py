@@ -70,3 +70,24 @@ def test_scored_where_counted_matches_oracle(ctx, frames, T, C, flip):
         assert np.array_equal(nodes[name][inner], on[name][inner]), name
     assert np.abs(nodes["score"][inner] - on["score"][inner]).max() <= 4e-16
     assert np.array_equal(hist, oh)
+
+
+def test_coarsened_places_train_alike(ctx, monkeypatch):
+    """190 trees over 700 frames of 1024x256 are 133000 (image, tree) segments a level: whole places (9 bits) would
+    pass 2^26 buckets and one bit is dropped.  The order only decides which lanes evaluate what: the trees are those
+    of levels that are not ordered by place."""
+    n, trees = 700, 190
+    rgb, depth, labels = random_u8_dataset(7, 1024, 256, seed=3)
+    im = cf.Images(ctx, n, 1024, 256)
+    for i in range(n):
+        im.set_rgbd_u8(i, rgb[i % 7], depth[i % 7])
+        im.set_labels(i, labels[i % 7])
+    cfg = cf.TrainingConfiguration(4711, trees, 20, 5, 5, 30, 6, 4, subsamplingType="pixelUniform")
+    forests = []
+    for order in ("1", "0"):
+        monkeypatch.setenv("CURFIL_ROW_ORDER", order)
+        forests.append(cf.RandomForestImage.train(ctx, im, cfg, trees, 6, cf.MODE_BATCHED))
+    im.close()
+    for t in range(trees):
+        (an, ah), (bn, bh) = forests[0].tree(t), forests[1].tree(t)
+        assert len(an) > 7 and an.tobytes() == bn.tobytes() and np.array_equal(ah, bh)

@@ -169,3 +169,24 @@ def test_tune_file_of_another_build_is_tuned_again(tmp_path):
     assert tuple(int(v) for v in line[2:6]) == cf.eval_shape_info(2)
     path.write_text(" ".join(line[:-1] + [str(int(line[-1]) - 1)]) + "\n")
     assert _tuner(path)[:2] == (0, 1)
+
+
+@pytest.mark.parametrize("width,height", [(1, 1), (160, 120), (640, 480), (1280, 960), (2048, 64), (32767, 32767)])
+def test_level_order_keeps_as_many_place_bits_as_fit(width, height):
+    """The keys of a level's order hold the (image, tree) segment and a sample's place in the image.  Where whole
+    places would pass 2^26 buckets they are coarsened bit by bit, not left out (65534 segments of 640x480 and one
+    more)."""
+    import ctypes
+    places_of = cf.lib._ZN2cf11levelPlacesEii
+    bits_of = cf.lib._ZN2cf14levelPlaceBitsEmiPi
+    bits_of.argtypes = [ctypes.c_uint64, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+    places = places_of(width, height)
+    assert places == -(-width // 128) * -(-height // 4)
+    full = (places - 1).bit_length()
+    for segments in (1, 100, 65534, 65535, 131070, 131071, 1 << 20, (1 << 25) - 2, (1 << 25) - 1, (1 << 26) - 2, (1 << 27) - 1):
+        shift = ctypes.c_int(-1)
+        bits = bits_of(segments, places, ctypes.byref(shift))
+        assert bits + shift.value == full and bits >= 0 and shift.value >= 0
+        assert ((places - 1) >> shift.value).bit_length() <= bits
+        assert bits == 0 or (segments + 2) << bits <= 1 << 26
+        assert bits == full or (segments + 2) << (bits + 1) > 1 << 26
