@@ -398,7 +398,10 @@ __device__ __forceinline__ bool scoreBetter(double best, double score) {
 // then resolved in order with the reference's predicate.  A segment whose list is full is scanned whole.
 // Bound by latency (one wave over all scores: 49 us for 500 x 50, 223 for 4000 x 32; now 16 and
 // 31).
-constexpr int kSeqWaves = 16, kSeqList = 64, kSeqAhead = 8;
+// Up to kSeqAlone scores one wave resolves all windows and lists none (a call on 1, 512, 1024, 2048, 5000 random
+// scores takes 29, 34, 34, 37, 48 us with one wave, 31, 41, 39, 40, 46 with sixteen; ascending ones 29, 74, 120, 214,
+// 490 and 31, 83, 136, 225, 479).
+constexpr int kSeqWaves = 16, kSeqList = 64, kSeqAhead = 8, kSeqAlone = 48 * 64;
 __global__ void __launch_bounds__(64 * kSeqWaves) k_seq_argmax(const double* __restrict__ allScores, int T, int F,
         NodeBest* __restrict__ allOut) {
     __shared__ int list[kSeqWaves][kSeqList], listed[kSeqWaves];   // windows of a segment, -1: all of them
@@ -407,12 +410,16 @@ __global__ void __launch_bounds__(64 * kSeqWaves) k_seq_argmax(const double* __r
     const long long n = static_cast<long long>(T) * F;
     // one node per workgroup: scores[T][F] and its result
     const double* scores = allScores + static_cast<size_t>(blockIdx.x) * n;
-    const int windows = static_cast<int>((n + 63) / 64), per = (windows + kSeqWaves - 1) / kSeqWaves;
+    const int waves = static_cast<int>(blockDim.x >> 6);   // 1 or kSeqWaves
+    const int windows = static_cast<int>((n + 63) / 64), per = (windows + waves - 1) / waves;
     auto scoreAt = [&](int w) {
         const long long i = static_cast<long long>(w) * 64 + lane;
         return i < n ? scores[i] : -__builtin_inf();
     };
-    {
+    if (waves == 1) {
+        if (lane == 0) listed[0] = -1;
+        __syncthreads();
+    } else {
         const int first = min(wave * per, windows), end = min(first + per, windows);
         double run = -__builtin_inf();
         int count = 0;
@@ -454,7 +461,7 @@ __global__ void __launch_bounds__(64 * kSeqWaves) k_seq_argmax(const double* __r
     if (wave != 0) return;
     double best = -__builtin_inf();
     long long pos = 0;
-    for (int s = 0; s < kSeqWaves; s++) {
+    for (int s = 0; s < waves; s++) {
         const int first = min(s * per, windows), end = min(first + per, windows);
         const int count = listed[s] < 0 ? end - first : listed[s];
         for (int k0 = 0; k0 < count; k0 += kSeqAhead) {
@@ -629,7 +636,8 @@ void launchReduce(hipStream_t s, const FeatSummary* summ, int numSlots, int F, N
 
 void launchSequentialArgmax(hipStream_t s, const double* scores, int T, int F, NodeBest* best, int numNodes) {
     if (numNodes <= 0) return;
-    hipLaunchKernelGGL(k_seq_argmax, dim3(static_cast<unsigned>(numNodes)), dim3(64 * kSeqWaves), 0, s, scores, T, F, best);
+    const int waves = static_cast<int64_t>(T) * F <= kSeqAlone ? 1 : kSeqWaves;
+    hipLaunchKernelGGL(k_seq_argmax, dim3(static_cast<unsigned>(numNodes)), dim3(64 * waves), 0, s, scores, T, F, best);
 }
 
 void launchCountersFromBins(hipStream_t s, const uint32_t* G, const FeatTables& tabs, int C, uint32_t* counters) {

@@ -65,3 +65,25 @@ def test_argmax_scan_edges(ctx, F, T, order):
     f, t, best = cf.argmax_scores(ctx, scores)
     bf, bt, bb = orc.argmax(scores)
     assert (f, t) == (bf, bt) and best == bb
+
+
+# the number of scores past which sixteen waves take them, and segments of a few windows behind it
+@pytest.mark.parametrize("F,T", [(3072, 1), (1024, 3), (3073, 1), (439, 7), (4097, 1), (512, 11)])
+@pytest.mark.parametrize("order", ["random", "ascending", "ties", "steps", "infinite"])
+def test_argmax_waves_edges(ctx, F, T, order):
+    rng = np.random.default_rng(F * T)
+    n = F * T
+    scores = rng.random(n)
+    if order == "ascending":
+        scores = np.sort(scores)
+    elif order == "ties":
+        scores = 0.5 + rng.integers(0, 40, n) * 0.3e-13
+    elif order == "steps":
+        scores = 0.5 + np.arange(n) * rng.choice([0.2e-13, 0.6e-13, 1.1e-13], n)
+    elif order == "infinite":
+        scores[:n // 2] = -np.inf
+        scores[rng.integers(0, n, 5)] = np.nan
+    scores = scores.reshape(T, F)
+    f, t, best = cf.argmax_scores(ctx, scores)
+    bf, bt, bb = orc.argmax(scores)
+    assert (f, t) == (bf, bt) and best == bb
