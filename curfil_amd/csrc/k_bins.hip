@@ -515,8 +515,6 @@ void launchEvalBins(hipStream_t s, const ImageSet& imgs, const cf_sample* sample
                 flipOffset, blockMax);                                                                           \
         return;                                                                                                  \
     }
-    CF_SHAPE(128, 1)
-    CF_SHAPE(128, 2)
     CF_SHAPE(256, 1)
     CF_SHAPE(256, 2)
     CF_SHAPE(256, 4)

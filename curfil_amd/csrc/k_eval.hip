@@ -36,7 +36,6 @@ constexpr int kEvalThreads = 256;
 constexpr int kEvalStep = 4;           // features whose corner gathers are issued together
 constexpr int kEvalTile = 16;          // features of a workgroup
 constexpr int kEvalSmallTile = 4;      // the same where there are few workgroups
-constexpr int kXcds = 8;               // MI355X: 8 XCDs, workgroups dispatched round-robin
 
 // One training pixel held in registers for the feature loop.
 struct RegSample {
@@ -92,8 +91,8 @@ __global__ void __launch_bounds__(kEvalThreads) k_eval_hist(const float* __restr
         uint32_t* __restrict__ G, NodeScoring scoring) {
     extern __shared__ double evalLds[];   // scoreFeatures' part where the tile is scored, the bins
     uint32_t* h = reinterpret_cast<uint32_t*>(evalLds) + (scoring.summ ? scoreLdsBytes(tile, T, C) / sizeof(uint32_t) : 0);
-    const int total = numChunks * tiles, per = (total + kXcds - 1) / kXcds;
-    const int item = static_cast<int>(blockIdx.x % kXcds) * per + static_cast<int>(blockIdx.x / kXcds);
+    const int total = numChunks * tiles, per = (total + kNumXcds - 1) / kNumXcds;
+    const int item = static_cast<int>(blockIdx.x % kNumXcds) * per + static_cast<int>(blockIdx.x / kNumXcds);
     if (item >= total) return;
     const int chunkIdx = item / tiles, tileIdx = item - chunkIdx * tiles;
     Chunk ch = node;
@@ -565,7 +564,7 @@ static void launchEval(hipStream_t s, const ImageSet& imgs, const cf_sample* sam
     const int tiles = (tabs.F + tile - 1) / tile;
     const size_t lds = static_cast<size_t>(tile) * (tabs.T + 1) * C * sizeof(uint32_t) +
             (scoring.summ ? scoreLdsBytes(tile, tabs.T, C) : 0);
-    const int64_t blocks = (static_cast<int64_t>(numChunks) * tiles + kXcds - 1) / kXcds * kXcds;
+    const int64_t blocks = (static_cast<int64_t>(numChunks) * tiles + kNumXcds - 1) / kNumXcds * kNumXcds;
     if (blocks > INT32_MAX) throw Error(CF_ERR_UNSUPPORTED, "too many samples in one evaluation launch");
     const dim3 grid(static_cast<unsigned>(blocks)), block(kEvalThreads);
     auto launch = [&](auto tm) {
