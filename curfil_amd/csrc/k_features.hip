@@ -799,6 +799,8 @@ void launchFeatureGeneration(hipStream_t s, const ImageSet& imgs, const FeatGenJ
     if (T > kMaxThresholds) throw Error(CF_ERR_ARG, "too many thresholds (max 256)");
     if (F > 8192) throw Error(CF_ERR_ARG, "too many features (max 8192)");
     if (boxRadius > 127 || regionSize > 127) throw Error(CF_ERR_ARG, "boxRadius/regionSize must fit int8");
+    // a candidate's second offset is drawn until it differs from the first: with one offset to draw, for ever
+    if (boxRadius < 1) throw Error(CF_ERR_ARG, "boxRadius must be at least 1");
     const int numCand = 3 * F;
     tabs.trees = numJobs;
     tabs.F = F;

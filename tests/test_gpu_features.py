@@ -44,3 +44,16 @@ def test_feature_walk_edges_match_oracle(ctx, frames, n, F, T, br, rs, missing):
     feats, thr = cf.generate_features(ctx, im, s, F + T, F, T, br, rs)
     assert np.array_equal(feats, want[0])
     assert np.array_equal(thr.view(np.uint32), want[1].view(np.uint32))
+
+
+def test_box_radius_of_zero_is_refused(ctx, frames):
+    """With boxRadius 0 there is one offset, and a feature's two cannot differ."""
+    depth, labels, im, _ = frames
+    s = random_samples(np.random.default_rng(1), 50, 4, 160, 120, depth.astype(np.int32), labels=labels)
+    s = s[s["depth_mm"] > 0]
+    with pytest.raises(cf.CurfilError, match="boxRadius"):
+        cf.generate_features(ctx, im, s, 1, 10, 4, 0, 5)
+    cfg = cf.TrainingConfiguration(1, 1, 10, 2, 3, 0, 5, 4)
+    for mode in (cf.MODE_BATCHED, cf.MODE_PLAIN):
+        with pytest.raises(cf.CurfilError, match="boxRadius"):
+            cf.RandomForestImage.train_tree_from_samples(ctx, im, cfg, 0, 6, 1, s, mode=mode)
