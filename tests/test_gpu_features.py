@@ -46,6 +46,47 @@ def test_feature_walk_edges_match_oracle(ctx, frames, n, F, T, br, rs, missing):
     assert np.array_equal(thr.view(np.uint32), want[1].view(np.uint32))
 
 
+# what the oracle cannot generate either: a third of the samples without depth where most responses are NaN already;
+# 50 features of 20 thresholds from one sample that has NaN for most of them
+EXCEEDS_CANDIDATES = {(2000, 60, 65, 127, 20, True), (2000, 16, 255, 127, 20, True), (1, 50, 20, 10, 5, False),
+                      (1, 50, 20, 10, 5, True)}
+
+
+@pytest.mark.parametrize("n,F,T,br,rs", [(700, 40, 1, 60, 10), (700, 90, 9, 127, 20), (1500, 400, 17, 127, 10),
+                                         (2000, 60, 65, 127, 20), (2000, 30, 129, 60, 10), (2000, 16, 255, 127, 20),
+                                         (1, 50, 20, 10, 5)])
+@pytest.mark.parametrize("missing", [False, True])
+def test_feature_walk_exceeds_only_where_expected(ctx, frames, n, F, T, br, rs, missing):
+    depth, labels, im, ds = frames
+    rng = np.random.default_rng(1000 * F + T)
+    s = random_samples(rng, 4 * n, 4, 160, 120, depth.astype(np.int32), labels=labels)
+    s = s[s["depth_mm"] > 0][:n]
+    if missing and n > 1:
+        s["depth_mm"][rng.random(n) < 0.3] = -1
+    if (n, F, T, br, rs, missing) in EXCEEDS_CANDIDATES:
+        with pytest.raises(RuntimeError, match="max loops exceeded"):
+            ds.generate_features(s, F + T, F, T, br, rs)
+        with pytest.raises(cf.CurfilError, match="max loops exceeded"):
+            cf.generate_features(ctx, im, s, F + T, F, T, br, rs)
+        return
+    want = ds.generate_features(s, F + T, F, T, br, rs)
+    feats, thr = cf.generate_features(ctx, im, s, F + T, F, T, br, rs)
+    assert np.array_equal(feats, want[0])
+    assert np.array_equal(thr.view(np.uint32), want[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("x,y", [(80, 60), (20, 100)])
+@pytest.mark.parametrize("T", [1, 20, 255])
+def test_feature_walk_of_one_sample(ctx, frames, x, y, T):
+    """One sample: every draw is the same, and a feature's thresholds are all its one response."""
+    depth, labels, im, ds = frames
+    s = cf.make_samples(np.array([x]), np.array([y]), np.array([1]), np.array([4000], np.int32), np.array([2]))
+    want = ds.generate_features(s, 3, 30, T, 40, 6)
+    feats, thr = cf.generate_features(ctx, im, s, 3, 30, T, 40, 6)
+    assert np.array_equal(feats, want[0])
+    assert np.array_equal(thr.view(np.uint32), want[1].view(np.uint32))
+
+
 def test_box_radius_of_zero_is_refused(ctx, frames):
     """With boxRadius 0 there is one offset, and a feature's two cannot differ."""
     depth, labels, im, _ = frames
