@@ -27,14 +27,15 @@
 // trees' workgroups of one feature group read the same planes of one image
 // and an XCD's L2 holds them.
 //
-// Pass 1 is bound by the vector memory path (the L1's misses in flight, about
-// 60 of 64 per CU, times the L2's latency of 150 cycles under this load), not by
-// arithmetic or HBM; its lookups are not far behind (0.94 per CU and cycle).
-// What counts is lines fetched per response: 3.33 with samples ordered by row,
-// 3.06 in strips, 2.76 with the waves of a workgroup on the same samples.  Eight
+// Pass 1 is bound by the vector memory path (58 lines in flight per CU times the
+// L2's latency of 152 cycles under this load; the L1 is stalled on them in 55% of
+// the cycles), not by arithmetic or HBM; its lookups are not far behind (0.90 per
+// CU and cycle).  What counts is lines fetched per response: 3.33 with samples
+// ordered by row, 3.06 in strips, 2.77 with the waves of a workgroup on the same
+// samples (21 frames, 3 trees, 2000 x 20, shape 0; 2.62 with shape 2).  Eight
 // waves per CU, each lane with one sample's 8 corner loads in flight, beat
 // configurations with more in flight: the blocks an XCD runs at once cover a few
-// feature groups of a segment, the planes they read fit the XCD's L2 (0.5%
+// feature groups of a segment, the planes they read fit the XCD's L2 (0.4%
 // misses) and requests return sooner.  The launch reserves LDS the kernel does
 // not use to hold the CU at the shape's workgroups.
 #include <algorithm>
@@ -116,8 +117,8 @@ constexpr int kBlockSampleBytes = sizeof(BinSample) + kBinGroup + sizeof(int);
 // covers one block of samples and a group of 16 features.  All its waves take the same 64 samples at a time,
 // wave w the features w, w + WAVES, ... of the group: neighbouring features of the table read the same plane with
 // nearly the same row offset, so the waves' corners fall on the same lines of a small patch, and a line that one
-// wave brought into the L1 serves the others.  (Waves with samples of their own and the same feature share
-// nothing: XX.)  A wave's features and thresholds are uniform and stay in scalar registers over the block.
+// wave brought into the L1 serves the others.  (Waves with samples of their own and the same feature share nothing:
+// 3.06 lines a response in place of 2.77.)  A wave's features and thresholds are uniform and stay in scalar registers over the block.
 template<int TM, int WAVES, int FPS>
 __global__ void __launch_bounds__(WAVES * 64) k_eval_bins(const float* __restrict__ colBase,
         const int2* __restrict__ depBase, int W, int H, const cf_sample* __restrict__ samples,
@@ -223,8 +224,9 @@ struct LevelScoring {
 // an order rotated by the sample, so that one LDS atomic instruction covers 4 samples of each of the 16
 // features: their histograms lie in different banks and at most 4 lanes can hit one address (all lanes counting
 // one feature, as for samples of an almost pure node, would collide on few bins).  Features past the table's last
-// hold anything in the rows; they are counted into histograms that nothing reads.  Of the LDS cycles, 70% of
-// the time, a third are banks met twice and a third equal addresses (samples of one class in one bin).
+// hold anything in the rows; they are counted into histograms that nothing reads.  With the scores of the
+// small nodes (50 frames, 5 trees, 4000 x 32) the LDS works in half of the cycles, two thirds of them conflicts, a
+// third on equal addresses (samples of one class in one bin).
 // One feature of a sample a lane took a byte load and three times the instructions for each atomic, and a
 // chunk was not cut into parts: 13 flipped frames, 500 x 50 108 us a level (now 36); 4 small frames 19 (5); 21
 // frames, 3 trees, 2000 x 20 199 (151); 50 frames, 5 trees, 4000 x 32 1562 (1245).
@@ -436,10 +438,12 @@ void launchLevelLabels(hipStream_t s, const cf_sample* samples, int n, uint8_t* 
 }
 
 // Launch shapes of pass 1 the tuner chooses from: {lanes, samples of a block per lane, features whose gathers
-// are issued together, workgroups per CU}.  Shape 0 is the default.  On large levels the shapes with two
-// workgroups are within 1% of each other and ahead (21 frames, 3 trees, 2000 x 20: 93.2, 92.2, 91.6, 96.5, 99.2 ms
-// of pass 1 a training in this order); on small ones with wide threshold rows the last two are (13 flipped
-// frames of 320x240, 2 trees, 500 x 50: 3.5, 3.9, 4.0, 3.0, 2.95 ms).
+// are issued together, workgroups per CU}.  Shape 0 is the default.  Which is ahead turns on the threshold rows:
+// with up to 32 thresholds the shapes of two workgroups, within 2% of each other, with more the compares count and
+// the last two overlap them with the gathers.  Pass 1 of 70 frames, 5 trees, 1.4 million entries in this order, ms:
+// 512 x 8 69.9, 68.6, 68.4, 72.5, 74.8; 512 x 32 70.1, 70.1, 70.9, 72.7, 75.0; 512 x 50 72.4, 76.0, 78.7, 73.0,
+// 75.2 and flipped 133.0, 141.6, 145.6, 127.8, 130.4; 256 x 100 79.7, 84.6, 86.5, 69.5, 66.5.  (Levels below the
+// tuner's smallest class run shape 0 whatever their rows.)
 constexpr EvalShape kEvalShapes[] = {
     {256, 1, 1, 2},
     {256, 1, 2, 2},

@@ -108,9 +108,10 @@ __device__ __forceinline__ bool cornerOffsets(const Feat& f, int px, int py, int
     return a && b;
 }
 
-// depthResponseFromCorners(d) <= thr.  The kernel keeps the vector units as busy as the vector L1 (170
-// instructions a pixel, tree and level before), and two correctly rounded double divisions are a third of a
-// depth split's (with the 24-bit offsets: 64 frames of 640x480, 10 trees of depth 18, 15.14 -> 14.45 ms).  The means in mm are first formed in float:
+// depthResponseFromCorners(d) <= thr.  The kernel kept the vector units as busy as the vector L1 (170
+// instructions a pixel, tree and level; now 142, the units 85% busy beside one lookup a cycle), and two correctly
+// rounded double divisions are a third of a depth split's (with the 24-bit offsets: 64 frames of 640x480, 10 trees of
+// depth 18, 15.14 -> 14.45 ms).  The means in mm are first formed in float:
 // relative error below 2^-21 each (the sums rounded to float, a reciprocal of 1 ulp, a product), so a
 // difference that clears the threshold by 2^-20 of the operands' sizes decides as the double one does.  Else
 // (and where a count is zero or anything is not finite: the comparison with NaN fails) the exact form.

@@ -547,7 +547,8 @@ __global__ void __launch_bounds__(256) k_responses_paired(const DevImage* __rest
 }
 
 // Chunks of at least 256 samples (one per lane) and at most 4096 (over which the zeroing and flushing of a
-// workgroup's histograms no longer shows), of a size that gives about 2048 workgroups: 8 per CU.
+// workgroup's histograms no longer shows), of a size that in between
+// gives 2048 to 4096 workgroups: 8 to 16 per CU.
 int evalChunkSamples(size_t samples, int F) {
     const size_t tiles = (static_cast<size_t>(F) + kEvalTile - 1) / kEvalTile;
     int c = 256;

@@ -633,8 +633,8 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             }
         };
         auto evalTwoPass = [&]() {
-            // (image, tree) segments of the sorted order -> blocks of <= kBinBlockSamples samples within a segment;
-            // the segments of one image form a group of consecutive blocks
+            // (image, tree) segments of the sorted order -> blocks of at most the launch shape's samples within a
+            // segment; the segments of one image form a group of consecutive blocks
             int* starts = reinterpret_cast<int*>(ws.hostStarts.get());
             timer.flush();
             if (starts[numKeys] < 0) starts[numKeys] = M;   // the end of the last segment
@@ -643,7 +643,8 @@ void trainTrees(cf_ctx* ctx, cf_images* images, const cf_train_config& cfg, int 
             // segment starts for each block size the tuner asks for; the work list of a batch of ngb feature
             // groups is then built on the device: each XCD takes an eighth of it in order, all feature groups of an
             // image group (feature group major, then tree, then block) before the next image group, so the trees'
-            // workgroups of one feature group read the same planes of one image from the XCD's L2; workgroup w runs on XCD w % 8, so the lists are interleaved
+            // workgroups of one feature group read the same planes of one image from the XCD's L2; workgroup w runs on
+            // XCD w % 8, so the lists are interleaved
             for (auto& kv : blockSets) kv.second.level = -1;
             auto blocksFor = [&](int blockSamples) -> BlockSet& {
                 BlockSet& bs = blockSets[blockSamples];

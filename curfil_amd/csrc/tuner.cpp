@@ -33,11 +33,10 @@ namespace cf {
 
 namespace {
 
-// Ratios per shape.  Timing the shapes in turn, without the default between them, chose shape 1 or 8 on
-// the 800-frame workload (17.57 and 17.50 s per step) where shape 7 pinned took 17.41 s: the launch order
-// and the levels' differences decided more than the shapes did.  With ratios, 3 rounds chose shape 3 in
-// three runs out of three (17.48 s per step); 6 rounds, which reach further down the tree, chose shape 7
-// in two runs out of two (17.44 s).
+// Ratios per shape.  Timing the shapes in turn, without the default between them, chose shapes of 17.57 and
+// 17.50 s per step of 800 frames where another of the list of that time, pinned, took 17.41 s: the launch order and
+// the levels' differences decided more than the shapes did.  With ratios, 3 rounds chose a shape of 17.48 s in three
+// runs out of three; 6 rounds, which reach further down the tree, the one of 17.44 s in two runs out of two.
 constexpr int kRounds = 6;
 // CURFIL_TUNE_ROUNDS=r overrides the ratios per shape (tests on small workloads, which have few launches)
 int tuneRounds() {
